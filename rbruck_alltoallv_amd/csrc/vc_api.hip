@@ -47,7 +47,8 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_header, sizeof(int64_t) * VC_HEADER_WORDS(VC_MAX_LAUNCHES), hipHostMallocCoherent);
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_header_dev, c->h_header, 0);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_launches, sizeof(VcLaunchInfo) * VC_MAX_LAUNCHES, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, 2 * sizeof(int), hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, VC_FLAG_WORDS * sizeof(int), hipHostMallocCoherent);
+    if (e == hipSuccess) memset(c->h_flags, 0, VC_FLAG_WORDS * sizeof(int));
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_flags_dev, c->h_flags, 0);
     if (e != hipSuccess) {
         (void)vc_comm_free(c);

@@ -168,6 +168,8 @@ hipError_t vc_launch_hop_bytes(const int *sc, int esz, int P, int n, const int *
                                hipStream_t st);
 hipError_t vc_launch_uniform_tables(int *counts, int *displs, int count, int P, hipStream_t st);
 hipError_t vc_launch_empty(hipStream_t st);
+// stores `value` to `word` (host memory) once everything enqueued on the stream before has ended
+hipError_t vc_launch_done(unsigned *word, unsigned value, hipStream_t st);
 
 // vc_plan.hip
 // header layout (int64), nl = number of launches:

@@ -113,7 +113,10 @@ struct vc_comm {
     const void *last_stage = nullptr;     // staging arena of the last call
     int64_t *h_header = nullptr;          // pinned, coherent: the planner writes its header straight into it
     int64_t *h_header_dev = nullptr;      // the same memory as the device sees it
-    int *h_flags = nullptr, *h_flags_dev = nullptr;   // pinned, coherent: the two flags of vc_displs_from_counts, as host and device see them
+    int *h_flags = nullptr, *h_flags_dev = nullptr;   // pinned, coherent: the two flags of vc_displs_from_counts, as host and device see
+                                          // them; in a cache line of its own behind them (VC_DONE_AT) the word vc_wait_stream waits for
+    unsigned done_value = 0;              // the value last enqueued for that word
+    std::mutex done_mutex;                // values go into the stream in order, also from several threads
     VcLaunchInfo *h_launches = nullptr;   // pinned
     std::vector<hipEvent_t> events;
     vc_stats_t stats;
@@ -150,8 +153,33 @@ struct BusyGuard {
     bool ok() const { return !c || mine; }
     void keep() { mine = false; }         // the call stays in progress after the entry point returns (vc_comm_wait ends it)
 };
+#define VC_DONE_AT 32
+#define VC_FLAG_WORDS 64
+#define VC_SPIN_US 10000
+
+// Waits for everything enqueued on the communicator's stream (see vc_done_kernel).  A call that takes longer than
+// VC_SPIN_US is waited for by the runtime (4 us are nothing then, and it reports what went wrong), as is a call with
+// per-launch timing on, whose events end behind its last kernel.
+inline hipError_t vc_wait_stream(vc_comm *c) {
+    if (c->timing) return hipStreamSynchronize(c->stream);
+    unsigned value;
+    {
+        std::lock_guard<std::mutex> lock(c->done_mutex);
+        value = ++c->done_value;
+        const hipError_t e = vc_launch_done(reinterpret_cast<unsigned *>(c->h_flags_dev) + VC_DONE_AT, value, c->stream);
+        if (e != hipSuccess) return e;
+    }
+    const unsigned *word = reinterpret_cast<const unsigned *>(c->h_flags) + VC_DONE_AT;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (unsigned spin = 1;; spin++) {
+        if ((int)(__atomic_load_n(word, __ATOMIC_ACQUIRE) - value) >= 0) return hipSuccess;
+        __builtin_ia32_pause();
+        if (spin % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(VC_SPIN_US)) return hipStreamSynchronize(c->stream);
+    }
+}
+
 // the host waits for the communicator's stream (counted: vc_stats_t.host_waits)
-#define VC_WAIT(c) ((c)->waits++, hipStreamSynchronize((c)->stream))
+#define VC_WAIT(c) ((c)->waits++, vc_wait_stream(c))
 
 #define VC_ONE_CALL(c)                                                                                              \
     BusyGuard busy_guard_(c);                                                                                       \

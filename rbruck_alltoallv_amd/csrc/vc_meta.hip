@@ -249,3 +249,16 @@ hipError_t vc_launch_empty(hipStream_t st) {
     hipLaunchKernelGGL(vc_empty_kernel, dim3(1), dim3(VC_WAVE), 0, st);
     return hipGetLastError();
 }
+
+// The last kernel of a blocking call: the kernels before it on the stream have ended, their stores released, when it runs.
+// Waiting for its word in pinned host memory takes the host 4 us less than hipStreamSynchronize, which enqueues a barrier
+// packet with a completion signal of its own behind the last kernel: a 5 us kernel launched and waited for 17.2 -> 13.2 us,
+// three of them 30.6 -> 26.5 (a kernel launched with a stop event gained 1 - 2 us alone and lost as much behind another).
+__global__ void vc_done_kernel(unsigned *word, unsigned value) {
+    if (threadIdx.x == 0) __hip_atomic_store(word, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t vc_launch_done(unsigned *word, unsigned value, hipStream_t st) {
+    hipLaunchKernelGGL(vc_done_kernel, dim3(1), dim3(VC_WAVE), 0, st, word, value);
+    return hipGetLastError();
+}

@@ -7,7 +7,7 @@
 extern "C" int vc_alltoall_counts(const int *sendcounts, int *recvcounts, vc_comm_t c) {
     if (!c || !sendcounts || !recvcounts) return fail_arg("vc_alltoall_counts: null argument");
     HIP_TRY(vc_launch_transpose(sendcounts, recvcounts, c->P, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(vc_wait_stream(c));
     return VC_OK;
 }
 
@@ -17,7 +17,7 @@ extern "C" int vc_displs_from_counts(const int *counts, int *displs, int64_t *ex
     // the kernel raises the two flags in pinned host memory: no clearing launch before it, no copy back after it
     c->h_flags[0] = c->h_flags[1] = 0;
     HIP_TRY(vc_launch_row_scan(counts, displs, extent_out, c->h_flags_dev, c->P, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(vc_wait_stream(c));
     if (c->h_flags[1]) return fail_arg("vc_displs_from_counts: negative count", VC_ERR_TABLES);
     if (c->h_flags[0]) return fail_arg("vc_displs_from_counts: a rank's counts sum past INT_MAX elements", VC_ERR_OVERFLOW);
     return VC_OK;
@@ -27,14 +27,14 @@ extern "C" int vc_bases_from_extents(const int64_t *extent, int elem_size, int64
                                      vc_comm_t c) {
     if (!c || !extent || !base_out || elem_size < 1 || align < 1) return fail_arg("vc_bases_from_extents: bad argument");
     HIP_TRY(vc_launch_bases(extent, elem_size, align, base_out, total_out, c->P, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(vc_wait_stream(c));
     return VC_OK;
 }
 
 extern "C" int vc_allreduce_max_count(const int *sendcounts, int *max_out, vc_comm_t c) {
     if (!c || !sendcounts || !max_out) return fail_arg("vc_allreduce_max_count: null argument");
     HIP_TRY(vc_launch_max(sendcounts, max_out, (int64_t)c->P * c->P, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(vc_wait_stream(c));
     return VC_OK;
 }
 

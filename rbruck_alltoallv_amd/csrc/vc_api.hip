@@ -64,7 +64,7 @@ extern "C" int vc_comm_free(vc_comm_t c) {
     (void)hipStreamSynchronize(c->stream);
     c->pending.active = false;
     for (DevBuf *b : {&c->slot_off, &c->row_tot, &c->row_base, &c->org_run_base, &c->item_row_tot, &c->item_row_base, &c->row_bytes, &c->desc, &c->header, &c->launches, &c->stage, &c->rd_packed,
-                      &c->uni_counts, &c->uni_displs, &c->scratch, &c->chain_row_tot, &c->chain_row_base, &c->strided_headers})
+                      &c->scratch, &c->max_state, &c->chain_row_tot, &c->chain_row_base, &c->strided_headers})
         b->release();
     free_retired_stage(c);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
@@ -893,19 +893,14 @@ static int run_uniform(VcFunc f, int n, int r, vc_comm *c, char *sendbuf, int se
     rc = make_schedule(c, q, forward, S, L);              // (validates the tunables before anything is enqueued)
     if (rc) return schedule_error(rc);
     S.recv_lo = (int)((uintptr_t)recvbuf & 4095);
-    const size_t PP = (size_t)c->P * c->P;
-    HIP_TRY(c->uni_counts.reserve(sizeof(int) * PP));
-    HIP_TRY(c->uni_displs.reserve(sizeof(int) * PP));
-    hipStream_t const own = c->stream;
-    if (async_stream) c->stream = static_cast<hipStream_t>(*async_stream);
-    const int *cnt = c->uni_counts.as<int>(), *dsp = c->uni_displs.as<int>();
-    hipError_t e = vc_launch_uniform_tables(c->uni_counts.as<int>(), c->uni_displs.as<int>(), sendcount, c->P, c->stream);
-    if (e != hipSuccess) { c->stream = own; return fail_hip(e, "vc_launch_uniform_tables", __LINE__); }
-    if (!async_stream) return run_schedule(c, q, sendbuf, recvbuf, make_tables(c, cnt, dsp, cnt, dsp), forward);
-    c->pending.own_stream = own;
-    rc = enqueue_async(c, q, S, L, sendbuf, recvbuf, make_tables(c, cnt, dsp, cnt, dsp));
+    const int *const any = reinterpret_cast<const int *>(c->sbase);      // (VcSched::table_mask: what is read there does not count)
+    const VcTables T = make_tables(c, any, any, any, any);
+    if (!async_stream) return run_schedule(c, q, sendbuf, recvbuf, T, forward);
+    c->pending.own_stream = c->stream;
+    c->stream = static_cast<hipStream_t>(*async_stream);
+    rc = enqueue_async(c, q, S, L, sendbuf, recvbuf, T);
     if (rc == VC_OK) busy_guard_.keep();
-    else c->stream = own;
+    else c->stream = c->pending.own_stream;
     return rc;
 }
 
@@ -1006,14 +1001,8 @@ extern "C" int vc_plan_create(const char *function, int n, int r, int batch, int
         rc = make_schedule(c, q, forward, S, L);          // validates the tunables before anything is allocated
         if (rc) return schedule_error(rc);
     }
-    if (uniform) {
-        const size_t PP = (size_t)c->P * c->P;
-        HIP_TRY(c->uni_counts.reserve(sizeof(int) * PP));
-        HIP_TRY(c->uni_displs.reserve(sizeof(int) * PP));
-        HIP_TRY(vc_launch_uniform_tables(c->uni_counts.as<int>(), c->uni_displs.as<int>(), batch, c->P, c->stream));
-        sendcounts = recvcounts = c->uni_counts.as<int>();
-        sdispls = rdispls = c->uni_displs.as<int>();
-    }
+    // (VcSched::table_mask: what is read there does not count)
+    if (uniform) sendcounts = sdispls = recvcounts = rdispls = reinterpret_cast<int *>(const_cast<int64_t *>(c->sbase));
     vc_plan *p = new vc_plan();
     p->comm = c;
     rc = build_plan(c, q, recvbuf_low_bits & 4095, make_tables(c, sendcounts, sdispls, recvcounts, rdispls), p->items, p->info, forward);

@@ -82,7 +82,10 @@ struct VcSched {
     int msd;          // 1: most significant digit first (twophase_rbruck_alltoallv, uniform intra phase)
     int esz;          // element size in bytes
     int packed_recv;  // 1: receive side is the packed source-ordered layout (TTPL_BT_alltoallv ignores rdispls)
-    int uniform;      // >0: equal blocks of this many elements, tables are implied (uniform_* functions)
+    int uniform;      // uniform_* functions: elements per block; else 0
+    int table_mask;   // -1; 0 in the uniform_* functions: equal blocks in rank order, there are no tables, and what is read in their
+                      // place (anything readable) is masked out (vc_sc; a branch around the reads would split the batch of
+                      // reads a block's addresses depend on: +10 us on 1 Mi blocks)
     int recv_lo;      // low 12 bits of the recvbuf pointer: staging slots copy the final destination's cache-line phase,
                       // long copies into recvbuf are cut at its 4 KiB boundaries
     int last_hop;     // which blocks make a hop that is no digit round and ends in recvbuf, besides every rank's block to
@@ -157,7 +160,8 @@ hipError_t vc_launch_transpose(const int *in, int *out, int P, hipStream_t st);
 // flags (device, 2 ints the caller has zeroed, or null): [0] set when a row's total passes INT_MAX, [1] when a count is negative
 hipError_t vc_launch_row_scan(const int *counts, int *displs, int64_t *extent, int *flags, int P, hipStream_t st);
 hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_t *base, int64_t *total, int P, hipStream_t st);
-hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, hipStream_t st);
+// state: 65 words, the first one zero before and after
+hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, int *state, hipStream_t st);
 hipError_t vc_launch_fill_payload(int mode, uint64_t seed, char *sendbuf, const int *sc, const int *sd, const int64_t *sbase,
                                   int esz, int P, hipStream_t st);
 hipError_t vc_launch_verify(const char *sendbuf, const char *recvbuf, VcTables t, int esz, int P, int packed,
@@ -166,7 +170,6 @@ hipError_t vc_launch_verify(const char *sendbuf, const char *recvbuf, VcTables t
 // items per candidate, the work items of the payload
 hipError_t vc_launch_hop_bytes(const int *sc, int esz, int P, int n, const int *cand_dev, int ncand, unsigned long long *moved_dev,
                                hipStream_t st);
-hipError_t vc_launch_uniform_tables(int *counts, int *displs, int count, int P, hipStream_t st);
 hipError_t vc_launch_empty(hipStream_t st);
 // stores `value` to `word` (host memory) once everything enqueued on the stream before has ended
 hipError_t vc_launch_done(unsigned *word, unsigned value, hipStream_t st);

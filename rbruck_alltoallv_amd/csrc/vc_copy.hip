@@ -268,8 +268,7 @@ __device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &
         const int64_t idx = wave * per_wave + u * VC_WAVE + lane;
         if (idx >= pairs) continue;
         const int to = vc_div((int)idx, S.dP), s = (int)idx - to * P;      // (idx < P^2 <= 2^30)
-        const int64_t i = (int64_t)to * P + s, k = (int64_t)s * P + to;
-        const int sc = T.sc[k], rc = T.rc[i];
+        const int sc = vc_sc(S, T, s, to), rc = vc_rc(S, T, to, s);
         const int64_t len = (int64_t)sc * S.esz;
         const int64_t cnt = sc > 0 ? vc_chain_count(S, T, s, to) : 0;
         payload += (int64_t)rc * S.esz;                   // (what the receivers expect, as the planner counts it)
@@ -345,10 +344,9 @@ __host__ __device__ __forceinline__ unsigned vc_totals_blocks(const VcSched &S, 
 // Whether the pair's own table entries allow its block to be moved: none negative, the receiver expecting what the
 // source sends, the block no longer than a slot and cut into no more pieces than the kernel was chosen for.
 __device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcTables &T, const VcListlessGuard &g, int s, int t) {
-    const int64_t i = (int64_t)t * S.P + s, k = (int64_t)s * S.P + t;
-    const int sc = T.sc[k];
-    if (sc < 0 || T.rc[i] != sc || T.sd[k] < 0 || (S.packed_recv ? T.rd_packed[i] < 0 : T.rd[i] < 0)) return false;
-    if (S.packed_recv && (int64_t)T.rd_packed[i] + sc > 0x7FFFFFFF) return false;
+    const int sc = vc_sc(S, T, s, t), rd = vc_rd(S, T, t, s);
+    if (sc < 0 || vc_rc(S, T, t, s) != sc || vc_sd(S, T, s, t) < 0 || rd < 0) return false;
+    if (S.packed_recv && (int64_t)rd + sc > 0x7FFFFFFF) return false;
     const int64_t len = (int64_t)sc * S.esz;
     if (g.max_len && len > g.max_len) return false;
     return !(g.max_pieces && sc > 0 && vc_chain_count(S, T, s, t) > g.max_pieces);
@@ -383,7 +381,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
     // Everything the block's addresses depend on is loaded before the planner's verdict is looked at: the loads are
     // independent of each other and of the verdict (tables are always readable), so they travel together instead of one
     // memory round trip after the other; nothing is stored before the verdict is known.
-    const int64_t len = (int64_t)T.sc[(int64_t)s * S.P + t] * S.esz;
+    const int64_t len = (int64_t)vc_sc(S, T, s, t) * S.esz;
     const int64_t send_off = vc_send_offset(S, T, s, t);
     const int64_t recv_off = vc_recv_offset(S, T, s, t);
     int64_t dst = 0;
@@ -435,7 +433,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
     const bool inside = idx < (int64_t)S.P * S.P;
     const int t = inside ? vc_div((int)idx, S.dP) : 0, s = inside ? (int)idx - t * S.P : 0;       // (idx < P^2 <= 2^30)
     // all loads the addresses depend on go out before the planner's verdict is looked at (see vc_copy_blocks_kernel)
-    const int64_t len = inside ? (int64_t)T.sc[(int64_t)s * S.P + t] * S.esz : 0;
+    const int64_t len = inside ? (int64_t)vc_sc(S, T, s, t) * S.esz : 0;
     const int64_t send_off = vc_send_offset(S, T, s, t);
     const int64_t recv_off = vc_recv_offset(S, T, s, t);
     // no lane leaves before the barrier below
@@ -493,7 +491,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
     const bool inside = idx < (int64_t)S.P * S.P;
     const int t = inside ? vc_div((int)idx, S.dP) : 0, s = inside ? (int)idx - t * S.P : 0;       // (idx < P^2 <= 2^30)
     // all loads the addresses depend on go out before the planner's verdict is looked at (see vc_copy_blocks_kernel)
-    const int64_t len = inside ? (int64_t)T.sc[(int64_t)s * S.P + t] * S.esz : 0;
+    const int64_t len = inside ? (int64_t)vc_sc(S, T, s, t) * S.esz : 0;
     const int64_t send_off = vc_send_offset(S, T, s, t);
     const int64_t recv_off = vc_recv_offset(S, T, s, t);
     const bool active = len > 0;

@@ -89,7 +89,7 @@ struct vc_comm {
     bool strided_clean = false;           // ... and the one the next call will use is known to be zero
     int strided_turn = 0;
     DevBuf slot_off, row_tot, row_base, org_run_base, item_row_tot, item_row_base, row_bytes, desc, header, launches, stage, rd_packed,
-        uni_counts, uni_displs, scratch;
+        scratch, max_state;
     double cal_copy_bytes_per_s = 0, cal_launch_s = 0, cal_sync_s = 0;   // calibrate(): the plain copy's rate, the cost of a
                                           // launch, of a launch the host waits for
     int bound_staging = 1;                // vc_comm_set_staging_bound

@@ -89,39 +89,47 @@ hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_
 // ---------------------------------------------------------------------------
 // MPI_Allreduce(MAX) of the block length (src/twophase_tunable_rbruckv.cpp:40-44).
 // ---------------------------------------------------------------------------
-// One atomic per workgroup (the wavefronts' maxima meet in LDS first): 256 atomics on the one word instead of one per
-// wavefront, which is what the call waited for at 1024 ranks.
-__global__ __launch_bounds__(VC_THREADS) void vc_max_kernel(const int *__restrict__ counts, int *__restrict__ out, int64_t n) {
-    __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
+// One launch: every workgroup leaves its maximum in state[1 + workgroup] and counts itself in state[0]; the last one takes
+// the maximum of these and leaves the count at zero for the next call.  A clearing kernel in front of a maximum by atomics was
+// one more launch, 4 us of a call of 18.  Atomics of many workgroups on one word go one after the other (256 of them twice: 4 us),
+// so the workgroups are few and large.
+#define VC_MAX_WORKGROUPS 64
+#define VC_MAX_LANES 1024
+__global__ __launch_bounds__(VC_MAX_LANES) void vc_max_kernel(const int *__restrict__ counts, int *__restrict__ out, int64_t n, int *state) {
+    __shared__ int wave_max[VC_MAX_LANES / VC_WAVE];
+    const int lane = threadIdx.x % VC_WAVE, wave = threadIdx.x / VC_WAVE;
     int m = INT_MIN;
-    for (int64_t i = (int64_t)blockIdx.x * VC_THREADS + threadIdx.x; i < n; i += (int64_t)gridDim.x * VC_THREADS) m = max(m, counts[i]);
-    const int64_t all = vc_block_max(m, lds);
-    if (threadIdx.x == 0) atomicMax(out, (int)all);
-}
-
-__global__ void vc_lowest_int_kernel(int *p) { *p = INT_MIN; }
-
-hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, hipStream_t st) {
-    hipLaunchKernelGGL(vc_lowest_int_kernel, dim3(1), dim3(1), 0, st, out);
-    int64_t blocks = (nelem + 4 * VC_THREADS - 1) / (4 * VC_THREADS);
-    if (blocks > 256) blocks = 256;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(vc_max_kernel, dim3((unsigned)blocks), dim3(VC_THREADS), 0, st, counts, out, nelem);
-    return hipGetLastError();
-}
-
-// Equal-block tables implied by the uniform_* functions: counts = count, displs[p][i] = i*count.
-__global__ void vc_uniform_tables_kernel(int *counts, int *displs, int count, int P) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < (int64_t)P * P) {
-        counts[i] = count;
-        displs[i] = (int)(i % P) * count;
+#pragma unroll 8
+    for (int64_t i = (int64_t)blockIdx.x * VC_MAX_LANES + threadIdx.x; i < n; i += (int64_t)gridDim.x * VC_MAX_LANES) m = max(m, counts[i]);
+#pragma unroll
+    for (int o = VC_WAVE / 2; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, VC_WAVE));
+    if (lane == 0) wave_max[wave] = m;
+    __syncthreads();
+    if (wave != 0) return;
+    m = lane < VC_MAX_LANES / VC_WAVE ? wave_max[lane] : INT_MIN;
+#pragma unroll
+    for (int o = VC_MAX_LANES / VC_WAVE / 2; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, VC_WAVE));
+    int last = 0;
+    if (lane == 0) {
+        __hip_atomic_store(&state[1 + blockIdx.x], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the store has been performed where the others will look
+        last = __hip_atomic_fetch_add(&state[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    }
+    if (!__shfl(last, 0, VC_WAVE)) return;
+    m = lane < (int)gridDim.x ? __hip_atomic_load(&state[1 + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : INT_MIN;
+#pragma unroll
+    for (int o = VC_WAVE / 2; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, VC_WAVE));
+    if (lane == 0) {
+        *out = m;
+        __hip_atomic_store(&state[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
-hipError_t vc_launch_uniform_tables(int *counts, int *displs, int count, int P, hipStream_t st) {
-    int64_t nb = ((int64_t)P * P + VC_THREADS - 1) / VC_THREADS;
-    hipLaunchKernelGGL(vc_uniform_tables_kernel, dim3((unsigned)nb), dim3(VC_THREADS), 0, st, counts, displs, count, P);
+hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, int *state, hipStream_t st) {
+    int64_t blocks = (nelem + 4 * VC_MAX_LANES - 1) / (4 * VC_MAX_LANES);
+    if (blocks > VC_MAX_WORKGROUPS) blocks = VC_MAX_WORKGROUPS;
+    if (blocks < 1) blocks = 1;
+    hipLaunchKernelGGL(vc_max_kernel, dim3((unsigned)blocks), dim3(VC_MAX_LANES), 0, st, counts, out, nelem, state);
     return hipGetLastError();
 }
 

@@ -106,7 +106,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_rows(VcSched S, VcLaunchPa
                 cnt[u] = 0;
                 if (chunk0 + u >= nchunk || s >= P) continue;
                 cnt[u] = vc_chain_count(S, T, s, to);
-                const int expected = T.rc[(int64_t)to * P + s], sent = T.sc[(int64_t)s * P + to];
+                const int expected = vc_rc(S, T, to, s), sent = vc_sc(S, T, s, to);
                 bad += vc_pair_bad_entries(S, T, s, to);
                 payload += (int64_t)expected * S.esz;
                 most = cnt[u] > most ? cnt[u] : most;
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_rows(VcSched S, VcLaunchPa
     }
     if (L == 0 && !forward)                               // forwarded execution has done this above
         for (int id = threadIdx.x; id < P; id += VC_THREADS) {
-            payload += (int64_t)T.rc[(int64_t)to * P + id] * S.esz;
+            payload += (int64_t)vc_rc(S, T, to, id) * S.esz;
             bad += vc_pair_bad_entries(S, T, id, to);
         }
     items = vc_block_sum(items, lds);
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
         }
         const int nhop = __popc(moves);
         if (!big) {
-            const int64_t src = VC_SPACE_SEND | vc_send_offset(S, T, s, t), len = (int64_t)T.sc[(int64_t)s * P + t] * S.esz;
+            const int64_t src = VC_SPACE_SEND | vc_send_offset(S, T, s, t), len = (int64_t)vc_sc(S, T, s, t) * S.esz;
             const int phase = vc_phase(S, T, s, t), cut = vc_chain_cut(S, T, s, t);
             for (int64_t c = 0; c < cnt; c++) {
                 int64_t lo, hi;
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
             const int64_t c = q - big_pre[lo];
             const int sb = s_lo + lo;
             if (cached)
-                vc_chain_piece(VC_SPACE_SEND | vc_send_offset(S, T, sb, t), (int64_t)T.sc[(int64_t)sb * P + t] * S.esz, vc_phase(S, T, sb, t),
+                vc_chain_piece(VC_SPACE_SEND | vc_send_offset(S, T, sb, t), (int64_t)vc_sc(S, T, sb, t) * S.esz, vc_phase(S, T, sb, t),
                                vc_chain_cut(S, T, sb, t), c, big_dst[lo], big_nhop[lo], items + (big_at[lo] + c) * stride);
             else
                 vc_chain_item(S, T, slot_off, row_base, sb, t, c, items + (big_at[lo] + c) * stride);

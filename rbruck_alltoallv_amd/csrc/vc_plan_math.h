@@ -123,9 +123,17 @@ VC_HD bool vc_inter_block(const VcSched &S, int x, int dist, int to, int id, VcE
     return true;
 }
 
+// Entries of the tables: what rank s sends to rank t, what rank t expects from rank s, and where, in elements.  (Ranks are
+// at most 32768: an index fits 30 bits.)
+VC_HD int vc_sc(const VcSched &S, const VcTables &T, int s, int t) { return (T.sc[(unsigned)((s * S.P + t) & S.table_mask)] & S.table_mask) + S.uniform; }
+VC_HD int vc_sd(const VcSched &S, const VcTables &T, int s, int t) { return (T.sd[(unsigned)((s * S.P + t) & S.table_mask)] & S.table_mask) + t * S.uniform; }
+VC_HD int vc_rc(const VcSched &S, const VcTables &T, int t, int s) { return (T.rc[(unsigned)((t * S.P + s) & S.table_mask)] & S.table_mask) + S.uniform; }
+VC_HD int vc_rd(const VcSched &S, const VcTables &T, int t, int s) {
+    return ((S.packed_recv ? T.rd_packed : T.rd)[(unsigned)((t * S.P + s) & S.table_mask)] & S.table_mask) + s * S.uniform;
+}
+
 VC_HD int64_t vc_recv_offset(const VcSched &S, const VcTables &T, int s, int t) {
-    const int *rd = S.packed_recv ? T.rd_packed : T.rd;
-    return T.rbase[t] + (int64_t)rd[(int64_t)t * S.P + s] * S.esz;
+    return T.rbase[t] + (int64_t)vc_rd(S, T, t, s) * S.esz;
 }
 
 // Staging slots start cache-line (VC_LINE) aligned; the data inside starts at the line phase
@@ -145,7 +153,7 @@ VC_HD int64_t vc_stage_slot_size(const VcSched &S, const VcTables &T, int x, int
     if (data_len) *data_len = 0;
     if (!vc_intra_block(S, x, dist, to, id, b) || !b.to_stage || b.to_org) return 0;
     if (st) { st[0] = b.s; st[1] = b.t; }
-    const int64_t len = (int64_t)T.sc[(int64_t)b.s * S.P + b.t] * S.esz;
+    const int64_t len = (int64_t)vc_sc(S, T, b.s, b.t) * S.esz;
     if (data_len) *data_len = len;
     return len ? ((len + vc_phase(S, T, b.s, b.t) + VC_LINE - 1) & ~(int64_t)(VC_LINE - 1)) : 0;
 }
@@ -164,7 +172,7 @@ VC_HD int64_t vc_region_slot_size(const VcSched &S, const VcTables &T, int y, in
     if (data_len) *data_len = 0;
     if (!vc_inter_block(S, y - S.w, dist, to, id, e, z) || e.xdst < 0) return 0;
     if (st) { st[0] = e.s; st[1] = e.t; }
-    const int64_t len = (int64_t)T.sc[(int64_t)e.s * S.P + e.t] * S.esz;
+    const int64_t len = (int64_t)vc_sc(S, T, e.s, e.t) * S.esz;
     if (data_len) *data_len = len;
     return len ? ((len + vc_phase(S, T, e.s, e.t) + VC_LINE - 1) & ~(int64_t)(VC_LINE - 1)) : 0;
 }
@@ -211,7 +219,7 @@ VC_HD int vc_block_hops(const VcSched &S, int s, int t) {
 }
 
 VC_HD int64_t vc_send_offset(const VcSched &S, const VcTables &T, int s, int t) {
-    return T.sbase[s] + (int64_t)T.sd[(int64_t)s * S.P + t] * S.esz;
+    return T.sbase[s] + (int64_t)vc_sd(S, T, s, t) * S.esz;
 }
 
 // ---- organized region (S.coalesce) ----
@@ -321,7 +329,7 @@ VC_HD bool vc_entry_block(const VcSched &S, const VcLaunchInfo &info, int to, in
 }
 
 VC_HD int64_t vc_entry_len(const VcSched &S, const VcTables &T, const VcEntry &e) {
-    if (e.nblk == 1) return (int64_t)T.sc[(int64_t)e.s * S.P + e.t] * S.esz;
+    if (e.nblk == 1) return (int64_t)vc_sc(S, T, e.s, e.t) * S.esz;
     const int gs = vc_div(e.s, S.dn), m0 = e.s - gs * S.n;
     return vc_org_run_prefix(S, T, gs, e.t, m0 + e.nblk) - vc_org_run_prefix(S, T, gs, e.t, m0);
 }
@@ -408,7 +416,7 @@ VC_HD int vc_chain_cut(const VcSched &S, const VcTables &T, int s, int t) {
 }
 
 VC_HD int64_t vc_chain_count(const VcSched &S, const VcTables &T, int s, int t) {
-    const int64_t len = (int64_t)T.sc[(int64_t)s * S.P + t] * S.esz;
+    const int64_t len = (int64_t)vc_sc(S, T, s, t) * S.esz;
     return vc_chunk_count(len, vc_phase(S, T, s, t), vc_chain_cut(S, T, s, t));
 }
 
@@ -417,9 +425,9 @@ VC_HD int64_t vc_chain_count(const VcSched &S, const VcTables &T, int s, int t) 
 // of the receiver's own row may be negative.  Summed over all pairs this is header word VC_HEADER_BAD, whoever adds it
 // up (the planner's row kernel, or the copy kernel that plans nothing).
 VC_HD int vc_pair_bad_entries(const VcSched &S, const VcTables &T, int s, int t) {
-    const int64_t i = (int64_t)t * S.P + s;
-    const int expected = T.rc[i], sent = T.sc[(int64_t)s * S.P + t];
-    return (expected != sent) + (int)((T.sc[i] < 0) | (T.sd[i] < 0) | (expected < 0) | (!S.packed_recv && T.rd[i] < 0));
+    const int expected = vc_rc(S, T, t, s), sent = vc_sc(S, T, s, t);
+    const int rd = S.packed_recv ? 0 : vc_rd(S, T, t, s);
+    return (expected != sent) + ((vc_sc(S, T, t, s) | vc_sd(S, T, t, s) | expected | rd) < 0);
 }
 
 // Layout of a chain item, in int64 words; `stride` = VC_CHAIN_HEAD + hop slots of the call.
@@ -593,7 +601,7 @@ VC_HD int vc_chain_route(const VcSched &S, const VcTables &T, const int64_t *slo
 // Writes piece c of block (s, t) to `item`.
 VC_HD void vc_chain_item(const VcSched &S, const VcTables &T, const int64_t *slot_off, const int64_t *row_base, int s, int t, int64_t c,
                          int64_t *item) {
-    const int64_t len = (int64_t)T.sc[(int64_t)s * S.P + t] * S.esz;
+    const int64_t len = (int64_t)vc_sc(S, T, s, t) * S.esz;
     const int nhop = vc_chain_route(S, T, slot_off, row_base, s, t, item + VC_CHAIN_HEAD);   // whole-block destinations first
     vc_chain_piece(VC_SPACE_SEND | vc_send_offset(S, T, s, t), len, vc_phase(S, T, s, t), vc_chain_cut(S, T, s, t), c,
                    item + VC_CHAIN_HEAD, nhop, item);

@@ -118,7 +118,7 @@ inline int vc_make_schedule(VcFunc f, int P, int n, int r, int batch, int esz, i
                             std::vector<VcLaunchInfo> &L, int batch2 = 0, bool forward = false) {
     memset(&S, 0, sizeof S);
     L.clear();
-    S.P = P; S.esz = esz; S.uniform = uniform_count;
+    S.P = P; S.esz = esz; S.uniform = uniform_count; S.table_mask = -1;
     if (forward) batch = batch2 = 0;                        // one kernel performs every hop: batches of rounds mean nothing
 
     int d = 0;
@@ -189,6 +189,7 @@ inline int vc_make_schedule(VcFunc f, int P, int n, int r, int batch, int esz, i
         if (r < 2) r = 2;                                                // :143
         if (n < 2 || n >= P || P % n != 0) return VC_ERR_GROUP;          // :18-22, :145-149 MPI_Abort
         if (r > n) r = n;
+        S.table_mask = 0;
         S.n = n; S.G = P / n; S.r = r; S.msd = 1; S.last_hop = 1;   // intra-node phase is most significant digit first (:69)
         vc_radix_params(n, S.r, S.w, d);
         vc_add_intra_launches(L, S, d, 0);

@@ -33,7 +33,11 @@ extern "C" int vc_bases_from_extents(const int64_t *extent, int elem_size, int64
 
 extern "C" int vc_allreduce_max_count(const int *sendcounts, int *max_out, vc_comm_t c) {
     if (!c || !sendcounts || !max_out) return fail_arg("vc_allreduce_max_count: null argument");
-    HIP_TRY(vc_launch_max(sendcounts, max_out, (int64_t)c->P * c->P, c->stream));
+    if (!c->max_state.p) {
+        HIP_TRY(c->max_state.reserve(512));
+        HIP_TRY(hipMemsetAsync(c->max_state.p, 0, 512, c->stream));
+    }
+    HIP_TRY(vc_launch_max(sendcounts, max_out, (int64_t)c->P * c->P, c->max_state.as<int>(), c->stream));
     HIP_TRY(vc_wait_stream(c));
     return VC_OK;
 }

@@ -64,7 +64,7 @@ extern "C" int vc_comm_free(vc_comm_t c) {
     (void)hipStreamSynchronize(c->stream);
     c->pending.active = false;
     for (DevBuf *b : {&c->slot_off, &c->row_tot, &c->row_base, &c->org_run_base, &c->item_row_tot, &c->item_row_base, &c->row_bytes, &c->desc, &c->header, &c->launches, &c->stage, &c->rd_packed,
-                      &c->scratch, &c->max_state, &c->chain_row_tot, &c->chain_row_base, &c->strided_headers})
+                      &c->scratch, &c->max_state, &c->ticket, &c->chain_row_tot, &c->chain_row_base, &c->strided_headers})
         b->release();
     free_retired_stage(c);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
@@ -224,6 +224,10 @@ static int reserve_plan_bufs(vc_comm *c, const VcSched &S, int nl, bool forward)
     if (forward) {
         HIP_TRY(c->chain_row_tot.reserve(z.chain_row_tot));
         HIP_TRY(c->chain_row_base.reserve(z.chain_row_base));
+        if (!c->ticket.p) {
+            HIP_TRY(c->ticket.reserve(VC_TICKET_BYTES));
+            HIP_TRY(hipMemsetAsync(c->ticket.p, 0, VC_TICKET_BYTES, c->stream));
+        }
     }
     if (S.packed_recv) HIP_TRY(c->rd_packed.reserve(z.rd_packed));
     PlanBufs &B = c->B;
@@ -232,6 +236,7 @@ static int reserve_plan_bufs(vc_comm *c, const VcSched &S, int nl, bool forward)
     B.item_row_base = c->item_row_base.as<int64_t>(); B.row_bytes = c->row_bytes.as<int64_t>();
     B.chain_row_tot = forward ? c->chain_row_tot.as<int64_t>() : nullptr;
     B.chain_row_base = forward ? c->chain_row_base.as<int64_t>() : nullptr;
+    B.ticket = c->ticket.as<unsigned>();
     B.header = c->header.as<int64_t>(); B.launches = c->launches.as<VcLaunchInfo>(); B.rd_packed = c->rd_packed.as<int>();
     return VC_OK;
 }
@@ -252,9 +257,12 @@ static int enqueue_plan_sizes(vc_comm *c, const VcSched &S, std::vector<VcLaunch
         HIP_TRY(vc_launch_row_scan(T.rc, B.rd_packed, nullptr, nullptr, P, st));
         T.rd_packed = B.rd_packed;
     }
-    HIP_TRY(vc_launch_plan_sizes(S, L.data(), B.launches, nl, T, B.slot_off, B.row_tot, B.row_base, B.org_run_base, B.item_row_tot,
-                                 B.item_row_base, B.row_bytes, forward ? B.chain_row_tot : nullptr,
-                                 forward ? B.chain_row_base : nullptr, B.header, c->h_header_dev, st));
+    if (forward)
+        HIP_TRY(vc_launch_plan_forward(S, T, B.slot_lines(), B.row_tot, B.row_base, B.row_bytes, B.chain_row_tot, B.chain_row_base, B.header,
+                                       c->h_header_dev, B.ticket, st));
+    else
+        HIP_TRY(vc_launch_plan_sizes(S, L.data(), B.launches, nl, T, B.slot_off, B.row_tot, B.row_base, B.org_run_base, B.item_row_tot,
+                                     B.item_row_base, B.row_bytes, B.header, c->h_header_dev, st));
     return VC_OK;
 }
 
@@ -313,7 +321,7 @@ static int plan_emit(vc_comm *c, const VcSched &S, std::vector<VcLaunchInfo> &L,
     if (pi.chain) {
         if (!c->B.chain_row_base || !c->B.chain_row_tot) return fail_arg("internal: chain items asked for a plan that was not sized for them", VC_ERR_HIP);
         HIP_TRY(items.reserve(sizeof(int64_t) * (size_t)pi.chain_stride * (size_t)std::max<int64_t>(pi.chain_items, 1)));
-        HIP_TRY(vc_launch_chain_plan(S, T, c->B.slot_off, c->B.row_base, c->B.chain_row_tot + 2 * (size_t)S.P, items.as<int64_t>(),
+        HIP_TRY(vc_launch_chain_plan(S, T, c->B.slot_lines(), c->B.row_base, c->B.chain_row_base, c->B.chain_row_tot, items.as<int64_t>(),
                                      pi.chain_items, st));
     } else {
         HIP_TRY(items.reserve(sizeof(VcDesc) * (size_t)std::max<int64_t>(pi.items_total, 1)));
@@ -505,7 +513,7 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
     if (c->hint.items > 2 * c->items_before_last) return 2;
     hipStream_t st = c->stream;
     const int lanes = vc_lanes_for_items(c->hint.payload, c->hint.items);
-    HIP_TRY(vc_launch_chain_plan(S, T, c->B.slot_off, c->B.row_base, c->B.chain_row_tot + 2 * (size_t)S.P, c->desc.as<int64_t>(), guess, st,
+    HIP_TRY(vc_launch_chain_plan(S, T, c->B.slot_lines(), c->B.row_base, c->B.chain_row_base, c->B.chain_row_tot, c->desc.as<int64_t>(), guess, st,
                                  c->B.header, guard.cap_items));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     int64_t done = 0;                                     // items the guarded launch was sized for
@@ -555,7 +563,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
                 if (attempt == 1) { std::swap(c->events[1], c->events[2]); c->plan_end = 1; }
                 HIP_TRY(hipEventRecord(c->events[2], st));
             }
-            HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_off, c->B.row_base, c->B.header, guard, pair_lanes, sendbuf, recvbuf,
+            HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, pair_lanes, sendbuf, recvbuf,
                                           c->stage.as<char>(), st));
             if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
             HIP_TRY(VC_WAIT(c));
@@ -598,7 +606,7 @@ static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std:
     const int lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes;
     const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
-    HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_off, c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+    HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     c->pending.active = true;
     c->pending.S = S; c->pending.T = T; c->pending.sendbuf = sendbuf; c->pending.recvbuf = recvbuf; c->pending.lanes = lanes;
@@ -642,7 +650,7 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
             c->plan_end = 1;
             HIP_TRY(hipEventRecord(c->events[2], c->stream));
         }
-        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, c->B.slot_off, c->B.row_base, c->B.header, guard, c->pending.lanes,
+        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, c->pending.lanes,
                                       c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], c->stream));
         HIP_TRY(VC_WAIT(c));
@@ -751,8 +759,9 @@ extern "C" int TTPL_rbruck_alltoallv(int n, int r, char *sendbuf, int *sendcount
 // listless execution of twophase_rbruck_alltoallv, with the plan tables and the staging arena carved out of the static
 // device array `scratch` instead of the communicator's grow-only buffers.  No hipMalloc, hipFree, event or stream
 // creation happens here; the pinned header the planner reports through was allocated by vc_comm_create.  Every call on
-// a GPU uses that GPU's one array, so calls that overlap on one GPU race.  Nothing in the array needs to start at
-// zero: the planning kernels overwrite every word they or the copy kernel later read.
+// a GPU uses that GPU's one array, so calls that overlap on one GPU race.  The first
+// words count the planning kernel's workgroups and are zero between the calls; of the rest nothing needs to start at zero: the
+// planning kernel overwrites every word it or the copy kernel later reads.
 static size_t carve(size_t &at, size_t bytes) {
     const size_t here = at;
     at += (bytes + 255) & ~(size_t)255;
@@ -792,6 +801,7 @@ extern "C" int twophase_rbruck_alltoallv_noalloc(int r, char *sendbuf, int *send
     size_t at = 0;
     PlanBufs &B = c->B;
     B = PlanBufs();
+    B.ticket = reinterpret_cast<unsigned *>(base + carve(at, VC_TICKET_BYTES));      // (nothing else ever lies here: zero from the start)
     B.header = reinterpret_cast<int64_t *>(base + carve(at, z.header));
     B.slot_off = reinterpret_cast<int64_t *>(base + carve(at, z.slot_off));
     B.row_tot = reinterpret_cast<int64_t *>(base + carve(at, z.row_tot));
@@ -811,7 +821,7 @@ extern "C" int twophase_rbruck_alltoallv_noalloc(int r, char *sendbuf, int *send
     rc = enqueue_plan_sizes(c, S, L, T, true, false);
     if (rc) return rc;
     const int lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes;
-    HIP_TRY(vc_launch_copy_blocks(S, T, B.slot_off, B.row_base, B.header, guard, lanes, sendbuf, recvbuf, stage, c->stream));
+    HIP_TRY(vc_launch_copy_blocks(S, T, B.slot_lines(), B.row_base, B.header, guard, lanes, sendbuf, recvbuf, stage, c->stream));
     HIP_TRY(VC_WAIT(c));
     PlanInfo pi;
     rc = plan_read(c, S, L, pi, true);

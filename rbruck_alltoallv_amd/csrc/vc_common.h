@@ -70,6 +70,26 @@ VC_HD VcDivisor vc_make_divisor(int d) {          // d >= 1
 VC_HD int vc_div(int x, const VcDivisor &v) { return (int)(((uint64_t)(unsigned)x * v.mul) >> v.shift); }
 VC_HD int vc_mod(int x, const VcDivisor &v) { return x - vc_div(x, v) * v.d; }
 
+// The same for what routes divide: ranks, slots, offsets and nodes, all below 2^16, by a divisor below 2^16.  One multiplication
+// whose high word is the quotient, and one operation for the divisor 1, whose constant would take 33 bits.
+// mul = floor(2^32 / d) + 1 for d > 1: x * (mul * d - 2^32) <= x * d < 2^32.
+struct VcRankDivisor {
+    int d;
+    unsigned mul;
+    unsigned one;      // all bits for d = 1, else 0
+};
+
+VC_HD VcRankDivisor vc_make_rank_divisor(int d) {          // d >= 1
+    VcRankDivisor v;
+    v.d = d;
+    v.mul = d > 1 ? (unsigned)(((uint64_t)1 << 32) / (uint64_t)d) + 1 : 0;
+    v.one = d > 1 ? 0 : ~0u;
+    return v;
+}
+
+VC_HD int vc_div(int x, const VcRankDivisor &v) { return (int)((unsigned)(((uint64_t)(unsigned)x * v.mul) >> 32) | ((unsigned)x & v.one)); }
+VC_HD int vc_mod(int x, const VcRankDivisor &v) { return x - vc_div(x, v) * v.d; }
+
 // What kind of algorithm the call runs; fixed for the whole call.
 struct VcSched {
     int P;            // ranks
@@ -104,13 +124,13 @@ struct VcSched {
                       //    is a contiguous copy (TTPL_BT_alltoallv, src/twophase_twolayer_rbruck.cpp:388-398, 430-453).
                       //    The organized region is staging region number w.
     // set by vc_set_divisors once n, G, r and P are final:
-    VcDivisor dn, dG, dr, dP;                     // division by n, G, r, P
+    VcRankDivisor dn, dr;                         // division of ranks, slots and offsets by n, r
+    VcDivisor dP;                                 // division of pair numbers by P
 };
 
 VC_HD void vc_set_divisors(VcSched &S) {
-    S.dn = vc_make_divisor(S.n > 0 ? S.n : 1);
-    S.dG = vc_make_divisor(S.G > 0 ? S.G : 1);
-    S.dr = vc_make_divisor(S.r > 0 ? S.r : 1);
+    S.dn = vc_make_rank_divisor(S.n > 0 ? S.n : 1);
+    S.dr = vc_make_rank_divisor(S.r > 0 ? S.r : 1);
     S.dP = vc_make_divisor(S.P > 0 ? S.P : 1);
 }
 
@@ -197,23 +217,25 @@ hipError_t vc_launch_done(unsigned *word, unsigned value, hipStream_t st);
 // ... set (in the host's copy of the header only) by a copying wavefront that gave up waiting for that: the call is redone
 #define VC_HEADER_STALLED (VC_HEADER_SYNC + 2)
 #define VC_HEADER_WORDS(nl) (VC_HEADER_FIXED + 2 * (nl))
-// Passes 1 and 2: staging prefix sums and the number of work items of every launch (sizes only).  The launch table
-// travels as a kernel argument when it has at most VC_LAUNCH_PACK entries (launches_dev is then not read).  With chain_row_tot /
-// chain_row_base ((2 + VC_TILES(P)) P and P int64, or null) also the chain items per final receiver, the first item of every
-// (receiver, tile of sources) in the list's tiled order (behind chain_row_tot's first 2 P words), their total in header[2] and the most
-// pieces of any block in header[4].
+// Launch-per-digit execution, passes 1 and 2: staging prefix sums and the number of work items of every launch (sizes only).
+// The launch table travels as a kernel argument when it has at most VC_LAUNCH_PACK entries (launches_dev is then not read).
 hipError_t vc_launch_plan_sizes(const VcSched &S, const VcLaunchInfo *launches_host, const VcLaunchInfo *launches_dev, int nlaunch,
                                 VcTables T, int64_t *slot_off,
                                 int64_t *row_tot, int64_t *row_base, int64_t *org_run_base, int64_t *item_row_tot,
-                                int64_t *item_row_base, int64_t *row_bytes, int64_t *chain_row_tot, int64_t *chain_row_base,
-                                int64_t *header, int64_t *header_host, hipStream_t st);
-// Forwarded execution: the chain items (every block's route in closed form, staging addresses from the plan tables).
-// chain_tile_base: [P][VC_TILES(P)] first item of every (receiver, tile of sources) (vc_launch_plan_sizes leaves it behind
-// chain_row_tot's first 2 P words).
+                                int64_t *item_row_base, int64_t *row_bytes, int64_t *header, int64_t *header_host, hipStream_t st);
+// Forwarded execution: the same in one kernel; slot_off in units of VC_LINE.  chain_row_tot ((2 + VC_TILES(P)) P int64) and chain_row_base (P) receive the chain items
+// per final receiver and tile of sources and the first item of every receiver (were the list ordered by receivers).  ticket:
+// VC_TICKET_BYTES that are zero before and after.
+#define VC_TICKET_BYTES 16384
+hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_off, int64_t *row_tot, int64_t *row_base, int64_t *row_bytes,
+                                  int64_t *chain_row_tot, int64_t *chain_row_base, int64_t *header, int64_t *header_host, unsigned *ticket,
+                                  hipStream_t st);
+// Forwarded execution: the chain items (every block's route in closed form, staging addresses from the plan tables;
+// chain_row_base and chain_row_tot as vc_launch_plan_forward leaves them).
 // header + cap_items (optional): the launch was enqueued before the host knew the plan; it writes nothing unless the
 // device header the sizing kernels left says the tables are in order and the list holds all header[2] items.
-hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const int64_t *slot_off, const int64_t *row_base,
-                                const int64_t *chain_tile_base, int64_t *items, int64_t nitems, hipStream_t st,
+hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base,
+                                const int64_t *chain_row_base, const int64_t *chain_row_tot, int64_t *items, int64_t nitems, hipStream_t st,
                                 const int64_t *header = nullptr, int64_t cap_items = 0);
 // Pass 3: writes the work items (needs the item buffer, sized from the header).
 hipError_t vc_launch_plan_emit(const VcSched &S, const VcLaunchInfo *launches_host, const VcLaunchInfo *launches_dev, int nlaunch,
@@ -283,7 +305,7 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 // the call as refused then.  With bad table entries nothing has been stored by then: the copying wavefronts hold their
 // stores back until the totalling ones have reported on all of the tables.  With a block longer than a slot the blocks of
 // the other pairs may already have been delivered; they are delivered again when the host redoes the call.
-hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const int64_t *slot_off, const int64_t *row_base, const int64_t *header,
+hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  int64_t *header_host = nullptr, int64_t *header_zero = nullptr, int64_t *totals = nullptr);
 // dst2 non-null: every vector is stored twice (one read, two writes)

@@ -362,7 +362,7 @@ __device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcTables
 // LANES = VC_THREADS: a workgroup of four wavefronts per pair; LANES = VC_WAVE: one wavefront per pair, for blocks of a
 // KiB or two (a quarter of the wavefronts to start, all of them with work).
 template <int LANES>
-__global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const int64_t *__restrict__ slot_off,
+__global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                const int64_t *__restrict__ row_base,
                                                                const int64_t *__restrict__ header, VcListlessGuard guard,
                                                                int64_t first_pair, const char *__restrict__ sendbuf,
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
 
 // The same for pairs whose blocks are a few hundred bytes: a quarter of a wavefront per pair, four pairs in a row per
 // wavefront.  Lane q of a group evaluates hop slots q and q + 16; the four routes of the wavefront go through LDS.
-__global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched S, VcTables T, const int64_t *__restrict__ slot_off,
+__global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                          const int64_t *__restrict__ row_base,
                                                                          const int64_t *__restrict__ header, VcListlessGuard guard,
                                                                          int64_t first_pair, const char *__restrict__ sendbuf,
@@ -473,7 +473,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
 // of the wavefront carries BATCH / 4 of the blocks, one after the other.  Measured on MI355X, 1024 ranks, blocks of 0 - 16
 // bytes (two hops each): 211 us with a quarter of a wavefront per pair, 105 / 87 / 79 us with BATCH = 16 / 32 / 64.
 template <int BATCH>
-__global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const int64_t *__restrict__ slot_off,
+__global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                        const int64_t *__restrict__ row_base,
                                                                        const int64_t *__restrict__ header, VcListlessGuard guard,
                                                                        int64_t first_pair, const char *__restrict__ sendbuf,
@@ -536,7 +536,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
 }
 
 template <int BATCH>
-static void vc_launch_batch(int64_t pairs, const VcSched &S, VcTables T, const int64_t *slot_off, const int64_t *row_base, const int64_t *header,
+static void vc_launch_batch(int64_t pairs, const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                             VcListlessGuard guard, int64_t first_pair, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                             int64_t *header_host, int64_t *header_zero) {
     const int64_t waves = (pairs + BATCH - 1) / BATCH;
@@ -545,7 +545,7 @@ static void vc_launch_batch(int64_t pairs, const VcSched &S, VcTables T, const i
                        T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, header_host, header_zero);
 }
 
-hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const int64_t *slot_off, const int64_t *row_base, const int64_t *header,
+hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  int64_t *header_host, int64_t *header_zero, int64_t *totals) {
     const int64_t npairs = (int64_t)S.P * S.P;

@@ -63,6 +63,8 @@ struct PlanBufs {
             *item_row_base = nullptr, *row_bytes = nullptr, *chain_row_tot = nullptr, *chain_row_base = nullptr, *header = nullptr;
     VcLaunchInfo *launches = nullptr;
     int *rd_packed = nullptr;
+    uint32_t *slot_lines() const { return reinterpret_cast<uint32_t *>(slot_off); }      // as a forwarded plan keeps them
+    unsigned *ticket = nullptr;           // vc_launch_plan_forward's count of finished workgroups: zero between the calls
 };
 
 // What a call asked for: enough to derive its schedule again in the other execution mode.
@@ -89,7 +91,7 @@ struct vc_comm {
     bool strided_clean = false;           // ... and the one the next call will use is known to be zero
     int strided_turn = 0;
     DevBuf slot_off, row_tot, row_base, org_run_base, item_row_tot, item_row_base, row_bytes, desc, header, launches, stage, rd_packed,
-        scratch, max_state;
+        scratch, max_state, ticket;
     double cal_copy_bytes_per_s = 0, cal_launch_s = 0, cal_sync_s = 0;   // calibrate(): the plain copy's rate, the cost of a
                                           // launch, of a launch the host waits for
     int bound_staging = 1;                // vc_comm_set_staging_bound

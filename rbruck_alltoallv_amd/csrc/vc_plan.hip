@@ -10,6 +10,7 @@
 // staging arena is compact; a second family of prefix sums numbers the work
 // items (block pieces of at most VC_CHUNK bytes) so that every launch gets a
 // dense list with no empty entries.
+#include <algorithm>
 #include <cstring>
 
 #include "vc_common.h"
@@ -17,23 +18,17 @@
 
 #include "vc_plan_math.h"
 
-// ---- pass 1: row-wise prefix sums ----
-// Launch-per-digit execution: grid (P, regions + nl).  Rows y < regions = w + w2: staging sizes of region y,
-// slot_off[(y*P + to)*P + id] = offset of the slot inside the row.  Later rows: work-item count and moved bytes of launch
-// y - regions; the first of them also sums the payload and counts negative table entries.
-// Forwarded execution (chain_row_tot != null, nl = 0): grid (P, regions + 1).  The region rows also sum the bytes of the
-// blocks themselves (every staged block is one hop), and the last row counts the chain items of the blocks that end on
-// the rank, the most pieces of any of them, the payload and the negative table entries.
-// row_bytes rows: [launch or region][P], then [payload][P], then [negative entries][P], then (forwarded) [longest block][P].
+// ---- launch-per-digit execution, pass 1: row-wise prefix sums ----
+// grid (P, regions + nl).  Rows y < regions = w + w2: staging sizes of region y, slot_off[(y*P + to)*P + id] = offset of the slot
+// inside the row.  Later rows: work-item count and moved bytes of launch y - regions; the first of them also sums the
+// payload and counts negative table entries.
+// row_bytes rows: [launch][P], then [payload][P], then [negative entries][P].
 __global__ __launch_bounds__(VC_THREADS) void vc_plan_rows(VcSched S, VcLaunchPack pack, const VcLaunchInfo *__restrict__ launches, int nl, VcTables T,
                                                            int64_t *__restrict__ slot_off, int64_t *__restrict__ row_tot,
-                                                           int64_t *__restrict__ item_row_tot, int64_t *__restrict__ row_bytes,
-                                                           int64_t *__restrict__ chain_row_tot) {
+                                                           int64_t *__restrict__ item_row_tot, int64_t *__restrict__ row_bytes) {
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
     const int to = blockIdx.x, P = S.P;
     const int nreg = S.w + S.w2;                          // the organized region is laid out by vc_plan_org_rows
-    const bool forward = chain_row_tot != nullptr;
-    const int nsum = forward ? nreg : nl;                 // rows of row_bytes before the payload row
     if ((int)blockIdx.y < nreg && S.recycle) {
         // reused staging: the slots of the region in one prefix sum per hop slot in which their blocks leave again
         __shared__ int64_t family_carry[VC_RECYCLE_MAX_SLOTS];
@@ -61,14 +56,13 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_rows(VcSched S, VcLaunchPa
     }
     if ((int)blockIdx.y < nreg) {
         const int y = blockIdx.y;
-        int64_t carry = 0, data = 0;
+        int64_t carry = 0;
         for (int base0 = 0; base0 < P; base0 += 4 * VC_THREADS) {       // four chunks at a time: their table reads travel together
-            int64_t v[4], len[4];
+            int64_t v[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const int id = base0 + u * VC_THREADS + threadIdx.x;
-                len[u] = 0;
-                v[u] = (id < P) ? vc_region_slot_size(S, T, y, to, id, &len[u]) : 0;
+                v[u] = (id < P) ? vc_region_slot_size(S, T, y, to, id) : 0;
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
@@ -78,72 +72,31 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_rows(VcSched S, VcLaunchPa
                 const int64_t ex = vc_block_exclusive_scan(v[u], lds, total);
                 if (id < P) slot_off[((int64_t)y * P + to) * P + id] = carry + ex;
                 carry += total;
-                data += len[u];
             }
         }
-        if (forward) data = vc_block_sum(data, lds);
-        if (threadIdx.x == 0) {
-            row_tot[(int64_t)y * P + to] = carry;
-            if (forward) row_bytes[(int64_t)y * P + to] = data;
-        }
+        if (threadIdx.x == 0) row_tot[(int64_t)y * P + to] = carry;
         return;
     }
-    int64_t items = 0, bytes = 0, payload = 0, most = 0, longest = 0;
+    int64_t items = 0, bytes = 0, payload = 0;
     int64_t bad = 0;                                      // entries of this rank's rows no rank could have passed
     const int L = blockIdx.y - nreg;
-    if (forward) {
-        // sources in chunks of VC_THREADS; the items of every tile of VC_TILE_RANKS sources (half a wavefront) are left for
-        // vc_plan_bases, which turns them into the first item of every (receiver, tile) in the list's tiled order.
-        // Four chunks at a time, so that the table reads of all of them travel together before the first sum needs them;
-        // the checks of this rank's own rows (the loop over ids below, for launch-per-digit execution) ride along.
-        const int nchunk = (P + VC_THREADS - 1) / VC_THREADS, ntile = VC_TILES(P);
-        int64_t before = 0;
-        for (int chunk0 = 0; chunk0 < nchunk; chunk0 += 4) {
-            int64_t cnt[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int s = (chunk0 + u) * VC_THREADS + threadIdx.x;
-                cnt[u] = 0;
-                if (chunk0 + u >= nchunk || s >= P) continue;
-                cnt[u] = vc_chain_count(S, T, s, to);
-                const int expected = vc_rc(S, T, to, s), sent = vc_sc(S, T, s, to);
-                bad += vc_pair_bad_entries(S, T, s, to);
-                payload += (int64_t)expected * S.esz;
-                most = cnt[u] > most ? cnt[u] : most;
-                const int64_t len = (int64_t)sent * S.esz;
-                longest = len > longest ? len : longest;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                if (chunk0 + u >= nchunk) break;
-                int64_t tile = cnt[u];
-#pragma unroll
-                for (int o = VC_TILE_RANKS / 2; o > 0; o >>= 1) tile += __shfl_xor(tile, o, VC_TILE_RANKS);
-                const int s = (chunk0 + u) * VC_THREADS + threadIdx.x;
-                if (threadIdx.x % VC_TILE_RANKS == 0 && s < P) chain_row_tot[2 * (int64_t)P + (int64_t)to * ntile + s / VC_TILE_RANKS] = tile;
-                before += vc_block_sum(cnt[u], lds);
-            }
-        }
-        items = threadIdx.x == 0 ? before : 0;            // vc_block_sum below adds the lanes up
-    } else {
-        const VcLaunchInfo info = launches ? launches[L] : pack.info[L];     // a short launch table travels as a kernel argument
-        const int nent = vc_entries_per_rank(S, info);
-        for (int id = threadIdx.x; id < nent; id += VC_THREADS) {
-            VcEntry e;
-            if (vc_entry_block(S, info, to, id, e)) {
-                const int64_t len = vc_entry_len(S, T, e);
-                items += vc_chunk_count(len, vc_entry_phase(S, T, e), vc_entry_cut(S, T, e));
-                bytes += len;
-            }
+    const VcLaunchInfo info = launches ? launches[L] : pack.info[L];     // a short launch table travels as a kernel argument
+    const int nent = vc_entries_per_rank(S, info);
+    for (int id = threadIdx.x; id < nent; id += VC_THREADS) {
+        VcEntry e;
+        if (vc_entry_block(S, info, to, id, e)) {
+            const int64_t len = vc_entry_len(S, T, e);
+            items += vc_chunk_count(len, vc_entry_phase(S, T, e), vc_entry_cut(S, T, e));
+            bytes += len;
         }
     }
-    if (L == 0 && !forward)                               // forwarded execution has done this above
+    if (L == 0)
         for (int id = threadIdx.x; id < P; id += VC_THREADS) {
             payload += (int64_t)vc_rc(S, T, to, id) * S.esz;
             bad += vc_pair_bad_entries(S, T, id, to);
         }
     items = vc_block_sum(items, lds);
-    if (forward) { most = vc_block_max(most, lds); longest = vc_block_max(longest, lds); } else bytes = vc_block_sum(bytes, lds);
+    bytes = vc_block_sum(bytes, lds);
     if (L == 0) {
         payload = vc_block_sum(payload, lds);
         bad = vc_block_sum(bad, lds);
@@ -151,9 +104,9 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_rows(VcSched S, VcLaunchPa
         if (S.packed_recv && payload > (int64_t)0x7FFFFFFF * S.esz) bad += VC_BAD_OVERFLOW;
     }
     if (threadIdx.x == 0) {
-        if (forward) { chain_row_tot[to] = items; chain_row_tot[P + to] = most; row_bytes[(int64_t)(nsum + 2) * P + to] = longest; }
-        else { item_row_tot[(int64_t)L * P + to] = items; row_bytes[(int64_t)L * P + to] = bytes; }
-        if (L == 0) { row_bytes[(int64_t)nsum * P + to] = payload; row_bytes[(int64_t)(nsum + 1) * P + to] = bad; }
+        item_row_tot[(int64_t)L * P + to] = items;
+        row_bytes[(int64_t)L * P + to] = bytes;
+        if (L == 0) { row_bytes[(int64_t)nl * P + to] = payload; row_bytes[(int64_t)(nl + 1) * P + to] = bad; }
     }
 }
 
@@ -179,68 +132,17 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_org_rows(VcSched S, VcTabl
         slot_off[((int64_t)S.w * P + to) * P + id] = org_run_base[(int64_t)to * G + vc_div(id, S.dn)] + vc_org_slot_rel(S, T, to, id);
 }
 
-// ---- pass 2: prefix sums over the rows ----
-// (A kernel of its own although a boundary between two kernels of one stream costs as much as the pass itself: folding it
-// into pass 1 — every workgroup counts itself when its rows are written, the last one does the prefix sums — needs a
-// device-wide release fence per workgroup, which on this chip writes the XCD's L2 back; measured, calls on 160 - 512 ranks
-// took twice as long that way.)
-// Launch-per-digit execution: grid (nl + 1).  Workgroup L < nl: item bases of launch L's rows (relative to the launch's
-// first item), its item count and moved bytes.  Workgroup nl: staging row bases, staging bytes, payload bytes, negative
-// table entries.  Forwarded execution (chain_row_tot != null, nl = 0): grid (2 + tile rows).  Workgroup 0 as workgroup nl above,
-// and the moved bytes = payload + bytes of the staged blocks as those of launch 0; workgroup 1: chain items per receiver summed up
-// (their total, the most pieces, the longest block); workgroup 2 + k: first item of every (receiver, tile of sources) of tile row k.
+// ---- launch-per-digit execution, pass 2: prefix sums over the rows ----
+// grid (nl + 1).  Workgroup L < nl: item bases of launch L's rows (relative to the launch's first item), its item count and
+// moved bytes.  Workgroup nl: staging row bases, staging bytes, payload bytes, negative table entries.
 __global__ __launch_bounds__(VC_THREADS) void vc_plan_bases(VcSched S, int P, int w, int nreg, int nl, const int64_t *__restrict__ row_tot,
                                                             int64_t *__restrict__ row_base, const int64_t *__restrict__ item_row_tot,
                                                             int64_t *__restrict__ item_row_base, const int64_t *__restrict__ row_bytes,
-                                                            int64_t *chain_row_tot, int64_t *__restrict__ chain_row_base,
                                                             int64_t *__restrict__ header, int64_t *__restrict__ header_host) {
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
     const int L = blockIdx.x;
-    const bool forward = chain_row_tot != nullptr, recycle = S.recycle != 0;
-    const int nsum = forward ? nreg : nl;                 // rows of row_bytes before the payload row
+    const bool recycle = S.recycle != 0;
     int64_t carry = 0, bytes = 0;
-    if (forward && L >= 2) {
-        // tile row L - 2: the receivers [t0, t1).  The list holds, tile row after tile row, the tiles of sources in turn and
-        // inside a tile the receivers in turn: an exclusive scan over (tile of sources, receiver) of the counts vc_plan_rows
-        // left, in place, started at the items of all receivers before t0.
-        const int ntile = VC_TILES(P), t0 = (L - 2) * VC_TILE_RANKS, rows = (t0 + VC_TILE_RANKS < P ? t0 + VC_TILE_RANKS : P) - t0;
-        int64_t *tile = chain_row_tot + 2 * (int64_t)P;
-        int64_t earlier = 0;
-        for (int i = threadIdx.x; i < t0; i += VC_THREADS) earlier += chain_row_tot[i];
-        carry = vc_block_sum(earlier, lds);
-        const int per = VC_THREADS / VC_TILE_RANKS;       // tiles of sources per pass
-        for (int sb0 = 0; sb0 < ntile; sb0 += per) {
-            const int sb = sb0 + threadIdx.x / VC_TILE_RANKS, row = threadIdx.x % VC_TILE_RANKS;
-            const bool inside = sb < ntile && row < rows;
-            int64_t total;
-            const int64_t ex = vc_block_exclusive_scan(inside ? tile[(int64_t)(t0 + row) * ntile + sb] : 0, lds, total);
-            if (inside) tile[(int64_t)(t0 + row) * ntile + sb] = carry + ex;
-            carry += total;
-        }
-        return;
-    }
-    if (forward && L == 1) {                              // first chain item of every final receiver
-        int64_t most = 0, longest = 0;
-        for (int b0 = 0; b0 < P; b0 += VC_THREADS) {
-            const int i = b0 + threadIdx.x;
-            int64_t total;
-            const int64_t ex = vc_block_exclusive_scan((i < P) ? chain_row_tot[i] : 0, lds, total);
-            if (i < P) {
-                chain_row_base[i] = carry + ex;
-                most = chain_row_tot[P + i] > most ? chain_row_tot[P + i] : most;
-                const int64_t len = row_bytes[(int64_t)(nsum + 2) * P + i];
-                longest = len > longest ? len : longest;
-            }
-            carry += total;
-        }
-        most = vc_block_max(most, lds);
-        longest = vc_block_max(longest, lds);
-        if (threadIdx.x == 0) {
-            header[2] = carry; header[VC_HEADER_MAX_PIECES] = most; header[VC_HEADER_MAX_LEN] = longest;
-            if (header_host) { header_host[2] = carry; header_host[VC_HEADER_MAX_PIECES] = most; header_host[VC_HEADER_MAX_LEN] = longest; }
-        }
-        return;
-    }
     if (L == nl && recycle) {
         // reused staging: row offsets inside every sub-region, the sizes of the sub-regions' pieces (the rows of
         // vc_recycle_rows_per_segment(P) consecutive receivers each), their places in the arena
@@ -279,7 +181,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_bases(VcSched S, int P, in
             if (piece_size[f * nseg + g] > 0) row_base[i] += piece_base[f * nseg + g] - start;
         }
         int64_t bad = 0;
-        for (int i = threadIdx.x; i < P; i += VC_THREADS) { bytes += row_bytes[(int64_t)nsum * P + i]; bad += row_bytes[(int64_t)(nsum + 1) * P + i]; }
+        for (int i = threadIdx.x; i < P; i += VC_THREADS) { bytes += row_bytes[(int64_t)nl * P + i]; bad += row_bytes[(int64_t)(nl + 1) * P + i]; }
         bytes = vc_block_sum(bytes, lds);
         bad = vc_block_sum(bad, lds);
         if (threadIdx.x == 0) {
@@ -298,20 +200,13 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_bases(VcSched S, int P, in
             if (i < nrows) row_base[i] = carry + ex;
             carry += total;
         }
-        int64_t bad = 0, staged = 0;
-        for (int i = threadIdx.x; i < P; i += VC_THREADS) { bytes += row_bytes[(int64_t)nsum * P + i]; bad += row_bytes[(int64_t)(nsum + 1) * P + i]; }
-        if (forward)
-            for (int64_t i = threadIdx.x; i < (int64_t)nreg * P; i += VC_THREADS) staged += row_bytes[i];
+        int64_t bad = 0;
+        for (int i = threadIdx.x; i < P; i += VC_THREADS) { bytes += row_bytes[(int64_t)nl * P + i]; bad += row_bytes[(int64_t)(nl + 1) * P + i]; }
         bytes = vc_block_sum(bytes, lds);
         bad = vc_block_sum(bad, lds);
-        if (forward) staged = vc_block_sum(staged, lds);
         if (threadIdx.x == 0) {
             header[0] = carry; header[1] = bytes; header[VC_HEADER_BAD] = bad;
             if (header_host) { header_host[0] = carry; header_host[1] = bytes; header_host[VC_HEADER_BAD] = bad; }
-            if (forward) {                                // every staged block is one hop, every block's last hop ends in recvbuf
-                header[VC_HEADER_FIXED] = bytes + staged;
-                if (header_host) header_host[VC_HEADER_FIXED] = bytes + staged;
-            }
         }
         return;
     }
@@ -331,7 +226,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_bases(VcSched S, int P, in
     }
 }
 
-// ---- pass 3: the work items ----
+// ---- launch-per-digit execution, pass 3: the work items ----
 // grid (P, nl, Z).  Repeats the row scan of pass 1 to place every block's pieces; Z workgroups share a receiver's entries
 // when there are few ranks (their blocks are then huge and have many pieces).
 __global__ __launch_bounds__(VC_THREADS) void vc_plan_emit(VcSched S, VcLaunchPack pack, const VcLaunchInfo *__restrict__ launches, VcTables T,
@@ -412,21 +307,17 @@ static VcLaunchPack vc_pack_launches(const VcLaunchInfo *host, int nl) {
     return pack;
 }
 
-hipError_t vc_launch_plan_sizes(const VcSched &S, const VcLaunchInfo *launches_host, const VcLaunchInfo *launches_dev, int nlaunch,
+hipError_t vc_launch_plan_sizes(const VcSched &S, const VcLaunchInfo *launches_host, const VcLaunchInfo *launches_dev, int nl,
                                 VcTables T, int64_t *slot_off,
                                 int64_t *row_tot, int64_t *row_base, int64_t *org_run_base, int64_t *item_row_tot,
-                                int64_t *item_row_base, int64_t *row_bytes, int64_t *chain_row_tot, int64_t *chain_row_base,
-                                int64_t *header, int64_t *header_host, hipStream_t st) {
-    const bool forward = chain_row_tot != nullptr;
-    const int nl = forward ? 0 : nlaunch;                 // forwarded execution has no use for the per-launch rows
+                                int64_t *item_row_base, int64_t *row_bytes, int64_t *header, int64_t *header_host, hipStream_t st) {
     const int nreg = S.w + S.w2;
-    hipLaunchKernelGGL(vc_plan_rows, dim3(S.P, nreg + (forward ? 1 : nl)), dim3(VC_THREADS), 0, st, S,
-                       vc_pack_launches(launches_host, nl), nl <= VC_LAUNCH_PACK ? nullptr : launches_dev, nl, T, slot_off,
-                       row_tot, item_row_tot, row_bytes, chain_row_tot);
+    hipLaunchKernelGGL(vc_plan_rows, dim3(S.P, nreg + nl), dim3(VC_THREADS), 0, st, S, vc_pack_launches(launches_host, nl),
+                       nl <= VC_LAUNCH_PACK ? nullptr : launches_dev, nl, T, slot_off, row_tot, item_row_tot, row_bytes);
     if (S.coalesce)
         hipLaunchKernelGGL(vc_plan_org_rows, dim3(S.P), dim3(VC_THREADS), 0, st, S, T, slot_off, row_tot, org_run_base);
-    hipLaunchKernelGGL(vc_plan_bases, dim3(forward ? 2 + VC_TILES(S.P) : nl + 1), dim3(VC_THREADS), 0, st, S, S.P, vc_regions(S), nreg, nl, row_tot, row_base,
-                       item_row_tot, item_row_base, row_bytes, chain_row_tot, chain_row_base, header, header_host);
+    hipLaunchKernelGGL(vc_plan_bases, dim3(nl + 1), dim3(VC_THREADS), 0, st, S, S.P, vc_regions(S), nreg, nl, row_tot, row_base,
+                       item_row_tot, item_row_base, row_bytes, header, header_host);
     return hipGetLastError();
 }
 
@@ -441,71 +332,322 @@ hipError_t vc_launch_plan_emit(const VcSched &S, const VcLaunchInfo *launches_ho
 }
 
 // ---- forwarded execution ----
-// grid (P, chunks x Z): the chain items of the blocks that end on rank t.  The list is ordered in tiles of VC_TILE_RANKS
-// receivers x VC_TILE_RANKS sources, receiver by receiver inside a tile (vc_plan_bases has left the first item of every
-// (receiver, tile of sources)); the sources come in chunks of VC_THREADS, and Z workgroups share a chunk (each a whole number
+#define VC_PLAN_XCDS 8
+// Workgroups count themselves on one of VC_TICKETS words, each in a cache line of its own, and the last of a word on the word
+// behind them: atomics on one word go one after the other, about 10 ns each (2048 workgroups on one word: +20 us).
+#define VC_TICKETS 64
+#define VC_TICKET_STRIDE 32
+// Rows a kernel gives a workgroup each: workgroup b runs on XCD b mod 8, and XCD k takes the k-th eighth of the ranks, so that
+// the table entries of neighbouring ranks, which share cache lines (the entries of a rank lie in a column), meet in one L2.
+static unsigned vc_rank_grid(int P, int rows) { return (unsigned)((P + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS) * VC_PLAN_XCDS * rows; }
+
+// What the last workgroup of a grid reads is stored and loaded past the L2 of the storing and the loading XCD.
+__device__ __forceinline__ void vc_share(int64_t *p, int64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ int64_t vc_shared(const int64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Everything that has to be known before the list or the blocks: grid vc_rank_grid(P, regions + 1).  Of the rows of rank `to`, row
+// y < regions = w + w2 sums up the staging slots of region y (slot_off[(y*P + to)*P + id] = offset of slot id inside the row, in lines) and
+// the bytes of the blocks in them (every staged block is one hop); the last row counts the chain items of the blocks that end
+// on the rank (by tile of VC_TILE_RANKS sources for vc_chain_emit), the payload, the table entries no rank could have
+// passed, the most pieces and the longest of its blocks.
+// row_bytes rows: [region][P] bytes of staged blocks, then [payload][P], [bad entries][P], [longest block][P].
+// chain_row_tot: [P] items, [P] most pieces, [P][tiles] items per tile of sources.
+// The workgroup that finishes last turns the row totals into first addresses (row_base, chain_row_base: exclusive sums) and
+// the header: a kernel of its own for that is a kernel boundary (2.6 us) more.  It learns that it is the last one from a count; no
+// release fence is needed (one per workgroup would write the XCD's L2 back each time: calls on 160 - 512 ranks took twice
+// as long that way), because the totals are stored past the L2 and waited for before the workgroup counts itself.
+// Latency bound below about 512 ranks.  Together with the prefix sums by data-parallel primitives and one reduction for
+// all totals: 150 ranks, four digits, 7.2 + 5.8 us (two kernels) -> 9.0,
+// 256 ranks, two digits, 7.2 + 4.8 -> 10.1, 1024 ranks in nodes of 32 27 + 7.5 -> 26.
+// PER: consecutive slots or sources per thread and round, so that one round takes all of them up to 1024 ranks.
+template <int PER>
+__global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTables T, uint32_t *__restrict__ slot_off, int64_t *row_tot,
+                                                              int64_t *__restrict__ row_base, int64_t *row_bytes, int64_t *chain_row_tot,
+                                                              int64_t *__restrict__ chain_row_base, int64_t *__restrict__ header,
+                                                              int64_t *__restrict__ header_host, unsigned *ticket) {
+    __shared__ int64_t lds[5 * VC_WAVES_PER_BLOCK];
+    __shared__ int is_last;
+    const int P = S.P, nreg = S.w + S.w2, nrow = nreg + 1, ranks_per_xcd = (P + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS;
+    const int at = blockIdx.x / VC_PLAN_XCDS, y = at % nrow, to = (int)(blockIdx.x % VC_PLAN_XCDS) * ranks_per_xcd + at / nrow;
+    if (to < P && y < nreg) {
+        int64_t carry = 0, data = 0;
+        uint32_t *const slots = slot_off + ((int64_t)y * P + to) * P;
+        for (int base = 0; base < P; base += PER * VC_THREADS) {
+            const int id0 = base + threadIdx.x * PER;
+            int64_t v[PER], rbase[PER], round = 0, total;
+            int count[PER], displ[PER];
+            bool there[PER];
+#pragma unroll
+            for (int u = 0; u < PER; u++) {                 // all reads first: none depends on another
+                int s, t;
+                const bool inside = id0 + u < P;
+                there[u] = vc_slot_block(S, y, to, inside ? id0 + u : 0, s, t) && inside;
+                count[u] = vc_sc(S, T, s, t); displ[u] = vc_rd(S, T, t, s); rbase[u] = T.rbase[t];
+            }
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                const int64_t len = there[u] ? (int64_t)count[u] * S.esz : 0, phase = (rbase[u] + (int64_t)displ[u] * S.esz + S.recv_lo) & (VC_LINE - 1);
+                v[u] = len ? (len + phase + VC_LINE - 1) & ~(int64_t)(VC_LINE - 1) : 0;
+                round += v[u];
+                data += len;
+            }
+            int64_t off = carry + vc_block_exclusive_scan(round, lds, total);
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                if (id0 + u < P) slots[id0 + u] = (uint32_t)(off / VC_LINE);
+                off += v[u];
+            }
+            carry += total;
+        }
+        data = vc_block_sum(data, lds);
+        if (threadIdx.x == 0) { vc_share(&row_tot[(int64_t)y * P + to], carry); vc_share(&row_bytes[(int64_t)y * P + to], data); }
+    } else if (to < P) {
+        const int ntile = VC_TILES(P), lanes = VC_TILE_RANKS / PER;              // threads per tile of sources
+        int64_t sum[5] = {0, 0, 0, 0, 0};                 // items, payload, bad entries; most pieces, longest block
+        for (int base = 0; base < P; base += PER * VC_THREADS) {
+            const int s0 = base + threadIdx.x * PER;
+            int64_t tile = 0;
+            VcPairEntries e[PER];
+#pragma unroll
+            for (int u = 0; u < PER; u++) {                 // all reads first
+                e[u] = vc_pair_entries(S, T, s0 + u < P ? s0 + u : 0, to);
+            }
+            const int64_t rbase = T.rbase[to];
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                if (s0 + u >= P) continue;
+                const int64_t len = (int64_t)e[u].sent * S.esz;
+                const int cut = (int)((rbase + (int64_t)e[u].rd * S.esz + S.recv_lo) & (VC_PIECE - 1));
+                const int64_t cnt = vc_chunk_count(len, cut & (VC_LINE - 1), cut);
+                tile += cnt;
+                sum[1] += (int64_t)e[u].expected * S.esz;
+                sum[2] += vc_bad_entries(S, e[u]);
+                sum[3] = cnt > sum[3] ? cnt : sum[3];
+                sum[4] = len > sum[4] ? len : sum[4];
+            }
+            sum[0] += tile;
+            for (int o = 1; o < lanes; o <<= 1) tile += __shfl_xor(tile, o, VC_WAVE);
+            if (threadIdx.x % lanes == 0 && s0 < P) chain_row_tot[2 * (int64_t)P + (int64_t)to * ntile + s0 / VC_TILE_RANKS] = tile;
+        }
+        vc_block_totals(sum, lds);
+        if (threadIdx.x == 0) {
+            // the packed receive layout is an int prefix sum of the rank's receive counts, like the reference's displacements
+            if (S.packed_recv && sum[1] > (int64_t)0x7FFFFFFF * S.esz) sum[2] += VC_BAD_OVERFLOW;
+            vc_share(&chain_row_tot[to], sum[0]);
+            vc_share(&chain_row_tot[P + to], sum[3]);
+            vc_share(&row_bytes[(int64_t)nreg * P + to], sum[1]);
+            vc_share(&row_bytes[(int64_t)(nreg + 1) * P + to], sum[2]);
+            vc_share(&row_bytes[(int64_t)(nreg + 2) * P + to], sum[4]);
+        }
+    }
+    if (threadIdx.x == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this workgroup's totals are where the last one will look
+        const unsigned mine = blockIdx.x % VC_TICKETS, words = gridDim.x < VC_TICKETS ? gridDim.x : VC_TICKETS;
+        unsigned *word = ticket + mine * VC_TICKET_STRIDE;
+        is_last = 0;
+        if (__hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (gridDim.x - mine + VC_TICKETS - 1) / VC_TICKETS - 1) {
+            __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            word = ticket + VC_TICKETS * VC_TICKET_STRIDE;
+            is_last = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == words - 1;
+        }
+    }
+    __syncthreads();
+    if (!is_last) return;
+    // rows are summed up in blocks of 4 per thread
+    int64_t carry = 0, items = 0, total;
+    const int64_t nrows = (int64_t)nreg * P;
+    int64_t sum[5] = {0, 0, 0, 0, 0};                     // payload, staged bytes, bad entries; most pieces, longest block
+    int64_t row_v[4], row_d[4];                           // the first round of the second loop, read together with the first loop's
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int64_t i = threadIdx.x * 4 + u;
+        row_v[u] = i < nrows ? vc_shared(&row_tot[i]) : 0;
+        row_d[u] = i < nrows ? vc_shared(&row_bytes[i]) : 0;
+    }
+    for (int64_t base = 0; base < P; base += 4 * VC_THREADS) {
+        int64_t v[4], pay[4], bad[4], most[4], longest[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int64_t i = base + threadIdx.x * 4 + u;
+            const bool inside = i < P;
+            v[u] = inside ? vc_shared(&chain_row_tot[i]) : 0;
+            most[u] = inside ? vc_shared(&chain_row_tot[P + i]) : 0;
+            pay[u] = inside ? vc_shared(&row_bytes[nreg * (int64_t)P + i]) : 0;
+            bad[u] = inside ? vc_shared(&row_bytes[(nreg + 1) * (int64_t)P + i]) : 0;
+            longest[u] = inside ? vc_shared(&row_bytes[(nreg + 2) * (int64_t)P + i]) : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            sum[0] += pay[u];
+            sum[2] += bad[u];
+            sum[3] = most[u] > sum[3] ? most[u] : sum[3];
+            sum[4] = longest[u] > sum[4] ? longest[u] : sum[4];
+        }
+        int64_t off = items + vc_block_exclusive_scan(v[0] + v[1] + v[2] + v[3], lds, total);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int64_t i = base + threadIdx.x * 4 + u;
+            if (i < P) chain_row_base[i] = off;
+            off += v[u];
+        }
+        items += total;
+    }
+    for (int64_t base = 0; base < nrows; base += 4 * VC_THREADS) {
+        sum[1] += row_d[0] + row_d[1] + row_d[2] + row_d[3];
+        int64_t off = carry + vc_block_exclusive_scan(row_v[0] + row_v[1] + row_v[2] + row_v[3], lds, total);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int64_t i = base + threadIdx.x * 4 + u, next = i + 4 * VC_THREADS;
+            if (i < nrows) row_base[i] = off;
+            off += row_v[u];
+            row_v[u] = next < nrows ? vc_shared(&row_tot[next]) : 0;
+            row_d[u] = next < nrows ? vc_shared(&row_bytes[next]) : 0;
+        }
+        carry += total;
+    }
+    __syncthreads();                                      // lds from the scans above
+    vc_block_totals(sum, lds);
+    if (threadIdx.x != 0) return;
+    // every staged block is one hop, every block's last hop ends in recvbuf
+    const int64_t words[VC_HEADER_MAX_LEN + 1] = {carry, sum[0], items, sum[2], sum[3], sum[0] + sum[1], sum[4]};
+#pragma unroll
+    for (int k = 0; k <= VC_HEADER_MAX_LEN; k++) { header[k] = words[k]; header_host[k] = words[k]; }
+    __hip_atomic_store(ticket + VC_TICKETS * VC_TICKET_STRIDE, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+static_assert((VC_TICKETS + 1) * VC_TICKET_STRIDE * sizeof(unsigned) <= VC_TICKET_BYTES, "room for the counts");
+static_assert(VC_HEADER_BAD == 3 && VC_HEADER_MAX_PIECES == 4 && VC_HEADER_FIXED == 5 && VC_HEADER_MAX_LEN == 6, "order of the words above");
+
+hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_off, int64_t *row_tot, int64_t *row_base, int64_t *row_bytes,
+                                  int64_t *chain_row_tot, int64_t *chain_row_base, int64_t *header, int64_t *header_host, unsigned *ticket,
+                                  hipStream_t st) {
+    const auto kernel = S.P <= VC_THREADS ? vc_plan_forward<1> : (S.P <= 2 * VC_THREADS ? vc_plan_forward<2> : vc_plan_forward<4>);
+    hipLaunchKernelGGL(kernel, dim3(vc_rank_grid(S.P, S.w + S.w2 + 1)), dim3(VC_THREADS), 0, st, S, T, slot_off, row_tot, row_base,
+                       row_bytes, chain_row_tot, chain_row_base, header, header_host, ticket);
+    return hipGetLastError();
+}
+
+// The chain items: grid vc_rank_grid(P, chunks x slices).  The list is ordered in tiles of VC_TILE_RANKS receivers x VC_TILE_RANKS sources, receiver by
+// receiver inside a tile; the sources come in chunks of VC_THREADS, and several workgroups share a chunk (each a whole number
 // of tiles) when there are few ranks, which would otherwise leave most of the chip idle: the kernel is a chain of dependent
-// table reads per workgroup, and one workgroup per compute unit hides none of them.  Big blocks are written by the whole
-// workgroup as in vc_plan_emit.
-__global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables T, const int64_t *__restrict__ slot_off,
-                                                            const int64_t *__restrict__ row_base,
-                                                            const int64_t *__restrict__ chain_tile_base, int slices,
+// table reads per workgroup, and one workgroup per compute unit hides none of them.
+// The items of a tile's blocks are neighbours in the list: where there are no more than VC_EMIT_TILE_ITEMS of them they are put
+// together in LDS and stored as whole cache lines (item by item a wavefront's store touches 64 places 40 bytes apart;
+// 1 Mi items: 34 -> 26 us with that and the reads of all hops together).
+// Big blocks are written by the whole workgroup as in vc_plan_emit.
+#define VC_EMIT_TILE_ITEMS 64
+// ROUTE: hop slots of a route kept in registers, 3 or 6 (two-layer calls and large radices have no more than 3, and the registers of 6
+// would cost them a third of the wavefronts in flight); with more the route is worked out again for every piece.
+#define VC_ROUTE_CACHE 6
+static_assert(VC_TILE_RANKS * VC_ROUTE_CACHE <= VC_EMIT_TILE_ITEMS * (VC_CHAIN_HEAD + 1), "routes of a tile's big blocks in the place of its items");
+template <int ROUTE>
+__global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
+                                                            const int64_t *__restrict__ row_base, const int64_t *__restrict__ chain_row_base,
+                                                            const int64_t *__restrict__ tile_items, int nchunk, int slices,
                                                             int64_t *__restrict__ items, const int64_t *__restrict__ header,
                                                             int64_t cap_items) {
-    // a launch that was enqueued before the host had seen the plan: nothing is written unless the tables are in order
-    // (their entries could point anywhere) and the list has room for every item
-    if (header && (header[VC_HEADER_BAD] != 0 || header[2] > cap_items)) return;
+    // [tiles of the workgroup][VC_EMIT_TILE_ITEMS][stride]: a tile's items, or, in a tile with blocks of many pieces, the routes of
+    // these, [VC_TILE_RANKS][ROUTE], while the whole workgroup writes their items
+    extern __shared__ int64_t tile_lds[];
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
     __shared__ int64_t big_at[VC_THREADS], big_pre[VC_THREADS];
-    // a block of many pieces keeps its route here while the whole workgroup writes its items (routes of more hops than
-    // fit are evaluated again for every piece)
-    const int VC_ROUTE_CACHE = 6;
-    __shared__ int64_t big_dst[VC_THREADS][VC_ROUTE_CACHE];
     __shared__ int big_nhop[VC_THREADS];
-    const int t = blockIdx.x, P = S.P;
+    const int P = S.P, ntile = VC_TILES(P), parts = nchunk * slices, ranks_per_xcd = (P + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS;
+    const int at_xcd = blockIdx.x / VC_PLAN_XCDS, part = at_xcd % parts, t = (int)(blockIdx.x % VC_PLAN_XCDS) * ranks_per_xcd + at_xcd / parts;
+    if (t >= P) return;
     const int stride = VC_CHAIN_HEAD + vc_hop_slots(S);
-    const bool cached = vc_hop_slots(S) <= VC_ROUTE_CACHE;
-    const int chunk = (int)blockIdx.y / slices, z = (int)blockIdx.y % slices;
+    const bool cached = vc_hop_slots(S) <= ROUTE;
+    const int chunk = part / slices, z = part % slices;
     const int c_lo = chunk * VC_THREADS, c_hi = c_lo + VC_THREADS < P ? c_lo + VC_THREADS : P;
-    const int per = ((c_hi - c_lo + slices - 1) / slices + VC_TILE_RANKS - 1) / VC_TILE_RANKS * VC_TILE_RANKS;      // whole tiles
-    const int s_lo = c_lo + z * per < c_hi ? c_lo + z * per : c_hi, s_hi = s_lo + per < c_hi ? s_lo + per : c_hi;
+    const int slice = ((c_hi - c_lo + slices - 1) / slices + VC_TILE_RANKS - 1) / VC_TILE_RANKS * VC_TILE_RANKS;      // whole tiles
+    const int s_lo = c_lo + z * slice < c_hi ? c_lo + z * slice : c_hi, s_hi = s_lo + slice < c_hi ? s_lo + slice : c_hi;
+    if (s_lo >= s_hi) return;
     const int s = s_lo + threadIdx.x;                     // one source per lane: a slice has at most VC_THREADS of them
-    const int64_t cnt = s < s_hi ? vc_chain_count(S, T, s, t) : 0;
-    // the block's first item: the first item of its (receiver, tile of sources) + the items of the tile's earlier sources
-    int64_t upto = cnt;
+    // everything the items depend on is read before any of it is used: the pair's table entries, the slots of its hops (hop
+    // slot k in slot[k], statically indexed), the tile counts below, the header
+    const int64_t header_bad = header ? header[VC_HEADER_BAD] : 0, header_items = header ? header[2] : 0;
+    const int nslots = vc_hop_slots(S), se = s < s_hi ? s : s_lo;
+    const int count = vc_sc(S, T, se, t);
+    const int64_t send_off = vc_send_offset(S, T, se, t), recv_off = vc_recv_offset(S, T, se, t);
+    VcHop hop[ROUTE];
+    int64_t slot_row[ROUTE];
+    uint32_t slot_at[ROUTE];                              // added up later: a sum here would wait for its two reads
+    VcWalk walk = vc_walk_start(S, se, t);
 #pragma unroll
-    for (int o = 1; o < VC_TILE_RANKS; o <<= 1) {
-        const int64_t below = __shfl_up(upto, o, VC_TILE_RANKS);
-        if ((int)(threadIdx.x % VC_TILE_RANKS) >= o) upto += below;
+    for (int k = 0; k < ROUTE; k++) {
+        slot_row[k] = slot_at[k] = 0;
+        hop[k].moves = 0;
+        if (!cached || k >= nslots) continue;
+        hop[k] = vc_walk_step(S, walk, se, t, k);
+        const int region_row = (k == nslots - 1 ? 0 : k) * P;      // (hop slot k's slots lie in region k; the last one has none)
+        slot_row[k] = (row_base + region_row)[(unsigned)(hop[k].row - region_row)];
+        slot_at[k] = (slot_off + (int64_t)region_row * P)[(unsigned)((hop[k].row - region_row) * P + hop[k].id)];
     }
-    const int64_t at = (s < s_hi ? chain_tile_base[(int64_t)t * VC_TILES(P) + s / VC_TILE_RANKS] : 0) + upto - cnt;
-    const bool big = cnt > 4;
-    if (cached && cnt > 0) {
-        // the block's route once, in registers (hop slot k in d[k], statically indexed; its table reads go out together); the
-        // pieces of a block of few pieces are then arithmetic and stores only — evaluating the route again for every piece
-        // was a chain of dependent reads per item
-        int64_t d[VC_ROUTE_CACHE];
-        unsigned moves = 0;
-        const int nslots = vc_hop_slots(S);
+    // first item of each of the workgroup's tiles: the items of all receivers before the tile row, of the tile row's tiles of
+    // earlier sources, and of the receivers before t in the tile
+    const int t0 = t / VC_TILE_RANKS * VC_TILE_RANKS, sb0 = s_lo / VC_TILE_RANKS, tiles = (s_hi - s_lo + VC_TILE_RANKS - 1) / VC_TILE_RANKS;
+    constexpr int COLS = VC_THREADS / VC_TILE_RANKS;      // 8 tiles at most, a thread per (receiver of the tile row, tile)
+    __shared__ int64_t share[VC_WAVES_PER_BLOCK][COLS];   // what a wavefront's receivers have before each of the workgroup's tiles
+    const int64_t row_first = chain_row_base[t0];
+    {
+        const int row = threadIdx.x / COLS, col = threadIdx.x % COLS, lane = threadIdx.x % VC_WAVE;
+        const bool there = t0 + row < P;
+        const int64_t *of_row = tile_items + (int64_t)(t0 + row) * ntile;
+        const int64_t here = there && col < tiles ? of_row[sb0 + col] : 0;
+        int64_t earlier = 0;                              // (only with more than VC_THREADS ranks)
+        for (int sb = col; sb < sb0; sb += COLS) earlier += there ? of_row[sb] : 0;
+        int64_t whole = here, mine = t0 + row < t ? here : 0;
 #pragma unroll
-        for (int k = 0; k < VC_ROUTE_CACHE; k++) {
-            d[k] = 0;
-            if (k < nslots && vc_block_hop(S, T, slot_off, row_base, s, t, k, d[k])) moves |= 1u << k;
+        for (int o = COLS; o < VC_WAVE; o <<= 1) {
+            whole += __shfl_xor(whole, o, VC_WAVE);
+            mine += __shfl_xor(mine, o, VC_WAVE);
+            earlier += __shfl_xor(earlier, o, VC_WAVE);
+        }
+#pragma unroll
+        for (int o = 1; o < COLS; o <<= 1) earlier += __shfl_xor(earlier, o, VC_WAVE);
+        // lanes 0 .. COLS - 1: the tiles of the earlier columns
+        int64_t before = vc_dpp_add<VC_DPP_SHR(1), 0xf>(whole);
+        before = vc_dpp_add<VC_DPP_SHR(2), 0xf>(before);
+        before = vc_dpp_add<VC_DPP_SHR(4), 0xf>(before) - whole;
+        if (lane < COLS) share[threadIdx.x / VC_WAVE][lane] = before + mine + earlier;
+    }
+    __syncthreads();
+    // a launch that was enqueued before the host had seen the plan: nothing is written unless the tables are in order
+    // (their entries could point anywhere) and the list has room for every item
+    if (header && (header_bad != 0 || header_items > cap_items)) return;
+    const int64_t len = (int64_t)count * S.esz;
+    const int cut = (int)((recv_off + S.recv_lo) & (VC_PIECE - 1)), phase = cut & (VC_LINE - 1);
+    const int64_t cnt = s < s_hi ? vc_chunk_count(len, phase, cut) : 0;
+    const int tile = threadIdx.x / VC_TILE_RANKS, lane_in_tile = threadIdx.x % VC_TILE_RANKS;
+    const int64_t upto = vc_half_inclusive_scan(cnt), in_tile = __shfl(upto, VC_TILE_RANKS - 1, VC_TILE_RANKS);
+    int64_t first = row_first;                            // the first item of the lane's tile
+#pragma unroll
+    for (int q = 0; q < VC_WAVES_PER_BLOCK; q++) first += share[q][tile];
+    const int64_t at = first + upto - cnt;
+    const bool big = cnt > 4;
+    const bool any_big = (__ballot(big) >> (threadIdx.x % VC_WAVE / VC_TILE_RANKS * VC_TILE_RANKS) & 0xFFFFFFFFull) != 0;
+    const bool together = cached && !any_big && in_tile <= VC_EMIT_TILE_ITEMS;
+    int64_t *const tile_buf = tile_lds + (int64_t)tile * VC_EMIT_TILE_ITEMS * stride;
+    if (cached && cnt > 0) {
+        int64_t d[ROUTE];
+        unsigned moves = 0;
+#pragma unroll
+        for (int k = 0; k < ROUTE; k++) {
+            d[k] = vc_hop_dst(S, hop[k], slot_row[k] + vc_slot_bytes(slot_at[k]), recv_off);
+            moves |= hop[k].moves ? 1u << k : 0u;
         }
         const int nhop = __popc(moves);
         if (!big) {
-            const int64_t src = VC_SPACE_SEND | vc_send_offset(S, T, s, t), len = (int64_t)vc_sc(S, T, s, t) * S.esz;
-            const int phase = vc_phase(S, T, s, t), cut = vc_chain_cut(S, T, s, t);
+            const int64_t src = VC_SPACE_SEND | send_off;
             for (int64_t c = 0; c < cnt; c++) {
                 int64_t lo, hi;
                 vc_piece_range(len, phase, cut, c, lo, hi);
-                int64_t *item = items + (at + c) * stride;
+                int64_t *item = together ? tile_buf + (upto - cnt + c) * stride : items + (at + c) * stride;
                 item[VC_CHAIN_SRC] = src + lo;
                 item[VC_CHAIN_LEN] = hi - lo;
                 item[VC_CHAIN_NHOP] = nhop;
                 int n = 0;
 #pragma unroll
-                for (int k = 0; k < VC_ROUTE_CACHE; k++)
+                for (int k = 0; k < ROUTE; k++)
                     if (moves >> k & 1) item[VC_CHAIN_HEAD + n++] = d[k] + lo;
             }
         } else {
@@ -513,15 +655,18 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
             big_nhop[threadIdx.x] = nhop;
             int n = 0;
 #pragma unroll
-            for (int k = 0; k < VC_ROUTE_CACHE; k++)
-                if (moves >> k & 1) big_dst[threadIdx.x][n++] = d[k];
+            for (int k = 0; k < ROUTE; k++)
+                if (moves >> k & 1) tile_buf[lane_in_tile * ROUTE + n++] = d[k];
         }
     } else if (!big) {
         for (int64_t c = 0; c < cnt; c++) vc_chain_item(S, T, slot_off, row_base, s, t, c, items + (at + c) * stride);
     } else {
         big_at[threadIdx.x] = at;
     }
-    if (__syncthreads_or(big)) {
+    const bool wg_big = __syncthreads_or(big);            // (also: the tiles in LDS are complete)
+    if (together)
+        for (int k = lane_in_tile; k < (int)in_tile * stride; k += VC_TILE_RANKS) items[first * stride + k] = tile_buf[k];
+    if (wg_big) {
         int64_t btotal;
         big_pre[threadIdx.x] = vc_block_exclusive_scan(big ? cnt : 0, lds, btotal);
         __syncthreads();
@@ -535,23 +680,28 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
             const int sb = s_lo + lo;
             if (cached)
                 vc_chain_piece(VC_SPACE_SEND | vc_send_offset(S, T, sb, t), (int64_t)vc_sc(S, T, sb, t) * S.esz, vc_phase(S, T, sb, t),
-                               vc_chain_cut(S, T, sb, t), c, big_dst[lo], big_nhop[lo], items + (big_at[lo] + c) * stride);
+                               vc_chain_cut(S, T, sb, t), c,
+                               tile_lds + (int64_t)(lo / VC_TILE_RANKS) * VC_EMIT_TILE_ITEMS * stride + lo % VC_TILE_RANKS * ROUTE, big_nhop[lo],
+                               items + (big_at[lo] + c) * stride);
             else
                 vc_chain_item(S, T, slot_off, row_base, sb, t, c, items + (big_at[lo] + c) * stride);
         }
     }
 }
 
-hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const int64_t *slot_off, const int64_t *row_base,
-                                const int64_t *chain_tile_base, int64_t *items, int64_t nitems, hipStream_t st, const int64_t *header,
-                                int64_t cap_items) {
+hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base,
+                                const int64_t *chain_row_base, const int64_t *chain_row_tot, int64_t *items, int64_t nitems, hipStream_t st,
+                                const int64_t *header, int64_t cap_items) {
     const int nchunk = (S.P + VC_THREADS - 1) / VC_THREADS;
     // at least ~1024 workgroups (four per compute unit), each a whole number of tiles of sources
     int slices = nchunk > 1 ? 1 : vc_emit_slices(nitems, S.P);
     if (nchunk == 1)
         while (slices < 8 && (int64_t)S.P * slices < 1024 && S.P / (slices * 2) >= VC_TILE_RANKS) slices *= 2;
-    hipLaunchKernelGGL(vc_chain_emit, dim3(S.P, nchunk * slices), dim3(VC_THREADS), 0, st, S, T, slot_off, row_base, chain_tile_base,
-                       slices, items, header, cap_items);
+    const int stride = VC_CHAIN_HEAD + vc_hop_slots(S), tiles = (std::min(S.P, VC_THREADS) + VC_TILE_RANKS - 1) / VC_TILE_RANKS;
+    const size_t lds = vc_hop_slots(S) <= VC_ROUTE_CACHE ? sizeof(int64_t) * tiles * VC_EMIT_TILE_ITEMS * stride : 0;
+    const auto kernel = vc_hop_slots(S) <= 3 ? vc_chain_emit<3> : vc_chain_emit<VC_ROUTE_CACHE>;
+    hipLaunchKernelGGL(kernel, dim3(vc_rank_grid(S.P, nchunk * slices)), dim3(VC_THREADS), lds, st, S, T, slot_off, row_base, chain_row_base,
+                       chain_row_tot + 2 * (size_t)S.P, nchunk, slices, items, header, cap_items);
     return hipGetLastError();
 }
 

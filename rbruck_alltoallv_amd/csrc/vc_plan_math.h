@@ -19,13 +19,13 @@ struct VcBlock {
     bool to_org;     // ... in its organized region (last intra-node hop of a block that still has to change node)
 };
 
-VC_HD int vc_top_digit(int v, const VcDivisor &r) {     // position of the highest non-zero digit, v > 0
+VC_HD int vc_top_digit(int v, const VcRankDivisor &r) {     // position of the highest non-zero digit, v > 0
     int x = -1;
     while (v) { v = vc_div(v, r); x++; }
     return x;
 }
 
-VC_HD int vc_low_digit(int v, const VcDivisor &r) {     // position of the lowest non-zero digit, v > 0
+VC_HD int vc_low_digit(int v, const VcRankDivisor &r) {     // position of the lowest non-zero digit, v > 0
     int x = 0;
     for (;;) {
         const int q = vc_div(v, r);
@@ -125,12 +125,15 @@ VC_HD bool vc_inter_block(const VcSched &S, int x, int dist, int to, int id, VcE
 
 // Entries of the tables: what rank s sends to rank t, what rank t expects from rank s, and where, in elements.  (Ranks are
 // at most 32768: an index fits 30 bits.)
-VC_HD int vc_sc(const VcSched &S, const VcTables &T, int s, int t) { return (T.sc[(unsigned)((s * S.P + t) & S.table_mask)] & S.table_mask) + S.uniform; }
-VC_HD int vc_sd(const VcSched &S, const VcTables &T, int s, int t) { return (T.sd[(unsigned)((s * S.P + t) & S.table_mask)] & S.table_mask) + t * S.uniform; }
-VC_HD int vc_rc(const VcSched &S, const VcTables &T, int t, int s) { return (T.rc[(unsigned)((t * S.P + s) & S.table_mask)] & S.table_mask) + S.uniform; }
-VC_HD int vc_rd(const VcSched &S, const VcTables &T, int t, int s) {
-    return ((S.packed_recv ? T.rd_packed : T.rd)[(unsigned)((t * S.P + s) & S.table_mask)] & S.table_mask) + s * S.uniform;
+// The offsets are 32-bit bytes: a scalar base and one register for the address.
+VC_HD int vc_entry(const int *table, const VcSched &S, int row, int col) {
+    const unsigned at = (unsigned)(((row * S.P + col) & S.table_mask) << 2);
+    return *reinterpret_cast<const int *>(reinterpret_cast<const char *>(table) + at) & S.table_mask;
 }
+VC_HD int vc_sc(const VcSched &S, const VcTables &T, int s, int t) { return vc_entry(T.sc, S, s, t) + S.uniform; }
+VC_HD int vc_sd(const VcSched &S, const VcTables &T, int s, int t) { return vc_entry(T.sd, S, s, t) + t * S.uniform; }
+VC_HD int vc_rc(const VcSched &S, const VcTables &T, int t, int s) { return vc_entry(T.rc, S, t, s) + S.uniform; }
+VC_HD int vc_rd(const VcSched &S, const VcTables &T, int t, int s) { return vc_entry(S.packed_recv ? T.rd_packed : T.rd, S, t, s) + s * S.uniform; }
 
 VC_HD int64_t vc_recv_offset(const VcSched &S, const VcTables &T, int s, int t) {
     return T.rbase[t] + (int64_t)vc_rd(S, T, t, s) * S.esz;
@@ -175,6 +178,28 @@ VC_HD int64_t vc_region_slot_size(const VcSched &S, const VcTables &T, int y, in
     const int64_t len = (int64_t)vc_sc(S, T, e.s, e.t) * S.esz;
     if (data_len) *data_len = len;
     return len ? ((len + vc_phase(S, T, e.s, e.t) + VC_LINE - 1) & ~(int64_t)(VC_LINE - 1)) : 0;
+}
+
+// Forwarded execution: the block (s, t) that staging region y keeps in slot `id` of rank `to`, if any (no organized region).  s
+// and t are ranks in any case, so that a kernel can read the tables for many slots at once without waiting to know which
+// of them are used: no branches here, and no reads.
+VC_HD bool vc_slot_block(const VcSched &S, int y, int to, int id, int &s, int &t) {
+    const int n = S.n, G = S.G;
+    const int gto = vc_div(to, S.dn), lr = to - gto * n, gid = vc_div(id, S.dn), lid = id - gid * n;
+    const bool intra = y < S.w;
+    // the block's offset inside the node / between the nodes, and where its holder stands among the ranks / nodes of that span
+    const int x = intra ? y : y - S.w, span = intra ? n : G;
+    const int j = intra ? vc_wrap(lid - lr + n, n) : gid, pos = intra ? lr : gto;
+    int dist;
+    const int upper = vc_upper_digits(S, j, x, span, dist), higher = vc_div(upper, S.dr), z = upper - higher * S.r;
+    const bool msd = intra && S.msd;
+    // z dist <= j < span ranks above the holder is the sender, `above` ranks above that one the source
+    const int above = msd ? higher * (dist * S.r) : j - upper * dist;
+    const bool last = msd ? upper * dist == j : higher == 0;
+    const int from = vc_wrap(pos + z * dist, span), src = vc_wrap(from + above, span), dst = vc_wrap(src - j + span, span);
+    s = intra ? gto * n + src : src * n + lid;
+    t = intra ? gid * n + dst : dst * n + lr;
+    return z != 0 && !(last && (!intra || gid == gto));
 }
 
 // Address (inside the staging arena) of the data of block (s, t) while it sits in slot `id`
@@ -424,11 +449,22 @@ VC_HD int64_t vc_chain_count(const VcSched &S, const VcTables &T, int s, int t) 
 // expect exactly what the source sends (the reference fails with an MPI truncation error), and no count or displacement
 // of the receiver's own row may be negative.  Summed over all pairs this is header word VC_HEADER_BAD, whoever adds it
 // up (the planner's row kernel, or the copy kernel that plans nothing).
-VC_HD int vc_pair_bad_entries(const VcSched &S, const VcTables &T, int s, int t) {
-    const int expected = vc_rc(S, T, t, s), sent = vc_sc(S, T, s, t);
-    const int rd = S.packed_recv ? 0 : vc_rd(S, T, t, s);
-    return (expected != sent) + ((vc_sc(S, T, t, s) | vc_sd(S, T, t, s) | expected | rd) < 0);
+struct VcPairEntries { int sent, expected, rd, own; };      // own: negative when an entry of the receiver's row is
+
+VC_HD VcPairEntries vc_pair_entries(const VcSched &S, const VcTables &T, int s, int t) {
+    VcPairEntries e;
+    e.sent = vc_sc(S, T, s, t);
+    e.expected = vc_rc(S, T, t, s);
+    e.rd = vc_rd(S, T, t, s);
+    e.own = vc_sc(S, T, t, s) | vc_sd(S, T, t, s);
+    return e;
 }
+
+VC_HD int vc_bad_entries(const VcSched &S, const VcPairEntries &e) {
+    return (e.expected != e.sent) + ((e.own | e.expected | (S.packed_recv ? 0 : e.rd)) < 0);
+}
+
+VC_HD int vc_pair_bad_entries(const VcSched &S, const VcTables &T, int s, int t) { return vc_bad_entries(S, vc_pair_entries(S, T, s, t)); }
 
 // Layout of a chain item, in int64 words; `stride` = VC_CHAIN_HEAD + hop slots of the call.
 #define VC_CHAIN_SRC 0    // space-tagged source offset of the piece (always in sendbuf)
@@ -549,30 +585,78 @@ VC_HD int vc_recycle_rows_per_segment(int P) { return (P + VC_RECYCLE_SEGMENTS -
 // significant first (offset div r^x) * r^x; it sits in slot (destination group) * n + (local offset + local rank) % n
 // of its holder (src/twophase_twolayer_rbruck.cpp:322), and lands in recvbuf when no digit is left and it is on its
 // destination's node.  The CPU check of the plan compares this with what the launches' entries say, block by block.
-VC_HD bool vc_block_hop(const VcSched &S, const VcTables &T, const int64_t *slot_off, const int64_t *row_base, int s, int t, int k,
-                        int64_t &dst) {
-    const int n = S.n, G = S.G, final_slot = S.w + S.w2;
-    const int64_t to_recv = VC_SPACE_RECV | vc_recv_offset(S, T, s, t);
-    if (s == t) { dst = to_recv; return k == final_slot; }
-    const int gs = vc_div(s, S.dn), gt = vc_div(t, S.dn), ls = s - gs * n, lt = t - gt * n;
-    if (k == final_slot) { dst = to_recv; return S.last_hop == 2 || (S.last_hop == 1 && gs != gt); }
-    const bool intra = k < S.w;
-    const int x = intra ? k : k - S.w;
+// Two steps, so that a kernel can work out several hops and read the tables for all of them together: where the hop goes
+// (arithmetic without branches; `row` and `id` name an existing slot also when the block does not move or goes to
+// recvbuf), then its address.
+struct VcHop {
+    int moves;       // the block moves in this slot
+    int staged;      // ... into slot `id` of staging row `row` (else into recvbuf)
+    int row, id;     // row = region * P + holder
+};
+
+// Hop slot after hop slot of one block, slot 0 first: one division by the radix each.
+struct VcWalk { int gs, gt, ls, lt, upper, dist; };
+
+VC_HD VcWalk vc_walk_start(const VcSched &S, int s, int t) {
+    VcWalk w;
+    w.gs = vc_div(s, S.dn); w.gt = vc_div(t, S.dn); w.ls = s - w.gs * S.n; w.lt = t - w.gt * S.n;
+    w.upper = vc_wrap(w.ls - w.lt + S.n, S.n);
+    w.dist = 1;
+    return w;
+}
+
+VC_HD VcHop vc_walk_step(const VcSched &S, VcWalk &w, int s, int t, int k) {
+    const int n = S.n, G = S.G;
+    const bool intra = k < S.w, final = k == S.w + S.w2;
     const int span = intra ? n : G;
-    const int j = intra ? vc_wrap(ls - lt + n, n) : vc_wrap(gs - gt + G, G);      // offset inside the node / between the nodes
-    int dist;
-    const int upper = vc_upper_digits(S, j, x, span, dist);       // the digits from x upwards
-    if (dist >= span) return false;
-    const int higher = vc_div(upper, S.dr);                       // ... from x + 1 upwards
-    if (upper == higher * S.r) return false;
+    const int j = intra ? vc_wrap(w.ls - w.lt + n, n) : vc_wrap(w.gs - w.gt + G, G);      // offset inside the node / between the nodes
+    if (k == S.w) { w.upper = j; w.dist = 1; }
+    const int upper = w.upper;                                    // the digits from k's upwards
+    const int higher = vc_div(upper, S.dr);                       // ... above k's
     const bool msd = intra && S.msd;
-    const int travelled = msd ? upper * dist : j - higher * dist * S.r;           // at most j < span
-    const bool last = msd ? upper * dist == j : higher == 0;
-    const int pos = vc_wrap((intra ? ls : gs) - travelled + span, span);            // local rank / node of the holder after the hop
-    const int to = intra ? gs * n + pos : pos * n + lt;
-    const int id = intra ? gt * n + vc_wrap(j + pos, n) : j * n + ls;
-    dst = (last && (intra ? gs == gt : true)) ? to_recv : (VC_SPACE_STAGE | vc_stage_addr(S, T, slot_off, row_base, k, to, id, s, t));
-    return true;
+    const int travelled = msd ? upper * w.dist : j - higher * w.dist * S.r;       // at most j < span
+    const bool last = msd ? upper * w.dist == j : higher == 0;
+    const int pos = vc_wrap((intra ? w.ls : w.gs) - travelled + span, span);        // local rank / node of the holder after the hop
+    const int to = intra ? w.gs * n + pos : pos * n + w.lt;
+    w.upper = higher;
+    if (!final) w.dist *= S.r;
+    VcHop h;
+    h.moves = final ? (s == t || S.last_hop == 2 || (S.last_hop == 1 && w.gs != w.gt)) : (s != t && upper != higher * S.r);
+    h.staged = !final && !(last && (!intra || w.gs == w.gt));
+    h.row = (final ? 0 : k) * S.P + to;
+    h.id = intra ? w.gt * n + vc_wrap(j + pos, n) : j * n + w.ls;
+    return h;
+}
+
+VC_HD VcHop vc_hop_place(const VcSched &S, int s, int t, int k) {
+    VcWalk w = vc_walk_start(S, s, t);
+    if (k >= S.w) w.upper = vc_wrap(w.gs - w.gt + S.G, S.G);
+    w.upper = vc_upper_digits(S, w.upper, k < S.w ? k : k - S.w, k < S.w ? S.n : S.G, w.dist);
+    return vc_walk_step(S, w, s, t, k);
+}
+
+// Address of the slot a hop goes to: a read of two plan tables, or a closed form with fixed-stride staging.  A forwarded plan
+// keeps the slots' places inside their rows in units of VC_LINE, 32 bits (a row of 2^32 lines is more than there is memory).
+VC_HD int64_t vc_slot_bytes(int64_t off) { return off; }
+VC_HD int64_t vc_slot_bytes(uint32_t lines) { return (int64_t)lines * VC_LINE; }
+
+template <class Slot>
+VC_HD int64_t vc_slot_addr(const VcSched &S, const Slot *slot_off, const int64_t *row_base, const VcHop &h) {
+    if (S.stride) return ((int64_t)h.row * S.P + h.id) * S.stride;
+    return row_base[h.row] + vc_slot_bytes(slot_off[(int64_t)h.row * S.P + h.id]);
+}
+
+// Destination of a hop: recv_off = vc_recv_offset(S, T, s, t).
+VC_HD int64_t vc_hop_dst(const VcSched &S, const VcHop &h, int64_t slot_addr, int64_t recv_off) {
+    return h.staged ? (VC_SPACE_STAGE | (slot_addr + ((recv_off + S.recv_lo) & (VC_LINE - 1)))) : (VC_SPACE_RECV | recv_off);
+}
+
+template <class Slot>
+VC_HD bool vc_block_hop(const VcSched &S, const VcTables &T, const Slot *slot_off, const int64_t *row_base, int s, int t, int k,
+                        int64_t &dst) {
+    const VcHop h = vc_hop_place(S, s, t, k);
+    dst = vc_hop_dst(S, h, h.moves && h.staged ? vc_slot_addr(S, slot_off, row_base, h) : 0, vc_recv_offset(S, T, s, t));
+    return h.moves != 0;
 }
 
 // Piece c of a block whose source and hop destinations (whole block) are known.
@@ -587,7 +671,8 @@ VC_HD void vc_chain_piece(int64_t src, int64_t len, int phase, int cut, int64_t 
 }
 
 // Hop destinations of block (s, t) in slot order; returns their number.
-VC_HD int vc_chain_route(const VcSched &S, const VcTables &T, const int64_t *slot_off, const int64_t *row_base, int s, int t,
+template <class Slot>
+VC_HD int vc_chain_route(const VcSched &S, const VcTables &T, const Slot *slot_off, const int64_t *row_base, int s, int t,
                          int64_t *dst) {
     int nhop = 0;
     const int nslots = vc_hop_slots(S);
@@ -599,7 +684,8 @@ VC_HD int vc_chain_route(const VcSched &S, const VcTables &T, const int64_t *slo
 }
 
 // Writes piece c of block (s, t) to `item`.
-VC_HD void vc_chain_item(const VcSched &S, const VcTables &T, const int64_t *slot_off, const int64_t *row_base, int s, int t, int64_t c,
+template <class Slot>
+VC_HD void vc_chain_item(const VcSched &S, const VcTables &T, const Slot *slot_off, const int64_t *row_base, int s, int t, int64_t c,
                          int64_t *item) {
     const int64_t len = (int64_t)vc_sc(S, T, s, t) * S.esz;
     const int nhop = vc_chain_route(S, T, slot_off, row_base, s, t, item + VC_CHAIN_HEAD);   // whole-block destinations first

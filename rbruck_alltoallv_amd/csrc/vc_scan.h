@@ -9,15 +9,47 @@
 #define VC_WAVE 64
 #define VC_WAVES_PER_BLOCK (VC_THREADS / VC_WAVE)
 
-// Inclusive prefix sum across the 64 lanes of a wavefront.
-__device__ __forceinline__ int64_t vc_wave_inclusive_scan(int64_t v) {
-    const int lane = threadIdx.x & (VC_WAVE - 1);
-#pragma unroll
-    for (int o = 1; o < VC_WAVE; o <<= 1) {
-        int64_t u = __shfl_up(v, o, VC_WAVE);
-        if (lane >= o) v += u;
-    }
-    return v;
+// One step of a sum over lanes by data-parallel primitives: v plus the value CTRL fetches from another lane (0 for lanes it
+// gives none, and in the rows of 16 lanes ROWS leaves out).  A few cycles; a lane exchange through LDS is about a hundred.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int64_t vc_dpp_add(int64_t v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+    return v + (((int64_t)hi << 32) | (unsigned)lo);
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int64_t vc_dpp_max(int64_t v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, false);
+    const int64_t u = ((int64_t)hi << 32) | (unsigned)lo;
+    return u > v ? u : v;
+}
+
+#define VC_DPP_SHR(n) (0x110 | (n))           // from n lanes below, inside a row of 16
+#define VC_DPP_BCAST15 0x142                  // last lane of a row to the next row
+#define VC_DPP_BCAST31 0x143                  // lane 31 to the upper half
+
+// Inclusive prefix sum across each half (32 lanes) of a wavefront.
+__device__ __forceinline__ int64_t vc_half_inclusive_scan(int64_t v) {
+    v = vc_dpp_add<VC_DPP_SHR(1), 0xf>(v);
+    v = vc_dpp_add<VC_DPP_SHR(2), 0xf>(v);
+    v = vc_dpp_add<VC_DPP_SHR(4), 0xf>(v);
+    v = vc_dpp_add<VC_DPP_SHR(8), 0xf>(v);
+    return vc_dpp_add<VC_DPP_BCAST15, 0xa>(v);
+}
+
+// Inclusive prefix sum across the 64 lanes of a wavefront (lane 63: the sum of all).
+__device__ __forceinline__ int64_t vc_wave_inclusive_scan(int64_t v) { return vc_dpp_add<VC_DPP_BCAST31, 0xc>(vc_half_inclusive_scan(v)); }
+
+// Lane 63 receives the maximum of the wavefront's values, none of them negative.
+__device__ __forceinline__ int64_t vc_wave_max_last(int64_t v) {
+    v = vc_dpp_max<VC_DPP_SHR(1), 0xf>(v);
+    v = vc_dpp_max<VC_DPP_SHR(2), 0xf>(v);
+    v = vc_dpp_max<VC_DPP_SHR(4), 0xf>(v);
+    v = vc_dpp_max<VC_DPP_SHR(8), 0xf>(v);
+    v = vc_dpp_max<VC_DPP_BCAST15, 0xa>(v);
+    return vc_dpp_max<VC_DPP_BCAST31, 0xc>(v);
 }
 
 // Exclusive prefix sum across a 256-thread workgroup; `total` receives the sum of all
@@ -61,4 +93,26 @@ __device__ __forceinline__ int64_t vc_block_max(int64_t v, int64_t *lds) {
 #pragma unroll
     for (int k = 1; k < VC_WAVES_PER_BLOCK; k++) m = lds[k] > m ? lds[k] : m;
     return m;
+}
+
+// Five totals of a 256-thread workgroup at once (one barrier): sums of v[0], v[1], v[2], maxima of v[3], v[4] (not negative).
+// Thread 0 receives them; lds holds 5 * VC_WAVES_PER_BLOCK int64.
+__device__ __forceinline__ void vc_block_totals(int64_t v[5], int64_t *lds) {
+    const int wave = threadIdx.x / VC_WAVE;
+#pragma unroll
+    for (int k = 0; k < 5; k++) v[k] = k < 3 ? vc_wave_inclusive_scan(v[k]) : vc_wave_max_last(v[k]);
+    if ((threadIdx.x & (VC_WAVE - 1)) == VC_WAVE - 1)
+#pragma unroll
+        for (int k = 0; k < 5; k++) lds[k * VC_WAVES_PER_BLOCK + wave] = v[k];
+    __syncthreads();
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+            v[k] = lds[k * VC_WAVES_PER_BLOCK];
+#pragma unroll
+            for (int q = 1; q < VC_WAVES_PER_BLOCK; q++) {
+                const int64_t u = lds[k * VC_WAVES_PER_BLOCK + q];
+                v[k] = k < 3 ? v[k] + u : (u > v[k] ? u : v[k]);
+            }
+        }
 }

@@ -28,7 +28,7 @@ extern "C" int rank_division_mismatches(int d_lo, int d_hi) {
 extern "C" int route_mismatches(int func, int P, int n, int r) {
     VcSched S;
     std::vector<VcLaunchInfo> L;
-    if (vc_make_schedule((VcFunc)func, P, n, r, 0, 1, 0, S, L, 0, true)) return -1;
+    if (vc_make_schedule((VcFunc)func, P, n, r, 0, 1, func == VC_F_UNIFORM_SPREADOUT || func == VC_F_UNIFORM_ISPLIT, S, L, 0, true)) return -1;
     std::vector<int> one((size_t)P * P, 1), zero((size_t)P * P, 0);
     std::vector<int64_t> base(P, 0);
     VcTables T = {one.data(), zero.data(), one.data(), zero.data(), base.data(), base.data(), zero.data()};

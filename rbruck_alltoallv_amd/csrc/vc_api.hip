@@ -44,7 +44,7 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
             if (e == hipSuccess) g_scratch_ptr[c->device] = static_cast<unsigned char *>(ptr);
         }
     }
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_header, sizeof(int64_t) * VC_HEADER_WORDS(VC_MAX_LAUNCHES), hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_header, sizeof(int64_t) * VC_HEADER_ROOM, hipHostMallocCoherent);
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_header_dev, c->h_header, 0);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_launches, sizeof(VcLaunchInfo) * VC_MAX_LAUNCHES, hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, VC_FLAG_WORDS * sizeof(int), hipHostMallocCoherent);
@@ -64,7 +64,7 @@ extern "C" int vc_comm_free(vc_comm_t c) {
     (void)hipStreamSynchronize(c->stream);
     c->pending.active = false;
     for (DevBuf *b : {&c->slot_off, &c->row_tot, &c->row_base, &c->org_run_base, &c->item_row_tot, &c->item_row_base, &c->row_bytes, &c->desc, &c->header, &c->launches, &c->stage, &c->rd_packed,
-                      &c->scratch, &c->max_state, &c->ticket, &c->chain_row_tot, &c->chain_row_base, &c->strided_headers})
+                      &c->scratch, &c->max_state, &c->ticket, &c->chain_row_tot, &c->chain_row_base, &c->verdicts})
         b->release();
     free_retired_stage(c);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
@@ -447,21 +447,19 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     S.stride = d.stride;
     const int64_t need = vc_strided_stage_bytes(S);
     hipStream_t st = c->stream;
-    // two headers in turn: the planner adds up into one (with atomics, so it must start from zero) while the copy kernel
-    // clears the other one for the next call
-    const size_t header_bytes = sizeof(int64_t) * 16;
-    if (!c->strided_headers.p) {
-        HIP_TRY(c->strided_headers.reserve(2 * header_bytes));
-        c->strided_clean = false;
+    // two sets of words in turn: a launch counts in one, which must start from zero, and clears the other one for the next call
+    if (!c->verdicts.p) {
+        HIP_TRY(c->verdicts.reserve(2 * VC_VERDICTS * VC_LINE));
+        c->verdict_clean = false;
     }
     HIP_TRY(reserve_stage(c, (size_t)need + 64));
     if (S.packed_recv) HIP_TRY(c->rd_packed.reserve(sizeof(int) * (size_t)S.P * S.P));
     if (c->timing) { int rc = ensure_events(c, 5); if (rc) return rc; HIP_TRY(hipEventRecord(c->events[0], st)); }
-    if (!c->strided_clean) HIP_TRY(hipMemsetAsync(c->strided_headers.p, 0, 2 * header_bytes, st));
-    c->strided_clean = false;                             // until the copy kernel that clears the other header is enqueued
-    int64_t *header = c->strided_headers.as<int64_t>() + (c->strided_turn ? 16 : 0);
-    int64_t *header_next = c->strided_headers.as<int64_t>() + (c->strided_turn ? 0 : 16);
-    c->strided_turn ^= 1;
+    if (!c->verdict_clean) HIP_TRY(hipMemsetAsync(c->verdicts.p, 0, 2 * VC_VERDICTS * VC_LINE, st));
+    c->verdict_clean = false;                             // until the kernel that clears the other set is enqueued
+    unsigned long long *verdict = c->verdicts.as<unsigned long long>() + (c->verdict_turn ? VC_VERDICTS * VC_LINE / 8 : 0);
+    unsigned long long *verdict_next = c->verdicts.as<unsigned long long>() + (c->verdict_turn ? 0 : VC_VERDICTS * VC_LINE / 8);
+    c->verdict_turn ^= 1;
     if (S.packed_recv) {
         HIP_TRY(vc_launch_row_scan(T.rc, c->rd_packed.as<int>(), nullptr, nullptr, S.P, st));
         T.rd_packed = c->rd_packed.as<int>();
@@ -469,19 +467,29 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     VcListlessGuard guard = d.guard;
     guard.stage_cap = (int64_t)c->stage.cap - 64;
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
-    c->h_header[VC_HEADER_STALLED] = 0;
-    // the one launch of the call: its first wavefronts check the tables and add their totals up into `header`; every pair
+    int64_t *totals = c->h_header + VC_TOTALS_AT;
+    totals[VC_TOTALS_STALLED] = 0;
+    // the one launch of the call: its first wavefronts check the tables and leave their totals in host memory; every pair
     // checks its own entries and the length of its block before it forms an address, and stores nothing before all of
     // the tables have been found in order
-    HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, header, guard, pair_lanes, sendbuf, recvbuf, c->stage.as<char>(), st, c->h_header_dev,
-                                  header_next, header));
-    c->strided_clean = true;
+    HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, nullptr, guard, pair_lanes, sendbuf, recvbuf, c->stage.as<char>(), st, verdict, verdict_next,
+                                  c->h_header_dev + VC_TOTALS_AT));
+    c->verdict_clean = true;
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     HIP_TRY(VC_WAIT(c));
+    int64_t *h = c->h_header;
+    for (int k = 0; k <= VC_HEADER_MAX_LEN; k++) h[k] = 0;
+    for (int64_t w = 0; w < vc_totals_waves(S.P); w++) {
+        const int64_t *slot = totals + w * VC_TOTALS_SLOT;
+        h[1] += slot[VC_TOTALS_PAYLOAD]; h[2] += slot[VC_TOTALS_ITEMS]; h[VC_HEADER_BAD] += slot[VC_TOTALS_BAD]; h[VC_HEADER_FIXED] += slot[VC_TOTALS_MOVED];
+        h[VC_HEADER_MAX_PIECES] = std::max(h[VC_HEADER_MAX_PIECES], slot[VC_TOTALS_MOST]);
+        h[VC_HEADER_MAX_LEN] = std::max(h[VC_HEADER_MAX_LEN], slot[VC_TOTALS_LONGEST]);
+    }
+    h[0] = need;
     PlanInfo pi;
     int rc = plan_read(c, S, L, pi, true);
     if (rc) return rc;
-    if (c->h_header[VC_HEADER_STALLED]) return 0;          // a copying wavefront gave up waiting for the verdict and moved nothing
+    if (totals[VC_TOTALS_STALLED]) return 0;          // a copying wavefront gave up waiting for the verdict and moved nothing
     if (!vc_listless_ok(c->h_header, guard)) return 0;     // longer blocks than the last call's, or not a call for this kernel
     pi.listless = pi.strided = true;
     pi.chain_lanes = pair_lanes;

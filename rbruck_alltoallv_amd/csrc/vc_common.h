@@ -209,14 +209,17 @@ hipError_t vc_launch_done(unsigned *word, unsigned value, hipStream_t st);
 // added to header[VC_HEADER_BAD] once per rank whose packed receive displacements would pass INT_MAX elements
 #define VC_BAD_OVERFLOW (1ll << 40)
 #define VC_HEADER_MAX_PIECES 4
-// fixed-stride staging: wavefronts that have added their part of the tables' totals into the header
-#define VC_HEADER_SYNC (VC_HEADER_MAX_LEN + 1)
-// ... wavefronts that have checked their part of the tables and added what they found to VC_HEADER_BAD: the copying
-// wavefronts of the same launch store nothing before all of them have
-#define VC_HEADER_CHECKED (VC_HEADER_SYNC + 1)
-// ... set (in the host's copy of the header only) by a copying wavefront that gave up waiting for that: the call is redone
-#define VC_HEADER_STALLED (VC_HEADER_SYNC + 2)
 #define VC_HEADER_WORDS(nl) (VC_HEADER_FIXED + 2 * (nl))
+// Fixed-stride staging: the totals of a call on P ranks are added up by vc_totals_waves(P) wavefronts, four pairs a lane, each leaving
+// a slot (a cache line) in host memory.
+#define VC_TOTALS_PER_LANE 4
+#define VC_TOTALS_SLOT 8
+// copies of the verdict on the tables, a cache line each (one per lane of the wavefronts that report)
+#define VC_VERDICTS 64
+enum { VC_TOTALS_PAYLOAD, VC_TOTALS_ITEMS, VC_TOTALS_BAD, VC_TOTALS_MOST, VC_TOTALS_MOVED, VC_TOTALS_LONGEST,
+       VC_TOTALS_STALLED = 7 };               // (first slot) a copying wavefront gave up waiting for the verdict: the call is redone
+#define VC_TOTALS_PER_WAVE (64 * VC_TOTALS_PER_LANE)
+__host__ __device__ __forceinline__ int64_t vc_totals_waves(int P) { return ((int64_t)P * P + VC_TOTALS_PER_WAVE - 1) / VC_TOTALS_PER_WAVE; }
 // Launch-per-digit execution, passes 1 and 2: staging prefix sums and the number of work items of every launch (sizes only).
 // The launch table travels as a kernel argument when it has at most VC_LAUNCH_PACK entries (launches_dev is then not read).
 hipError_t vc_launch_plan_sizes(const VcSched &S, const VcLaunchInfo *launches_host, const VcLaunchInfo *launches_dev, int nlaunch,
@@ -293,13 +296,10 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 // planning kernels before it on the stream have written and does nothing unless vc_listless_ok(header, guard).
 // lanes: VC_THREADS (a workgroup per pair), VC_WAVE (a wavefront per pair, blocks of a KiB or two) or VC_QUARTER (a quarter of a
 // wavefront per pair, for blocks of a few hundred bytes).
-// header_host (pinned, may be null): the first workgroup copies the fixed words of `header` there, for planners that add
-// the header up with atomics and cannot write it to the host themselves.  header_zero (may be null): ... and clears the
-// fixed words there: the header the next call's planner will add up into.
-// totals (device, non-null: fixed-stride staging, S.stride > 0, at most VC_MAX_GRID pairs): the kernel needs no planner
-// before it.  Its first wavefronts add up the tables' totals — validation, payload, block pieces, longest block,
-// hop-weighted bytes — into `totals` (words 0 .. VC_HEADER_SYNC zeroed by the caller) and the last of them to finish
-// copies the words to header_host, with [0] = the bytes the fixed-stride arena takes; `header` is not read.  Every pair
+// verdict (device, non-null: fixed-stride staging, S.stride > 0, at most VC_MAX_GRID pairs): the kernel needs no planner
+// before it and `header` is not read.  Its first wavefronts check the tables, count themselves in the VC_VERDICTS words at `verdict` (zero at the
+// start; the kernel clears those at `verdict_next` for the call after this one) and leave what the host wants to know — payload, block pieces, longest block, ... —
+// in `totals` (host memory, vc_totals_waves(P) slots).  Every pair
 // checks its own table entries and the guard's max_len / max_pieces and leaves its block alone when one of them fails, so
 // no address is formed from a bad entry; the host, which evaluates the same conditions on the totals afterwards, reports
 // the call as refused then.  With bad table entries nothing has been stored by then: the copying wavefronts hold their
@@ -307,6 +307,7 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 // the other pairs may already have been delivered; they are delivered again when the host redoes the call.
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
-                                 int64_t *header_host = nullptr, int64_t *header_zero = nullptr, int64_t *totals = nullptr);
+                                 unsigned long long *verdict = nullptr, unsigned long long *verdict_next = nullptr,
+                                 int64_t *totals = nullptr);
 // dst2 non-null: every vector is stored twice (one read, two writes)
 hipError_t vc_launch_calibration_copy(const char *src, char *dst, char *dst2, int64_t nbytes, hipStream_t st);

@@ -56,42 +56,63 @@ __device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, ch
 // before the first and after the last of them are moved byte-wise (lanes 0..15 the head, lanes 16..31 the tail: one byte
 // load and one byte store each).  The planner guarantees len + (dst & 127) <= VC_CHUNK.
 // With nhop > 1 this is forwarded execution: the piece is read once, from sendbuf, and every hop stores the same
-// registers (all destinations of a block share the offset inside their cache line, so one mapping of lanes to window
-// vectors serves them all).  dst_of(k) is where hop k puts the piece.
+// registers (all destinations of a block share the offset inside their cache line, `w`, so one mapping of lanes to window
+// vectors serves them all).  next_dst() is where the next hop puts the piece.
 // go() is asked once, after the loads have been issued and before the first store: false leaves the piece where it is.
+#define VC_WAIT_VMCNT0 0x0F70              // s_waitcnt vmcnt(0): loads have arrived and stores have been acknowledged
 struct VcAlwaysGo { __device__ __forceinline__ bool operator()() const { return true; } };
 
-template <int LANES, class DstOf, class Go = VcAlwaysGo>
-__device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, int nhop, DstOf dst_of, Go go = Go()) {
+template <int LANES, class NextDst, class Go = VcAlwaysGo>
+__device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, int nhop, int w, NextDst next_dst, Go go = Go()) {
     constexpr int VECS = VC_CHUNK / 16 / LANES;           // window vectors per lane: 2 for a workgroup of 256, 8 for one wavefront
-    char *dst = dst_of(0);
     const int t = threadIdx.x;
-    const int64_t w = (int64_t)((uintptr_t)dst & (VC_LINE - 1));
-    const int64_t first_full = (w + 15) >> 4, end_full = (w + len) >> 4;
+    const int n = (int)len;                               // (a piece fits the window)
+    if (n == VC_PIECE && w == 0) {
+        // A whole aligned piece, the inside of a long block: no vector to leave out and no edge.  A wavefront waits for each of its
+        // stores before the next one: on lists of these the memory runs a few per cent faster with fewer writes in flight
+        // (64 ranks, 1.3 MB blocks, two hops: 2436 us -> 2361).
+        constexpr int WHOLE = VC_PIECE / 16 / LANES;
+        vc_u32x4 v[WHOLE];
+#pragma unroll
+        for (int i = 0; i < WHOLE; i++) v[i] = vc_load16(src + ((t + i * LANES) << 4));
+        if (!go()) return;
+        for (int k = 0; k < nhop; k++) {
+            char *dst = next_dst();
+#pragma unroll
+            for (int i = 0; i < WHOLE; i++) {
+                if (k || i) __builtin_amdgcn_s_waitcnt(VC_WAIT_VMCNT0);
+                vc_store16(dst + ((t + i * LANES) << 4), v[i]);
+            }
+        }
+        return;
+    }
+    const int first_full = (w + 15) >> 4, end_full = (w + n) >> 4;
     const char *sw = src - w;
     vc_u32x4 v[VECS];
     bool has[VECS];
 #pragma unroll
     for (int i = 0; i < VECS; i++) {
-        const int64_t j = t + i * LANES;
+        const int j = t + i * LANES;
         has[i] = (i > 0 || j >= first_full) && j < end_full;
         if (has[i]) v[i] = vc_load16(sw + (j << 4));
     }
-    int64_t head = (first_full << 4) - w;
-    if (head > len) head = len;
-    int64_t done = (end_full << 4) - w;
+    int head = (first_full << 4) - w;
+    if (head > n) head = n;
+    int done = (end_full << 4) - w;
     if (done < head) done = head;
-    const int64_t edge = t < 16 ? (t < head ? t : -1) : (t < 32 && done + (t - 16) < len ? done + (t - 16) : -1);
+    const int edge = t < 16 ? (t < head ? t : -1) : (t < 32 && done + (t - 16) < n ? done + (t - 16) : -1);
     char edge_byte = 0;
     if (edge >= 0) edge_byte = src[edge];
     if (!go()) return;
+    // all at once and after the last load has arrived, so that the writes of one line reach the L2 together (512 ranks, 1 KiB: 107 us
+    // -> 99; 1024 ranks, 4 KiB: 2475 -> 2434)
+    __builtin_amdgcn_s_waitcnt(VC_WAIT_VMCNT0);
     for (int k = 0; k < nhop; k++) {
-        if (k) dst = dst_of(k);
-        char *dw = dst - w;
+        char *dst = next_dst(), *dw = dst - w;
         if (edge >= 0) dst[edge] = edge_byte;
 #pragma unroll
         for (int i = 0; i < VECS; i++)
-            if (has[i]) vc_store16(dw + ((int64_t)(t + i * LANES) << 4), v[i]);
+            if (has[i]) vc_store16(dw + ((t + i * LANES) << 4), v[i]);
     }
 }
 
@@ -113,8 +134,17 @@ __global__ __launch_bounds__(LANES) void vc_copy_chains_kernel(const int64_t *__
     const int64_t len = it[VC_CHAIN_LEN];
     const int nhop = (int)it[VC_CHAIN_NHOP];
     if (len <= 0 || nhop <= 0) return;
-    vc_forward_piece<LANES>(vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage), len, nhop,
-                            [&](int k) { return vc_resolve(it[VC_CHAIN_HEAD + k], sendbuf, recvbuf, stage); });
+    const char *src = vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage);
+    char *dst = vc_resolve(it[VC_CHAIN_HEAD], sendbuf, recvbuf, stage);
+    const int w = (int)((uintptr_t)dst & (VC_LINE - 1)), lane = threadIdx.x % VC_WAVE;
+    // the hops after the first in one read, a word per lane: a load between the stores would wait for the stores before it
+    int64_t word = 0;
+    if (lane < nhop) word = it[VC_CHAIN_HEAD + lane];
+    int at = 0;
+    vc_forward_piece<LANES>(src, len, nhop, w, [&]() {
+        const unsigned lo = __builtin_amdgcn_readlane((int)word, at), hi = __builtin_amdgcn_readlane((int)(word >> 32), at);
+        return at++ ? vc_resolve((int64_t)hi << 32 | lo, sendbuf, recvbuf, stage) : dst;
+    });
 }
 
 // Launch-per-digit execution: one hop of one piece per item.
@@ -129,7 +159,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_items_kernel(const VcDesc *__re
     const VcDesc d = items[idx];
     if (d.len <= 0) return;
     char *dst = vc_resolve(d.dst, sendbuf, recvbuf, stage);
-    vc_forward_piece<LANES>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, [&](int) { return dst; });
+    vc_forward_piece<LANES>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, (int)((uintptr_t)dst & (VC_LINE - 1)), [&]() { return dst; });
 }
 
 // A quarter of a wavefront (16 lanes) per item, four items per wavefront, for lists of pieces of a few hundred bytes:
@@ -167,6 +197,95 @@ __device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_
             if (has1) vc_store16(dw + ((j + 16) << 4), v1);
         }
         first_pass = false;
+    }
+}
+
+// ---- blocks of a few hundred bytes, without byte-wise edges ----
+// What bounds these is the number of requests the copying sends to the L2 (about 75 per ns on this chip, whoever sends them: a
+// request writes at most 64 bytes), so every byte-wise head and tail counts as much as a whole vector.  Edges are moved as
+// 16-byte vectors that start or end with the block and overlap the aligned ones (the same bytes, twice).
+struct __attribute__((packed, aligned(1))) VcU64 { unsigned long long v; };
+struct __attribute__((packed, aligned(1))) VcU32 { unsigned v; };
+struct __attribute__((packed, aligned(1))) VcU16 { unsigned short v; };
+
+// A block of 1 .. VC_LANE_BLOCK bytes in one lane's registers: its first and its last 16 (8, 4, 2, 1) bytes, which overlap.
+#define VC_LANE_BLOCK 32
+struct VcLaneBlock { vc_u32x4 first, last; };
+
+__device__ __forceinline__ VcLaneBlock vc_lane_load(const char *src, int len) {
+    VcLaneBlock b;
+    b.first = b.last = vc_u32x4(0);
+    if (len >= 16) {
+        b.first = reinterpret_cast<const VcU128 *>(src)->v;
+        b.last = reinterpret_cast<const VcU128 *>(src + len - 16)->v;
+    } else if (len >= 8) {
+        const unsigned long long x = reinterpret_cast<const VcU64 *>(src)->v, y = reinterpret_cast<const VcU64 *>(src + len - 8)->v;
+        b.first.x = (unsigned)x; b.first.y = (unsigned)(x >> 32); b.last.x = (unsigned)y; b.last.y = (unsigned)(y >> 32);
+    } else if (len >= 4) {
+        b.first.x = reinterpret_cast<const VcU32 *>(src)->v;
+        b.last.x = reinterpret_cast<const VcU32 *>(src + len - 4)->v;
+    } else if (len >= 2) {
+        b.first.x = reinterpret_cast<const VcU16 *>(src)->v;
+        b.last.x = reinterpret_cast<const VcU16 *>(src + len - 2)->v;
+    } else {
+        b.first.x = *reinterpret_cast<const unsigned char *>(src);
+    }
+    return b;
+}
+
+__device__ __forceinline__ void vc_lane_store(const VcLaneBlock &b, char *dst, int len) {
+    if (len >= 16) {
+        reinterpret_cast<VcU128 *>(dst)->v = b.first;
+        reinterpret_cast<VcU128 *>(dst + len - 16)->v = b.last;
+    } else if (len >= 8) {
+        reinterpret_cast<VcU64 *>(dst)->v = (unsigned long long)b.first.y << 32 | b.first.x;
+        reinterpret_cast<VcU64 *>(dst + len - 8)->v = (unsigned long long)b.last.y << 32 | b.last.x;
+    } else if (len >= 4) {
+        reinterpret_cast<VcU32 *>(dst)->v = b.first.x;
+        reinterpret_cast<VcU32 *>(dst + len - 4)->v = b.last.x;
+    } else if (len >= 2) {
+        reinterpret_cast<VcU16 *>(dst)->v = (unsigned short)b.first.x;
+        reinterpret_cast<VcU16 *>(dst + len - 2)->v = (unsigned short)b.last.x;
+    } else {
+        *dst = (char)b.first.x;
+    }
+}
+
+// A piece moved by LANES neighbouring lanes of a wavefront: lane t owns window vectors t, t + LANES, ... (the window starts at the
+// cache line of the destination, `w` bytes before it), VECS of them in flight at once.  Staging is stored past the caches
+// (nothing reads it again); recvbuf is not: a line that two neighbouring blocks share is then put together in the L2.
+template <int LANES, int VECS, class DstOf, class Go = VcAlwaysGo>
+__device__ __forceinline__ void vc_forward_short(const char *src, int len, int nhop, int w, DstOf dst_of, Go go = Go()) {
+    const int t = threadIdx.x % LANES;
+    if (len < 16) {
+        VcLaneBlock b;
+        if (t == 0) b = vc_lane_load(src, len);
+        if (!go()) return;
+        if (t == 0)
+            for (int k = 0; k < nhop; k++) vc_lane_store(b, dst_of(k), len);
+        return;
+    }
+    const int last = (w + len + 15) >> 4;                 // vectors of the window, the ones below the block included
+    for (int j0 = t; j0 - t < last; j0 += VECS * LANES) {
+        vc_u32x4 v[VECS];
+        int at[VECS];                                     // where the vector starts inside the block
+#pragma unroll
+        for (int i = 0; i < VECS; i++) {
+            const int lo = ((j0 + i * LANES) << 4) - w;
+            at[i] = lo <= -16 || lo >= len ? -1 : (lo < 0 ? 0 : (lo > len - 16 ? len - 16 : lo));
+            if (at[i] >= 0) v[i] = vc_load16(src + at[i]);
+        }
+        if (j0 == t && !go()) return;
+        for (int k = 0; k < nhop - 1; k++) {
+            char *dst = dst_of(k);
+#pragma unroll
+            for (int i = 0; i < VECS; i++)
+                if (at[i] >= 0) __builtin_nontemporal_store(v[i], &reinterpret_cast<VcU128 *>(dst + at[i])->v);
+        }
+        char *dst = dst_of(nhop - 1);
+#pragma unroll
+        for (int i = 0; i < VECS; i++)
+            if (at[i] >= 0) reinterpret_cast<VcU128 *>(dst + at[i])->v = v[i];
     }
 }
 
@@ -211,204 +330,181 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_items_quarter_kernel(const Vc
     }
 }
 
-// ---- fixed-stride staging in one launch (the `totals` of vc_launch_copy_blocks) ----
-__device__ __forceinline__ int64_t vc_wave_sum(int64_t v) {
-#pragma unroll
-    for (int o = VC_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, VC_WAVE);
-    return v;
-}
-
-__device__ __forceinline__ int64_t vc_wave_max(int64_t v) {
-#pragma unroll
-    for (int o = VC_WAVE / 2; o > 0; o >>= 1) {
-        const int64_t u = __shfl_xor(v, o, VC_WAVE);
-        v = u > v ? u : v;
-    }
-    return v;
-}
-
+// ---- fixed-stride staging in one launch (the `verdict` of vc_launch_copy_blocks) ----
 // The wavefronts of the first vc_totals_blocks workgroups of the grid: four pairs of ranks per lane (by receiver, then
-// source; the atomics on the same few words are what limits this at many ranks), the wavefront's
-// sums and maxima added into `totals` with one atomic each: [1] payload, [2] block pieces, [3] table entries no rank could
-// have passed, [4] the most pieces of a block, [5] hop-weighted bytes, [6] the longest block.  The wavefront that finishes
-// last hands the words to the host.
-#define VC_TOTALS_PER_LANE 4
-// wavefronts that add up the totals of a call on P ranks
-__host__ __device__ __forceinline__ int64_t vc_totals_waves(int P) {
-    const int64_t per_wave = VC_WAVE * VC_TOTALS_PER_LANE;
-    return ((int64_t)P * P + per_wave - 1) / per_wave;
-}
-
-__device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &T, int64_t *totals, int64_t *header_host) {
-    const int P = S.P;
-    const int64_t pairs = (int64_t)P * P, per_wave = VC_WAVE * VC_TOTALS_PER_LANE, nwaves = vc_totals_waves(P);
-    const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / VC_WAVE) + threadIdx.x / VC_WAVE;
+// source).  Each puts its sums and maxima into a slot of its own in host memory, and the host adds the slots up when the launch
+// is over; their verdict goes into VC_VERDICTS copies of one word, and every copying wavefront looks at one of them.  (With an atomic
+// per wavefront on each of six shared words, and one verdict word that all wavefronts polled, these were what the launch waited for:
+// atomics on one address follow each other at about 10 ns.  128 ranks, 2 KiB blocks: 57 us -> 26; 64 ranks: 14 -> 13.)
+__device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &T, unsigned long long *verdict, int64_t *totals) {
+    const int P = S.P, pairs = P * P, per_wave = VC_TOTALS_PER_WAVE, nwaves = (int)vc_totals_waves(P);      // P^2 <= VC_STRIDED_MAX_PAIRS
+    const int wave = (int)blockIdx.x * (int)(blockDim.x / VC_WAVE) + (int)threadIdx.x / VC_WAVE;
     if (wave >= nwaves) return;
     const int lane = threadIdx.x & (VC_WAVE - 1);
-    unsigned long long *h = reinterpret_cast<unsigned long long *>(totals);
-    int64_t payload = 0, items = 0, bad = 0, most = 0, moved = 0, longest = 0;
-    // The verdict on the tables first, with nothing but one round of loads in front of it: the copying wavefronts of this
-    // launch hold their stores back until every totalling wavefront has reported (vc_wait_verdict).
+    // The verdict on the tables first, with nothing but one round of reads in front of it (all of a lane's pairs together): the
+    // copying wavefronts of this launch hold their stores back until every totalling wavefront has reported (VcVerdictGate).
+    VcPairEntries e[VC_TOTALS_PER_LANE];
+    int64_t rbase[VC_TOTALS_PER_LANE];
+    int src[VC_TOTALS_PER_LANE], dst[VC_TOTALS_PER_LANE];
 #pragma unroll
     for (int u = 0; u < VC_TOTALS_PER_LANE; u++) {
-        const int64_t idx = wave * per_wave + u * VC_WAVE + lane;
-        if (idx >= pairs) continue;
-        const int to = vc_div((int)idx, S.dP), s = (int)idx - to * P;      // (idx < P^2 <= 2^30)
-        const int64_t i = (int64_t)to * P + s;
-        bad += vc_pair_bad_entries(S, T, s, to);          // the same count the planner's row kernel makes
-        // (a packed receive layout past INT_MAX elements shows as a negative packed displacement of a later source)
-        if (S.packed_recv && (T.rd_packed[i] < 0 || (s == P - 1 && (int64_t)T.rd_packed[i] + T.rc[i] > 0x7FFFFFFF))) bad += VC_BAD_OVERFLOW;
+        const int idx = wave * per_wave + u * VC_WAVE + lane, in = idx < pairs ? idx : 0;
+        dst[u] = vc_div(in, S.dP);
+        src[u] = in - dst[u] * P;
+        e[u] = vc_pair_entries(S, T, src[u], dst[u]);
+        rbase[u] = T.rbase[dst[u]];
     }
-    bad = vc_wave_sum(bad);
-    // one word says it all, so one atomic publishes it: wavefronts that have reported in the low half, wavefronts that
-    // found something wrong in the high half
-    if (lane == 0) atomicAdd(&h[VC_HEADER_CHECKED], 1ull | (bad ? 1ull << 32 : 0ull));
+    int64_t bad = 0;
 #pragma unroll
     for (int u = 0; u < VC_TOTALS_PER_LANE; u++) {
-        const int64_t idx = wave * per_wave + u * VC_WAVE + lane;
-        if (idx >= pairs) continue;
-        const int to = vc_div((int)idx, S.dP), s = (int)idx - to * P;      // (idx < P^2 <= 2^30)
-        const int sc = vc_sc(S, T, s, to), rc = vc_rc(S, T, to, s);
-        const int64_t len = (int64_t)sc * S.esz;
-        const int64_t cnt = sc > 0 ? vc_chain_count(S, T, s, to) : 0;
-        payload += (int64_t)rc * S.esz;                   // (what the receivers expect, as the planner counts it)
+        if (wave * per_wave + u * VC_WAVE + lane >= pairs) continue;
+        bad += vc_bad_entries(S, e[u]);                   // the same count the planner makes
+        // (a packed receive layout past INT_MAX elements shows as a negative packed displacement of a later source)
+        if (S.packed_recv && (e[u].rd < 0 || (src[u] == P - 1 && (int64_t)e[u].rd + e[u].expected > 0x7FFFFFFF))) bad += VC_BAD_OVERFLOW;
+    }
+    // one word says it all, so one atomic instruction publishes it in every copy: wavefronts that have reported in the low half,
+    // wavefronts that found something wrong in the high half
+    const unsigned long long report = __ballot(bad != 0) ? 1ull | 1ull << 32 : 1ull;
+    if (lane < VC_VERDICTS) atomicAdd(verdict + lane * (VC_LINE / 8), report);
+    bad = vc_wave_inclusive_scan(bad);                    // (lane 63 has the sum)
+    int64_t payload = 0, items = 0, most = 0, moved = 0, longest = 0;
+#pragma unroll
+    for (int u = 0; u < VC_TOTALS_PER_LANE; u++) {
+        if (wave * per_wave + u * VC_WAVE + lane >= pairs) continue;
+        const int64_t len = (int64_t)e[u].sent * S.esz;
+        const int cut = (int)((rbase[u] + (int64_t)e[u].rd * S.esz + S.recv_lo) & (VC_PIECE - 1));
+        const int64_t cnt = vc_chunk_count(len, cut & (VC_LINE - 1), cut);
+        payload += (int64_t)e[u].expected * S.esz;        // (what the receivers expect, as the planner counts it)
         items += cnt;
-        moved += len * vc_block_hops(S, s, to);
+        moved += len * vc_block_hops(S, src[u], dst[u]);
         most = cnt > most ? cnt : most;
         longest = len > longest ? len : longest;
     }
-    payload = vc_wave_sum(payload);
-    items = vc_wave_sum(items);
-    moved = vc_wave_sum(moved);
-    most = vc_wave_max(most);
-    longest = vc_wave_max(longest);
-    int last = 0;
-    if (lane == 0) {
-        // The count below must not be seen before the words above.  A release fence would do, but at device scope it writes
-        // this XCD's L2 back, once per wavefront here.  Instead every atomic returns its old value: when the values are
-        // back the atomics have been performed where the count is kept too, and the count's operand is made from them.
-        unsigned long long seen = 0;
-        if (payload) seen += atomicAdd(&h[1], (unsigned long long)payload);
-        if (items) seen += atomicAdd(&h[2], (unsigned long long)items);
-        if (bad) seen += atomicAdd(&h[VC_HEADER_BAD], (unsigned long long)bad);
-        if (moved) seen += atomicAdd(&h[VC_HEADER_FIXED], (unsigned long long)moved);
-        if (most) seen += atomicMax(&h[VC_HEADER_MAX_PIECES], (unsigned long long)most);
-        if (longest) seen += atomicMax(&h[VC_HEADER_MAX_LEN], (unsigned long long)longest);
-        unsigned zero;
-        asm volatile("v_mov_b32 %0, 0" : "=v"(zero) : "v"((unsigned)seen), "v"((unsigned)(seen >> 32)));      // (opaque to the compiler)
-        last = atomicAdd(&h[VC_HEADER_SYNC], 1ull + zero) == (unsigned long long)(nwaves - 1);
+    payload = vc_wave_inclusive_scan(payload);
+    items = vc_wave_inclusive_scan(items);
+    moved = vc_wave_inclusive_scan(moved);
+    most = vc_wave_max_last(most);
+    longest = vc_wave_max_last(longest);
+    if (lane == VC_WAVE - 1) {
+        int64_t *slot = totals + wave * VC_TOTALS_SLOT;
+        slot[VC_TOTALS_PAYLOAD] = payload; slot[VC_TOTALS_ITEMS] = items; slot[VC_TOTALS_BAD] = bad;
+        slot[VC_TOTALS_MOST] = most; slot[VC_TOTALS_MOVED] = moved; slot[VC_TOTALS_LONGEST] = longest;
     }
-    last = __shfl(last, 0, VC_WAVE);
-    if (last && lane <= VC_HEADER_MAX_LEN)
-        header_host[lane] = lane == 0 ? vc_strided_stage_bytes(S)
-                                      : (int64_t)__hip_atomic_load(&h[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // A copying wavefront of the single launch asks before its first store: have all totalling wavefronts checked their part of
 // the tables, and did they find them in order?  The totalling workgroups are the first of the grid, so they are resident
 // before any copying one; the wait is bounded all the same (VC_CHECK_SPINS polls, a few milliseconds): a wavefront that
-// gives up moves nothing and says so in the host's copy of the header, and the host redoes the call the general way.
+// gives up moves nothing and says so in the first slot of the totals, and the host redoes the call the general way.
 #define VC_CHECK_SPINS (1 << 15)
-__device__ __forceinline__ unsigned long long vc_verdict_word(int64_t *totals) {
-    return __hip_atomic_load(reinterpret_cast<unsigned long long *>(totals) + VC_HEADER_CHECKED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ unsigned long long vc_verdict_word(unsigned long long *verdict) {
+    return __hip_atomic_load(verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Asked by the piece movers between their loads and their stores (see vc_forward_piece).  Without `totals` there is nothing
+// Asked by the piece movers between their loads and their stores (see vc_forward_piece).  Without `verdict` there is nothing
 // to wait for (the planner's verdict was checked before the block's route was worked out).  look() reads the word once
 // ahead of the block's loads, so that a verdict that is already in costs no round trip of its own.
 struct VcVerdictGate {
-    int64_t *totals, *header_host;
+    unsigned long long *verdict;
+    int64_t *totals;
     unsigned long long nwaves, word;
     int state;                                            // 0 not known yet, 1 go, 2 leave everything where it is
-    __device__ __forceinline__ void look() { if (totals) word = vc_verdict_word(totals); }
+    __device__ __forceinline__ void look() { if (verdict) word = vc_verdict_word(verdict); }
     __device__ __forceinline__ bool operator()() {
-        if (!totals) return true;
+        if (!verdict) return true;
         for (int spin = 0; state == 0; spin++) {
             if ((word & 0xFFFFFFFFull) >= nwaves) state = (word >> 32) ? 2 : 1;
-            else if (spin >= VC_CHECK_SPINS) { header_host[VC_HEADER_STALLED] = 1; state = 2; }
-            else { __builtin_amdgcn_s_sleep(4); word = vc_verdict_word(totals); }
+            else if (spin >= VC_CHECK_SPINS) { totals[VC_TOTALS_STALLED] = 1; state = 2; }
+            else { __builtin_amdgcn_s_sleep(1); word = vc_verdict_word(verdict); }
         }
         return state == 1;
     }
 };
 
-// Workgroups at the head of the grid that only add up the totals (none without `totals`): their round trips run beside the
+// Workgroups at the head of the grid that only add up the totals (none without `verdict`): their round trips run beside the
 // copying instead of in front of it.  A multiple of VC_XCDS, so that the workgroups behind them keep their XCDs.
-__host__ __device__ __forceinline__ unsigned vc_totals_blocks(const VcSched &S, const int64_t *totals, int lanes) {
-    if (!totals) return 0;
-    const int64_t per_wave = VC_WAVE * VC_TOTALS_PER_LANE;
-    const int64_t waves = ((int64_t)S.P * S.P + per_wave - 1) / per_wave, per = lanes / VC_WAVE;
+__host__ __device__ __forceinline__ unsigned vc_totals_blocks(const VcSched &S, const void *verdict, int lanes) {
+    if (!verdict) return 0;
+    const int64_t waves = vc_totals_waves(S.P), per = lanes / VC_WAVE;
     return (unsigned)(((waves + per - 1) / per + VC_XCDS - 1) / VC_XCDS * VC_XCDS);
 }
 
-// Whether the pair's own table entries allow its block to be moved: none negative, the receiver expecting what the
-// source sends, the block no longer than a slot and cut into no more pieces than the kernel was chosen for.
-__device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcTables &T, const VcListlessGuard &g, int s, int t) {
-    const int sc = vc_sc(S, T, s, t), rd = vc_rd(S, T, t, s);
-    if (sc < 0 || vc_rc(S, T, t, s) != sc || vc_sd(S, T, s, t) < 0 || rd < 0) return false;
-    if (S.packed_recv && (int64_t)rd + sc > 0x7FFFFFFF) return false;
-    const int64_t len = (int64_t)sc * S.esz;
-    if (g.max_len && len > g.max_len) return false;
-    return !(g.max_pieces && sc > 0 && vc_chain_count(S, T, s, t) > g.max_pieces);
+// Everything the addresses of a pair's block depend on, read at once.
+struct VcPairRead { int sent, expected, sd, rd; int64_t sbase, rbase; };
+
+__device__ __forceinline__ VcPairRead vc_pair_read(const VcSched &S, const VcTables &T, int s, int t) {
+    VcPairRead p;
+    p.sent = vc_sc(S, T, s, t); p.expected = vc_rc(S, T, t, s); p.sd = vc_sd(S, T, s, t); p.rd = vc_rd(S, T, t, s);
+    p.sbase = T.sbase[s]; p.rbase = T.rbase[t];
+    return p;
+}
+
+// Whether the pair's own table entries allow its block to be moved (the single launch has no planner that checked them):
+// none negative, the receiver expecting what the source sends, the block no longer than a slot and cut into no more pieces
+// than the kernel was chosen for.
+__device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcPairRead &p, const VcListlessGuard &g) {
+    const int64_t len = (int64_t)p.sent * S.esz;
+    const int cut = (int)((p.rbase + (int64_t)p.rd * S.esz + S.recv_lo) & (VC_PIECE - 1));
+    bool ok = (p.sent | p.sd | p.rd) >= 0 && p.expected == p.sent;
+    ok = ok && !(S.packed_recv && (int64_t)p.rd + p.sent > 0x7FFFFFFF);
+    ok = ok && !(g.max_len && len > g.max_len);
+    return ok && !(g.max_pieces && vc_chunk_count(len, cut & (VC_LINE - 1), cut) > g.max_pieces);
 }
 
 // Forwarded execution without a work-item list, for calls whose planning would otherwise cost more than their copying:
-// one workgroup per (source, destination) pair, in the order of the chain items (by destination, then source, an eighth
-// of the pairs per XCD).  The workgroup works out the route of its block in closed form from the plan tables (lane k
-// evaluates hop slot k), then carries the block through it piece by piece.  The kernel is enqueued right behind the
-// planning kernels, before the host has seen their result, so it checks that result itself: nothing is touched when the
+// one workgroup (LANES = VC_THREADS) or one wavefront (VC_WAVE: blocks of a KiB or two) per (source, destination)
+// pair, in the order of the chain items (by destination, then source, an eighth
+// of the pairs per XCD).  Every wavefront works out the route of its block in closed form from the plan tables (lane k
+// evaluates hop slot k) and carries the block through it piece by piece, taking one hop's destination after the other from
+// its lane into scalar registers.  The kernel is enqueued right behind the
+// planning kernel, before the host has seen its result, so it checks that result itself: nothing is touched when the
 // plan needs more staging than there is, the tables hold negative entries, or the call is not of the kind the host
 // expected when it chose this kernel (the host, which evaluates the same condition afterwards, then takes another path).
-// LANES = VC_THREADS: a workgroup of four wavefronts per pair; LANES = VC_WAVE: one wavefront per pair, for blocks of a
-// KiB or two (a quarter of the wavefronts to start, all of them with work).
+// Everything the block's addresses depend on is read before the planner's verdict is looked at: the reads are
+// independent of each other and of the verdict (tables are always readable), so they travel together instead of one
+// memory round trip after the other; nothing is stored before the verdict is known.
 template <int LANES>
 __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                const int64_t *__restrict__ row_base,
                                                                const int64_t *__restrict__ header, VcListlessGuard guard,
                                                                int64_t first_pair, const char *__restrict__ sendbuf,
                                                                char *__restrict__ recvbuf, char *__restrict__ stage,
-                                                               int64_t *__restrict__ header_host, int64_t *__restrict__ header_zero,
+                                                               unsigned long long *verdict, unsigned long long *verdict_next,
                                                                int64_t *totals) {
-    __shared__ int64_t route[VC_MAX_HOP_SLOTS];
-    __shared__ int route_len;
-    const unsigned head = vc_totals_blocks(S, totals, LANES);
-    if (blockIdx.x < head) { vc_add_totals(S, T, totals, header_host); return; }
+    const unsigned head = vc_totals_blocks(S, verdict, LANES);
+    if (blockIdx.x < head) { vc_add_totals(S, T, verdict, totals); return; }
     const unsigned block = blockIdx.x - head;
     const int64_t per = (gridDim.x - head) / VC_XCDS;
     const int64_t idx = first_pair + (int64_t)(block % VC_XCDS) * per + block / VC_XCDS;
     const bool inside = idx < (int64_t)S.P * S.P;
     const int t = inside ? vc_div((int)idx, S.dP) : 0, s = inside ? (int)idx - t * S.P : 0;       // (idx < P^2 <= 2^30)
-    // Everything the block's addresses depend on is loaded before the planner's verdict is looked at: the loads are
-    // independent of each other and of the verdict (tables are always readable), so they travel together instead of one
-    // memory round trip after the other; nothing is stored before the verdict is known.
-    const int64_t len = (int64_t)vc_sc(S, T, s, t) * S.esz;
-    const int64_t send_off = vc_send_offset(S, T, s, t);
-    const int64_t recv_off = vc_recv_offset(S, T, s, t);
-    int64_t dst = 0;
-    const bool moves = threadIdx.x < VC_WAVE && (int)threadIdx.x < vc_hop_slots(S) && vc_block_hop(S, T, slot_off, row_base, s, t, threadIdx.x, dst);
-    if (block == 0 && first_pair == 0 && threadIdx.x <= VC_HEADER_CHECKED) {
-        if (header_host && !totals && threadIdx.x <= VC_HEADER_MAX_LEN) header_host[threadIdx.x] = header[threadIdx.x];
-        if (header_zero) header_zero[threadIdx.x] = 0;    // the header the next call will add up into
-    }
+    const VcPairRead p = vc_pair_read(S, T, s, t);
+    const int lane = threadIdx.x % VC_WAVE, nslots = vc_hop_slots(S);
+    const VcHop hop = vc_hop_place(S, s, t, lane < nslots ? lane : 0);
+    const int64_t slot = vc_slot_addr(S, slot_off, row_base, hop);
+    if (verdict && block == 0 && threadIdx.x < VC_VERDICTS) verdict_next[threadIdx.x * (VC_LINE / 8)] = 0;      // the words of the next call
+    const int64_t len = (int64_t)p.sent * S.esz;
     if (!inside || len <= 0) return;
-    if (totals ? !vc_pair_allowed(S, T, guard, s, t) : !vc_listless_ok(header, guard)) return;
-    if (threadIdx.x < VC_WAVE) {                          // hop slots <= VC_MAX_HOP_SLOTS < lanes of the first wavefront
-        const unsigned long long mask = __ballot(moves);
-        if (moves) route[__popcll(mask & ((1ull << threadIdx.x) - 1))] = dst;
-        if (threadIdx.x == 0) route_len = __popcll(mask);
-    }
-    __syncthreads();
-    const int nhop = route_len;
-    if (nhop <= 0) return;
-    const char *src = sendbuf + send_off;
-    const int phase = (int)((recv_off + S.recv_lo) & (VC_LINE - 1)), cut = (int)((recv_off + S.recv_lo) & (VC_PIECE - 1));
+    if (verdict ? !vc_pair_allowed(S, p, guard) : !vc_listless_ok(header, guard)) return;
+    const int64_t recv_off = p.rbase + (int64_t)p.rd * S.esz;
+    const int64_t dst = vc_hop_dst(S, hop, slot, recv_off);
+    const unsigned long long moves = __ballot(lane < nslots && hop.moves);
+    const char *src = sendbuf + p.sbase + (int64_t)p.sd * S.esz;
+    const int cut = (int)((recv_off + S.recv_lo) & (VC_PIECE - 1)), phase = cut & (VC_LINE - 1);
     const int64_t pieces = vc_chunk_count(len, phase, cut);
-    VcVerdictGate gate = {totals, header_host, (unsigned long long)vc_totals_waves(S.P), 0, 0};
+    VcVerdictGate gate = {verdict ? verdict + block % VC_VERDICTS * (VC_LINE / 8) : nullptr, totals, (unsigned long long)vc_totals_waves(S.P), 0, 0};
     gate.look();
     for (int64_t c = 0; c < pieces; c++) {                // the same cuts as the chain items of this block
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
-        vc_forward_piece<LANES>(src + lo, hi - lo, nhop, [&](int k) { return vc_resolve(route[k] + lo, sendbuf, recvbuf, stage); },
+        unsigned long long left = moves;
+        vc_forward_piece<LANES>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
+                                [&]() {
+                                    const int k = __ffsll(left) - 1;
+                                    left &= left - 1;
+                                    const unsigned d_lo = __builtin_amdgcn_readlane((int)dst, k), d_hi = __builtin_amdgcn_readlane((int)(dst >> 32), k);
+                                    return vc_resolve(((int64_t)d_hi << 32 | d_lo) + lo, sendbuf, recvbuf, stage);
+                                },
                                 [&]() { return gate(); });
     }
 }
@@ -420,11 +516,11 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
                                                                          const int64_t *__restrict__ header, VcListlessGuard guard,
                                                                          int64_t first_pair, const char *__restrict__ sendbuf,
                                                                          char *__restrict__ recvbuf, char *__restrict__ stage,
-                                                                         int64_t *__restrict__ header_host, int64_t *__restrict__ header_zero,
+                                                                         unsigned long long *verdict, unsigned long long *verdict_next,
                                                                          int64_t *totals) {
     __shared__ int64_t route[VC_ITEMS_PER_WAVE][VC_MAX_HOP_SLOTS];
-    const unsigned head = vc_totals_blocks(S, totals, VC_WAVE);
-    if (blockIdx.x < head) { vc_add_totals(S, T, totals, header_host); return; }
+    const unsigned head = vc_totals_blocks(S, verdict, VC_WAVE);
+    if (blockIdx.x < head) { vc_add_totals(S, T, verdict, totals); return; }
     const unsigned block = blockIdx.x - head;
     const int64_t per = (gridDim.x - head) / VC_XCDS;
     const int64_t wave = (int64_t)(block % VC_XCDS) * per + block / VC_XCDS;
@@ -432,97 +528,126 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
     const int64_t idx = first_pair + wave * VC_ITEMS_PER_WAVE + g;
     const bool inside = idx < (int64_t)S.P * S.P;
     const int t = inside ? vc_div((int)idx, S.dP) : 0, s = inside ? (int)idx - t * S.P : 0;       // (idx < P^2 <= 2^30)
-    // all loads the addresses depend on go out before the planner's verdict is looked at (see vc_copy_blocks_kernel)
-    const int64_t len = inside ? (int64_t)vc_sc(S, T, s, t) * S.esz : 0;
-    const int64_t send_off = vc_send_offset(S, T, s, t);
-    const int64_t recv_off = vc_recv_offset(S, T, s, t);
-    // no lane leaves before the barrier below
-    const bool active = len > 0 && (!totals || vc_pair_allowed(S, T, guard, s, t));
+    // all reads the addresses depend on go out before the planner's verdict is looked at (see vc_copy_blocks_kernel)
+    const VcPairRead p = vc_pair_read(S, T, s, t);
     const int nslots = vc_hop_slots(S);
-    int64_t d0 = 0, d1 = 0;
-    const bool m0 = active && q < nslots && vc_block_hop(S, T, slot_off, row_base, s, t, q, d0);
-    const bool m1 = active && q + VC_QUARTER < nslots && vc_block_hop(S, T, slot_off, row_base, s, t, q + VC_QUARTER, d1);
-    if (block == 0 && first_pair == 0 && threadIdx.x <= VC_HEADER_CHECKED) {
-        if (header_host && !totals && threadIdx.x <= VC_HEADER_MAX_LEN) header_host[threadIdx.x] = header[threadIdx.x];
-        if (header_zero) header_zero[threadIdx.x] = 0;
-    }
-    if (!totals && !vc_listless_ok(header, guard)) return;      // the same for every lane of the grid
+    const VcHop h0 = vc_hop_place(S, s, t, q < nslots ? q : 0);
+    const int64_t slot0 = vc_slot_addr(S, slot_off, row_base, h0);
+    if (verdict && block == 0 && threadIdx.x < VC_VERDICTS) verdict_next[threadIdx.x * (VC_LINE / 8)] = 0;
+    if (!verdict && !vc_listless_ok(header, guard)) return;      // the same for every lane of the grid
+    const int64_t len = inside ? (int64_t)p.sent * S.esz : 0, recv_off = p.rbase + (int64_t)p.rd * S.esz;
+    // no lane leaves before the barrier below
+    const bool active = len > 0 && (!verdict || vc_pair_allowed(S, p, guard));
+    const bool m0 = active && q < nslots && h0.moves;
     const unsigned g0 = (unsigned)(__ballot(m0) >> (g * VC_QUARTER)) & 0xFFFFu;      // the group's hops among slots 0..15
-    const unsigned g1 = (unsigned)(__ballot(m1) >> (g * VC_QUARTER)) & 0xFFFFu;      // ... among slots 16..31
-    if (m0) route[g][__popc(g0 & ((1u << q) - 1))] = d0;
-    if (m1) route[g][__popc(g0) + __popc(g1 & ((1u << q) - 1))] = d1;
+    if (m0) route[g][__popc(g0 & ((1u << q) - 1))] = vc_hop_dst(S, h0, slot0, recv_off);
+    int nhop = __popc(g0);
+    if (nslots > VC_QUARTER) {                            // ... among slots 16..31
+        int64_t d1 = 0;
+        const bool m1 = active && q + VC_QUARTER < nslots && vc_block_hop(S, T, slot_off, row_base, s, t, q + VC_QUARTER, d1);
+        const unsigned g1 = (unsigned)(__ballot(m1) >> (g * VC_QUARTER)) & 0xFFFFu;
+        if (m1) route[g][nhop + __popc(g1 & ((1u << q) - 1))] = d1;
+        nhop += __popc(g1);
+    }
     __syncthreads();
-    const int nhop = __popc(g0) + __popc(g1);
     if (!active || nhop <= 0) return;
-    const char *src = sendbuf + send_off;
-    const int phase = (int)((recv_off + S.recv_lo) & (VC_LINE - 1)), cut = (int)((recv_off + S.recv_lo) & (VC_PIECE - 1));
+    const char *src = sendbuf + p.sbase + (int64_t)p.sd * S.esz;
+    const int cut = (int)((recv_off + S.recv_lo) & (VC_PIECE - 1)), phase = cut & (VC_LINE - 1);
     const int64_t pieces = vc_chunk_count(len, phase, cut);
-    VcVerdictGate gate = {totals, header_host, (unsigned long long)vc_totals_waves(S.P), 0, 0};
+    VcVerdictGate gate = {verdict ? verdict + block % VC_VERDICTS * (VC_LINE / 8) : nullptr, totals, (unsigned long long)vc_totals_waves(S.P), 0, 0};
     gate.look();
     for (int64_t c = 0; c < pieces; c++) {
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
-        vc_forward_piece_quarter(src + lo, hi - lo, nhop, [&](int k) { return vc_resolve(route[g][k] + lo, sendbuf, recvbuf, stage); },
-                                 [&]() { return gate(); });
+        vc_forward_short<VC_QUARTER, 8>(src + lo, (int)(hi - lo), nhop, c ? 0 : phase, [&](int k) { return vc_resolve(route[g][k] + lo, sendbuf, recvbuf, stage); },
+                                        [&]() { return gate(); });
     }
 }
 
 // The same again for calls of many short blocks, where the wavefronts above live for one pass over four blocks and the
-// round trips and the arithmetic of working out a route, not the bytes, set the pace: a wavefront takes BATCH pairs in a
-// row.  64 / BATCH lanes per pair evaluate its hop slots, one lane per pair compacts the route in LDS, then every quarter
-// of the wavefront carries BATCH / 4 of the blocks, one after the other.  Measured on MI355X, 1024 ranks, blocks of 0 - 16
-// bytes (two hops each): 211 us with a quarter of a wavefront per pair, 105 / 87 / 79 us with BATCH = 16 / 32 / 64.
+// round trips and the arithmetic of working out a route, not the bytes, set the pace: a wavefront takes BATCH pairs, a tile of
+// TS sources x TR receivers, so that its table entries, the blocks it reads (of one source, for neighbouring receivers) and
+// the blocks it writes (of one receiver, from neighbouring sources) share cache lines.
+// 64 / BATCH lanes per pair evaluate its hop slots and leave the route in LDS.  Blocks of no more than VC_LANE_BLOCK bytes are then moved by
+// a lane each, when all blocks of the wavefront are that short; else every quarter of the wavefront carries BATCH / 4 of them, one
+// after the other.  Measured on MI355X, 1024 ranks, two hops for most blocks: 0 - 16 bytes 80 us (pairs of one receiver
+// in a row, every block a quarter of a wavefront) -> 40; 0 - 512 bytes 280 us either way.
 template <int BATCH>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                        const int64_t *__restrict__ row_base,
                                                                        const int64_t *__restrict__ header, VcListlessGuard guard,
-                                                                       int64_t first_pair, const char *__restrict__ sendbuf,
-                                                                       char *__restrict__ recvbuf, char *__restrict__ stage,
-                                                                       int64_t *__restrict__ header_host, int64_t *__restrict__ header_zero) {
+                                                                       int64_t first_wave, const char *__restrict__ sendbuf,
+                                                                       char *__restrict__ recvbuf, char *__restrict__ stage) {
+    constexpr int TS = BATCH == 16 ? 4 : 8, TR = BATCH / TS, SHARE = VC_WAVE / BATCH;
     extern __shared__ int64_t batch_lds[];
-    const int nslots = vc_hop_slots(S);
+    const int nslots = vc_hop_slots(S), P = S.P;
     int64_t *route = batch_lds;                           // [BATCH][nslots]
     int64_t *b_len = route + BATCH * nslots, *b_src = b_len + BATCH;
     int *b_nhop = reinterpret_cast<int *>(b_src + BATCH), *b_cut = b_nhop + BATCH;
-    const int64_t per = gridDim.x / VC_XCDS;
-    const int64_t wave = (int64_t)(blockIdx.x % VC_XCDS) * per + blockIdx.x / VC_XCDS;
+    const unsigned per = gridDim.x / VC_XCDS, tiles_s = (unsigned)(P + TS - 1) / TS;
+    const unsigned wave = (unsigned)first_wave + (blockIdx.x % VC_XCDS) * per + blockIdx.x / VC_XCDS;
+    const unsigned tile_t = wave / tiles_s, tile_s = wave - tile_t * tiles_s;
     const int p = threadIdx.x % BATCH, kq = threadIdx.x / BATCH;
-    const int64_t idx = first_pair + wave * BATCH + p;
-    const bool inside = idx < (int64_t)S.P * S.P;
-    const int t = inside ? vc_div((int)idx, S.dP) : 0, s = inside ? (int)idx - t * S.P : 0;       // (idx < P^2 <= 2^30)
-    // all loads the addresses depend on go out before the planner's verdict is looked at (see vc_copy_blocks_kernel)
-    const int64_t len = inside ? (int64_t)vc_sc(S, T, s, t) * S.esz : 0;
-    const int64_t send_off = vc_send_offset(S, T, s, t);
-    const int64_t recv_off = vc_recv_offset(S, T, s, t);
-    const bool active = len > 0;
-    for (int k = kq; k < nslots; k += VC_WAVE / BATCH) {
-        int64_t d = 0;
-        const bool moves = active && vc_block_hop(S, T, slot_off, row_base, s, t, k, d);
-        route[p * nslots + k] = moves ? d : -1;           // destinations carry their space in bits 60 and 61: never negative
-    }
-    if (blockIdx.x == 0 && first_pair == 0 && threadIdx.x <= VC_HEADER_MAX_LEN) {
-        if (header_host) header_host[threadIdx.x] = header[threadIdx.x];
-        if (header_zero) header_zero[threadIdx.x] = 0;
-    }
-    if (!vc_listless_ok(header, guard)) return;           // the same for every lane of the grid
-    __syncthreads();
-    if (kq == 0) {
-        int nhop = 0;
-        for (int k = 0; k < nslots; k++) {
-            const int64_t d = route[p * nslots + k];
-            if (d >= 0) route[p * nslots + nhop++] = d;
+    const int s_at = (int)tile_s * TS + p % TS, t_at = (int)tile_t * TR + p / TS;
+    const bool inside = s_at < P && t_at < P;
+    const int s = inside ? s_at : 0, t = inside ? t_at : 0;
+    // all reads the addresses depend on go out before the planner's verdict is looked at (see vc_copy_blocks_kernel)
+    const int sent = vc_sc(S, T, s, t);
+    const int64_t send_off = vc_send_offset(S, T, s, t), recv_off = vc_recv_offset(S, T, s, t);
+    const bool ok = vc_listless_ok(header, guard);
+    const int64_t len = inside ? (int64_t)sent * S.esz : 0;
+    int nhop = 0;
+    if (SHARE == 1) {
+        VcWalk walk = vc_walk_start(S, s, t);
+        for (int k0 = 0; k0 < nslots; k0 += 4) {          // four slots at a time: their reads travel together
+            VcHop hop[4];
+            int64_t at_row[4];
+            uint32_t at[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                hop[u].moves = 0; at_row[u] = 0; at[u] = 0;
+                if (k0 + u >= nslots) continue;
+                hop[u] = vc_walk_step(S, walk, s, t, k0 + u);
+                at_row[u] = row_base[hop[u].row];
+                at[u] = slot_off[(int64_t)hop[u].row * P + hop[u].id];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (hop[u].moves) route[p * nslots + nhop++] = vc_hop_dst(S, hop[u], at_row[u] + vc_slot_bytes(at[u]), recv_off);
         }
-        b_len[p] = len;
+    } else {
+        for (int k = kq; k < nslots; k += SHARE) {
+            const VcHop hop = vc_hop_place(S, s, t, k);
+            const int64_t d = vc_hop_dst(S, hop, vc_slot_addr(S, slot_off, row_base, hop), recv_off);
+            route[p * nslots + k] = hop.moves ? d : -1;   // destinations carry their space in bits 60 and 61: never negative
+        }
+        __syncthreads();
+        for (int k = 0; k < nslots; k++) {                // (every lane of the pair on its own copy of the count; one writes)
+            const int64_t d = route[p * nslots + k];
+            if (d >= 0) { if (kq == 0) route[p * nslots + nhop] = d; nhop++; }
+        }
+    }
+    if (!ok) return;                                      // the same for every lane of the grid
+    const bool active = len > 0 && nhop > 0;
+    if (__ballot(active && len > VC_LANE_BLOCK) == 0) {
+        __syncthreads();
+        if (active && kq == 0) {
+            const VcLaneBlock b = vc_lane_load(sendbuf + send_off, (int)len);
+            for (int k = 0; k < nhop; k++) vc_lane_store(b, vc_resolve(route[p * nslots + k], sendbuf, recvbuf, stage), (int)len);
+        }
+        return;
+    }
+    if (kq == 0) {
+        b_len[p] = active ? len : 0;
         b_src[p] = send_off;
-        b_nhop[p] = active ? nhop : 0;
+        b_nhop[p] = nhop;
         b_cut[p] = (int)((recv_off + S.recv_lo) & (VC_PIECE - 1));
     }
     __syncthreads();
     for (int it = 0; it < BATCH / VC_ITEMS_PER_WAVE; it++) {
         const int b = it * VC_ITEMS_PER_WAVE + threadIdx.x / VC_QUARTER;
         const int64_t blen = b_len[b];
-        const int nhop = b_nhop[b];
-        if (blen <= 0 || nhop <= 0) continue;
+        if (blen <= 0) continue;
         const char *src = sendbuf + b_src[b];
         const int cut = b_cut[b], phase = cut & (VC_LINE - 1);
         const int64_t *dsts = route + b * nslots;
@@ -530,49 +655,43 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
         for (int64_t c = 0; c < pieces; c++) {            // the same cuts as the chain items of this block
             int64_t lo, hi;
             vc_piece_range(blen, phase, cut, c, lo, hi);
-            vc_forward_piece_quarter(src + lo, hi - lo, nhop, [&](int k) { return vc_resolve(dsts[k] + lo, sendbuf, recvbuf, stage); });
+            vc_forward_short<VC_QUARTER, 4>(src + lo, (int)(hi - lo), b_nhop[b], c ? 0 : phase, [&](int k) { return vc_resolve(dsts[k] + lo, sendbuf, recvbuf, stage); });
         }
     }
 }
 
 template <int BATCH>
-static void vc_launch_batch(int64_t pairs, const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
-                            VcListlessGuard guard, int64_t first_pair, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
-                            int64_t *header_host, int64_t *header_zero) {
-    const int64_t waves = (pairs + BATCH - 1) / BATCH;
+static void vc_launch_batch(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
+                            VcListlessGuard guard, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st) {
+    const int64_t ts = BATCH == 16 ? 4 : 8, waves = ((S.P + ts - 1) / ts) * ((S.P + BATCH / ts - 1) / (BATCH / ts));
     const size_t lds = sizeof(int64_t) * BATCH * (vc_hop_slots(S) + 2) + sizeof(int) * BATCH * 2;
-    hipLaunchKernelGGL(vc_copy_blocks_batch_kernel<BATCH>, dim3((unsigned)((waves + VC_XCDS - 1) / VC_XCDS * VC_XCDS)), dim3(VC_WAVE), lds, st, S,
-                       T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, header_host, header_zero);
+    for (int64_t done = 0; done < waves; done += VC_MAX_GRID) {
+        const int64_t now = waves - done < VC_MAX_GRID ? waves - done : VC_MAX_GRID;
+        hipLaunchKernelGGL(vc_copy_blocks_batch_kernel<BATCH>, dim3((unsigned)((now + VC_XCDS - 1) / VC_XCDS * VC_XCDS)), dim3(VC_WAVE), lds, st, S,
+                           T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage);
+    }
 }
 
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
-                                 int64_t *header_host, int64_t *header_zero, int64_t *totals) {
+                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals) {
     const int64_t npairs = (int64_t)S.P * S.P;
-    const int64_t step = lanes == VC_QUARTER || lanes == VC_BATCHED ? VC_MAX_GRID * VC_ITEMS_PER_WAVE : VC_MAX_GRID;
+    if (lanes == VC_BATCHED) {
+        if (verdict) return hipErrorInvalidValue;         // the batches are for more pairs than one launch with totals takes
+        const int batch = vc_batch_pairs(npairs);
+        (batch == 64 ? vc_launch_batch<64> : (batch == 32 ? vc_launch_batch<32> : vc_launch_batch<16>))(
+            S, T, slot_off, row_base, header, guard, sendbuf, recvbuf, stage, st);
+        return hipGetLastError();
+    }
+    const int64_t step = lanes == VC_QUARTER ? VC_MAX_GRID * VC_ITEMS_PER_WAVE : VC_MAX_GRID;
     for (int64_t done = 0; done < npairs; done += step) {
         const int64_t now = npairs - done < step ? npairs - done : step;
         const int64_t units = lanes == VC_QUARTER ? (now + VC_ITEMS_PER_WAVE - 1) / VC_ITEMS_PER_WAVE : now;
-        if (totals && done) return hipErrorInvalidValue;    // the totals belong to a call that one launch takes
-        const dim3 grid((unsigned)((units + VC_XCDS - 1) / VC_XCDS * VC_XCDS) + vc_totals_blocks(S, totals, lanes == VC_THREADS ? VC_THREADS : VC_WAVE));
-        if (lanes == VC_BATCHED) {
-            if (totals) return hipErrorInvalidValue;      // the batches are for more pairs than one launch with totals takes
-            const int batch = vc_batch_pairs(npairs);
-            if (batch == 64)
-                vc_launch_batch<64>(now, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, st, header_host, header_zero);
-            else if (batch == 32)
-                vc_launch_batch<32>(now, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, st, header_host, header_zero);
-            else
-                vc_launch_batch<16>(now, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, st, header_host, header_zero);
-        } else if (lanes == VC_QUARTER)
-            hipLaunchKernelGGL(vc_copy_blocks_quarter_kernel, grid, dim3(VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done,
-                               sendbuf, recvbuf, stage, header_host, header_zero, totals);
-        else if (lanes == VC_WAVE)
-            hipLaunchKernelGGL(vc_copy_blocks_kernel<VC_WAVE>, grid, dim3(VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done,
-                               sendbuf, recvbuf, stage, header_host, header_zero, totals);
-        else
-            hipLaunchKernelGGL(vc_copy_blocks_kernel<VC_THREADS>, grid, dim3(VC_THREADS), 0, st, S, T, slot_off, row_base, header, guard,
-                               done, sendbuf, recvbuf, stage, header_host, header_zero, totals);
+        if (verdict && done) return hipErrorInvalidValue;    // the totals belong to a call that one launch takes
+        const dim3 grid((unsigned)((units + VC_XCDS - 1) / VC_XCDS * VC_XCDS) + vc_totals_blocks(S, verdict, lanes == VC_THREADS ? VC_THREADS : VC_WAVE));
+        const auto kernel = lanes == VC_QUARTER ? vc_copy_blocks_quarter_kernel : (lanes == VC_WAVE ? vc_copy_blocks_kernel<VC_WAVE> : vc_copy_blocks_kernel<VC_THREADS>);
+        hipLaunchKernelGGL(kernel, grid, dim3(lanes == VC_THREADS ? VC_THREADS : VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done,
+                           sendbuf, recvbuf, stage, verdict, verdict_next, totals);
     }
     return hipGetLastError();
 }

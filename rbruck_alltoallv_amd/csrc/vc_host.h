@@ -87,9 +87,9 @@ struct vc_comm {
     int waits = 0;                        // times the host has waited for the stream in the call in progress
     int64_t items_before_last = 0;        // block pieces of the forwarded call before the one `hint` describes (0: there was none)
     DevBuf chain_row_tot, chain_row_base;
-    DevBuf strided_headers;               // fixed-stride calls: two headers used in turn
-    bool strided_clean = false;           // ... and the one the next call will use is known to be zero
-    int strided_turn = 0;
+    DevBuf verdicts;                      // fixed-stride calls: two sets of VC_VERDICTS words used in turn
+    bool verdict_clean = false;           // ... and the set the next call will use is known to be zero
+    int verdict_turn = 0;
     DevBuf slot_off, row_tot, row_base, org_run_base, item_row_tot, item_row_base, row_bytes, desc, header, launches, stage, rd_packed,
         scratch, max_state, ticket;
     double cal_copy_bytes_per_s = 0, cal_launch_s = 0, cal_sync_s = 0;   // calibrate(): the plain copy's rate, the cost of a
@@ -115,6 +115,7 @@ struct vc_comm {
     const void *last_stage = nullptr;     // staging arena of the last call
     int64_t *h_header = nullptr;          // pinned, coherent: the planner writes its header straight into it
     int64_t *h_header_dev = nullptr;      // the same memory as the device sees it
+                                          // (VC_TOTALS_AT words in: the totals of a call on fixed-stride staging, slot by slot)
     int *h_flags = nullptr, *h_flags_dev = nullptr;   // pinned, coherent: the two flags of vc_displs_from_counts, as host and device see
                                           // them; in a cache line of its own behind them (VC_DONE_AT) the word vc_wait_stream waits for
     unsigned done_value = 0;              // the value last enqueued for that word
@@ -156,6 +157,9 @@ struct BusyGuard {
     void keep() { mine = false; }         // the call stays in progress after the entry point returns (vc_comm_wait ends it)
 };
 #define VC_DONE_AT 32
+// words of h_header: the planner's header, then (in cache lines of their own) the slots of vc_totals_waves(P) wavefronts
+#define VC_TOTALS_AT ((VC_HEADER_WORDS(VC_MAX_LAUNCHES) + VC_TOTALS_SLOT - 1) / VC_TOTALS_SLOT * VC_TOTALS_SLOT)
+#define VC_HEADER_ROOM (VC_TOTALS_AT + VC_TOTALS_SLOT * (VC_STRIDED_MAX_PAIRS / VC_TOTALS_PER_WAVE))
 #define VC_FLAG_WORDS 64
 #define VC_SPIN_US 10000
 

@@ -1,0 +1,52 @@
+"""Calls served without a work-item list, at the edges of what their kernels do: blocks moved by one lane (up to 32 bytes), by a quarter
+of a wavefront or by a wavefront, rank counts that fill no tile of sources x receivers, blocks cut into pieces, whole aligned pieces."""
+import numpy as np
+import pytest
+import torch
+
+from rbruck_alltoallv_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def api():
+    from rbruck_alltoallv_amd import api
+    return api
+
+
+# ranks, longest block in bytes, radix, executions allowed after the first call (2: listless, 3: fixed-stride staging)
+@pytest.mark.parametrize("P,top,r,kinds", [(5, 33, 2, {3}), (64, 2050, 2, {3}), (127, 1500, 3, {3}), (191, 700, 8, {2, 3}), (197, 16, 2, {2}),
+                                           (321, 33, 4, {2}), (363, 200, 3, {2}), (725, 17, 3, {2}), (1021, 48, 32, {2})])
+def test_short_blocks_at_every_length(api, P, top, r, kinds):
+    rng = np.random.default_rng(P)
+    counts = rng.integers(0, top + 1, (P, P)).astype(np.int32)
+    counts[: min(P, 8), : min(P, 34)] = np.arange(min(P, 34))[None] * (np.arange(min(P, 34)) <= top)      # every short length
+    prob = W.make_problem(counts, 1, 1, 1)
+    dp = api.DeviceProblem(prob)
+    ds, want, got = dp.new_send_arena(), dp.new_recv_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, P, ds)
+    want.fill_(0xA5)
+    dp.comm.set_forwarding(0)
+    assert api.twophase_rbruck_alltoallv(r, dp, ds, want) == 0 and dp.verify(ds, want) == 0
+    dp.comm.set_forwarding(1)
+    for call in range(3):
+        got.fill_(0xA5)
+        assert api.twophase_rbruck_alltoallv(r, dp, ds, got) == 0, dp.comm.error()
+        assert torch.equal(got, want), (P, top, call)
+        assert call == 0 or dp.comm.last_stats().execution in kinds
+    dp.comm.free()
+
+
+@pytest.mark.parametrize("P,length", [(16, 4096), (16, 20000), (48, 8191)])
+def test_whole_pieces_on_fixed_stride_staging(api, P, length):
+    counts = np.full((P, P), length, dtype=np.int32)
+    counts[::3, ::2] -= 1
+    prob = W.make_problem(counts, 1, 0, 0)
+    dp = api.DeviceProblem(prob)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 9, ds)
+    for _ in range(3):
+        dr.zero_()
+        assert api.twophase_rbruck_alltoallv(2, dp, ds, dr) == 0 and dp.verify(ds, dr) == 0
+    dp.comm.free()

@@ -112,7 +112,9 @@ int vc_comm_set_forwarding(vc_comm_t comm, int enable);
  *    (hops - 1) x bytes (configuration 5 with radix 2: 60 GB);
  *  - forwarded execution keeps every hop's copy of every block, because nothing reads them and so nothing says when one
  *    may be overwritten.  A call whose staging would pass both the allowance (an eighth of the device's memory, at least
- *    1 GiB) and three times its payload is therefore run one launch per digit instead (vc_stats_t.execution says so).
+ *    1 GiB) and three times its payload is therefore run in batches of receivers that use the same staging memory one after
+ *    the other (blocking calls in the default mode of vc_comm_set_forwarding, when 8 batches suffice and none of them needs
+ *    more than 1.25 x the allowance), or one launch per digit instead (vc_stats_t.execution and n_launches say so).
  * Unbounded: every digit phase has its own region and forwarded calls stay forwarded, whatever they need. */
 int vc_comm_set_staging_bound(vc_comm_t comm, int enable);
 
@@ -324,7 +326,7 @@ int vc_comm_calibration(vc_comm_t comm, double *copy_bytes_per_s_out, double *la
 #define VC_MAX_LAUNCHES 1024
 
 typedef struct {
-    int32_t n_launches;          /* data-moving kernel launches of the last call (1 in forwarded execution) */
+    int32_t n_launches;          /* data-moving kernel launches of the last call (forwarded execution: 1, or one per batch) */
     int32_t n_digits;            /* digit phases among them */
     int64_t payload_bytes;       /* S: sum of all blocks */
     int64_t moved_bytes;         /* sum over all hops of the bytes copied (each hop counted once) */
@@ -335,7 +337,7 @@ typedef struct {
     float inter_ms;              /* launches between the nodes (orgData_time, prepSP_time, SP_time; intra_time / iteration_time of
                                     src/twolayer_communicator_linear.cpp:10-11 likewise).  Forwarded execution has one launch
                                     for both: its time is in intra_ms and inter_ms is 0. */
-    int64_t launch_bytes[VC_MAX_LAUNCHES];   /* bytes the hops of a launch copy (forwarded execution: [0] = moved_bytes) */
+    int64_t launch_bytes[VC_MAX_LAUNCHES];   /* bytes the hops of a launch copy (forwarded execution in one launch: [0] = moved_bytes) */
     float launch_ms[VC_MAX_LAUNCHES];  /* per data-moving launch, HIP events on the comm's stream */
     int32_t execution;           /* how the call ran: 0 launch per digit, 1 forwarded through a work-item list, 2 forwarded
                                     without one, 3 forwarded without one on fixed-stride staging (see vc_comm_set_forwarding) */

@@ -169,9 +169,20 @@ bool staging_out_of_bound(const vc_comm *c, int64_t stage_bytes, int64_t payload
     return c->bound_staging && stage_bytes > c->staging_allowance && stage_bytes > 3 * payload_bytes;
 }
 
+// In the default mode such a call stays forwarded where it can: in batches of receivers that use the same staging memory one after the
+// other, each within the allowance.  0: more than VC_MAX_BATCHES of them, or a mode that runs the call one launch per digit.
+// Measured on MI355X: configuration 5 with radix 2 (512 ranks, 17.2 GB, 60 GB of staging) 25.9 ms -> 14.8.  (Not more batches than it
+// takes: every one is planned and listed for itself, 0.2 ms.)
+#define VC_MAX_BATCHES 8
+int staging_batches(const vc_comm *c, int64_t stage_bytes) {
+    const int64_t batches = (stage_bytes + c->staging_allowance - 1) / c->staging_allowance;
+    return c->forward == 1 && batches <= std::min(VC_MAX_BATCHES, c->P) ? (int)batches : 0;
+}
+
 // What the planner leaves behind for the copy launches.
 struct PlanInfo {
     int nl = 0, n_digits = 0;
+    int batches = 1;                                // launches of forwarded execution
     int recv_lo = 0;
     int64_t stage_bytes = 0, payload_bytes = 0;
     std::vector<int64_t> first, count, bytes;       // per launch: first work item, item count, bytes moved
@@ -365,7 +376,7 @@ static int launch_items(vc_comm *c, const PlanInfo &pi, const void *items_any, c
 
 // After the final synchronisation: the statistics of the call.
 static int finish_stats(vc_comm *c, const PlanInfo &pi, const void *items_any, bool planned_now) {
-    const int nl = pi.chain ? 1 : pi.nl;              // kernel launches of this execution
+    const int nl = pi.chain ? pi.batches : pi.nl;     // kernel launches of this execution
     vc_stats_t &s = c->stats;
     s.n_launches = nl;
     s.n_digits = pi.n_digits;
@@ -379,12 +390,14 @@ static int finish_stats(vc_comm *c, const PlanInfo &pi, const void *items_any, b
     s.bad_table_entries = 0;
     s.host_waits = c->waits;
     s.plan_ms = s.total_ms = s.intra_ms = s.inter_ms = 0.f;
-    if (pi.chain) {                                   // one launch that performs the hops of every digit
-        for (int k = 0; k < pi.nl; k++) s.moved_bytes += pi.bytes[k];
-        s.launch_bytes[0] = s.moved_bytes;
-        s.launch_ms[0] = 0.f;
-        if (c->timing) HIP_TRY(hipEventElapsedTime(&s.launch_ms[0], c->events[2], c->events[3]));
-        s.intra_ms = s.launch_ms[0];
+    if (pi.chain) {                                   // launches that perform the hops of every digit
+        for (int k = 0; k < nl; k++) {
+            s.launch_bytes[k] = pi.bytes[k];
+            s.moved_bytes += pi.bytes[k];
+            s.launch_ms[k] = 0.f;
+            if (c->timing) HIP_TRY(hipEventElapsedTime(&s.launch_ms[k], c->events[2 + 2 * k], c->events[3 + 2 * k]));
+            s.intra_ms += s.launch_ms[k];
+        }
         s.lanes_per_item = pi.chain_lanes;
         c->items_before_last = c->hint.valid ? c->hint.items : 0;
         c->hint = VcHint{1, pi.chain_items, pi.payload_bytes, pi.max_pieces, pi.max_len};
@@ -403,7 +416,7 @@ static int finish_stats(vc_comm *c, const PlanInfo &pi, const void *items_any, b
     }
     if (c->timing) {
         if (planned_now) HIP_TRY(hipEventElapsedTime(&s.plan_ms, c->events[0], c->events[c->plan_end]));
-        HIP_TRY(hipEventElapsedTime(&s.total_ms, c->events[planned_now ? 0 : 2], c->events[2 + nl]));
+        HIP_TRY(hipEventElapsedTime(&s.total_ms, c->events[planned_now ? 0 : 2], c->events[pi.chain ? 1 + 2 * nl : 2 + nl]));
     }
     c->last_nlaunch = pi.chain ? 0 : nl;              // per-launch traffic can only be inspected after launch-per-digit execution
     c->last_items = static_cast<const VcDesc *>(items_any);
@@ -543,6 +556,40 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
     return rc ? rc : 1;
 }
 
+// A forwarded call out of the staging bound in `batches` batches of receivers: each is planned, listed and copied for itself on the
+// same staging memory (S.recv_from, S.recv_num).  `all`: the plan of the whole call, which has been read and found in order.
+// Returns 1: served; 0: a batch needs more staging than the communicator allows (very uneven receivers), < 0: errors.
+static int run_batches(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, VcTables T, const char *sendbuf, char *recvbuf, PlanInfo all, int batches) {
+    hipStream_t st = c->stream;
+    if (c->timing) { int rc = ensure_events(c, 2 + 2 * (size_t)batches); if (rc) return rc; }
+    all.stage_bytes = 0;
+    all.batches = batches;
+    all.bytes.assign(batches, 0);
+    for (int b = 0; b < batches; b++) {
+        S.recv_from = (int)((int64_t)c->P * b / batches);
+        S.recv_num = (int)((int64_t)c->P * (b + 1) / batches) - S.recv_from;
+        int rc = enqueue_plan_sizes(c, S, L, T, true, false);
+        if (rc) return rc;
+        HIP_TRY(VC_WAIT(c));
+        PlanInfo pi;
+        rc = plan_read(c, S, L, pi, true);
+        if (rc) return rc;
+        if (pi.stage_bytes > c->staging_allowance + (c->staging_allowance >> 2)) return 0;
+        rc = plan_emit(c, S, L, T, c->desc, pi);
+        if (rc) return rc;
+        HIP_TRY(reserve_stage(c, (size_t)pi.stage_bytes + 64));
+        if (c->timing) HIP_TRY(hipEventRecord(c->events[2 + 2 * b], st));
+        HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>(), pi.chain_stride, pi.chain_items, all.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+        if (c->timing) HIP_TRY(hipEventRecord(c->events[3 + 2 * b], st));
+        all.stage_bytes = std::max(all.stage_bytes, pi.stage_bytes);
+        all.bytes[b] = pi.bytes[0];
+    }
+    HIP_TRY(VC_WAIT(c));
+    const int rc = finish_stats(c, all, c->desc.p, true);
+    c->hint.valid = 0;                                    // (the next call of the kind looks at its plan before it sends out a list)
+    return rc ? rc : 1;
+}
+
 static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, char *recvbuf, VcTables T, bool forward, bool reuse = false) {
     VcSched S;
     std::vector<VcLaunchInfo> L;
@@ -596,7 +643,12 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
         rc = plan_read(c, S, L, pi, forward);
         if (rc) return rc;
     }
-    if (forward && staging_out_of_bound(c, pi.stage_bytes, pi.payload_bytes)) return run_schedule(c, q, sendbuf, recvbuf, T, false, true);
+    if (forward && staging_out_of_bound(c, pi.stage_bytes, pi.payload_bytes)) {
+        const int batches = staging_batches(c, pi.stage_bytes);
+        rc = batches ? run_batches(c, S, L, T, sendbuf, recvbuf, pi, batches) : 0;
+        if (rc) return rc < 0 ? rc : VC_OK;
+        return run_schedule(c, q, sendbuf, recvbuf, T, false, true);
+    }
     if (!forward && worth_reusing(c, S, pi.stage_bytes)) return run_schedule(c, q, sendbuf, recvbuf, T, false, true);
     rc = plan_emit(c, S, L, T, c->desc, pi);
     if (rc) return rc;

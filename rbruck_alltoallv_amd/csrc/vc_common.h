@@ -123,10 +123,14 @@ struct VcSched {
                       //    holds for one destination rank back to back in source order — so that an inter-node message
                       //    is a contiguous copy (TTPL_BT_alltoallv, src/twophase_twolayer_rbruck.cpp:388-398, 430-453).
                       //    The organized region is staging region number w.
+    int recv_from, recv_num;    // forwarded execution through a list: the plan and the list hold the blocks for receivers recv_from ..
+                      //    recv_from + recv_num - 1 only (all of them unless a call runs in batches)
     // set by vc_set_divisors once n, G, r and P are final:
     VcRankDivisor dn, dr;                         // division of ranks, slots and offsets by n, r
     VcDivisor dP;                                 // division of pair numbers by P
 };
+
+VC_HD bool vc_receives_now(const VcSched &S, int t) { return (unsigned)(t - S.recv_from) < (unsigned)S.recv_num; }
 
 VC_HD void vc_set_divisors(VcSched &S) {
     S.dn = vc_make_rank_divisor(S.n > 0 ? S.n : 1);

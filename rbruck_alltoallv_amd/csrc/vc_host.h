@@ -194,4 +194,5 @@ inline hipError_t vc_wait_stream(vc_comm *c) {
 // ---- defined in vc_api.hip, used by vc_tools.hip ----
 int ensure_events(vc_comm *c, size_t n);
 bool staging_out_of_bound(const vc_comm *c, int64_t stage_bytes, int64_t payload_bytes);
+int staging_batches(const vc_comm *c, int64_t stage_bytes);
 VcTables make_tables(vc_comm *c, const int *sc, const int *sd, const int *rc, const int *rd);

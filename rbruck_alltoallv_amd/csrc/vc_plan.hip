@@ -350,6 +350,7 @@ __device__ __forceinline__ int64_t vc_shared(const int64_t *p) { return __hip_at
 // the bytes of the blocks in them (every staged block is one hop); the last row counts the chain items of the blocks that end
 // on the rank (by tile of VC_TILE_RANKS sources for vc_chain_emit), the payload, the table entries no rank could have
 // passed, the most pieces and the longest of its blocks.
+// A call in batches counts the slots, items and bytes of the blocks for the receivers of the batch only, and checks all of the tables.
 // row_bytes rows: [region][P] bytes of staged blocks, then [payload][P], [bad entries][P], [longest block][P].
 // chain_row_tot: [P] items, [P] most pieces, [P][tiles] items per tile of sources.
 // The workgroup that finishes last turns the row totals into first addresses (row_base, chain_row_base: exclusive sums) and
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTable
             for (int u = 0; u < PER; u++) {                 // all reads first: none depends on another
                 int s, t;
                 const bool inside = id0 + u < P;
-                there[u] = vc_slot_block(S, y, to, inside ? id0 + u : 0, s, t) && inside;
+                there[u] = vc_slot_block(S, y, to, inside ? id0 + u : 0, s, t) && inside && vc_receives_now(S, t);
                 count[u] = vc_sc(S, T, s, t); displ[u] = vc_rd(S, T, t, s); rbase[u] = T.rbase[t];
             }
 #pragma unroll
@@ -403,6 +404,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTable
         if (threadIdx.x == 0) { vc_share(&row_tot[(int64_t)y * P + to], carry); vc_share(&row_bytes[(int64_t)y * P + to], data); }
     } else if (to < P) {
         const int ntile = VC_TILES(P), lanes = VC_TILE_RANKS / PER;              // threads per tile of sources
+        const bool now = vc_receives_now(S, to);
         int64_t sum[5] = {0, 0, 0, 0, 0};                 // items, payload, bad entries; most pieces, longest block
         for (int base = 0; base < P; base += PER * VC_THREADS) {
             const int s0 = base + threadIdx.x * PER;
@@ -418,9 +420,9 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTable
                 if (s0 + u >= P) continue;
                 const int64_t len = (int64_t)e[u].sent * S.esz;
                 const int cut = (int)((rbase + (int64_t)e[u].rd * S.esz + S.recv_lo) & (VC_PIECE - 1));
-                const int64_t cnt = vc_chunk_count(len, cut & (VC_LINE - 1), cut);
+                const int64_t cnt = now ? vc_chunk_count(len, cut & (VC_LINE - 1), cut) : 0;
                 tile += cnt;
-                sum[1] += (int64_t)e[u].expected * S.esz;
+                sum[1] += now ? (int64_t)e[u].expected * S.esz : 0;
                 sum[2] += vc_bad_entries(S, e[u]);
                 sum[3] = cnt > sum[3] ? cnt : sum[3];
                 sum[4] = len > sum[4] ? len : sum[4];
@@ -533,17 +535,31 @@ hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_o
 // The items of a tile's blocks are neighbours in the list: where there are no more than VC_EMIT_TILE_ITEMS of them they are put
 // together in LDS and stored as whole cache lines (item by item a wavefront's store touches 64 places 40 bytes apart;
 // 1 Mi items: 34 -> 26 us with that and the reads of all hops together).
-// Big blocks are written by the whole workgroup as in vc_plan_emit.
+// Blocks of many pieces are written by the whole workgroup, and `shares` workgroups share those of a slice.  512 ranks, 32 blocks of 256
+// pieces each, nine hop slots, one of two batches: 460 us (an item a thread, its route worked out again for every piece) -> 86.
 #define VC_EMIT_TILE_ITEMS 64
+#define VC_EMIT_UNIT 256
+#define VC_EMIT_GROUP 32
+static_assert(VC_MAX_HOP_SLOTS <= VC_EMIT_GROUP, "a hop slot per lane");
 // ROUTE: hop slots of a route kept in registers, 3 or 6 (two-layer calls and large radices have no more than 3, and the registers of 6
 // would cost them a third of the wavefronts in flight); with more the route is worked out again for every piece.
 #define VC_ROUTE_CACHE 6
 static_assert(VC_TILE_RANKS * VC_ROUTE_CACHE <= VC_EMIT_TILE_ITEMS * (VC_CHAIN_HEAD + 1), "routes of a tile's big blocks in the place of its items");
+// The last of VC_THREADS ascending numbers that is no larger than x (the first one is 0).
+__device__ __forceinline__ int vc_last_at_or_below(const int64_t *of, int64_t x) {
+    int lo = 0, hi = VC_THREADS - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (of[mid] <= x) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
 template <int ROUTE>
 __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                             const int64_t *__restrict__ row_base, const int64_t *__restrict__ chain_row_base,
                                                             const int64_t *__restrict__ tile_items, int nchunk, int slices,
-                                                            int64_t *__restrict__ items, const int64_t *__restrict__ header,
+                                                            int shares, int64_t *__restrict__ items, const int64_t *__restrict__ header,
                                                             int64_t cap_items) {
     // [tiles of the workgroup][VC_EMIT_TILE_ITEMS][stride]: a tile's items, or, in a tile with blocks of many pieces, the routes of
     // these, [VC_TILE_RANKS][ROUTE], while the whole workgroup writes their items
@@ -551,12 +567,14 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
     __shared__ int64_t big_at[VC_THREADS], big_pre[VC_THREADS];
     __shared__ int big_nhop[VC_THREADS];
-    const int P = S.P, ntile = VC_TILES(P), parts = nchunk * slices, ranks_per_xcd = (P + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS;
-    const int at_xcd = blockIdx.x / VC_PLAN_XCDS, part = at_xcd % parts, t = (int)(blockIdx.x % VC_PLAN_XCDS) * ranks_per_xcd + at_xcd / parts;
-    if (t >= P) return;
+    __shared__ int64_t field[VC_THREADS / VC_EMIT_GROUP][VC_CHAIN_HEAD + VC_MAX_HOP_SLOTS];
+    const int P = S.P, ntile = VC_TILES(P), ranks_per_xcd = (P + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS;
+    // (part by part, the ranks of the XCD in each: ranks with work only in some of the parts keep every compute unit busy)
+    const int at_xcd = blockIdx.x / VC_PLAN_XCDS, part = at_xcd / ranks_per_xcd, t = (int)(blockIdx.x % VC_PLAN_XCDS) * ranks_per_xcd + at_xcd % ranks_per_xcd;
+    if (t >= P || !vc_receives_now(S, t)) return;
     const int stride = VC_CHAIN_HEAD + vc_hop_slots(S);
     const bool cached = vc_hop_slots(S) <= ROUTE;
-    const int chunk = part / slices, z = part % slices;
+    const int share_no = part / (nchunk * slices), chunk = part / slices % nchunk, z = part % slices;
     const int c_lo = chunk * VC_THREADS, c_hi = c_lo + VC_THREADS < P ? c_lo + VC_THREADS : P;
     const int slice = ((c_hi - c_lo + slices - 1) / slices + VC_TILE_RANKS - 1) / VC_TILE_RANKS * VC_TILE_RANKS;      // whole tiles
     const int s_lo = c_lo + z * slice < c_hi ? c_lo + z * slice : c_hi, s_hi = s_lo + slice < c_hi ? s_lo + slice : c_hi;
@@ -627,7 +645,8 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
     const bool any_big = (__ballot(big) >> (threadIdx.x % VC_WAVE / VC_TILE_RANKS * VC_TILE_RANKS) & 0xFFFFFFFFull) != 0;
     const bool together = cached && !any_big && in_tile <= VC_EMIT_TILE_ITEMS;
     int64_t *const tile_buf = tile_lds + (int64_t)tile * VC_EMIT_TILE_ITEMS * stride;
-    if (cached && cnt > 0) {
+    const bool small = cnt > 0 && !big && share_no == 0;
+    if (cached && (small || big)) {
         int64_t d[ROUTE];
         unsigned moves = 0;
 #pragma unroll
@@ -651,41 +670,65 @@ __global__ __launch_bounds__(VC_THREADS) void vc_chain_emit(VcSched S, VcTables 
                     if (moves >> k & 1) item[VC_CHAIN_HEAD + n++] = d[k] + lo;
             }
         } else {
-            big_at[threadIdx.x] = at;
             big_nhop[threadIdx.x] = nhop;
             int n = 0;
 #pragma unroll
             for (int k = 0; k < ROUTE; k++)
                 if (moves >> k & 1) tile_buf[lane_in_tile * ROUTE + n++] = d[k];
         }
-    } else if (!big) {
+    } else if (small) {
         for (int64_t c = 0; c < cnt; c++) vc_chain_item(S, T, slot_off, row_base, s, t, c, items + (at + c) * stride);
-    } else {
-        big_at[threadIdx.x] = at;
     }
+    big_at[threadIdx.x] = at;
     const bool wg_big = __syncthreads_or(big);            // (also: the tiles in LDS are complete)
-    if (together)
+    if (together && share_no == 0)
         for (int k = lane_in_tile; k < (int)in_tile * stride; k += VC_TILE_RANKS) items[first * stride + k] = tile_buf[k];
-    if (wg_big) {
+    if (!wg_big) return;
+    if (cached) {                                         // an item a thread
         int64_t btotal;
         big_pre[threadIdx.x] = vc_block_exclusive_scan(big ? cnt : 0, lds, btotal);
         __syncthreads();
-        for (int64_t q = threadIdx.x; q < btotal; q += VC_THREADS) {
-            int lo = 0, hi = VC_THREADS - 1;              // last lane whose pieces start at or before q
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (big_pre[mid] <= q) lo = mid; else hi = mid - 1;
-            }
-            const int64_t c = q - big_pre[lo];
-            const int sb = s_lo + lo;
-            if (cached)
-                vc_chain_piece(VC_SPACE_SEND | vc_send_offset(S, T, sb, t), (int64_t)vc_sc(S, T, sb, t) * S.esz, vc_phase(S, T, sb, t),
-                               vc_chain_cut(S, T, sb, t), c,
-                               tile_lds + (int64_t)(lo / VC_TILE_RANKS) * VC_EMIT_TILE_ITEMS * stride + lo % VC_TILE_RANKS * ROUTE, big_nhop[lo],
-                               items + (big_at[lo] + c) * stride);
-            else
-                vc_chain_item(S, T, slot_off, row_base, sb, t, c, items + (big_at[lo] + c) * stride);
+        for (int64_t q = share_no * VC_THREADS + threadIdx.x; q < btotal; q += shares * VC_THREADS) {
+            const int b = vc_last_at_or_below(big_pre, q), sb = s_lo + b;
+            vc_chain_piece(VC_SPACE_SEND | vc_send_offset(S, T, sb, t), (int64_t)vc_sc(S, T, sb, t) * S.esz, vc_phase(S, T, sb, t),
+                           vc_chain_cut(S, T, sb, t), q - big_pre[b],
+                           tile_lds + (int64_t)(b / VC_TILE_RANKS) * VC_EMIT_TILE_ITEMS * stride + b % VC_TILE_RANKS * ROUTE, big_nhop[b],
+                           items + (big_at[b] + q - big_pre[b]) * stride);
         }
+        return;
+    }
+    // With more hop slots than a thread keeps, half a wavefront takes VC_EMIT_UNIT pieces of a block at a time: a hop slot per lane, then
+    // the items word by word, whole cache lines at once.
+    int64_t units;
+    big_pre[threadIdx.x] = vc_block_exclusive_scan(big ? (cnt + VC_EMIT_UNIT - 1) / VC_EMIT_UNIT : 0, lds, units);
+    __syncthreads();
+    const int lane = threadIdx.x % VC_EMIT_GROUP, group = threadIdx.x / VC_EMIT_GROUP, groups = VC_THREADS / VC_EMIT_GROUP;
+    const int step_c = VC_EMIT_GROUP / stride, step_f = VC_EMIT_GROUP % stride;
+    int64_t *const f_of = field[group];
+    for (int64_t u = share_no * groups + group; u < units; u += shares * groups) {
+        const int b = vc_last_at_or_below(big_pre, u), sb = s_lo + b;
+        const int64_t to = vc_recv_offset(S, T, sb, t), from = vc_send_offset(S, T, sb, t), blen = (int64_t)vc_sc(S, T, sb, t) * S.esz;
+        const VcHop h = vc_hop_place(S, sb, t, lane < nslots ? lane : 0);
+        const int64_t dst = vc_hop_dst(S, h, vc_slot_addr(S, slot_off, row_base, h), to);
+        const unsigned moves = (unsigned)(__ballot(lane < nslots && h.moves) >> (threadIdx.x % VC_WAVE - lane));
+        const int bcut = (int)((to + S.recv_lo) & (VC_PIECE - 1)), nhop = __popc(moves), fields = VC_CHAIN_HEAD + nhop;
+        if (lane == 0) { f_of[VC_CHAIN_SRC] = VC_SPACE_SEND | from; f_of[VC_CHAIN_LEN] = 0; f_of[VC_CHAIN_NHOP] = nhop; }
+        if (moves >> lane & 1) f_of[VC_CHAIN_HEAD + __popc(moves & ((1u << lane) - 1))] = dst;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int64_t begin = (u - big_pre[b]) * VC_EMIT_UNIT, left = vc_chunk_count(blen, bcut & (VC_LINE - 1), bcut) - begin;
+        const int words = (int)(left < VC_EMIT_UNIT ? left : VC_EMIT_UNIT) * stride;
+        int64_t *const out = items + (big_at[b] + begin) * stride;
+        int f = lane % stride;
+        int64_t start = (begin + lane / stride) * VC_PIECE - bcut;      // of the piece inside the block (below 0: the first one's)
+        for (int q = lane; q < words; q += VC_EMIT_GROUP) {
+            const int64_t lo = start > 0 ? start : 0, hi = start + VC_PIECE < blen ? start + VC_PIECE : blen;
+            if (f < fields) out[q] = f_of[f] + (f == VC_CHAIN_LEN ? hi - lo : (f == VC_CHAIN_NHOP ? 0 : lo));
+            start += step_c * VC_PIECE; f += step_f;
+            if (f >= stride) { f -= stride; start += VC_PIECE; }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();                  // (the fields are read before the next unit's take their place)
     }
 }
 
@@ -694,14 +737,16 @@ hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const uint32_t *sl
                                 const int64_t *header, int64_t cap_items) {
     const int nchunk = (S.P + VC_THREADS - 1) / VC_THREADS;
     // at least ~1024 workgroups (four per compute unit), each a whole number of tiles of sources
-    int slices = nchunk > 1 ? 1 : vc_emit_slices(nitems, S.P);
-    if (nchunk == 1)
-        while (slices < 8 && (int64_t)S.P * slices < 1024 && S.P / (slices * 2) >= VC_TILE_RANKS) slices *= 2;
+    int slices = 1;
+    while (nchunk == 1 && slices < 8 && (int64_t)S.P * slices < 1024 && S.P / (slices * 2) >= VC_TILE_RANKS) slices *= 2;
+    // workgroups that share the long blocks of a slice: one per ~2048 items of an average slice
+    const int64_t per_slice = nitems / ((int64_t)S.P * nchunk * slices);
+    const int shares = (int)std::max<int64_t>(1, std::min<int64_t>(64, per_slice / 2048));
     const int stride = VC_CHAIN_HEAD + vc_hop_slots(S), tiles = (std::min(S.P, VC_THREADS) + VC_TILE_RANKS - 1) / VC_TILE_RANKS;
     const size_t lds = vc_hop_slots(S) <= VC_ROUTE_CACHE ? sizeof(int64_t) * tiles * VC_EMIT_TILE_ITEMS * stride : 0;
     const auto kernel = vc_hop_slots(S) <= 3 ? vc_chain_emit<3> : vc_chain_emit<VC_ROUTE_CACHE>;
-    hipLaunchKernelGGL(kernel, dim3(vc_rank_grid(S.P, nchunk * slices)), dim3(VC_THREADS), lds, st, S, T, slot_off, row_base, chain_row_base,
-                       chain_row_tot + 2 * (size_t)S.P, nchunk, slices, items, header, cap_items);
+    hipLaunchKernelGGL(kernel, dim3(vc_rank_grid(S.P, nchunk * slices * shares)), dim3(VC_THREADS), lds, st, S, T, slot_off, row_base, chain_row_base,
+                       chain_row_tot + 2 * (size_t)S.P, nchunk, slices, shares, items, header, cap_items);
     return hipGetLastError();
 }
 

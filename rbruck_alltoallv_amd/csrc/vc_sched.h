@@ -118,7 +118,7 @@ inline int vc_make_schedule(VcFunc f, int P, int n, int r, int batch, int esz, i
                             std::vector<VcLaunchInfo> &L, int batch2 = 0, bool forward = false) {
     memset(&S, 0, sizeof S);
     L.clear();
-    S.P = P; S.esz = esz; S.uniform = uniform_count; S.table_mask = -1;
+    S.P = P; S.esz = esz; S.uniform = uniform_count; S.table_mask = -1; S.recv_num = P;
     if (forward) batch = batch2 = 0;                        // one kernel performs every hop: batches of rounds mean nothing
 
     int d = 0;

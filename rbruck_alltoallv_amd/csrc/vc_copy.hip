@@ -129,11 +129,12 @@ __global__ __launch_bounds__(LANES) void vc_copy_chains_kernel(const int64_t *__
     const unsigned per = gridDim.x / VC_XCDS;
     const unsigned idx = (blockIdx.x % VC_XCDS) * per + blockIdx.x / VC_XCDS;
     if (idx >= nitems) return;
-    if (GUARDED && (!vc_chain_guard_ok(header, guard) || (int64_t)idx >= header[2])) return;
-    const int64_t *it = items + (int64_t)idx * stride;
+    const int64_t *it = items + (int64_t)idx * stride;    // (there is room for nitems items, whatever is in them)
     const int64_t len = it[VC_CHAIN_LEN];
     const int nhop = (int)it[VC_CHAIN_NHOP];
-    if (len <= 0 || nhop <= 0) return;
+    bool ok = (len > 0) & (nhop > 0);                     // (one condition: item and header are read together)
+    if (GUARDED) ok = ok & vc_chain_guard_ok(header, guard) & ((int64_t)idx < header[2]);
+    if (!ok) return;
     const char *src = vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage);
     char *dst = vc_resolve(it[VC_CHAIN_HEAD], sendbuf, recvbuf, stage);
     const int w = (int)((uintptr_t)dst & (VC_LINE - 1)), lane = threadIdx.x % VC_WAVE;

@@ -739,9 +739,10 @@ hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const uint32_t *sl
     // at least ~1024 workgroups (four per compute unit), each a whole number of tiles of sources
     int slices = 1;
     while (nchunk == 1 && slices < 8 && (int64_t)S.P * slices < 1024 && S.P / (slices * 2) >= VC_TILE_RANKS) slices *= 2;
-    // workgroups that share the long blocks of a slice: one per ~2048 items of an average slice
-    const int64_t per_slice = nitems / ((int64_t)S.P * nchunk * slices);
-    const int shares = (int)std::max<int64_t>(1, std::min<int64_t>(64, per_slice / 2048));
+    // workgroups that share the long blocks of a slice: one per ~2048 items of an average slice, and of slices with 256 items or more as
+    // many as bring the grid to that size
+    const int64_t wgs = (int64_t)S.P * nchunk * slices, per_slice = nitems / wgs;
+    const int shares = (int)std::min<int64_t>(64, std::max<int64_t>(1, std::max(per_slice / 2048, std::min(per_slice / 256, 1024 / wgs))));
     const int stride = VC_CHAIN_HEAD + vc_hop_slots(S), tiles = (std::min(S.P, VC_THREADS) + VC_TILE_RANKS - 1) / VC_TILE_RANKS;
     const size_t lds = vc_hop_slots(S) <= VC_ROUTE_CACHE ? sizeof(int64_t) * tiles * VC_EMIT_TILE_ITEMS * stride : 0;
     const auto kernel = vc_hop_slots(S) <= 3 ? vc_chain_emit<3> : vc_chain_emit<VC_ROUTE_CACHE>;

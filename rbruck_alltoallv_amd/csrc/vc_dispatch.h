@@ -15,6 +15,9 @@
 //  * ... a batch of 16 - 64 pairs per wavefront when the blocks are so short that working out the routes costs more than
 //    moving the bytes: on 192 - 2048 ranks 5 - 40 % faster than the quarter up to an average block of 256 bytes, even at
 //    512, 3 - 16 % slower beyond.  Not on at most 128 ranks, where batches would leave most of the chip without a wavefront.
+//  * ... for the functions that send every block straight to its destination (nothing is staged, the plan is the check of the
+//    tables) a quarter of a wavefront up to an average block of 3 KiB on at most 362 ranks: 150 ranks, 1 and 2 KiB 31 -> 24 and
+//    39 -> 36, 300 ranks 61 -> 60 and 97 -> 91; even on 512 ranks, where a list makes up for itself.
 //  * ... a wavefront (average piece below 3 KiB) or a workgroup per pair: at most 128 ranks and 32768 pieces (26 - 42
 //    against 40 - 57 through the list at 16 and 64 ranks with blocks up to 8 KB, 31 - 77 against 48 - 92 up to 32 KB; a few
 //    per cent at 128 ranks; at 256 ranks the list wins).
@@ -37,6 +40,7 @@
 #define VC_LISTLESS_WG_MAX_PIECES 16          // pieces of one block: wavefront or workgroup per pair
 #define VC_LISTLESS_QUARTER_BELOW 768         // average piece below which pairs get a quarter of a wavefront, more than 128 ranks
 #define VC_LISTLESS_BATCH_BELOW 384           // average piece below which a wavefront takes a batch of pairs
+#define VC_LISTLESS_DIRECT_PAIRS (1 << 17)    // direct functions: a quarter of a wavefront per pair up to VC_LISTLESS_WAVE_BELOW
 #define VC_LISTLESS_WAVE_BELOW 3072           // average piece below which a pair gets a wavefront instead of a workgroup
 #define VC_LISTLESS_MAX_AVERAGE 4096          // a call the short-block kernels were chosen for must stay below this average
 #define VC_STRIDED_MAX_BYTES ((int64_t)256 << 20)
@@ -90,6 +94,8 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
         d.lanes = VC_THREADS;
     else if (h.valid && small_comm && h.max_pieces <= VC_LISTLESS_WG_MAX_PIECES && h.items <= VC_LISTLESS_MAX_ITEMS)
         d.lanes = average < VC_LISTLESS_WAVE_BELOW ? VC_WAVE : VC_THREADS;
+    else if (h.valid && S.w + S.w2 == 0 && pairs <= VC_LISTLESS_DIRECT_PAIRS && h.max_pieces <= VC_LISTLESS_MAX_PIECES && average < VC_LISTLESS_WAVE_BELOW)
+        d.lanes = VC_QUARTER;
     else
         return d;                                         // no hint yet, or long blocks: the list
     if (listless_only) return d;                          // nothing to fall back to: whatever the call turns out to be, it runs

@@ -50,3 +50,18 @@ def test_whole_pieces_on_fixed_stride_staging(api, P, length):
         dr.zero_()
         assert api.twophase_rbruck_alltoallv(2, dp, ds, dr) == 0 and dp.verify(ds, dr) == 0
     dp.comm.free()
+
+
+# ranks, block length around which the lengths lie, execution after the first call: the list beyond 362 ranks or 3 KiB
+@pytest.mark.parametrize("P,around,execution", [(150, 1000, 3), (150, 2900, 3), (200, 2000, 2), (363, 2000, 1), (200, 3500, 1)])
+def test_direct_functions(api, P, around, execution):
+    counts = np.random.default_rng(P).integers(around - 900, around + 100, (P, P)).astype(np.int32)
+    prob = W.make_problem(counts, 1, 1, 1)
+    dp = api.DeviceProblem(prob)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 4, ds)
+    for call in range(3):
+        dr.zero_()
+        assert api.spreadout_alltoallv(dp, ds, dr) == 0 and dp.verify(ds, dr) == 0, dp.comm.error()
+        assert call == 0 or dp.comm.last_stats().execution == execution
+    dp.comm.free()

@@ -50,6 +50,11 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, VC_FLAG_WORDS * sizeof(int), hipHostMallocCoherent);
     if (e == hipSuccess) memset(c->h_flags, 0, VC_FLAG_WORDS * sizeof(int));
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_flags_dev, c->h_flags, 0);
+    if (e == hipSuccess) e = c->ticket.reserve(VC_TICKET_BYTES);
+    if (e == hipSuccess) {
+        const std::vector<char> zeros(VC_TICKET_BYTES, 0);
+        e = hipMemcpy(c->ticket.p, zeros.data(), zeros.size(), hipMemcpyHostToDevice);
+    }
     if (e != hipSuccess) {
         (void)vc_comm_free(c);
         return fail_hip(e, "vc_comm_create", __LINE__);
@@ -235,10 +240,6 @@ static int reserve_plan_bufs(vc_comm *c, const VcSched &S, int nl, bool forward)
     if (forward) {
         HIP_TRY(c->chain_row_tot.reserve(z.chain_row_tot));
         HIP_TRY(c->chain_row_base.reserve(z.chain_row_base));
-        if (!c->ticket.p) {
-            HIP_TRY(c->ticket.reserve(VC_TICKET_BYTES));
-            HIP_TRY(hipMemsetAsync(c->ticket.p, 0, VC_TICKET_BYTES, c->stream));
-        }
     }
     if (S.packed_recv) HIP_TRY(c->rd_packed.reserve(z.rd_packed));
     PlanBufs &B = c->B;

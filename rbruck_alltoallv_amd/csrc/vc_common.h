@@ -180,12 +180,15 @@ struct VcTables {
 // ---- launchers implemented in the .hip files (all asynchronous on `st`) ----
 
 // vc_meta.hip
-hipError_t vc_launch_transpose(const int *in, int *out, int P, hipStream_t st);
+// The word in pinned host memory a kernel stores `value` to when all it was launched for has been stored (vc_signal); ticket:
+// VC_TICKET_BYTES that are zero before and after.  word null: it does not.
+struct VcSignal { unsigned *word; unsigned value; unsigned *ticket; };
+hipError_t vc_launch_transpose(const int *in, int *out, int P, hipStream_t st, VcSignal sig);
 // flags (device, 2 ints the caller has zeroed, or null): [0] set when a row's total passes INT_MAX, [1] when a count is negative
-hipError_t vc_launch_row_scan(const int *counts, int *displs, int64_t *extent, int *flags, int P, hipStream_t st);
-hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_t *base, int64_t *total, int P, hipStream_t st);
+hipError_t vc_launch_row_scan(const int *counts, int *displs, int64_t *extent, int *flags, int P, hipStream_t st, VcSignal sig = VcSignal());
+hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_t *base, int64_t *total, int P, hipStream_t st, VcSignal sig);
 // state: 65 words, the first one zero before and after
-hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, int *state, hipStream_t st);
+hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, int *state, hipStream_t st, VcSignal sig);
 hipError_t vc_launch_fill_payload(int mode, uint64_t seed, char *sendbuf, const int *sc, const int *sd, const int64_t *sbase,
                                   int esz, int P, hipStream_t st);
 hipError_t vc_launch_verify(const char *sendbuf, const char *recvbuf, VcTables t, int esz, int P, int packed,

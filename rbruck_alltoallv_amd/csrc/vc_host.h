@@ -163,25 +163,31 @@ struct BusyGuard {
 #define VC_FLAG_WORDS 64
 #define VC_SPIN_US 10000
 
-// Waits for everything enqueued on the communicator's stream (see vc_done_kernel).  A call that takes longer than
-// VC_SPIN_US is waited for by the runtime (4 us are nothing then, and it reports what went wrong), as is a call with
-// per-launch timing on, whose events end behind its last kernel.
-inline hipError_t vc_wait_stream(vc_comm *c) {
-    if (c->timing) return hipStreamSynchronize(c->stream);
-    unsigned value;
+// Enqueues launch(sig), whose last kernel tells the host by `sig` that everything before it on the stream and it itself are done, and waits
+// for that.  A call that takes longer than VC_SPIN_US is waited for by the runtime (4 us are nothing then, and it reports what went
+// wrong), as is a call with per-launch timing on, whose events end behind its last kernel.
+template <class Launch> inline hipError_t vc_run_and_wait(vc_comm *c, Launch launch) {
+    VcSignal sig;
     {
         std::lock_guard<std::mutex> lock(c->done_mutex);
-        value = ++c->done_value;
-        const hipError_t e = vc_launch_done(reinterpret_cast<unsigned *>(c->h_flags_dev) + VC_DONE_AT, value, c->stream);
+        sig = VcSignal{reinterpret_cast<unsigned *>(c->h_flags_dev) + VC_DONE_AT, ++c->done_value, c->ticket.as<unsigned>()};
+        const hipError_t e = launch(sig);
         if (e != hipSuccess) return e;
     }
+    if (c->timing) return hipStreamSynchronize(c->stream);
     const unsigned *word = reinterpret_cast<const unsigned *>(c->h_flags) + VC_DONE_AT;
     const auto t0 = std::chrono::steady_clock::now();
     for (unsigned spin = 1;; spin++) {
-        if ((int)(__atomic_load_n(word, __ATOMIC_ACQUIRE) - value) >= 0) return hipSuccess;
+        if ((int)(__atomic_load_n(word, __ATOMIC_ACQUIRE) - sig.value) >= 0) return hipSuccess;
         __builtin_ia32_pause();
         if (spin % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(VC_SPIN_US)) return hipStreamSynchronize(c->stream);
     }
+}
+
+// ... everything enqueued so far (see vc_done_kernel)
+inline hipError_t vc_wait_stream(vc_comm *c) {
+    if (c->timing) return hipStreamSynchronize(c->stream);
+    return vc_run_and_wait(c, [&](VcSignal sig) { return vc_launch_done(sig.word, sig.value, c->stream); });
 }
 
 // the host waits for the communicator's stream (counted: vc_stats_t.host_waits)

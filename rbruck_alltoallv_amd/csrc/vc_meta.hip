@@ -14,10 +14,10 @@
 // ---------------------------------------------------------------------------
 #define VC_TILE 32
 
-__global__ __launch_bounds__(VC_THREADS) void vc_transpose_kernel(const int *__restrict__ in, int *__restrict__ out, int P) {
+__global__ __launch_bounds__(VC_THREADS) void vc_transpose_kernel(const int *__restrict__ in, int *__restrict__ out, int P, VcSignal sig) {
     __shared__ int tile[VC_TILE][VC_TILE + 1];
     const int tx = threadIdx.x % VC_TILE, ty = threadIdx.x / VC_TILE;   // ty in [0, 8)
-    const int c0 = blockIdx.x * VC_TILE, r0 = blockIdx.y * VC_TILE;
+    const int tiles = (P + VC_TILE - 1) / VC_TILE, c0 = (int)(blockIdx.x % tiles) * VC_TILE, r0 = (int)(blockIdx.x / tiles) * VC_TILE;
 #pragma unroll
     for (int k = 0; k < VC_TILE; k += VC_THREADS / VC_TILE) {
         int r = r0 + ty + k, c = c0 + tx;
@@ -27,13 +27,14 @@ __global__ __launch_bounds__(VC_THREADS) void vc_transpose_kernel(const int *__r
 #pragma unroll
     for (int k = 0; k < VC_TILE; k += VC_THREADS / VC_TILE) {
         int r = c0 + ty + k, c = r0 + tx;                                // transposed coordinates
-        if (r < P && c < P) out[(int64_t)r * P + c] = tile[tx][ty + k];
+        if (r < P && c < P) vc_store_through(&out[(int64_t)r * P + c], tile[tx][ty + k]);
     }
+    vc_signal(sig);
 }
 
-hipError_t vc_launch_transpose(const int *in, int *out, int P, hipStream_t st) {
-    int t = (P + VC_TILE - 1) / VC_TILE;
-    hipLaunchKernelGGL(vc_transpose_kernel, dim3(t, t), dim3(VC_THREADS), 0, st, in, out, P);
+hipError_t vc_launch_transpose(const int *in, int *out, int P, hipStream_t st, VcSignal sig) {
+    const unsigned t = (P + VC_TILE - 1) / VC_TILE;
+    hipLaunchKernelGGL(vc_transpose_kernel, dim3(t * t), dim3(VC_THREADS), 0, st, in, out, P, sig);
     return hipGetLastError();
 }
 
@@ -43,7 +44,7 @@ hipError_t vc_launch_transpose(const int *in, int *out, int P, hipStream_t st) {
 // rows longer than the workgroup.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(VC_THREADS) void vc_row_scan_kernel(const int *__restrict__ counts, int *__restrict__ displs,
-                                                                 int64_t *__restrict__ extent, int *__restrict__ flags, int P) {
+                                                                 int64_t *__restrict__ extent, int *__restrict__ flags, int P, VcSignal sig) {
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
     const int p = blockIdx.x;
     int64_t carry = 0;
@@ -51,23 +52,24 @@ __global__ __launch_bounds__(VC_THREADS) void vc_row_scan_kernel(const int *__re
         int i = base + threadIdx.x;
         int64_t v = (i < P) ? counts[(int64_t)p * P + i] : 0, total;
         int64_t ex = vc_block_exclusive_scan(v, lds, total);
-        if (i < P) displs[(int64_t)p * P + i] = (int)(carry + ex);
-        if (flags && v < 0) flags[1] = 1;                 // a negative count
+        if (i < P) vc_store_through(&displs[(int64_t)p * P + i], (int)(carry + ex));
+        if (flags && v < 0) vc_store_through(&flags[1], 1);      // a negative count
         carry += total;
     }
-    if (extent && threadIdx.x == 0) extent[p] = carry;
+    if (extent && threadIdx.x == 0) vc_store_through(&extent[p], carry);
     // the last displacement is the largest when no count is negative
-    if (flags && threadIdx.x == 0 && carry > 0x7FFFFFFFll) flags[0] = 1;
+    if (flags && threadIdx.x == 0 && carry > 0x7FFFFFFFll) vc_store_through(&flags[0], 1);
+    if (sig.word) vc_signal(sig);
 }
 
-hipError_t vc_launch_row_scan(const int *counts, int *displs, int64_t *extent, int *flags, int P, hipStream_t st) {
-    hipLaunchKernelGGL(vc_row_scan_kernel, dim3(P), dim3(VC_THREADS), 0, st, counts, displs, extent, flags, P);
+hipError_t vc_launch_row_scan(const int *counts, int *displs, int64_t *extent, int *flags, int P, hipStream_t st, VcSignal sig) {
+    hipLaunchKernelGGL(vc_row_scan_kernel, dim3(P), dim3(VC_THREADS), 0, st, counts, displs, extent, flags, P, sig);
     return hipGetLastError();
 }
 
 // base[p] = sum_{q<p} roundup(extent[q]*esz, align); one workgroup.
 __global__ __launch_bounds__(VC_THREADS) void vc_bases_kernel(const int64_t *__restrict__ extent, int esz, int64_t align,
-                                                              int64_t *__restrict__ base, int64_t *__restrict__ total_out, int P) {
+                                                              int64_t *__restrict__ base, int64_t *__restrict__ total_out, int P, VcSignal sig) {
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
     int64_t carry = 0;
     for (int b0 = 0; b0 < P; b0 += VC_THREADS) {
@@ -75,14 +77,15 @@ __global__ __launch_bounds__(VC_THREADS) void vc_bases_kernel(const int64_t *__r
         int64_t v = 0, total;
         if (i < P) v = (extent[i] * esz + align - 1) / align * align;
         int64_t ex = vc_block_exclusive_scan(v, lds, total);
-        if (i < P) base[i] = carry + ex;
+        if (i < P) vc_store_through(&base[i], carry + ex);
         carry += total;
     }
-    if (total_out && threadIdx.x == 0) *total_out = carry;
+    if (total_out && threadIdx.x == 0) vc_store_through(total_out, carry);
+    vc_signal(sig);
 }
 
-hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_t *base, int64_t *total, int P, hipStream_t st) {
-    hipLaunchKernelGGL(vc_bases_kernel, dim3(1), dim3(VC_THREADS), 0, st, extent, esz, align, base, total, P);
+hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_t *base, int64_t *total, int P, hipStream_t st, VcSignal sig) {
+    hipLaunchKernelGGL(vc_bases_kernel, dim3(1), dim3(VC_THREADS), 0, st, extent, esz, align, base, total, P, sig);
     return hipGetLastError();
 }
 
@@ -95,7 +98,7 @@ hipError_t vc_launch_bases(const int64_t *extent, int esz, int64_t align, int64_
 // so the workgroups are few and large.
 #define VC_MAX_WORKGROUPS 64
 #define VC_MAX_LANES 1024
-__global__ __launch_bounds__(VC_MAX_LANES) void vc_max_kernel(const int *__restrict__ counts, int *__restrict__ out, int64_t n, int *state) {
+__global__ __launch_bounds__(VC_MAX_LANES) void vc_max_kernel(const int *__restrict__ counts, int *__restrict__ out, int64_t n, int *state, VcSignal sig) {
     __shared__ int wave_max[VC_MAX_LANES / VC_WAVE];
     const int lane = threadIdx.x % VC_WAVE, wave = threadIdx.x / VC_WAVE;
     int m = INT_MIN;
@@ -120,16 +123,18 @@ __global__ __launch_bounds__(VC_MAX_LANES) void vc_max_kernel(const int *__restr
 #pragma unroll
     for (int o = VC_WAVE / 2; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, VC_WAVE));
     if (lane == 0) {
-        *out = m;
+        vc_store_through(out, m);
         __hip_atomic_store(&state[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        vc_store_through(sig.word, sig.value);            // (this workgroup is the last one)
     }
 }
 
-hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, int *state, hipStream_t st) {
+hipError_t vc_launch_max(const int *counts, int *out, int64_t nelem, int *state, hipStream_t st, VcSignal sig) {
     int64_t blocks = (nelem + 4 * VC_MAX_LANES - 1) / (4 * VC_MAX_LANES);
     if (blocks > VC_MAX_WORKGROUPS) blocks = VC_MAX_WORKGROUPS;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(vc_max_kernel, dim3((unsigned)blocks), dim3(VC_MAX_LANES), 0, st, counts, out, nelem, state);
+    hipLaunchKernelGGL(vc_max_kernel, dim3((unsigned)blocks), dim3(VC_MAX_LANES), 0, st, counts, out, nelem, state, sig);
     return hipGetLastError();
 }
 

@@ -333,10 +333,6 @@ hipError_t vc_launch_plan_emit(const VcSched &S, const VcLaunchInfo *launches_ho
 
 // ---- forwarded execution ----
 #define VC_PLAN_XCDS 8
-// Workgroups count themselves on one of VC_TICKETS words, each in a cache line of its own, and the last of a word on the word
-// behind them: atomics on one word go one after the other, about 10 ns each (2048 workgroups on one word: +20 us).
-#define VC_TICKETS 64
-#define VC_TICKET_STRIDE 32
 // Rows a kernel gives a workgroup each: workgroup b runs on XCD b mod 8, and XCD k takes the k-th eighth of the ranks, so that
 // the table entries of neighbouring ranks, which share cache lines (the entries of a rank lie in a column), meet in one L2.
 static unsigned vc_rank_grid(int P, int rows) { return (unsigned)((P + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS) * VC_PLAN_XCDS * rows; }
@@ -444,14 +440,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTable
     }
     if (threadIdx.x == 0) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this workgroup's totals are where the last one will look
-        const unsigned mine = blockIdx.x % VC_TICKETS, words = gridDim.x < VC_TICKETS ? gridDim.x : VC_TICKETS;
-        unsigned *word = ticket + mine * VC_TICKET_STRIDE;
-        is_last = 0;
-        if (__hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (gridDim.x - mine + VC_TICKETS - 1) / VC_TICKETS - 1) {
-            __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            word = ticket + VC_TICKETS * VC_TICKET_STRIDE;
-            is_last = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == words - 1;
-        }
+        is_last = vc_last_workgroup(ticket);
     }
     __syncthreads();
     if (!is_last) return;
@@ -514,9 +503,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTable
     const int64_t words[VC_HEADER_MAX_LEN + 1] = {carry, sum[0], items, sum[2], sum[3], sum[0] + sum[1], sum[4]};
 #pragma unroll
     for (int k = 0; k <= VC_HEADER_MAX_LEN; k++) { header[k] = words[k]; header_host[k] = words[k]; }
-    __hip_atomic_store(ticket + VC_TICKETS * VC_TICKET_STRIDE, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-static_assert((VC_TICKETS + 1) * VC_TICKET_STRIDE * sizeof(unsigned) <= VC_TICKET_BYTES, "room for the counts");
 static_assert(VC_HEADER_BAD == 3 && VC_HEADER_MAX_PIECES == 4 && VC_HEADER_FIXED == 5 && VC_HEADER_MAX_LEN == 6, "order of the words above");
 
 hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_off, int64_t *row_tot, int64_t *row_base, int64_t *row_bytes,

@@ -486,11 +486,20 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     // the one launch of the call: its first wavefronts check the tables and leave their totals in host memory; every pair
     // checks its own entries and the length of its block before it forms an address, and stores nothing before all of
     // the tables have been found in order
-    HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, nullptr, guard, pair_lanes, sendbuf, recvbuf, c->stage.as<char>(), st, verdict, verdict_next,
-                                  c->h_header_dev + VC_TOTALS_AT));
-    c->verdict_clean = true;
-    if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
-    HIP_TRY(VC_WAIT(c));
+    const auto launch = [&](VcSignal sig) {
+        const hipError_t e = vc_launch_copy_blocks(S, T, nullptr, nullptr, nullptr, guard, pair_lanes, sendbuf, recvbuf, c->stage.as<char>(), st, verdict,
+                                                   verdict_next, c->h_header_dev + VC_TOTALS_AT, sig);
+        if (e == hipSuccess) c->verdict_clean = true;
+        return e;
+    };
+    if (d.self && !c->timing) {
+        c->waits++;
+        HIP_TRY(vc_run_and_wait(c, launch));
+    } else {
+        HIP_TRY(launch(VcSignal()));
+        if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
+        HIP_TRY(VC_WAIT(c));
+    }
     int64_t *h = c->h_header;
     for (int k = 0; k <= VC_HEADER_MAX_LEN; k++) h[k] = 0;
     for (int64_t w = 0; w < vc_totals_waves(S.P); w++) {
@@ -599,7 +608,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     S.recv_lo = (int)((uintptr_t)recvbuf & 4095);
     PlanInfo pi;
     hipStream_t st = c->stream;
-    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, {0, 0, 0, 0, 0}};
+    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, false, {0, 0, 0, 0, 0}};
     const int pair_lanes = d.lanes;
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;

@@ -306,7 +306,7 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 // verdict (device, non-null: fixed-stride staging, S.stride > 0, at most VC_MAX_GRID pairs): the kernel needs no planner
 // before it and `header` is not read.  Its first wavefronts check the tables, count themselves in the VC_VERDICTS words at `verdict` (zero at the
 // start; the kernel clears those at `verdict_next` for the call after this one) and leave what the host wants to know — payload, block pieces, longest block, ... —
-// in `totals` (host memory, vc_totals_waves(P) slots).  Every pair
+// in `totals` (host memory, vc_totals_waves(P) slots).  sig (with `verdict` and a wavefront or workgroup per pair only): the kernel signals its own end.  Every pair
 // checks its own table entries and the guard's max_len / max_pieces and leaves its block alone when one of them fails, so
 // no address is formed from a bad entry; the host, which evaluates the same conditions on the totals afterwards, reports
 // the call as refused then.  With bad table entries nothing has been stored by then: the copying wavefronts hold their
@@ -315,6 +315,6 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  unsigned long long *verdict = nullptr, unsigned long long *verdict_next = nullptr,
-                                 int64_t *totals = nullptr);
+                                 int64_t *totals = nullptr, VcSignal sig = VcSignal());
 // dst2 non-null: every vector is stored twice (one read, two writes)
 hipError_t vc_launch_calibration_copy(const char *src, char *dst, char *dst2, int64_t nbytes, hipStream_t st);

@@ -36,6 +36,11 @@ __device__ __forceinline__ void vc_store16(char *p, vc_u32x4 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<vc_u32x4 *>(p));
 }
 
+// ... past the caches (THROUGH: for a kernel that signals its own end, vc_signal), to any byte address
+__device__ __forceinline__ void vc_store16_through(char *p, vc_u32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+}
+
 __device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, char *recvbuf, char *stage) {
     const int64_t off = loc & VC_OFFSET_MASK;
     const int space = (int)(loc >> VC_SPACE_SHIFT);
@@ -62,12 +67,12 @@ __device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, ch
 #define VC_WAIT_VMCNT0 0x0F70              // s_waitcnt vmcnt(0): loads have arrived and stores have been acknowledged
 struct VcAlwaysGo { __device__ __forceinline__ bool operator()() const { return true; } };
 
-template <int LANES, class NextDst, class Go = VcAlwaysGo>
+template <int LANES, bool THROUGH = false, class NextDst, class Go = VcAlwaysGo>
 __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, int nhop, int w, NextDst next_dst, Go go = Go()) {
     constexpr int VECS = VC_CHUNK / 16 / LANES;           // window vectors per lane: 2 for a workgroup of 256, 8 for one wavefront
     const int t = threadIdx.x;
     const int n = (int)len;                               // (a piece fits the window)
-    if (n == VC_PIECE && w == 0) {
+    if (!THROUGH && n == VC_PIECE && w == 0) {
         // A whole aligned piece, the inside of a long block: no vector to leave out and no edge.  A wavefront waits for each of its
         // stores before the next one: on lists of these the memory runs a few per cent faster with fewer writes in flight
         // (64 ranks, 1.3 MB blocks, two hops: 2436 us -> 2361).
@@ -109,10 +114,10 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
     __builtin_amdgcn_s_waitcnt(VC_WAIT_VMCNT0);
     for (int k = 0; k < nhop; k++) {
         char *dst = next_dst(), *dw = dst - w;
-        if (edge >= 0) dst[edge] = edge_byte;
+        if (edge >= 0) { if (THROUGH) vc_store_through(dst + edge, edge_byte); else dst[edge] = edge_byte; }
 #pragma unroll
         for (int i = 0; i < VECS; i++)
-            if (has[i]) vc_store16(dw + ((t + i * LANES) << 4), v[i]);
+            if (has[i]) { if (THROUGH) vc_store16_through(dw + ((t + i * LANES) << 4), v[i]); else vc_store16(dw + ((t + i * LANES) << 4), v[i]); }
     }
 }
 
@@ -386,11 +391,13 @@ __device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &
     moved = vc_wave_inclusive_scan(moved);
     most = vc_wave_max_last(most);
     longest = vc_wave_max_last(longest);
-    if (lane == VC_WAVE - 1) {
-        int64_t *slot = totals + wave * VC_TOTALS_SLOT;
-        slot[VC_TOTALS_PAYLOAD] = payload; slot[VC_TOTALS_ITEMS] = items; slot[VC_TOTALS_BAD] = bad;
-        slot[VC_TOTALS_MOST] = most; slot[VC_TOTALS_MOVED] = moved; slot[VC_TOTALS_LONGEST] = longest;
-    }
+    // six words in one store: each store past the caches is a write of its own to host memory (90 ranks of 4-byte blocks: one
+    // store per word 21 us)
+    const int64_t all[] = {vc_last_lane(payload), vc_last_lane(items), vc_last_lane(bad), vc_last_lane(most), vc_last_lane(moved), vc_last_lane(longest)};
+    int64_t v = all[VC_TOTALS_PAYLOAD];
+#pragma unroll
+    for (int k = VC_TOTALS_PAYLOAD + 1; k <= VC_TOTALS_LONGEST; k++) v = lane == k ? all[k] : v;
+    if (lane <= VC_TOTALS_LONGEST) vc_store_through(&totals[wave * VC_TOTALS_SLOT + lane], v);
 }
 
 // A copying wavefront of the single launch asks before its first store: have all totalling wavefronts checked their part of
@@ -415,7 +422,7 @@ struct VcVerdictGate {
         if (!verdict) return true;
         for (int spin = 0; state == 0; spin++) {
             if ((word & 0xFFFFFFFFull) >= nwaves) state = (word >> 32) ? 2 : 1;
-            else if (spin >= VC_CHECK_SPINS) { totals[VC_TOTALS_STALLED] = 1; state = 2; }
+            else if (spin >= VC_CHECK_SPINS) { vc_store_through(&totals[VC_TOTALS_STALLED], (int64_t)1); state = 2; }
             else { __builtin_amdgcn_s_sleep(1); word = vc_verdict_word(verdict); }
         }
         return state == 1;
@@ -464,14 +471,14 @@ __device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcPairRe
 // Everything the block's addresses depend on is read before the planner's verdict is looked at: the reads are
 // independent of each other and of the verdict (tables are always readable), so they travel together instead of one
 // memory round trip after the other; nothing is stored before the verdict is known.
-template <int LANES>
-__global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
-                                                               const int64_t *__restrict__ row_base,
-                                                               const int64_t *__restrict__ header, VcListlessGuard guard,
-                                                               int64_t first_pair, const char *__restrict__ sendbuf,
-                                                               char *__restrict__ recvbuf, char *__restrict__ stage,
-                                                               unsigned long long *verdict, unsigned long long *verdict_next,
-                                                               int64_t *totals) {
+template <int LANES, bool SELF>
+__device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T, const uint32_t *__restrict__ slot_off,
+                                             const int64_t *__restrict__ row_base,
+                                             const int64_t *__restrict__ header, VcListlessGuard guard,
+                                             int64_t first_pair, const char *__restrict__ sendbuf,
+                                             char *__restrict__ recvbuf, char *__restrict__ stage,
+                                             unsigned long long *verdict, unsigned long long *verdict_next,
+                                             int64_t *totals) {
     const unsigned head = vc_totals_blocks(S, verdict, LANES);
     if (blockIdx.x < head) { vc_add_totals(S, T, verdict, totals); return; }
     const unsigned block = blockIdx.x - head;
@@ -483,7 +490,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
     const int lane = threadIdx.x % VC_WAVE, nslots = vc_hop_slots(S);
     const VcHop hop = vc_hop_place(S, s, t, lane < nslots ? lane : 0);
     const int64_t slot = vc_slot_addr(S, slot_off, row_base, hop);
-    if (verdict && block == 0 && threadIdx.x < VC_VERDICTS) verdict_next[threadIdx.x * (VC_LINE / 8)] = 0;      // the words of the next call
+    if (verdict && block == 0 && threadIdx.x < VC_VERDICTS) vc_store_through(&verdict_next[threadIdx.x * (VC_LINE / 8)], 0ull);      // the words of the next call
     const int64_t len = (int64_t)p.sent * S.esz;
     if (!inside || len <= 0) return;
     if (verdict ? !vc_pair_allowed(S, p, guard) : !vc_listless_ok(header, guard)) return;
@@ -499,7 +506,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
         unsigned long long left = moves;
-        vc_forward_piece<LANES>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
+        vc_forward_piece<LANES, SELF>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
                                 [&]() {
                                     const int k = __ffsll(left) - 1;
                                     left &= left - 1;
@@ -508,6 +515,22 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
                                 },
                                 [&]() { return gate(); });
     }
+}
+
+// SELF: one launch on fixed-stride staging that tells the host itself that it is done (vc_signal), with everything it stores stored past
+// the caches.  A kernel behind this one that only does that costs the boundary between the two: 8 ranks 13.5 -> 13.0 us,
+// 24 ranks of 0 - 32 KiB blocks 30.6 -> 26.7.  The quarter kernel has no such instance: its lanes' short stores past the caches each
+// cost a write to memory (64 ranks, 1 KiB blocks: 16.6 -> 21.9 us).
+template <int LANES, bool SELF>
+__global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
+                                                               const int64_t *__restrict__ row_base,
+                                                               const int64_t *__restrict__ header, VcListlessGuard guard,
+                                                               int64_t first_pair, const char *__restrict__ sendbuf,
+                                                               char *__restrict__ recvbuf, char *__restrict__ stage,
+                                                               unsigned long long *verdict, unsigned long long *verdict_next,
+                                                               int64_t *totals, VcSignal sig) {
+    vc_copy_pair<LANES, SELF>(S, T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, verdict, verdict_next, totals);
+    if (SELF) vc_signal(sig);
 }
 
 // The same for pairs whose blocks are a few hundred bytes: a quarter of a wavefront per pair, four pairs in a row per
@@ -534,7 +557,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
     const int nslots = vc_hop_slots(S);
     const VcHop h0 = vc_hop_place(S, s, t, q < nslots ? q : 0);
     const int64_t slot0 = vc_slot_addr(S, slot_off, row_base, h0);
-    if (verdict && block == 0 && threadIdx.x < VC_VERDICTS) verdict_next[threadIdx.x * (VC_LINE / 8)] = 0;
+    if (verdict && block == 0 && threadIdx.x < VC_VERDICTS) vc_store_through(&verdict_next[threadIdx.x * (VC_LINE / 8)], 0ull);
     if (!verdict && !vc_listless_ok(header, guard)) return;      // the same for every lane of the grid
     const int64_t len = inside ? (int64_t)p.sent * S.esz : 0, recv_off = p.rbase + (int64_t)p.rd * S.esz;
     // no lane leaves before the barrier below
@@ -675,8 +698,9 @@ static void vc_launch_batch(const VcSched &S, VcTables T, const uint32_t *slot_o
 
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
-                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals) {
+                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig) {
     const int64_t npairs = (int64_t)S.P * S.P;
+    if (sig.word && (!verdict || (lanes != VC_WAVE && lanes != VC_THREADS))) return hipErrorInvalidValue;
     if (lanes == VC_BATCHED) {
         if (verdict) return hipErrorInvalidValue;         // the batches are for more pairs than one launch with totals takes
         const int batch = vc_batch_pairs(npairs);
@@ -690,9 +714,16 @@ hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *s
         const int64_t units = lanes == VC_QUARTER ? (now + VC_ITEMS_PER_WAVE - 1) / VC_ITEMS_PER_WAVE : now;
         if (verdict && done) return hipErrorInvalidValue;    // the totals belong to a call that one launch takes
         const dim3 grid((unsigned)((units + VC_XCDS - 1) / VC_XCDS * VC_XCDS) + vc_totals_blocks(S, verdict, lanes == VC_THREADS ? VC_THREADS : VC_WAVE));
-        const auto kernel = lanes == VC_QUARTER ? vc_copy_blocks_quarter_kernel : (lanes == VC_WAVE ? vc_copy_blocks_kernel<VC_WAVE> : vc_copy_blocks_kernel<VC_THREADS>);
-        hipLaunchKernelGGL(kernel, grid, dim3(lanes == VC_THREADS ? VC_THREADS : VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done,
-                           sendbuf, recvbuf, stage, verdict, verdict_next, totals);
+        if (lanes == VC_QUARTER) {
+            hipLaunchKernelGGL(vc_copy_blocks_quarter_kernel, grid, dim3(VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf,
+                               recvbuf, stage, verdict, verdict_next, totals);
+            continue;
+        }
+        const bool self = sig.word != nullptr;
+        const auto kernel = lanes == VC_WAVE ? (self ? vc_copy_blocks_kernel<VC_WAVE, true> : vc_copy_blocks_kernel<VC_WAVE, false>)
+                                             : (self ? vc_copy_blocks_kernel<VC_THREADS, true> : vc_copy_blocks_kernel<VC_THREADS, false>);
+        hipLaunchKernelGGL(kernel, grid, dim3(lanes), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, verdict,
+                           verdict_next, totals, sig);
     }
     return hipGetLastError();
 }

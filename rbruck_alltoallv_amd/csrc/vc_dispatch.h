@@ -45,6 +45,10 @@
 #define VC_LISTLESS_MAX_AVERAGE 4096          // a call the short-block kernels were chosen for must stay below this average
 #define VC_STRIDED_MAX_BYTES ((int64_t)256 << 20)
 #define VC_STRIDED_MAX_PAIRS 36864            // 192 ranks
+// the launch signals its own end: calls with cold caches gain up to 32 ranks (0 - 2 KiB blocks even, 0 - 32 KiB 26.7 us against 30.6 on 24
+// ranks) and lose on 64 (0 - 4 KiB 23.2 -> 25.1): stores past the caches fill a memory queue that the L2s would have filled later
+#define VC_SELF_MAX_PAIRS 1024
+#define VC_SELF_MAX_BYTES ((int64_t)64 << 20)
 // list-driven copy kernels: lanes per work item by the average piece of the launch
 #define VC_ITEM_QUARTER_BELOW 448
 #define VC_ITEM_WAVE_BELOW 3072
@@ -68,6 +72,7 @@ struct VcDispatch {
                              // VC_THREADS, VC_WAVE, VC_QUARTER, or VC_BATCHED (a batch of pairs per wavefront)
     int stride;              // > 0: first try one launch on fixed-stride staging with slots of this many bytes ...
     int stride_lanes;        // ... with this many lanes per pair (the batches come without the totals: a quarter of a wavefront)
+    bool self;               // ... that tells the host itself when it is done
     VcListlessGuard guard;   // what the call must look like for the listless kernel to move anything, checked on the device
                              // against the plan (the hint is only a guess); stage_cap is the caller's to fill in
 };
@@ -77,7 +82,7 @@ VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 :
 // mode: vc_comm_set_forwarding (0 launch per digit, 1 the library's choice, 2 the list, 3 / 4 / 5 listless with a workgroup / a
 // quarter of a wavefront per pair / batches).  S: the call's schedule (ranks, digits, whether it has an organized region).
 inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const VcSched &S) {
-    VcDispatch d = {0, 0, 0, {0, 0, 0, 0, 0}};
+    VcDispatch d = {0, 0, 0, false, {0, 0, 0, 0, 0}};
     if (mode == 3) { d.lanes = VC_THREADS; return d; }
     if (mode == 4) { d.lanes = VC_QUARTER; return d; }
     if (mode == 5) { d.lanes = VC_BATCHED; return d; }
@@ -113,6 +118,7 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
             d.stride = (int)stride;
             d.stride_lanes = d.lanes == VC_BATCHED ? VC_QUARTER : d.lanes;
             d.guard.max_len = stride - VC_LINE + 1;
+            d.self = d.stride_lanes != VC_QUARTER && pairs <= VC_SELF_MAX_PAIRS && h.payload * vc_hop_slots(S) <= VC_SELF_MAX_BYTES;
         }
     }
     return d;

@@ -52,6 +52,12 @@ __device__ __forceinline__ int64_t vc_wave_max_last(int64_t v) {
     return vc_dpp_max<VC_DPP_BCAST31, 0xc>(v);
 }
 
+// Lane 63's value, in every lane.
+__device__ __forceinline__ int64_t vc_last_lane(int64_t v) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, VC_WAVE - 1), hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), VC_WAVE - 1);
+    return (int64_t)((unsigned long long)hi << 32 | lo);
+}
+
 // Exclusive prefix sum across a 256-thread workgroup; `total` receives the sum of all
 // lanes.  `lds` must hold VC_WAVES_PER_BLOCK int64 and is safe to reuse after return.
 __device__ __forceinline__ int64_t vc_block_exclusive_scan(int64_t v, int64_t *lds, int64_t &total) {

@@ -65,3 +65,25 @@ def test_direct_functions(api, P, around, execution):
         assert api.spreadout_alltoallv(dp, ds, dr) == 0 and dp.verify(ds, dr) == 0, dp.comm.error()
         assert call == 0 or dp.comm.last_stats().execution == execution
     dp.comm.free()
+
+
+# up to 32 ranks the launch stores past the caches and signals its own end: what it wrote is read at once from another stream
+@pytest.mark.parametrize("P,top", [(2, 40), (9, 3000), (16, 70000), (32, 6000), (32, 30000), (33, 6000)])
+def test_everything_is_there_when_the_call_returns(api, P, top):
+    counts = np.random.default_rng(P).integers(top // 2, top + 1, (P, P)).astype(np.int32)
+    prob = W.make_problem(counts, 1, 1, 1)
+    dp = api.DeviceProblem(prob)
+    ds, want, got = dp.new_send_arena(), dp.new_recv_arena(), dp.new_recv_arena()
+    other = torch.cuda.Stream()
+    for call in range(4):
+        dp.fill_payload(0, call, ds)
+        want.fill_(0xA5)
+        got.fill_(0xA5)
+        dp.comm.set_forwarding(0)
+        assert api.twophase_rbruck_alltoallv(3, dp, ds, want) == 0 and dp.verify(ds, want) == 0
+        dp.comm.set_forwarding(1)
+        torch.cuda.synchronize()
+        assert api.twophase_rbruck_alltoallv(3, dp, ds, got) == 0, dp.comm.error()
+        with torch.cuda.stream(other):
+            assert torch.equal(got.cpu(), want.cpu()), (P, top, call)
+    dp.comm.free()

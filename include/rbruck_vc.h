@@ -121,7 +121,9 @@ int vc_comm_set_staging_bound(vc_comm_t comm, int enable);
 /* Text of the most recent failure on this thread ("" if none). */
 const char *vc_last_error_string(void);
 
-/* ---- caller-side steps of the reference drivers, as kernels ---- */
+/* ---- caller-side steps of the reference drivers, as kernels ----
+ * All of them wait for their result.  vc_alltoall_counts, vc_bases_from_extents and vc_allreduce_max_count may run beside a call on the
+ * communicator, also from several threads (they take turns); vc_displs_from_counts is a call like the collectives. */
 
 /* MPI_Alltoall of one int per pair (examples/rbruckv_example.cpp:76): recvcounts[t][s] = sendcounts[s][t].
  * LDS-tiled P x P transpose. */

@@ -50,15 +50,22 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, VC_FLAG_WORDS * sizeof(int), hipHostMallocCoherent);
     if (e == hipSuccess) memset(c->h_flags, 0, VC_FLAG_WORDS * sizeof(int));
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_flags_dev, c->h_flags, 0);
-    if (e == hipSuccess) e = c->ticket.reserve(VC_TICKET_BYTES);
+    if (e == hipSuccess) e = c->counting.reserve(VC_COUNTING_BYTES);
     if (e == hipSuccess) {
-        const std::vector<char> zeros(VC_TICKET_BYTES, 0);
-        e = hipMemcpy(c->ticket.p, zeros.data(), zeros.size(), hipMemcpyHostToDevice);
+        const std::vector<char> zeros(VC_COUNTING_BYTES, 0);
+        e = hipMemcpy(c->counting.p, zeros.data(), zeros.size(), hipMemcpyHostToDevice);
     }
     if (e != hipSuccess) {
         (void)vc_comm_free(c);
         return fail_hip(e, "vc_comm_create", __LINE__);
     }
+    const auto done = [c](int word, int ticket) {
+        return VcDone{reinterpret_cast<const unsigned *>(c->h_flags) + word, reinterpret_cast<unsigned *>(c->h_flags_dev) + word,
+                      reinterpret_cast<unsigned *>(c->counting.as<char>() + ticket * VC_TICKET_BYTES), 0};
+    };
+    c->of_call = done(VC_CALL_DONE_AT, 0);
+    c->of_meta = done(VC_META_DONE_AT, 1);
+    c->max_state = reinterpret_cast<int *>(c->counting.as<char>() + 2 * VC_TICKET_BYTES);
     c->staging_allowance = default_staging_allowance();
     *comm_out = c;
     return VC_OK;
@@ -69,7 +76,7 @@ extern "C" int vc_comm_free(vc_comm_t c) {
     (void)hipStreamSynchronize(c->stream);
     c->pending.active = false;
     for (DevBuf *b : {&c->slot_off, &c->row_tot, &c->row_base, &c->org_run_base, &c->item_row_tot, &c->item_row_base, &c->row_bytes, &c->desc, &c->header, &c->launches, &c->stage, &c->rd_packed,
-                      &c->scratch, &c->max_state, &c->ticket, &c->chain_row_tot, &c->chain_row_base, &c->verdicts})
+                      &c->scratch, &c->counting, &c->chain_row_tot, &c->chain_row_base, &c->verdicts})
         b->release();
     free_retired_stage(c);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
@@ -248,7 +255,7 @@ static int reserve_plan_bufs(vc_comm *c, const VcSched &S, int nl, bool forward)
     B.item_row_base = c->item_row_base.as<int64_t>(); B.row_bytes = c->row_bytes.as<int64_t>();
     B.chain_row_tot = forward ? c->chain_row_tot.as<int64_t>() : nullptr;
     B.chain_row_base = forward ? c->chain_row_base.as<int64_t>() : nullptr;
-    B.ticket = c->ticket.as<unsigned>();
+    B.ticket = c->of_call.ticket;
     B.header = c->header.as<int64_t>(); B.launches = c->launches.as<VcLaunchInfo>(); B.rd_packed = c->rd_packed.as<int>();
     return VC_OK;
 }
@@ -486,7 +493,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     // the one launch of the call: its first wavefronts check the tables and leave their totals in host memory; every pair
     // checks its own entries and the length of its block before it forms an address, and stores nothing before all of
     // the tables have been found in order
-    const auto launch = [&](VcSignal sig) {
+    const auto launch = [&](hipStream_t, VcSignal sig) {
         const hipError_t e = vc_launch_copy_blocks(S, T, nullptr, nullptr, nullptr, guard, pair_lanes, sendbuf, recvbuf, c->stage.as<char>(), st, verdict,
                                                    verdict_next, c->h_header_dev + VC_TOTALS_AT, sig);
         if (e == hipSuccess) c->verdict_clean = true;
@@ -494,9 +501,9 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     };
     if (d.self && !c->timing) {
         c->waits++;
-        HIP_TRY(vc_run_and_wait(c, launch));
+        HIP_TRY(vc_run_and_wait(c, c->of_call, launch));
     } else {
-        HIP_TRY(launch(VcSignal()));
+        HIP_TRY(launch(st, VcSignal()));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
         HIP_TRY(VC_WAIT(c));
     }
@@ -688,7 +695,8 @@ static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std:
 extern "C" int vc_comm_wait(vc_comm_t c) {
     if (!c) return fail_arg("null communicator");
     if (!c->pending.active) {
-        HIP_TRY(VC_WAIT(c));
+        std::lock_guard<std::mutex> lock(c->meta_mutex);
+        HIP_TRY(vc_wait_stream(c, c->of_meta));
         return VC_OK;
     }
     // whatever happens below, the call is over when this function returns: the communicator is free again and launches

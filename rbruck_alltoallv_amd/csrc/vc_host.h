@@ -73,10 +73,19 @@ struct CallParams {
     int n, r, batch, esz, uniform, batch2;
 };
 
+// What a kernel needs to tell the host that it is done (VcSignal).  The words serve one kernel at a time: who launches it has them to
+// itself until the wait is over.
+struct VcDone {
+    const unsigned *word = nullptr;       // pinned, as the host sees it ...
+    unsigned *word_dev = nullptr;         // ... and the device
+    unsigned *ticket = nullptr;           // VC_TICKET_BYTES, zero between the calls
+    unsigned value = 0;                   // the value last enqueued for the word
+};
+
 struct vc_comm {
     int P = 0;
     int device = 0;
-    hipStream_t stream = nullptr;
+    std::atomic<hipStream_t> stream{nullptr};        // (the metadata steps read it beside a call that moves the communicator to the caller's)
     const int64_t *sbase = nullptr, *rbase = nullptr;
     bool timing = false;
     int forward = 1;                      // vc_comm_set_forwarding: 0 launch per digit, 1 forwarded (list or listless as the last
@@ -91,7 +100,7 @@ struct vc_comm {
     bool verdict_clean = false;           // ... and the set the next call will use is known to be zero
     int verdict_turn = 0;
     DevBuf slot_off, row_tot, row_base, org_run_base, item_row_tot, item_row_base, row_bytes, desc, header, launches, stage, rd_packed,
-        scratch, max_state, ticket;
+        scratch, counting;
     double cal_copy_bytes_per_s = 0, cal_launch_s = 0, cal_sync_s = 0;   // calibrate(): the plain copy's rate, the cost of a
                                           // launch, of a launch the host waits for
     int bound_staging = 1;                // vc_comm_set_staging_bound
@@ -117,9 +126,11 @@ struct vc_comm {
     int64_t *h_header_dev = nullptr;      // the same memory as the device sees it
                                           // (VC_TOTALS_AT words in: the totals of a call on fixed-stride staging, slot by slot)
     int *h_flags = nullptr, *h_flags_dev = nullptr;   // pinned, coherent: the two flags of vc_displs_from_counts, as host and device see
-                                          // them; in a cache line of its own behind them (VC_DONE_AT) the word vc_wait_stream waits for
-    unsigned done_value = 0;              // the value last enqueued for that word
-    std::mutex done_mutex;                // values go into the stream in order, also from several threads
+                                          // them; behind them the words of the two signals, a cache line each
+    VcDone of_call;                       // for what runs under VC_ONE_CALL, or between an _async call and its vc_comm_wait
+    VcDone of_meta;                       // for the metadata steps and vc_comm_wait without a call, which do not refuse to run beside one:
+    std::mutex meta_mutex;                // they take turns, each from its launch to the end of its wait
+    int *max_state = nullptr;             // counting words of vc_allreduce_max_count (under meta_mutex)
     VcLaunchInfo *h_launches = nullptr;   // pinned
     std::vector<hipEvent_t> events;
     vc_stats_t stats;
@@ -156,42 +167,50 @@ struct BusyGuard {
     bool ok() const { return !c || mine; }
     void keep() { mine = false; }         // the call stays in progress after the entry point returns (vc_comm_wait ends it)
 };
-#define VC_DONE_AT 32
 // words of h_header: the planner's header, then (in cache lines of their own) the slots of vc_totals_waves(P) wavefronts
 #define VC_TOTALS_AT ((VC_HEADER_WORDS(VC_MAX_LAUNCHES) + VC_TOTALS_SLOT - 1) / VC_TOTALS_SLOT * VC_TOTALS_SLOT)
 #define VC_HEADER_ROOM (VC_TOTALS_AT + VC_TOTALS_SLOT * (VC_STRIDED_MAX_PAIRS / VC_TOTALS_PER_WAVE))
-#define VC_FLAG_WORDS 64
+// words of h_flags: the flags, the word of of_call, the word of of_meta
+#define VC_CALL_DONE_AT 32
+#define VC_META_DONE_AT 64
+#define VC_FLAG_WORDS 96
+// `counting` (device, zero from the start): the tickets of of_call and of_meta, max_state
+#define VC_MAX_STATE_BYTES 512
+#define VC_COUNTING_BYTES (2 * VC_TICKET_BYTES + VC_MAX_STATE_BYTES)
 #define VC_SPIN_US 10000
 
-// Enqueues launch(sig), whose last kernel tells the host by `sig` that everything before it on the stream and it itself are done, and waits
-// for that.  A call that takes longer than VC_SPIN_US is waited for by the runtime (4 us are nothing then, and it reports what went
-// wrong), as is a call with per-launch timing on, whose events end behind its last kernel.
-template <class Launch> inline hipError_t vc_run_and_wait(vc_comm *c, Launch launch) {
-    VcSignal sig;
-    {
-        std::lock_guard<std::mutex> lock(c->done_mutex);
-        sig = VcSignal{reinterpret_cast<unsigned *>(c->h_flags_dev) + VC_DONE_AT, ++c->done_value, c->ticket.as<unsigned>()};
-        const hipError_t e = launch(sig);
-        if (e != hipSuccess) return e;
-    }
-    if (c->timing) return hipStreamSynchronize(c->stream);
-    const unsigned *word = reinterpret_cast<const unsigned *>(c->h_flags) + VC_DONE_AT;
+// Enqueues launch(st, sig), whose last kernel tells the host by `sig` that everything before it on the stream and it itself are done, and
+// waits for that.  `d` is the caller's own until the return (the call holds the communicator, or meta_mutex).  A call that takes longer than
+// VC_SPIN_US is waited for by the runtime (4 us are nothing then, and it reports what went wrong), as is a call with per-launch timing on,
+// whose events end behind its last kernel.
+template <class Launch> inline hipError_t vc_run_and_wait(vc_comm *c, VcDone &d, Launch launch) {
+    const hipStream_t st = c->stream;
+    const VcSignal sig = {d.word_dev, ++d.value, d.ticket};
+    const hipError_t e = launch(st, sig);
+    if (e != hipSuccess) return e;
+    if (c->timing) return hipStreamSynchronize(st);
     const auto t0 = std::chrono::steady_clock::now();
     for (unsigned spin = 1;; spin++) {
-        if ((int)(__atomic_load_n(word, __ATOMIC_ACQUIRE) - sig.value) >= 0) return hipSuccess;
+        if (__atomic_load_n(d.word, __ATOMIC_ACQUIRE) == sig.value) return hipSuccess;
         __builtin_ia32_pause();
-        if (spin % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(VC_SPIN_US)) return hipStreamSynchronize(c->stream);
+        if (spin % 1024 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(VC_SPIN_US)) return hipStreamSynchronize(st);
     }
 }
 
 // ... everything enqueued so far (see vc_done_kernel)
-inline hipError_t vc_wait_stream(vc_comm *c) {
+inline hipError_t vc_wait_stream(vc_comm *c, VcDone &d) {
     if (c->timing) return hipStreamSynchronize(c->stream);
-    return vc_run_and_wait(c, [&](VcSignal sig) { return vc_launch_done(sig.word, sig.value, c->stream); });
+    return vc_run_and_wait(c, d, [](hipStream_t st, VcSignal sig) { return vc_launch_done(sig.word, sig.value, st); });
 }
 
-// the host waits for the communicator's stream (counted: vc_stats_t.host_waits)
-#define VC_WAIT(c) ((c)->waits++, vc_wait_stream(c))
+// A metadata step: it has the words of of_meta to itself until it is over.
+template <class Launch> inline hipError_t vc_run_meta(vc_comm *c, Launch launch) {
+    std::lock_guard<std::mutex> lock(c->meta_mutex);
+    return vc_run_and_wait(c, c->of_meta, launch);
+}
+
+// a call waits for the communicator's stream (counted: vc_stats_t.host_waits)
+#define VC_WAIT(c) ((c)->waits++, vc_wait_stream((c), (c)->of_call))
 
 #define VC_ONE_CALL(c)                                                                                              \
     BusyGuard busy_guard_(c);                                                                                       \

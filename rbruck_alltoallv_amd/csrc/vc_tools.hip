@@ -6,7 +6,7 @@
 
 extern "C" int vc_alltoall_counts(const int *sendcounts, int *recvcounts, vc_comm_t c) {
     if (!c || !sendcounts || !recvcounts) return fail_arg("vc_alltoall_counts: null argument");
-    HIP_TRY(vc_run_and_wait(c, [&](VcSignal sig) { return vc_launch_transpose(sendcounts, recvcounts, c->P, c->stream, sig); }));
+    HIP_TRY(vc_run_meta(c, [&](hipStream_t st, VcSignal sig) { return vc_launch_transpose(sendcounts, recvcounts, c->P, st, sig); }));
     return VC_OK;
 }
 
@@ -15,7 +15,7 @@ extern "C" int vc_displs_from_counts(const int *counts, int *displs, int64_t *ex
     VC_ONE_CALL(c);
     // the kernel raises the two flags in pinned host memory: no clearing launch before it, no copy back after it
     c->h_flags[0] = c->h_flags[1] = 0;
-    HIP_TRY(vc_run_and_wait(c, [&](VcSignal sig) { return vc_launch_row_scan(counts, displs, extent_out, c->h_flags_dev, c->P, c->stream, sig); }));
+    HIP_TRY(vc_run_and_wait(c, c->of_call, [&](hipStream_t st, VcSignal sig) { return vc_launch_row_scan(counts, displs, extent_out, c->h_flags_dev, c->P, st, sig); }));
     if (c->h_flags[1]) return fail_arg("vc_displs_from_counts: negative count", VC_ERR_TABLES);
     if (c->h_flags[0]) return fail_arg("vc_displs_from_counts: a rank's counts sum past INT_MAX elements", VC_ERR_OVERFLOW);
     return VC_OK;
@@ -24,17 +24,13 @@ extern "C" int vc_displs_from_counts(const int *counts, int *displs, int64_t *ex
 extern "C" int vc_bases_from_extents(const int64_t *extent, int elem_size, int64_t align, int64_t *base_out, int64_t *total_out,
                                      vc_comm_t c) {
     if (!c || !extent || !base_out || elem_size < 1 || align < 1) return fail_arg("vc_bases_from_extents: bad argument");
-    HIP_TRY(vc_run_and_wait(c, [&](VcSignal sig) { return vc_launch_bases(extent, elem_size, align, base_out, total_out, c->P, c->stream, sig); }));
+    HIP_TRY(vc_run_meta(c, [&](hipStream_t st, VcSignal sig) { return vc_launch_bases(extent, elem_size, align, base_out, total_out, c->P, st, sig); }));
     return VC_OK;
 }
 
 extern "C" int vc_allreduce_max_count(const int *sendcounts, int *max_out, vc_comm_t c) {
     if (!c || !sendcounts || !max_out) return fail_arg("vc_allreduce_max_count: null argument");
-    if (!c->max_state.p) {
-        HIP_TRY(c->max_state.reserve(512));
-        HIP_TRY(hipMemsetAsync(c->max_state.p, 0, 512, c->stream));
-    }
-    HIP_TRY(vc_run_and_wait(c, [&](VcSignal sig) { return vc_launch_max(sendcounts, max_out, (int64_t)c->P * c->P, c->max_state.as<int>(), c->stream, sig); }));
+    HIP_TRY(vc_run_meta(c, [&](hipStream_t st, VcSignal sig) { return vc_launch_max(sendcounts, max_out, (int64_t)c->P * c->P, c->max_state, st, sig); }));
     return VC_OK;
 }
 

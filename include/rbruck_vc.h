@@ -235,7 +235,8 @@ int spreadout_alltoallv(char *sendbuf, int *sendcounts, int *sdispls, int sendty
  * becomes the communicator's stream): the planning kernels and the copy kernel are enqueued and the call returns without
  * having waited for the device.  The execution is the forwarded one without a work-item list (the copy kernel derives
  * every block's route itself and checks the planner's verdict on the device before it touches anything), so the batching
- * tunables have no effect; a workgroup serves each pair of ranks, or a quarter of a wavefront after a call of short blocks.
+ * tunables have no effect; a workgroup serves each pair of ranks, or after a call of short blocks a quarter of a wavefront or less.
+ * A communicator's first call, which finds no staging arena, is only planned, and copied in vc_comm_wait.
  * Calls of very long blocks are served faster by a persistent plan (vc_plan_execute_async).
  * Until vc_comm_wait the communicator is busy (other calls on it return VC_ERR_BUSY) and the tables, bases and buffers
  * must stay valid.  The return code covers what the host can check (0, -1, -2, -3, -5); vc_comm_wait reports the rest. */
@@ -256,7 +257,7 @@ int uniform_inverse_isplit_r_bruck_async(int n, int r1, int r2, char *sendbuf, i
 /* Waits for the communicator's stream and completes the call an _async entry point enqueued: returns VC_ERR_TABLES /
  * VC_ERR_OVERFLOW when the planner refused the tables (recvbuf is then untouched), VC_ERR_HIP for a runtime failure; when the
  * staging arena was too small for the call (the copy kernel has then moved nothing) it grows the arena and runs the copy
- * kernel again before returning.  0 with nothing pending.  vc_comm_last_stats describes the call afterwards. */
+ * kernel again before returning, in the shape the plan asks for.  0 with nothing pending.  vc_comm_last_stats describes the call afterwards. */
 int vc_comm_wait(vc_comm_t comm);
 
 /* No counterpart in the reference.  twophase_rbruck_alltoallv for callers that cannot allocate device memory: code whose

@@ -674,16 +674,20 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
 
 // The _async entry points: planning kernels and the listless copy kernel are enqueued and the call returns.  The copy
 // kernel checks the planner's verdict on the device (tables, staging arena) and touches nothing when it is bad;
-// vc_comm_wait reads the same verdict and reports it, or grows the arena and runs the copy again.
+// vc_comm_wait reads the same verdict and reports it, or grows the arena and runs the copy again, in the shape the plan asks for.
+// Without any arena (the first call of a communicator, which has no hint to choose a shape by either) a call that stages is only planned
+// here: a copy kernel could do nothing but refuse (1024 ranks, 0 - 512 B: a workgroup per pair, once to refuse and once to copy, 4.4 ms a
+// first call; planned, then batches 0.57).
 static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf,
                          VcTables T) {
     int rc = plan_sizes(c, S, L, T, true);
     if (rc) return rc;
     hipStream_t st = c->stream;
-    const int lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes;
+    const int lanes = c->stage.cap || !vc_may_stage(S) ? vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes : 0;
     const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
-    HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+    if (lanes)
+        HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     c->pending.active = true;
     c->pending.S = S; c->pending.T = T; c->pending.sendbuf = sendbuf; c->pending.recvbuf = recvbuf; c->pending.lanes = lanes;
@@ -716,25 +720,27 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
     int rc = plan_read(c, S, L, pi, true);
     if (rc) return rc;
     VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
-    if (!vc_listless_ok(c->h_header, guard)) {            // the arena was too small: nothing has been moved yet
-        // a call whose forwarded staging is out of the communicator's bound runs one launch per digit on reused staging,
-        // like its blocking twin
+    int lanes = c->pending.lanes;
+    if (!lanes || !vc_listless_ok(c->h_header, guard)) {  // no arena, or one too small: nothing has been moved yet
+        // a call whose forwarded staging is out of the communicator's bound runs one launch per digit on reused staging (its blocking
+        // twin: in batches of receivers where it can)
         if (staging_out_of_bound(c, pi.stage_bytes, pi.payload_bytes))
             return run_schedule(c, c->pending.q, c->pending.sendbuf, c->pending.recvbuf, c->pending.T, false, true);
         HIP_TRY(reserve_stage(c, (size_t)pi.stage_bytes + 64));
         guard.stage_cap = (int64_t)c->stage.cap - 64;
+        lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, VcHint{1, pi.chain_items, pi.payload_bytes, pi.max_pieces, pi.max_len}, S).lanes;
         if (c->timing) {
             std::swap(c->events[1], c->events[2]);        // (the planning ended where the first attempt began)
             c->plan_end = 1;
             HIP_TRY(hipEventRecord(c->events[2], c->stream));
         }
-        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, c->pending.lanes,
+        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes,
                                       c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], c->stream));
         HIP_TRY(VC_WAIT(c));
     }
     pi.listless = true;
-    pi.chain_lanes = c->pending.lanes;
+    pi.chain_lanes = lanes;
     return finish_stats(c, pi, nullptr, true);
 }
 

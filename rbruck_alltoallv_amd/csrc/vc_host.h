@@ -115,7 +115,7 @@ struct vc_comm {
         VcTables T;
         const char *sendbuf = nullptr;
         char *recvbuf = nullptr;
-        int lanes = 0;
+        int lanes = 0;                    // 0: only planned so far
         int n_launch_infos = 0;
         hipStream_t own_stream = nullptr; // the communicator's stream while the call runs on the caller's
         CallParams q;                     // what was asked for (the call may have to be run again another way)

@@ -222,6 +222,9 @@ VC_HD int64_t vc_stage_addr(const VcSched &S, const VcTables &T, const int64_t *
 // Bytes of staging arena a fixed-stride layout takes.
 VC_HD int64_t vc_strided_stage_bytes(const VcSched &S) { return (int64_t)(S.w + S.w2) * S.P * S.P * S.stride; }
 
+// Whether any block of a call can make two hops, the first one into staging.
+VC_HD bool vc_may_stage(const VcSched &S) { return S.w + S.w2 + (S.last_hop == 1 && S.G > 1 ? 1 : 0) > 1; }
+
 // Hops of block (s, t): the digit rounds it moves in, plus the hop that is no digit round (vc_block_hop's last slot).
 VC_HD int vc_block_hops(const VcSched &S, int s, int t) {
     if (s == t) return 1;

@@ -87,3 +87,38 @@ def test_everything_is_there_when_the_call_returns(api, P, top):
         with torch.cuda.stream(other):
             assert torch.equal(got.cpu(), want.cpu()), (P, top, call)
     dp.comm.free()
+
+
+# ranks, longest block in bytes, radix, lanes per pair of the copy kernel (1: batches) of a communicator's first _async call: what its plan
+# asks for, not a shape chosen before there is a plan; with one hop per block (radix = ranks) nothing is staged and the copy goes out at once
+@pytest.mark.parametrize("timing", [False, True])
+@pytest.mark.parametrize("P,top,r,lanes", [(300, 500, 4, 1), (300, 1300, 4, 16), (64, 1500, 2, 16), (64, 20000, 2, 256), (40, 900, 40, 256)])
+def test_first_async_call(api, P, top, r, lanes, timing):
+    prob = W.make_problem(W.counts_uniform_random(P, top, seed=P), 1, 1, 1)
+    dp = api.DeviceProblem(prob)
+    dp.comm.set_timing(timing)
+    side = torch.cuda.Stream()
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, P, ds)
+    torch.cuda.synchronize()
+    for call in range(3):
+        dr.fill_(0xA5)
+        torch.cuda.synchronize()
+        assert api.call_async("twophase_rbruck_alltoallv", (r,), dp, ds, dr, side) == 0, dp.comm.error()
+        if r == P:
+            side.synchronize()
+            assert dp.verify(ds, dr) == 0
+        assert dp.comm.wait() == 0 and dp.verify(ds, dr) == 0, dp.comm.error()
+        st = dp.comm.last_stats()
+        assert call or (st.execution, st.lanes_per_item, st.host_waits) == (2, lanes, 1 if r == P else 2)
+        assert (st.total_ms > 0) == (st.launch_ms[0] > 0) == timing
+    # a longer call than the arena holds: its own plan decides again
+    counts = np.full((P, P), 40000, dtype=np.int32)
+    longer = W.make_problem(counts, 1, 0, 0)
+    dl = api.DeviceProblem(longer, comm=dp.comm)
+    ls, lr = dl.new_send_arena(), dl.new_recv_arena()
+    dl.fill_payload(0, 3, ls)
+    torch.cuda.synchronize()
+    assert api.call_async("twophase_rbruck_alltoallv", (2,), dl, ls, lr, side) == 0 and dl.comm.wait() == 0, dl.comm.error()
+    assert dl.verify(ls, lr) == 0 and dl.comm.last_stats().lanes_per_item == 256
+    dp.comm.free()

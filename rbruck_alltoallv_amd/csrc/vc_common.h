@@ -132,6 +132,12 @@ struct VcSched {
 
 VC_HD bool vc_receives_now(const VcSched &S, int t) { return (unsigned)(t - S.recv_from) < (unsigned)S.recv_num; }
 
+// The b-th of `batches` batches of receivers.
+VC_HD void vc_take_batch(VcSched &S, int b, int batches) {
+    S.recv_from = (int)((int64_t)S.P * b / batches);
+    S.recv_num = (int)((int64_t)S.P * (b + 1) / batches) - S.recv_from;
+}
+
 VC_HD void vc_set_divisors(VcSched &S) {
     S.dn = vc_make_rank_divisor(S.n > 0 ? S.n : 1);
     S.dr = vc_make_rank_divisor(S.r > 0 ? S.r : 1);
@@ -240,6 +246,8 @@ hipError_t vc_launch_plan_sizes(const VcSched &S, const VcLaunchInfo *launches_h
 hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_off, int64_t *row_tot, int64_t *row_base, int64_t *row_bytes,
                                   int64_t *chain_row_tot, int64_t *chain_row_base, int64_t *header, int64_t *header_host, unsigned *ticket,
                                   hipStream_t st);
+// Forwarded execution: staging[t] = bytes of staging the blocks for receiver t take (P int64, device).
+hipError_t vc_launch_receiver_staging(const VcSched &S, VcTables T, int64_t *staging, hipStream_t st);
 // Forwarded execution: the chain items (every block's route in closed form, staging addresses from the plan tables;
 // chain_row_base and chain_row_tot as vc_launch_plan_forward leaves them).
 // header + cap_items (optional): the launch was enqueued before the host knew the plan; it writes nothing unless the

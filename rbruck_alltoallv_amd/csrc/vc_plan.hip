@@ -515,6 +515,21 @@ hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_o
     return hipGetLastError();
 }
 
+// What a call that runs in batches of receivers has to know before the first of them: grid (P).
+__global__ __launch_bounds__(VC_THREADS) void vc_receiver_staging_kernel(VcSched S, VcTables T, int64_t *__restrict__ staging) {
+    __shared__ int64_t lds[VC_WAVES_PER_BLOCK];
+    const int t = blockIdx.x;
+    int64_t sum = 0;
+    for (int s = threadIdx.x; s < S.P; s += VC_THREADS) sum += vc_block_staging(S, T, s, t);
+    sum = vc_block_sum(sum, lds);
+    if (threadIdx.x == 0) staging[t] = sum;
+}
+
+hipError_t vc_launch_receiver_staging(const VcSched &S, VcTables T, int64_t *staging, hipStream_t st) {
+    hipLaunchKernelGGL(vc_receiver_staging_kernel, dim3(S.P), dim3(VC_THREADS), 0, st, S, T, staging);
+    return hipGetLastError();
+}
+
 // The chain items: grid vc_rank_grid(P, chunks x slices).  The list is ordered in tiles of VC_TILE_RANKS receivers x VC_TILE_RANKS sources, receiver by
 // receiver inside a tile; the sources come in chunks of VC_THREADS, and several workgroups share a chunk (each a whole number
 // of tiles) when there are few ranks, which would otherwise leave most of the chip idle: the kernel is a chain of dependent

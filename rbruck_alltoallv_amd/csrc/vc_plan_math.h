@@ -246,6 +246,12 @@ VC_HD int vc_block_hops(const VcSched &S, int s, int t) {
     return hops;
 }
 
+// Forwarded execution: bytes of staging the slots of block (s, t) take, one for every hop but the last.
+VC_HD int64_t vc_block_staging(const VcSched &S, const VcTables &T, int s, int t) {
+    const int64_t len = (int64_t)vc_sc(S, T, s, t) * S.esz;
+    return len ? (vc_block_hops(S, s, t) - 1) * ((len + vc_phase(S, T, s, t) + VC_LINE - 1) & ~(int64_t)(VC_LINE - 1)) : 0;
+}
+
 VC_HD int64_t vc_send_offset(const VcSched &S, const VcTables &T, int s, int t) {
     return T.sbase[s] + (int64_t)vc_sd(S, T, s, t) * S.esz;
 }

@@ -59,6 +59,19 @@ def emulate(func, prob, send, recv, n=0, r=2, batch=0, uniform_count=0, recv_lo=
     return Result(rc, stats, traffic)
 
 
+def emulate_batches(func, prob, send, recv, batches, n=0, r=2, uniform_count=0, recv_lo=0):
+    """A forwarded call in batches of receivers: (errors, staging of the largest batch, staging of all batches together)."""
+    global _lib
+    if _lib is None:
+        _lib = C.CDLL(build())
+    stats = np.zeros(3, dtype=np.int64)
+    rc = _lib.batches_emulate(C.c_int(func), C.c_int(prob.P), C.c_int(n), C.c_int(r), C.c_int(prob.esz), C.c_int(uniform_count), _p(send),
+                              C.c_int64(send.size), _p(recv), C.c_int64(recv.size), _p(prob.sbase), _p(prob.rbase), _p(prob.sendcounts),
+                              _p(prob.sdispls), _p(prob.recvcounts), _p(prob.rdispls), C.c_int(recv_lo), C.c_int(batches), _p(stats))
+    assert rc == 0, rc
+    return tuple(int(v) for v in stats)
+
+
 # the reference's names, returning the return code and remembering the last Result
 last = None
 # module-wide switch: emulate forwarded execution (and check it against the launch-per-digit execution)

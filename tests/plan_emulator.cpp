@@ -294,6 +294,80 @@ extern "C" int plan_emulate(int func, int P, int n, int r, int batch, int esz, i
     return 0;
 }
 
+// A forwarded call in batches of receivers on one staging arena (run_batches in csrc/vc_api.hip, vc_plan_forward and vc_chain_emit in
+// csrc/vc_plan.hip): every batch's slots from the blocks for its receivers alone, its chain items copied.  Checks every range
+// against its arena, that the items of a batch do not overlap, that the blocks of the batch take exactly the staging that
+// vc_block_staging says, and that every block is in exactly one batch.  stats_out: errors, the largest batch's staging, the
+// staging of the batches together.
+extern "C" int batches_emulate(int func, int P, int n, int r, int esz, int uniform_count, const char *send, int64_t send_bytes, char *recv,
+                               int64_t recv_bytes, const int64_t *sbase, const int64_t *rbase, const int *sc, const int *sd, const int *rc,
+                               const int *rd, int recv_lo, int batches, int64_t *stats_out) {
+    VcSched S;
+    std::vector<VcLaunchInfo> L;
+    const int code = vc_make_schedule((VcFunc)func, P, n, r, 0, esz, uniform_count, S, L, 0, true);
+    if (code) return code;
+    S.recv_lo = recv_lo;
+    const int64_t PP = (int64_t)P * P;
+    std::vector<int> rdp;
+    VcTables T = {sc, sd, rc, rd, sbase, rbase, nullptr};
+    const int any = 0;
+    if (!S.table_mask) T.sc = T.sd = T.rc = T.rd = &any;
+    if (S.packed_recv) {
+        rdp.resize(PP);
+        for (int t = 0; t < P; t++) { int acc = 0; for (int s = 0; s < P; s++) { rdp[(int64_t)t * P + s] = acc; acc += rc[(int64_t)t * P + s]; } }
+        T.rd_packed = rdp.data();
+    }
+    const int nreg = S.w + S.w2, nslots = vc_hop_slots(S);
+    int64_t errors = 0, most = 0, all = 0;
+    std::vector<int> served(PP, 0);
+    for (int b = 0; b < batches; b++) {
+        vc_take_batch(S, b, batches);
+        std::vector<uint32_t> slot_off(PP * std::max(nreg, 1), 0);
+        std::vector<int64_t> row_base((int64_t)P * std::max(nreg, 1), 0), item(VC_CHAIN_HEAD + nslots);
+        int64_t stage_bytes = 0, of_blocks = 0;
+        for (int y = 0; y < nreg; y++)
+            for (int to = 0; to < P; to++) {
+                int64_t acc = 0;
+                row_base[(int64_t)y * P + to] = stage_bytes;
+                for (int id = 0; id < P; id++) {
+                    int s, t;
+                    const bool there = vc_slot_block(S, y, to, id, s, t) && vc_receives_now(S, t);
+                    const int64_t len = there ? (int64_t)vc_sc(S, T, s, t) * esz : 0;
+                    slot_off[((int64_t)y * P + to) * P + id] = (uint32_t)(acc / VC_LINE);
+                    acc += len ? (len + vc_phase(S, T, s, t) + VC_LINE - 1) & ~(int64_t)(VC_LINE - 1) : 0;
+                }
+                stage_bytes += acc;
+            }
+        std::vector<char> stage((size_t)stage_bytes + 1);
+        std::vector<Range> dst_ranges, none;
+        for (int t = 0; t < P; t++) {
+            if (!vc_receives_now(S, t)) continue;
+            for (int s = 0; s < P; s++) {
+                served[(int64_t)s * P + t]++;
+                of_blocks += vc_block_staging(S, T, s, t);
+                for (int64_t c = 0; c < vc_chain_count(S, T, s, t); c++) {
+                    vc_chain_item(S, T, slot_off.data(), row_base.data(), s, t, c, item.data());
+                    const int64_t so = item[VC_CHAIN_SRC] & VC_OFFSET_MASK, len = item[VC_CHAIN_LEN];
+                    if (so + len > send_bytes) { errors++; continue; }
+                    for (int64_t k = 0; k < item[VC_CHAIN_NHOP]; k++) {
+                        const int64_t d = item[VC_CHAIN_HEAD + k], dof = d & VC_OFFSET_MASK;
+                        const int space = (int)(d >> VC_SPACE_SHIFT);
+                        if (dof < 0 || dof + len > (space == 1 ? recv_bytes : (space == 2 ? stage_bytes : -1))) { errors++; continue; }
+                        dst_ranges.push_back({dof, dof + len, space});
+                        memcpy((space == 1 ? recv : stage.data()) + dof, send + so, (size_t)len);
+                    }
+                }
+            }
+        }
+        errors += count_overlaps(dst_ranges, none) + (of_blocks != stage_bytes);
+        most = std::max(most, stage_bytes);
+        all += stage_bytes;
+    }
+    for (int64_t i = 0; i < PP; i++) errors += served[i] != 1;
+    stats_out[0] = errors; stats_out[1] = most; stats_out[2] = all;
+    return 0;
+}
+
 // The staging allocator of the planning kernel on its own: sizes per piece of every (arrival, departure) family in
 // (VC_RECYCLE_SEGMENTS pieces per family), bases out.
 extern "C" int64_t staging_allocate(int w, int w2, int msd, int coalesce, const int64_t *size, int64_t *base) {

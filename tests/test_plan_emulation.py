@@ -635,3 +635,23 @@ def test_multiply_and_shift_division_is_exact():
     assert E.division_mismatches(1 << 30, 1 << 30) == 0
     for d in (32769, 65535, 65536, 65537, 1000003, (1 << 24) - 1, (1 << 30) - 1, (1 << 30) + 1, (1 << 31) - 1):
         assert E.division_mismatches(d, d, 4096) == 0, d
+
+
+@pytest.mark.parametrize("P,n,r,func", [(24, 0, 2, E.F_TWOPHASE), (37, 0, 3, E.F_TWOPHASE), (32, 0, 2, E.F_OM), (41, 0, 2, E.F_TUNA), (24, 8, 2, E.F_TTPL),
+                                        (36, 6, 6, E.F_TTPL_S1), (48, 4, 2, E.F_TTPL_RBRUCK), (24, 6, 2, E.F_UNIFORM_ISPLIT), (9, 0, 2, E.F_SPREADOUT)])
+@pytest.mark.parametrize("batches", [1, 2, 5, 8])
+def test_batches_of_receivers(P, n, r, func, batches):
+    """The batches' plans cover every block once, their staging is what the blocks' own says and adds up to that of the call in one."""
+    count = 301 if func == E.F_UNIFORM_ISPLIT else 0
+    if count:
+        prob = W.make_uniform_problem(P, count, 2)
+    else:
+        counts = W.counts_uniform_random(P, 700, seed=P)
+        counts[counts % 5 == 0] = 0
+        counts[1, :] = 9000                               # several pieces
+        prob = W.make_problem(counts, 2, 1, 0 if func == E.F_TTPL else 1)
+    send, recv = W.fill_send_arena(prob, 0, 3), np.full(prob.recv_bytes, 0xEE, dtype=np.uint8)
+    errors, most, staging = E.emulate_batches(func, prob, send, recv, batches, n, r, count, recv_lo=80)
+    assert errors == 0 and np.array_equal(recv, W.expected_recv_arena(prob, send))
+    whole = E.emulate(func, prob, send, np.full(prob.recv_bytes, 0xEE, dtype=np.uint8), n=n, r=r, uniform_count=count, recv_lo=80, forward=True)
+    assert (whole.rc, whole.errors) == (0, 0) and staging == whole.stage_bytes and most <= staging

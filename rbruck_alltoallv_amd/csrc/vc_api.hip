@@ -172,19 +172,18 @@ static bool worth_reusing(const vc_comm *c, const VcSched &S, int64_t stage_byte
 
 // Forwarded execution keeps every hop's copy of every block (nothing reads them, so nothing says when one could be
 // overwritten): its staging is the sum over the blocks of (hops - 1) x bytes, 3.5 x the payload for a radix-2 Bruck
-// over 512 ranks.  A communicator that bounds its staging runs such a call one launch per digit instead, where staging
-// memory is reused (and stays below about twice the payload): beyond three times the payload, and only when it
-// matters (more than an eighth of the device's memory, 36 GB here; vc_comm_set_staging_bound takes another allowance).
-// Measured on MI355X: configuration 5 with radix 2, 60 GB forwarded in 17.4 ms against 30 GB in 25.5 ms; a radix-4
+// over 512 ranks.  A communicator that bounds its staging does not run such a call that way: beyond three times the payload, and
+// only when it matters (more than an eighth of the device's memory, 36 GB here; vc_comm_set_staging_bound takes another allowance).
+// A blocking call in the default mode then runs in batches of receivers where that can be done (staging_batches, run_batches).  Other
+// modes, _async calls and plans run one launch per digit, where staging memory is reused and stays below about twice the payload.
+// Measured on MI355X: configuration 5 with radix 2, 30 GB in batches 14.5 ms, 20 GB one launch per digit 25.8; a radix-4
 // two-layer Bruck at configuration 4 (13 GB, 3.1 x its payload) stays forwarded: 4.8 ms against 6.8.
 bool staging_out_of_bound(const vc_comm *c, int64_t stage_bytes, int64_t payload_bytes) {
     return c->bound_staging && stage_bytes > c->staging_allowance && stage_bytes > 3 * payload_bytes;
 }
 
-// In the default mode such a call stays forwarded where it can: in batches of receivers that use the same staging memory one after the
-// other, each within the allowance.  0: more than VC_MAX_BATCHES of them, or a mode that runs the call one launch per digit.
-// Measured on MI355X: configuration 5 with radix 2 (512 ranks, 17.2 GB, 60 GB of staging) 25.9 ms -> 14.8.  (Not more batches than it
-// takes: every one is planned and listed for itself, 0.2 ms.)
+// As many batches of receivers, using the same staging memory one after the other, as keep each of them within the allowance (not more:
+// every one is planned and listed for itself, 0.2 ms).  0: more than VC_MAX_BATCHES, or a mode that runs the call one launch per digit.
 #define VC_MAX_BATCHES 8
 int staging_batches(const vc_comm *c, int64_t stage_bytes) {
     const int64_t batches = (stage_bytes + c->staging_allowance - 1) / c->staging_allowance;

@@ -75,7 +75,8 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
     if (!THROUGH && n == VC_PIECE && w == 0) {
         // A whole aligned piece, the inside of a long block: no vector to leave out and no edge.  A wavefront waits for each of its
         // stores before the next one: on lists of these the memory runs a few per cent faster with fewer writes in flight
-        // (64 ranks, 1.3 MB blocks, two hops: 2436 us -> 2361).
+        // (64 ranks, 1.3 MB blocks, two hops, builds in turn in one process, quartiles within 0.4 %: without this path 2430 us, with it but
+        // without the waits 2407, so 2349; 512 ranks, 1 MiB blocks 6527 / 6494 / 6474).
         constexpr int WHOLE = VC_PIECE / 16 / LANES;
         vc_u32x4 v[WHOLE];
 #pragma unroll
@@ -109,8 +110,8 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
     char edge_byte = 0;
     if (edge >= 0) edge_byte = src[edge];
     if (!go()) return;
-    // all at once and after the last load has arrived, so that the writes of one line reach the L2 together (512 ranks, 1 KiB: 107 us
-    // -> 99; 1024 ranks, 4 KiB: 2475 -> 2434)
+    // all at once and after the last load has arrived, so that the writes of one line reach the L2 together (calls, builds in turn in one
+    // process: 512 ranks, 1 KiB 197 us -> 188; 1024 ranks, 4 KiB 2486 -> 2453; 256 ranks, Zipf 165.0 -> 166.2)
     __builtin_amdgcn_s_waitcnt(VC_WAIT_VMCNT0);
     for (int k = 0; k < nhop; k++) {
         char *dst = next_dst(), *dw = dst - w;
@@ -518,8 +519,8 @@ __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T
 }
 
 // SELF: one launch on fixed-stride staging that tells the host itself that it is done (vc_signal), with everything it stores stored past
-// the caches.  A kernel behind this one that only does that costs the boundary between the two: 8 ranks 13.5 -> 13.0 us,
-// 24 ranks of 0 - 32 KiB blocks 30.6 -> 26.7.  The quarter kernel has no such instance: its lanes' short stores past the caches each
+// the caches.  A kernel behind this one that only does that costs the boundary between the two: 8 ranks of 0 - 64 ints 13.0 -> 12.8 us,
+// 32 ranks of 0 - 2 KiB 14.0 -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3.  The quarter kernel has no such instance: its lanes' short stores past the caches each
 // cost a write to memory (64 ranks, 1 KiB blocks: 16.6 -> 21.9 us).
 template <int LANES, bool SELF>
 __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
@@ -535,6 +536,9 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
 
 // The same for pairs whose blocks are a few hundred bytes: a quarter of a wavefront per pair, four pairs in a row per
 // wavefront.  Lane q of a group evaluates hop slots q and q + 16; the four routes of the wavefront go through LDS.
+// Eight vectors of a lane in flight, 2 KiB a group: 87 VGPRs, 5 wavefronts per SIMD.  With four (62 VGPRs, 7) the loads of a second round
+// wait for the stores of the first: calls of blocks of 512 B - 2.5 KiB on average on 64 - 200 ranks 3 - 5 % slower (128 ranks, 2 KiB 33.0
+// us -> 34.2; 192 ranks, 600 B 38.3 -> 40.4), 1024 ranks, 700 B 596 -> 605, and only direct calls on 300 ranks faster (91.9 -> 89.9).
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                          const int64_t *__restrict__ row_base,
                                                                          const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -594,8 +598,8 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
 // the blocks it writes (of one receiver, from neighbouring sources) share cache lines.
 // 64 / BATCH lanes per pair evaluate its hop slots and leave the route in LDS.  Blocks of no more than VC_LANE_BLOCK bytes are then moved by
 // a lane each, when all blocks of the wavefront are that short; else every quarter of the wavefront carries BATCH / 4 of them, one
-// after the other.  Measured on MI355X, 1024 ranks, two hops for most blocks: 0 - 16 bytes 80 us (pairs of one receiver
-// in a row, every block a quarter of a wavefront) -> 40; 0 - 512 bytes 280 us either way.
+// after the other.  Measured on MI355X, 1024 ranks, two hops for most blocks: 0 - 16 bytes 76 us (pairs of one receiver
+// in a row, every block a quarter of a wavefront) -> 28; 0 - 512 bytes 277 -> 250.
 template <int BATCH>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                        const int64_t *__restrict__ row_base,

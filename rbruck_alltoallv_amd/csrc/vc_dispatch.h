@@ -45,8 +45,9 @@
 #define VC_LISTLESS_MAX_AVERAGE 4096          // a call the short-block kernels were chosen for must stay below this average
 #define VC_STRIDED_MAX_BYTES ((int64_t)256 << 20)
 #define VC_STRIDED_MAX_PAIRS 36864            // 192 ranks
-// the launch signals its own end: calls with cold caches gain up to 32 ranks (0 - 2 KiB blocks even, 0 - 32 KiB 26.7 us against 30.6 on 24
-// ranks) and lose on 64 (0 - 4 KiB 23.2 -> 25.1): stores past the caches fill a memory queue that the L2s would have filled later
+// the launch signals its own end: gains up to 32 ranks (32 ranks of 0 - 2 KiB 14.0 us -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3), is even
+// on 48 (0 - 4 KiB 17.0), and on 64 loses with cold caches what it gains with warm ones (0 - 4 KiB 23.2 -> 25.1, 21.5 -> 19.9): stores past
+// the caches fill a memory queue that the L2s would have filled later
 #define VC_SELF_MAX_PAIRS 1024
 #define VC_SELF_MAX_BYTES ((int64_t)64 << 20)
 // list-driven copy kernels: lanes per work item by the average piece of the launch

@@ -85,22 +85,6 @@ __device__ __forceinline__ int64_t vc_block_sum(int64_t v, int64_t *lds) {
     return total;
 }
 
-// Maximum across a 256-thread workgroup (every thread gets the result).
-__device__ __forceinline__ int64_t vc_block_max(int64_t v, int64_t *lds) {
-#pragma unroll
-    for (int o = VC_WAVE / 2; o > 0; o >>= 1) {
-        const int64_t u = __shfl_xor(v, o, VC_WAVE);
-        v = u > v ? u : v;
-    }
-    __syncthreads();                       // protects lds from the previous use
-    if ((threadIdx.x & (VC_WAVE - 1)) == 0) lds[threadIdx.x / VC_WAVE] = v;
-    __syncthreads();
-    int64_t m = lds[0];
-#pragma unroll
-    for (int k = 1; k < VC_WAVES_PER_BLOCK; k++) m = lds[k] > m ? lds[k] : m;
-    return m;
-}
-
 // Five totals of a 256-thread workgroup at once (one barrier): sums of v[0], v[1], v[2], maxima of v[3], v[4] (not negative).
 // Thread 0 receives them; lds holds 5 * VC_WAVES_PER_BLOCK int64.
 __device__ __forceinline__ void vc_block_totals(int64_t v[5], int64_t *lds) {

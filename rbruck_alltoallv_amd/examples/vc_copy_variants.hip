@@ -111,7 +111,8 @@ __device__ __forceinline__ void piece_store(char *dst, const PieceRegs &R) {
         if (R.has[i]) vc_store16(dw + ((int64_t)(t + i * VC_THREADS) << 4), R.v[i]);
 }
 
-// M      items in a row per workgroup (1: the library's shape)
+// M      items in a row per workgroup (1: the library's shape).  The variants do not wait for all loads before the first store, nor read
+//        the later hops' destinations ahead, as the library's kernel does: the base they build on is a row of its own.
 // PIPE   M > 1: the loads of item m + 1 go out before the stores of item m (two register sets); else all loads first
 // ALIGNED see piece_load
 // AHEAD  > 0: lane 0 of every workgroup touches the item AHEAD workgroups further down its XCD's range, so that the
@@ -377,7 +378,7 @@ int main(int argc, char **argv) {
         hipLaunchKernelGGL((variant_kernel<M, PIPE, ALIGNED, AHEAD, WHOLE, 0>), dim3((unsigned)(N / M)), dim3(VC_THREADS), 0, 0, items_dev, \
                            (unsigned)N, (unsigned)(N / M / VC_XCDS), sendbuf, recvbuf, stage);                                      \
     })
-    VARIANT("the same kernel restated in this file", 1, false, false, 0, false);
+    VARIANT("base of the variants: stores as loads arrive, hops read one by one", 1, false, false, 0, false);
     VARIANT("item fetched in one scalar round trip", 1, false, false, 0, true);
     VARIANT("item's cache line touched 256 workgroups ahead", 1, false, false, 256, false);
     VARIANT("item's cache line touched 1024 workgroups ahead", 1, false, false, 1024, false);
@@ -410,9 +411,9 @@ int main(int argc, char **argv) {
         const auto launch = [&](auto kernel, unsigned lds_kib) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)N), dim3(VC_THREADS), lds_kib << 10, 0, items_dev, (unsigned)N, (unsigned)(N / VC_XCDS), sendbuf, recvbuf, stage);
         };
-        failures += row("restated kernel + 26 KiB of unused LDS per workgroup (fewer resident)", [&] { launch(variant_kernel<1, false, false, 0, false, 26>, 26); });
-        failures += row("restated kernel + 40 KiB of unused LDS per workgroup", [&] { launch(variant_kernel<1, false, false, 0, false, 40>, 40); });
-        failures += row("restated kernel + 53 KiB of unused LDS per workgroup", [&] { launch(variant_kernel<1, false, false, 0, false, 53>, 53); });
+        failures += row("base + 26 KiB of unused LDS per workgroup (fewer resident)", [&] { launch(variant_kernel<1, false, false, 0, false, 26>, 26); });
+        failures += row("base + 40 KiB of unused LDS per workgroup", [&] { launch(variant_kernel<1, false, false, 0, false, 40>, 40); });
+        failures += row("base + 53 KiB of unused LDS per workgroup", [&] { launch(variant_kernel<1, false, false, 0, false, 53>, 53); });
     }
     failures += row("vc_copy_chains_kernel<256> once more", product);
     // what contiguous copies of the payload sustain in the same process

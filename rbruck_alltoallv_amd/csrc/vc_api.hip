@@ -44,17 +44,19 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
             if (e == hipSuccess) g_scratch_ptr[c->device] = static_cast<unsigned char *>(ptr);
         }
     }
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_header, sizeof(int64_t) * VC_HEADER_ROOM, hipHostMallocCoherent);
+    // one pinned allocation (12 us each): header and totals, flags, launch table
+    const size_t flags_at = (sizeof(int64_t) * VC_HEADER_ROOM + VC_LINE - 1) / VC_LINE * VC_LINE, launches_at = flags_at + sizeof(int) * VC_FLAG_WORDS;
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_header, launches_at + sizeof(VcLaunchInfo) * VC_MAX_LAUNCHES, hipHostMallocCoherent);
     if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_header_dev, c->h_header, 0);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_launches, sizeof(VcLaunchInfo) * VC_MAX_LAUNCHES, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, VC_FLAG_WORDS * sizeof(int), hipHostMallocCoherent);
-    if (e == hipSuccess) memset(c->h_flags, 0, VC_FLAG_WORDS * sizeof(int));
-    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->h_flags_dev, c->h_flags, 0);
-    if (e == hipSuccess) e = c->counting.reserve(VC_COUNTING_BYTES);
     if (e == hipSuccess) {
-        const std::vector<char> zeros(VC_COUNTING_BYTES, 0);
-        e = hipMemcpy(c->counting.p, zeros.data(), zeros.size(), hipMemcpyHostToDevice);
+        c->h_flags = reinterpret_cast<int *>(reinterpret_cast<char *>(c->h_header) + flags_at);
+        c->h_flags_dev = reinterpret_cast<int *>(reinterpret_cast<char *>(c->h_header_dev) + flags_at);
+        c->h_launches = reinterpret_cast<VcLaunchInfo *>(reinterpret_cast<char *>(c->h_header) + launches_at);
+        memset(c->h_flags, 0, VC_FLAG_WORDS * sizeof(int));
     }
+    if (e == hipSuccess) e = c->counting.reserve(VC_COUNTING_BYTES);
+    if (e == hipSuccess) e = hipMemset(c->counting.p, 0, VC_COUNTING_BYTES);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);          // (the calls may run on a stream that does not wait for this one)
     if (e != hipSuccess) {
         (void)vc_comm_free(c);
         return fail_hip(e, "vc_comm_create", __LINE__);
@@ -80,9 +82,7 @@ extern "C" int vc_comm_free(vc_comm_t c) {
         b->release();
     free_retired_stage(c);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
-    if (c->h_header) (void)hipHostFree(c->h_header);
-    if (c->h_launches) (void)hipHostFree(c->h_launches);
-    if (c->h_flags) (void)hipHostFree(c->h_flags);
+    if (c->h_header) (void)hipHostFree(c->h_header);      // (flags and launch table with it)
     delete c;
     return VC_OK;
 }

@@ -527,7 +527,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
 }
 
 // A forwarded call through the work-item list, without the host's look at the plan in mid-call (a round trip of ~10 us):
-// the list kernel and the copy kernel go out right behind the sizing kernels, the list's length guessed from the last
+// the list kernel and the copy kernel go out right behind the planning kernel, the list's length guessed from the last
 // forwarded call on the communicator, and check on the device what the host checks otherwise — tables in order, the list
 // and the staging arena large enough, the staging within the communicator's bound (VcChainGuard).  The host reads the
 // same header after the one synchronisation of the call: a plan the launches could not serve has moved nothing and goes

@@ -251,7 +251,7 @@ hipError_t vc_launch_receiver_staging(const VcSched &S, VcTables T, int64_t *sta
 // Forwarded execution: the chain items (every block's route in closed form, staging addresses from the plan tables;
 // chain_row_base and chain_row_tot as vc_launch_plan_forward leaves them).
 // header + cap_items (optional): the launch was enqueued before the host knew the plan; it writes nothing unless the
-// device header the sizing kernels left says the tables are in order and the list holds all header[2] items.
+// device header the planning kernel left says the tables are in order and the list holds all header[2] items.
 hipError_t vc_launch_chain_plan(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base,
                                 const int64_t *chain_row_base, const int64_t *chain_row_tot, int64_t *items, int64_t nitems, hipStream_t st,
                                 const int64_t *header = nullptr, int64_t cap_items = 0);
@@ -269,7 +269,7 @@ hipError_t vc_launch_copy_items(const VcDesc *items, int64_t nitems, int lanes, 
                                 hipStream_t st);
 hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf,
                                  char *stage, hipStream_t st);
-// What the plan of a call must look like for a list and a copy launch that were enqueued right behind the sizing kernels,
+// What the plan of a call must look like for a list and a copy launch that were enqueued right behind the planning kernel,
 // before the host had seen the plan, to do their work.  Kernels and host evaluate it on the same header, so both agree on
 // whether anything was moved.
 struct VcChainGuard {

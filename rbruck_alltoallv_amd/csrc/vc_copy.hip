@@ -342,7 +342,8 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_items_quarter_kernel(const Vc
 // source).  Each puts its sums and maxima into a slot of its own in host memory, and the host adds the slots up when the launch
 // is over; their verdict goes into VC_VERDICTS copies of one word, and every copying wavefront looks at one of them.  (With an atomic
 // per wavefront on each of six shared words, and one verdict word that all wavefronts polled, these were what the launch waited for:
-// atomics on one address follow each other at about 10 ns.  128 ranks, 2 KiB blocks: 57 us -> 26; 64 ranks: 14 -> 13.)
+// atomics on one address follow each other at about 10 ns.  Kernel times with warm caches: 128 ranks, 2 KiB blocks 27.6 us -> 24.5; 64 ranks
+// of 0 - 4 KiB 14.3 -> 12.8.)
 __device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &T, unsigned long long *verdict, int64_t *totals) {
     const int P = S.P, pairs = P * P, per_wave = VC_TOTALS_PER_WAVE, nwaves = (int)vc_totals_waves(P);      // P^2 <= VC_STRIDED_MAX_PAIRS
     const int wave = (int)blockIdx.x * (int)(blockDim.x / VC_WAVE) + (int)threadIdx.x / VC_WAVE;

@@ -144,8 +144,8 @@ extern "C" int vc_suggest_tunables(const int *sendcounts, int elem_size, int n, 
     unsigned long long got[2 * (VC_MAX_CANDIDATES + 1)];
     HIP_TRY(hipMemcpyAsync(got, moved_dev, sizeof(unsigned long long) * words, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    // Time model.  A blocking call waits for the stream twice (after sizing the plan, at the end) and launches three planning
-    // kernels besides its copy kernels.  Every launch costs one launch latency; bytes move at the rate
+    // Time model.  A blocking call waits twice (after planning, at the end) and launches three kernels (planning, list, end) besides its
+    // copy kernels.  Every launch costs one launch latency; bytes move at the rate
     // of the plain copy times what the block movers keep of it.  One launch per digit: every hop reads and writes its
     // bytes and its 32-byte work items are written and read once.  Forwarded execution: one launch; the payload is read
     // once, every hop writes its bytes, and every piece has one item of 24 + 8 x (hop slots) bytes.  The planning kernels

@@ -96,7 +96,7 @@ int vc_comm_set_bases(vc_comm_t comm, const int64_t *sbase_bytes, const int64_t 
  *    where the previous hop left it.  This is the mode whose launches vc_comm_last_stats and vc_comm_last_traffic
  *    describe one by one.
  * Results are the same in all of them, and so are the staging contents wherever two modes use the same staging layout
- * (a region per digit phase: staging bound off, no fixed stride).  Applies to calls and to plans created afterwards
+ * (a region per digit phase: staging bound off, no window, no fixed stride).  Applies to calls and to plans created afterwards
  * (plans always hold a list). */
 int vc_comm_set_forwarding(vc_comm_t comm, int enable);
 
@@ -110,9 +110,13 @@ int vc_comm_set_forwarding(vc_comm_t comm, int enable);
  *    some tens of microseconds, and such a call is planned twice); the
  *    peak then stays below about 1.5 x the payload where separate regions need the sum over the blocks of
  *    (hops - 1) x bytes (configuration 5 with radix 2: 60 GB);
- *  - forwarded execution keeps every hop's copy of every block, because nothing reads them and so nothing says when one
- *    may be overwritten.  A call whose staging would pass both the allowance (an eighth of the device's memory, at least
- *    1 GiB) and three times its payload is therefore run in batches of receivers that use the same staging memory one after
+ *  - forwarded execution in the default mode with the default bound (1) stages in a window of 32 MiB: a slot at offset x of the layout lies
+ *    at x mod 32 MiB, piece by piece.  A piece makes its next hop out of the registers of the workgroup that staged it, so nothing reads
+ *    what it left behind, and the window stays in the memory-side cache.  Calls on fixed-stride slots with a
+ *    wavefront or a workgroup per pair of ranks have an arena of up to 256 MiB instead;
+ *  - forwarded execution in another mode or with an allowance keeps every hop's copy of every block in a place of its own.  A call whose
+ *    staging would pass both the allowance (an eighth of the device's memory, at least
+ *    1 GiB) and three times its payload is run in batches of receivers that use the same staging memory one after
  *    the other (blocking calls in the default mode of vc_comm_set_forwarding, when 8 batches suffice and none of them needs
  *    more than 1.25 x the allowance), or one launch per digit instead (vc_stats_t.execution and n_launches say so).
  * Unbounded: every digit phase has its own region and forwarded calls stay forwarded, whatever they need. */
@@ -371,8 +375,9 @@ int vc_comm_last_stats(vc_comm_t comm, vc_stats_t *out);
 int vc_comm_last_traffic(vc_comm_t comm, int launch, int64_t *matrix_out);
 
 /* The staging arena as the last call left it: DEVICE pointer and the bytes that call used (what the reference keeps in
- * extra_buffer / temp_recv_buffer between rounds, src/twophase_tunable_rbruckv.cpp:59-61).  Both execution modes leave
- * the same bytes there; tests compare them.  The pointer is valid until a call on this communicator needs more. */
+ * extra_buffer / temp_recv_buffer between rounds, src/twophase_tunable_rbruckv.cpp:59-61).  Where every slot has a place of
+ * its own (vc_comm_set_staging_bound(comm, 0)) both execution modes leave the same bytes there; tests compare them.  A window holds what went
+ * through it last.  The pointer is valid until a call on this communicator needs more. */
 int vc_comm_staging(vc_comm_t comm, void **ptr_out, int64_t *bytes_out);
 
 /* ---- harness utilities (payload of the reference drivers, examples/rbruckv_example.cpp:88-92, and a

@@ -127,6 +127,7 @@ extern "C" int vc_comm_set_staging_bound(vc_comm_t c, int enable) {
     if (!c) return fail_arg("null communicator");
     if (enable < 0) return fail_arg("vc_comm_set_staging_bound: 0, 1 or an allowance in MiB");
     c->bound_staging = enable != 0;
+    c->own_allowance = enable > 1;
     c->staging_allowance = enable > 1 ? (int64_t)enable << 20 : default_staging_allowance();
     return VC_OK;
 }
@@ -150,6 +151,10 @@ int ensure_events(vc_comm *c, size_t n) {
 
 static int schedule_error(int code);
 
+// Forwarded calls and plans of a communicator in the default mode with the default bound stage in a window (VC_STAGE_WINDOW); where the caller
+// asked for a mode, an allowance or no bound, every slot has a place of its own.
+bool stages_in_window(const vc_comm *c) { return c->forward == 1 && c->bound_staging && !c->own_allowance; }
+
 // The schedule of a call in one of the two execution modes.  Launch-per-digit execution reuses staging memory when the
 // communicator bounds its staging (the default) and there is something to reuse: with fewer than three staging regions
 // no sub-region is written after another one has been read for the last time.
@@ -159,6 +164,7 @@ static int make_schedule(const vc_comm *c, const CallParams &q, bool forward, Vc
     if (rc) return rc;
     const int nreg = S.w + S.w2;
     if (!forward && reuse && c->bound_staging && nreg >= 3 && nreg + 1 <= VC_RECYCLE_MAX_SLOTS) S.recycle = 1;
+    if (forward && stages_in_window(c) && vc_may_stage(S)) S.window = VC_STAGE_WINDOW;
     return VC_OK;
 }
 
@@ -170,14 +176,13 @@ static bool worth_reusing(const vc_comm *c, const VcSched &S, int64_t stage_byte
     return c->bound_staging && !S.recycle && nreg >= 3 && nreg + 1 <= VC_RECYCLE_MAX_SLOTS && stage_bytes > (c->staging_allowance >> 5);
 }
 
-// Forwarded execution keeps every hop's copy of every block (nothing reads them, so nothing says when one could be
-// overwritten): its staging is the sum over the blocks of (hops - 1) x bytes, 3.5 x the payload for a radix-2 Bruck
-// over 512 ranks.  A communicator that bounds its staging does not run such a call that way: beyond three times the payload, and
-// only when it matters (more than an eighth of the device's memory, 36 GB here; vc_comm_set_staging_bound takes another allowance).
-// A blocking call in the default mode then runs in batches of receivers where that can be done (staging_batches, run_batches).  Other
+// Without a window forwarded execution keeps every hop's copy of every block: its staging is the sum over the blocks of (hops - 1) x
+// bytes, 3.5 x the payload for a radix-2 Bruck over 512 ranks.  A communicator that bounds its staging does not run such a call that way:
+// beyond three times the payload, and only when it matters (more than an eighth of the device's memory, 36 GB here;
+// vc_comm_set_staging_bound takes another allowance).  A blocking call in the default mode, with an allowance of the caller's, then runs in batches of receivers where that can be done (staging_batches, run_batches).  Other
 // modes, _async calls and plans run one launch per digit, where staging memory is reused and stays below about twice the payload.
-// Measured on MI355X: configuration 5 with radix 2, 30 GB in batches 14.5 ms, 20 GB one launch per digit 25.8; a radix-4
-// two-layer Bruck at configuration 4 (13 GB, 3.1 x its payload) stays forwarded: 4.8 ms against 6.8.
+// Measured on MI355X: configuration 5 with radix 2, 30 GB in batches 14.5 ms, 20 GB one launch per digit 25.8 (in a window 10.8); a
+// radix-4 two-layer Bruck at configuration 4 (13 GB, 3.1 x its payload) stays forwarded: 4.8 ms against 6.8.
 bool staging_out_of_bound(const vc_comm *c, int64_t stage_bytes, int64_t payload_bytes) {
     return c->bound_staging && stage_bytes > c->staging_allowance && stage_bytes > 3 * payload_bytes;
 }
@@ -195,6 +200,7 @@ struct PlanInfo {
     int nl = 0, n_digits = 0;
     int batches = 1;                                // launches of forwarded execution
     int recv_lo = 0;
+    int window = 0;                                 // VcSched::window
     int64_t stage_bytes = 0, payload_bytes = 0;
     std::vector<int64_t> first, count, bytes;       // per launch: first work item, item count, bytes moved
     std::vector<char> inter;                        // per launch: its messages cross nodes
@@ -307,7 +313,7 @@ static int plan_read(vc_comm *c, const VcSched &S, const std::vector<VcLaunchInf
     if (h[VC_HEADER_BAD] != 0)    // such tables would send the copy kernels outside the arenas
         return fail_arg("sendcounts / sdispls / recvcounts / rdispls hold negative entries, or recvcounts[t][s] != sendcounts[s][t]",
                         VC_ERR_TABLES);
-    out.nl = nl; out.n_digits = S.w + S.w2; out.recv_lo = S.recv_lo;
+    out.nl = nl; out.n_digits = S.w + S.w2; out.recv_lo = S.recv_lo; out.window = S.window;
     out.stage_bytes = h[0]; out.payload_bytes = h[1];
     out.first.assign(nl, 0); out.count.assign(nl, 0); out.bytes.assign(nl, 0); out.inter.assign(nl, 0); out.lanes.assign(nl, VC_THREADS);
     if (forward) {
@@ -372,7 +378,7 @@ static int launch_items(vc_comm *c, const PlanInfo &pi, const void *items_any, c
     if (c->stage.cap < (size_t)pi.stage_bytes + 64) return fail_arg("staging arena smaller than the plan needs");
     if (pi.chain) {
         HIP_TRY(vc_launch_copy_chains(static_cast<const int64_t *>(items_any), pi.chain_stride, pi.chain_items,
-                                      pi.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), c->stream));
+                                      pi.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), c->stream, pi.window));
         return VC_OK;
     }
     const VcDesc *items = static_cast<const VcDesc *>(items_any);
@@ -465,7 +471,8 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     if (d.stride <= 0) return 0;
     const int pair_lanes = d.stride_lanes;
     S.stride = d.stride;
-    const int64_t need = vc_strided_stage_bytes(S);
+    if (pair_lanes != VC_QUARTER) S.window = 0;           // (no more than VC_STRIDED_MAX_BYTES: a window would only save memory)
+    const int64_t need = vc_window_bytes(vc_strided_stage_bytes(S), S.window);
     hipStream_t st = c->stream;
     // two sets of words in turn: a launch counts in one, which must start from zero, and clears the other one for the next call
     if (!c->verdicts.p) {
@@ -555,7 +562,7 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     int64_t done = 0;                                     // items the guarded launch was sized for
     HIP_TRY(vc_launch_copy_chains_guarded(c->desc.as<int64_t>(), stride, guess, lanes, sendbuf, recvbuf, c->stage.as<char>(), st, c->B.header,
-                                          guard, &done));
+                                          guard, &done, S.window));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     HIP_TRY(VC_WAIT(c));
     int rc = plan_read(c, S, L, pi, true);
@@ -564,7 +571,7 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
     pi.chain_lanes = lanes;
     if (pi.chain_items > done) {                          // more pieces than the last call had
         HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>() + done * stride, stride, pi.chain_items - done, lanes, sendbuf, recvbuf,
-                                      c->stage.as<char>(), st));
+                                      c->stage.as<char>(), st, S.window));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
         HIP_TRY(VC_WAIT(c));
     }
@@ -610,7 +617,8 @@ static int run_batches(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, VcTa
         rc = plan_emit(c, S, L, T, c->desc, pi);
         if (rc) return rc;
         if (c->timing) HIP_TRY(hipEventRecord(c->events[2 + 2 * b], st));
-        HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>(), pi.chain_stride, pi.chain_items, all.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+        HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>(), pi.chain_stride, pi.chain_items, all.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+                                      S.window));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3 + 2 * b], st));
         all.bytes[b] = pi.bytes[0];
     }
@@ -697,13 +705,16 @@ static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std:
     if (rc) return rc;
     hipStream_t st = c->stream;
     const int lanes = c->stage.cap || !vc_may_stage(S) ? vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes : 0;
-    const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
+    // (an arena with a window holds any call: one of long blocks behind short ones must not run in the shape of these)
+    const int64_t max_pieces = S.window && vc_may_stage(S) && (lanes == VC_QUARTER || lanes == VC_BATCHED) ? VC_LISTLESS_MAX_PIECES : 0;
+    const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, max_pieces, 0, 0, 0};
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
         HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     c->pending.active = true;
     c->pending.S = S; c->pending.T = T; c->pending.sendbuf = sendbuf; c->pending.recvbuf = recvbuf; c->pending.lanes = lanes;
+    c->pending.max_pieces = max_pieces;
     c->pending.n_launch_infos = (int)L.size();
     c->pending.q = q;
     return VC_OK;
@@ -732,15 +743,15 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
     PlanInfo pi;
     int rc = plan_read(c, S, L, pi, true);
     if (rc) return rc;
-    VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
+    VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, c->pending.max_pieces, 0, 0, 0};
     int lanes = c->pending.lanes;
-    if (!lanes || !vc_listless_ok(c->h_header, guard)) {  // no arena, or one too small: nothing has been moved yet
+    if (!lanes || !vc_listless_ok(c->h_header, guard)) {  // no arena, or one too small, or longer blocks: nothing has been moved yet
         // a call whose forwarded staging is out of the communicator's bound runs one launch per digit on reused staging (its blocking
         // twin: in batches of receivers where it can)
         if (staging_out_of_bound(c, pi.stage_bytes, pi.payload_bytes))
             return run_schedule(c, c->pending.q, c->pending.sendbuf, c->pending.recvbuf, c->pending.T, false, true);
         HIP_TRY(reserve_stage(c, (size_t)pi.stage_bytes + 64));
-        guard.stage_cap = (int64_t)c->stage.cap - 64;
+        guard = {(int64_t)c->stage.cap - 64, 0, 0, 0, 0};
         lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, VcHint{1, pi.chain_items, pi.payload_bytes, pi.max_pieces, pi.max_len}, S).lanes;
         if (c->timing) {
             std::swap(c->events[1], c->events[2]);        // (the planning ended where the first attempt began)

@@ -30,6 +30,16 @@
 #define VC_SPACE_STAGE (2ll << VC_SPACE_SHIFT)
 #define VC_OFFSET_MASK ((1ll << VC_SPACE_SHIFT) - 1)
 
+// Forwarded execution in the default mode keeps its staging in a window: a piece (at most VC_CHUNK bytes) of a slot at offset x of the
+// layout lies at x mod `window` of the arena.  The piece has made its next hop by the time another one takes its place (one group of
+// lanes performs all hops of a piece and reads the staging of none), so slots that share a place need no order between them.
+// What bounds calls that stage is the traffic of the memory; 32 MiB of staging stay in the 256 MiB memory-side cache, and its writes
+// to HBM with them, if they are stored with an ordinary store (a non-temporal one bypasses that cache).  Contiguous copy with a second write to
+// a window: window >= 512 MiB 2250 us, <= 256 MiB 1705 (plain); 2110 - 2190 (non-temporal, any size).  Calls, no window / 128 / 64 / 32 MiB:
+// 1024 ranks, 4 KiB 2447 / 2234 / 1973 / 1893 us; 256 ranks, Zipf 166 / 156 / 138 / 135; 512 ranks, 1 MiB, radix 2 14400 / 12060 / 11330 / 10680.
+// No smaller one: about 29 MiB of pieces are in flight at once on routes of nine digits.
+#define VC_STAGE_WINDOW (32 << 20)
+
 // One block copy: `len` bytes from `src` to `dst` (space-tagged offsets), sent by
 // virtual rank `from` to virtual rank `to`.
 struct VcDesc {
@@ -119,6 +129,8 @@ struct VcSched {
                       //    leaves in a later one; blocks with the same (arrival, departure) pair of hop slots form a sub-region,
                       //    and a sub-region may take the memory of another one whose blocks have all left before it is written
                       //    (the reference reuses its extra_buffer slots the same way, src/twophase_tunable_rbruckv-om.cpp:52-75).
+    int window;       // forwarded execution: > 0: staging lies in a window of that many bytes, a power of two (VC_STAGE_WINDOW); 0: every slot has
+                      //    a place of its own
     int coalesce;     // 1: blocks that are about to leave their node wait in "organized" runs — the n blocks one rank
                       //    holds for one destination rank back to back in source order — so that an inter-node message
                       //    is a contiguous copy (TTPL_BT_alltoallv, src/twophase_twolayer_rbruck.cpp:388-398, 430-453).
@@ -129,6 +141,10 @@ struct VcSched {
     VcRankDivisor dn, dr;                         // division of ranks, slots and offsets by n, r
     VcDivisor dP;                                 // division of pair numbers by P
 };
+
+// What a staging offset of the layout is taken with, and the arena a layout of `bytes` takes (the last piece of a window may pass its end).
+VC_HD int64_t vc_window_mask(int window) { return window ? (int64_t)window - 1 : -1; }
+VC_HD int64_t vc_window_bytes(int64_t bytes, int window) { return window && bytes > window ? (int64_t)window + VC_CHUNK : bytes; }
 
 VC_HD bool vc_receives_now(const VcSched &S, int t) { return (unsigned)(t - S.recv_from) < (unsigned)S.recv_num; }
 
@@ -267,8 +283,9 @@ hipError_t vc_launch_traffic(const VcDesc *desc, int64_t ndesc, int64_t *matrix,
 // a wavefront, for lists of pieces of a few hundred bytes)
 hipError_t vc_launch_copy_items(const VcDesc *items, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf, char *stage,
                                 hipStream_t st);
+// window: VcSched::window of the plan the list was made for
 hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf,
-                                 char *stage, hipStream_t st);
+                                 char *stage, hipStream_t st, int window = 0);
 // What the plan of a call must look like for a list and a copy launch that were enqueued right behind the planning kernel,
 // before the host had seen the plan, to do their work.  Kernels and host evaluate it on the same header, so both agree on
 // whether anything was moved.
@@ -287,7 +304,8 @@ VC_HD bool vc_chain_guard_ok(const int64_t *header, const VcChainGuard &g) {
 // workgroup checks vc_chain_guard_ok on the device header and takes an item only if there is one at its index
 // (header[2] items exist).  Items beyond `covered` (grid_items, or what one launch holds) are left for a second, ordinary launch.
 hipError_t vc_launch_copy_chains_guarded(const int64_t *items, int stride, int64_t grid_items, int lanes, const char *sendbuf,
-                                         char *recvbuf, char *stage, hipStream_t st, const int64_t *header, VcChainGuard guard, int64_t *covered);
+                                         char *recvbuf, char *stage, hipStream_t st, const int64_t *header, VcChainGuard guard, int64_t *covered,
+                                         int window);
 // What the plan of a call must look like for the listless kernels to run it; 0 = no limit.  The kernels evaluate it on
 // the device header, the host on its copy after the synchronisation: both then agree on whether anything was moved.
 struct VcListlessGuard {

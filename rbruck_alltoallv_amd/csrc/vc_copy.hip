@@ -41,9 +41,18 @@ __device__ __forceinline__ void vc_store16_through(char *p, vc_u32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
 }
 
-__device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, char *recvbuf, char *stage) {
-    const int64_t off = loc & VC_OFFSET_MASK;
+// ... of a call that stages in a window: an ordinary store, so that the window stays in the caches.  What goes to recvbuf is stored the same
+// way (non-temporal: 1024 ranks, 4 KiB 1993 us -> 2066; 256 ranks, Zipf 148 -> 181), but not in calls that stage nothing (512 ranks, 1 KiB
+// 200 -> 191).  Calls with and without a window have kernels of their own: of two branches that only differ in the kind of their
+// stores the compiler makes one, with ordinary stores.
+template <bool WINDOW> __device__ __forceinline__ void vc_store16_of(char *p, vc_u32x4 v) {
+    if (WINDOW) *reinterpret_cast<vc_u32x4 *>(p) = v; else vc_store16(p, v);
+}
+
+// mask: vc_window_mask of the call, for the place of a piece in the staging arena
+__device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, char *recvbuf, char *stage, int64_t mask = -1) {
     const int space = (int)(loc >> VC_SPACE_SHIFT);
+    const int64_t off = loc & VC_OFFSET_MASK & (space >= 2 ? mask : -1);
     char *base = space == 0 ? const_cast<char *>(sendbuf) : (space == 1 ? recvbuf : stage);
     return base + off;
 }
@@ -63,18 +72,19 @@ __device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, ch
 // With nhop > 1 this is forwarded execution: the piece is read once, from sendbuf, and every hop stores the same
 // registers (all destinations of a block share the offset inside their cache line, `w`, so one mapping of lanes to window
 // vectors serves them all).  next_dst() is where the next hop puts the piece.
+// WINDOW: the call stages in a window (vc_store16_of).
 // go() is asked once, after the loads have been issued and before the first store: false leaves the piece where it is.
 #define VC_WAIT_VMCNT0 0x0F70              // s_waitcnt vmcnt(0): loads have arrived and stores have been acknowledged
 struct VcAlwaysGo { __device__ __forceinline__ bool operator()() const { return true; } };
 
-template <int LANES, bool THROUGH = false, class NextDst, class Go = VcAlwaysGo>
+template <int LANES, bool THROUGH, bool WINDOW, class NextDst, class Go = VcAlwaysGo>
 __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, int nhop, int w, NextDst next_dst, Go go = Go()) {
     constexpr int VECS = VC_CHUNK / 16 / LANES;           // window vectors per lane: 2 for a workgroup of 256, 8 for one wavefront
     const int t = threadIdx.x;
     const int n = (int)len;                               // (a piece fits the window)
     if (!THROUGH && n == VC_PIECE && w == 0) {
-        // A whole aligned piece, the inside of a long block: no vector to leave out and no edge.  A wavefront waits for each of its
-        // stores before the next one: on lists of these the memory runs a few per cent faster with fewer writes in flight
+        // A whole aligned piece, the inside of a long block: no vector to leave out and no edge.  Without a window a wavefront waits for each
+        // of its stores before the next one: on lists of these the memory runs a few per cent faster with fewer writes in flight
         // (64 ranks, 1.3 MB blocks, two hops, builds in turn in one process, quartiles within 0.4 %: without this path 2430 us, with it but
         // without the waits 2407, so 2349; 512 ranks, 1 MiB blocks 6527 / 6494 / 6474).
         constexpr int WHOLE = VC_PIECE / 16 / LANES;
@@ -86,8 +96,8 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
             char *dst = next_dst();
 #pragma unroll
             for (int i = 0; i < WHOLE; i++) {
-                if (k || i) __builtin_amdgcn_s_waitcnt(VC_WAIT_VMCNT0);
-                vc_store16(dst + ((t + i * LANES) << 4), v[i]);
+                if (!WINDOW && (k || i)) __builtin_amdgcn_s_waitcnt(VC_WAIT_VMCNT0);
+                vc_store16_of<WINDOW>(dst + ((t + i * LANES) << 4), v[i]);
             }
         }
         return;
@@ -118,7 +128,7 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
         if (edge >= 0) { if (THROUGH) vc_store_through(dst + edge, edge_byte); else dst[edge] = edge_byte; }
 #pragma unroll
         for (int i = 0; i < VECS; i++)
-            if (has[i]) { if (THROUGH) vc_store16_through(dw + ((t + i * LANES) << 4), v[i]); else vc_store16(dw + ((t + i * LANES) << 4), v[i]); }
+            if (has[i]) { if (THROUGH) vc_store16_through(dw + ((t + i * LANES) << 4), v[i]); else vc_store16_of<WINDOW>(dw + ((t + i * LANES) << 4), v[i]); }
     }
 }
 
@@ -127,11 +137,12 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
 // unit, and no wavefronts that start only to find nothing left for them in a piece of a few hundred bytes.
 // GUARDED: the launch was enqueued before the host had seen the plan (see VcChainGuard): `nitems` is a guess, header[2] the
 // truth, and nothing moves unless the plan is one this launch can serve.
-template <int LANES, bool GUARDED = false>
+// WINDOW: the plan stages in a window of `window` bytes.
+template <int LANES, bool GUARDED, bool WINDOW>
 __global__ __launch_bounds__(LANES) void vc_copy_chains_kernel(const int64_t *__restrict__ items, int stride, unsigned nitems,
                                                                const char *__restrict__ sendbuf, char *__restrict__ recvbuf,
-                                                               char *__restrict__ stage, const int64_t *__restrict__ header = nullptr,
-                                                               VcChainGuard guard = VcChainGuard()) {
+                                                               char *__restrict__ stage, const int64_t *__restrict__ header,
+                                                               VcChainGuard guard, int window) {
     const unsigned per = gridDim.x / VC_XCDS;
     const unsigned idx = (blockIdx.x % VC_XCDS) * per + blockIdx.x / VC_XCDS;
     if (idx >= nitems) return;
@@ -142,15 +153,16 @@ __global__ __launch_bounds__(LANES) void vc_copy_chains_kernel(const int64_t *__
     if (GUARDED) ok = ok & vc_chain_guard_ok(header, guard) & ((int64_t)idx < header[2]);
     if (!ok) return;
     const char *src = vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage);
-    char *dst = vc_resolve(it[VC_CHAIN_HEAD], sendbuf, recvbuf, stage);
+    const int64_t mask = WINDOW ? vc_window_mask(window) : -1;
+    char *dst = vc_resolve(it[VC_CHAIN_HEAD], sendbuf, recvbuf, stage, mask);
     const int w = (int)((uintptr_t)dst & (VC_LINE - 1)), lane = threadIdx.x % VC_WAVE;
     // the hops after the first in one read, a word per lane: a load between the stores would wait for the stores before it
     int64_t word = 0;
     if (lane < nhop) word = it[VC_CHAIN_HEAD + lane];
     int at = 0;
-    vc_forward_piece<LANES>(src, len, nhop, w, [&]() {
+    vc_forward_piece<LANES, false, WINDOW>(src, len, nhop, w, [&]() {
         const unsigned lo = __builtin_amdgcn_readlane((int)word, at), hi = __builtin_amdgcn_readlane((int)(word >> 32), at);
-        return at++ ? vc_resolve((int64_t)hi << 32 | lo, sendbuf, recvbuf, stage) : dst;
+        return at++ ? vc_resolve((int64_t)hi << 32 | lo, sendbuf, recvbuf, stage, mask) : dst;
     });
 }
 
@@ -166,15 +178,15 @@ __global__ __launch_bounds__(LANES) void vc_copy_items_kernel(const VcDesc *__re
     const VcDesc d = items[idx];
     if (d.len <= 0) return;
     char *dst = vc_resolve(d.dst, sendbuf, recvbuf, stage);
-    vc_forward_piece<LANES>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, (int)((uintptr_t)dst & (VC_LINE - 1)), [&]() { return dst; });
+    vc_forward_piece<LANES, false, false>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, (int)((uintptr_t)dst & (VC_LINE - 1)), [&]() { return dst; });
 }
 
 // A quarter of a wavefront (16 lanes) per item, four items per wavefront, for lists of pieces of a few hundred bytes:
 // such a launch is bound by how many items are in flight, not by HBM, and a piece of 100 bytes has work for 7 lanes.
 // Every group of 16 lanes reads its own item; lane t of the group owns window vectors t, t + 16 of every 512-byte pass
 // (most items need one pass; longer ones loop), and moves head byte t and tail byte t.
-template <class DstOf, class Go = VcAlwaysGo>
-__device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_t len, int nhop, DstOf dst_of, Go go = Go()) {
+template <bool WINDOW, class DstOf>
+__device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_t len, int nhop, DstOf dst_of) {
     const int t = threadIdx.x & 15;
     char *dst = dst_of(0);
     const int64_t w = (int64_t)((uintptr_t)dst & (VC_LINE - 1));
@@ -194,14 +206,13 @@ __device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_
         vc_u32x4 v0, v1;
         if (has0) v0 = vc_load16(sw + (j << 4));
         if (has1) v1 = vc_load16(sw + ((j + 16) << 4));
-        if (first_pass && !go()) return;
         for (int k = 0; k < nhop; k++) {
             if (k || !first_pass) dst = dst_of(k);
             char *dw = dst - w;
             if (first_pass && has_head) dst[t] = head_byte;
             if (first_pass && has_tail) dst[done + t] = tail_byte;
-            if (has0) vc_store16(dw + (j << 4), v0);
-            if (has1) vc_store16(dw + ((j + 16) << 4), v1);
+            if (has0) vc_store16_of<WINDOW>(dw + (j << 4), v0);
+            if (has1) vc_store16_of<WINDOW>(dw + ((j + 16) << 4), v1);
         }
         first_pass = false;
     }
@@ -259,9 +270,9 @@ __device__ __forceinline__ void vc_lane_store(const VcLaneBlock &b, char *dst, i
 }
 
 // A piece moved by LANES neighbouring lanes of a wavefront: lane t owns window vectors t, t + LANES, ... (the window starts at the
-// cache line of the destination, `w` bytes before it), VECS of them in flight at once.  Staging is stored past the caches
-// (nothing reads it again); recvbuf is not: a line that two neighbouring blocks share is then put together in the L2.
-template <int LANES, int VECS, class DstOf, class Go = VcAlwaysGo>
+// cache line of the destination, `w` bytes before it), VECS of them in flight at once.  Staging without a window is stored past the
+// caches (nothing reads it again); recvbuf is not: a line that two neighbouring blocks share is then put together in the L2.
+template <int LANES, int VECS, bool WINDOW, class DstOf, class Go = VcAlwaysGo>
 __device__ __forceinline__ void vc_forward_short(const char *src, int len, int nhop, int w, DstOf dst_of, Go go = Go()) {
     const int t = threadIdx.x % LANES;
     if (len < 16) {
@@ -287,7 +298,10 @@ __device__ __forceinline__ void vc_forward_short(const char *src, int len, int n
             char *dst = dst_of(k);
 #pragma unroll
             for (int i = 0; i < VECS; i++)
-                if (at[i] >= 0) __builtin_nontemporal_store(v[i], &reinterpret_cast<VcU128 *>(dst + at[i])->v);
+                if (at[i] >= 0) {
+                    if (WINDOW) reinterpret_cast<VcU128 *>(dst + at[i])->v = v[i];
+                    else __builtin_nontemporal_store(v[i], &reinterpret_cast<VcU128 *>(dst + at[i])->v);
+                }
         }
         char *dst = dst_of(nhop - 1);
 #pragma unroll
@@ -301,12 +315,12 @@ __device__ __forceinline__ void vc_forward_short(const char *src, int len, int n
 // gridDim.x wavefronts, a multiple of VC_XCDS; XCD k works through the k-th eighth of them, each taking four items in a row
 // `rounds`: groups of four items in a row a wavefront takes, one after the other (long lists of very short pieces: fewer
 // wavefronts, each paying its start-up once for more items)
-template <bool GUARDED = false>
+template <bool GUARDED, bool WINDOW>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_chains_quarter_kernel(const int64_t *__restrict__ items, int stride, unsigned nitems,
                                                                          int rounds, const char *__restrict__ sendbuf,
                                                                          char *__restrict__ recvbuf, char *__restrict__ stage,
-                                                                         const int64_t *__restrict__ header = nullptr,
-                                                                         VcChainGuard guard = VcChainGuard()) {
+                                                                         const int64_t *__restrict__ header,
+                                                                         VcChainGuard guard, int window) {
     const unsigned per = gridDim.x / VC_XCDS;
     const unsigned wave = (blockIdx.x % VC_XCDS) * per + blockIdx.x / VC_XCDS;
     if (GUARDED && !vc_chain_guard_ok(header, guard)) return;
@@ -317,8 +331,9 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_chains_quarter_kernel(const i
         const int64_t len = it[VC_CHAIN_LEN];
         const int nhop = (int)it[VC_CHAIN_NHOP];
         if (len <= 0 || nhop <= 0) continue;
-        vc_forward_piece_quarter(vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage), len, nhop,
-                                 [&](int k) { return vc_resolve(it[VC_CHAIN_HEAD + k], sendbuf, recvbuf, stage); });
+        const int64_t mask = WINDOW ? vc_window_mask(window) : -1;
+        vc_forward_piece_quarter<WINDOW>(vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage), len, nhop,
+                                         [&](int k) { return vc_resolve(it[VC_CHAIN_HEAD + k], sendbuf, recvbuf, stage, mask); });
     }
 }
 
@@ -333,7 +348,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_items_quarter_kernel(const Vc
         const VcDesc d = items[idx];
         if (d.len <= 0) continue;
         char *dst = vc_resolve(d.dst, sendbuf, recvbuf, stage);
-        vc_forward_piece_quarter(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, [&](int) { return dst; });
+        vc_forward_piece_quarter<false>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, [&](int) { return dst; });
     }
 }
 
@@ -473,7 +488,7 @@ __device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcPairRe
 // Everything the block's addresses depend on is read before the planner's verdict is looked at: the reads are
 // independent of each other and of the verdict (tables are always readable), so they travel together instead of one
 // memory round trip after the other; nothing is stored before the verdict is known.
-template <int LANES, bool SELF>
+template <int LANES, bool SELF, bool WINDOW>
 __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T, const uint32_t *__restrict__ slot_off,
                                              const int64_t *__restrict__ row_base,
                                              const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -508,12 +523,12 @@ __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
         unsigned long long left = moves;
-        vc_forward_piece<LANES, SELF>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
+        vc_forward_piece<LANES, SELF, WINDOW>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
                                 [&]() {
                                     const int k = __ffsll(left) - 1;
                                     left &= left - 1;
                                     const unsigned d_lo = __builtin_amdgcn_readlane((int)dst, k), d_hi = __builtin_amdgcn_readlane((int)(dst >> 32), k);
-                                    return vc_resolve(((int64_t)d_hi << 32 | d_lo) + lo, sendbuf, recvbuf, stage);
+                                    return vc_resolve(((int64_t)d_hi << 32 | d_lo) + lo, sendbuf, recvbuf, stage, WINDOW ? vc_window_mask(S.window) : -1);
                                 },
                                 [&]() { return gate(); });
     }
@@ -523,7 +538,8 @@ __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T
 // the caches.  A kernel behind this one that only does that costs the boundary between the two: 8 ranks of 0 - 64 ints 13.0 -> 12.8 us,
 // 32 ranks of 0 - 2 KiB 14.0 -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3.  The quarter kernel has no such instance: its lanes' short stores past the caches each
 // cost a write to memory (64 ranks, 1 KiB blocks: 16.6 -> 21.9 us).
-template <int LANES, bool SELF>
+// WINDOW: S.window.
+template <int LANES, bool SELF, bool WINDOW>
 __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                const int64_t *__restrict__ row_base,
                                                                const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -531,7 +547,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
                                                                char *__restrict__ recvbuf, char *__restrict__ stage,
                                                                unsigned long long *verdict, unsigned long long *verdict_next,
                                                                int64_t *totals, VcSignal sig) {
-    vc_copy_pair<LANES, SELF>(S, T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, verdict, verdict_next, totals);
+    vc_copy_pair<LANES, SELF, WINDOW>(S, T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, verdict, verdict_next, totals);
     if (SELF) vc_signal(sig);
 }
 
@@ -540,6 +556,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
 // Eight vectors of a lane in flight, 2 KiB a group: 87 VGPRs, 5 wavefronts per SIMD.  With four (62 VGPRs, 7) the loads of a second round
 // wait for the stores of the first: calls of blocks of 512 B - 2.5 KiB on average on 64 - 200 ranks 3 - 5 % slower (128 ranks, 2 KiB 33.0
 // us -> 34.2; 192 ranks, 600 B 38.3 -> 40.4), 1024 ranks, 700 B 596 -> 605, and only direct calls on 300 ranks faster (91.9 -> 89.9).
+template <bool WINDOW>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                          const int64_t *__restrict__ row_base,
                                                                          const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -588,8 +605,9 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
     for (int64_t c = 0; c < pieces; c++) {
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
-        vc_forward_short<VC_QUARTER, 8>(src + lo, (int)(hi - lo), nhop, c ? 0 : phase, [&](int k) { return vc_resolve(route[g][k] + lo, sendbuf, recvbuf, stage); },
-                                        [&]() { return gate(); });
+        vc_forward_short<VC_QUARTER, 8, WINDOW>(src + lo, (int)(hi - lo), nhop, c ? 0 : phase,
+                                                [&](int k) { return vc_resolve(route[g][k] + lo, sendbuf, recvbuf, stage, WINDOW ? vc_window_mask(S.window) : -1); },
+                                                [&]() { return gate(); });
     }
 }
 
@@ -601,7 +619,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
 // a lane each, when all blocks of the wavefront are that short; else every quarter of the wavefront carries BATCH / 4 of them, one
 // after the other.  Measured on MI355X, 1024 ranks, two hops for most blocks: 0 - 16 bytes 76 us (pairs of one receiver
 // in a row, every block a quarter of a wavefront) -> 28; 0 - 512 bytes 277 -> 250.
-template <int BATCH>
+template <int BATCH, bool WINDOW>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                        const int64_t *__restrict__ row_base,
                                                                        const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -610,6 +628,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
     constexpr int TS = BATCH == 16 ? 4 : 8, TR = BATCH / TS, SHARE = VC_WAVE / BATCH;
     extern __shared__ int64_t batch_lds[];
     const int nslots = vc_hop_slots(S), P = S.P;
+    const int64_t mask = WINDOW ? vc_window_mask(S.window) : -1;
     int64_t *route = batch_lds;                           // [BATCH][nslots]
     int64_t *b_len = route + BATCH * nslots, *b_src = b_len + BATCH;
     int *b_nhop = reinterpret_cast<int *>(b_src + BATCH), *b_cut = b_nhop + BATCH;
@@ -662,7 +681,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
         __syncthreads();
         if (active && kq == 0) {
             const VcLaneBlock b = vc_lane_load(sendbuf + send_off, (int)len);
-            for (int k = 0; k < nhop; k++) vc_lane_store(b, vc_resolve(route[p * nslots + k], sendbuf, recvbuf, stage), (int)len);
+            for (int k = 0; k < nhop; k++) vc_lane_store(b, vc_resolve(route[p * nslots + k], sendbuf, recvbuf, stage, mask), (int)len);
         }
         return;
     }
@@ -684,7 +703,8 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
         for (int64_t c = 0; c < pieces; c++) {            // the same cuts as the chain items of this block
             int64_t lo, hi;
             vc_piece_range(blen, phase, cut, c, lo, hi);
-            vc_forward_short<VC_QUARTER, 4>(src + lo, (int)(hi - lo), b_nhop[b], c ? 0 : phase, [&](int k) { return vc_resolve(dsts[k] + lo, sendbuf, recvbuf, stage); });
+            vc_forward_short<VC_QUARTER, 4, WINDOW>(src + lo, (int)(hi - lo), b_nhop[b], c ? 0 : phase,
+                                                    [&](int k) { return vc_resolve(dsts[k] + lo, sendbuf, recvbuf, stage, mask); });
         }
     }
 }
@@ -696,7 +716,8 @@ static void vc_launch_batch(const VcSched &S, VcTables T, const uint32_t *slot_o
     const size_t lds = sizeof(int64_t) * BATCH * (vc_hop_slots(S) + 2) + sizeof(int) * BATCH * 2;
     for (int64_t done = 0; done < waves; done += VC_MAX_GRID) {
         const int64_t now = waves - done < VC_MAX_GRID ? waves - done : VC_MAX_GRID;
-        hipLaunchKernelGGL(vc_copy_blocks_batch_kernel<BATCH>, dim3((unsigned)((now + VC_XCDS - 1) / VC_XCDS * VC_XCDS)), dim3(VC_WAVE), lds, st, S,
+        const auto kernel = S.window ? vc_copy_blocks_batch_kernel<BATCH, true> : vc_copy_blocks_batch_kernel<BATCH, false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((now + VC_XCDS - 1) / VC_XCDS * VC_XCDS)), dim3(VC_WAVE), lds, st, S,
                            T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage);
     }
 }
@@ -705,7 +726,7 @@ hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *s
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig) {
     const int64_t npairs = (int64_t)S.P * S.P;
-    if (sig.word && (!verdict || (lanes != VC_WAVE && lanes != VC_THREADS))) return hipErrorInvalidValue;
+    if (sig.word && (!verdict || S.window || (lanes != VC_WAVE && lanes != VC_THREADS))) return hipErrorInvalidValue;
     if (lanes == VC_BATCHED) {
         if (verdict) return hipErrorInvalidValue;         // the batches are for more pairs than one launch with totals takes
         const int batch = vc_batch_pairs(npairs);
@@ -720,13 +741,15 @@ hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *s
         if (verdict && done) return hipErrorInvalidValue;    // the totals belong to a call that one launch takes
         const dim3 grid((unsigned)((units + VC_XCDS - 1) / VC_XCDS * VC_XCDS) + vc_totals_blocks(S, verdict, lanes == VC_THREADS ? VC_THREADS : VC_WAVE));
         if (lanes == VC_QUARTER) {
-            hipLaunchKernelGGL(vc_copy_blocks_quarter_kernel, grid, dim3(VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf,
-                               recvbuf, stage, verdict, verdict_next, totals);
+            const auto kernel = S.window ? vc_copy_blocks_quarter_kernel<true> : vc_copy_blocks_quarter_kernel<false>;
+            hipLaunchKernelGGL(kernel, grid, dim3(VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, verdict,
+                               verdict_next, totals);
             continue;
         }
         const bool self = sig.word != nullptr;
-        const auto kernel = lanes == VC_WAVE ? (self ? vc_copy_blocks_kernel<VC_WAVE, true> : vc_copy_blocks_kernel<VC_WAVE, false>)
-                                             : (self ? vc_copy_blocks_kernel<VC_THREADS, true> : vc_copy_blocks_kernel<VC_THREADS, false>);
+        const auto wave = self ? vc_copy_blocks_kernel<VC_WAVE, true, false> : (S.window ? vc_copy_blocks_kernel<VC_WAVE, false, true> : vc_copy_blocks_kernel<VC_WAVE, false, false>);
+        const auto workgroup = self ? vc_copy_blocks_kernel<VC_THREADS, true, false> : (S.window ? vc_copy_blocks_kernel<VC_THREADS, false, true> : vc_copy_blocks_kernel<VC_THREADS, false, false>);
+        const auto kernel = lanes == VC_WAVE ? wave : workgroup;
         hipLaunchKernelGGL(kernel, grid, dim3(lanes), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, verdict,
                            verdict_next, totals, sig);
     }
@@ -742,43 +765,42 @@ static unsigned vc_grid_for(int64_t items, int lanes) {
     return (unsigned)((units + VC_XCDS - 1) / VC_XCDS * VC_XCDS);
 }
 
+// One launch of the list-driven kernel with LANES lanes per item, in the instance for calls with or without a window.
+template <bool GUARDED>
+static void vc_launch_chains_once(const int64_t *items, int stride, unsigned nitems, int lanes, const char *sendbuf, char *recvbuf, char *stage,
+                                  hipStream_t st, const int64_t *header, VcChainGuard guard, int window) {
+    const dim3 grid(vc_grid_for(nitems, lanes));
+    if (lanes == VC_QUARTER) {
+        const auto kernel = window ? vc_copy_chains_quarter_kernel<GUARDED, true> : vc_copy_chains_quarter_kernel<GUARDED, false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(VC_WAVE), 0, st, items, stride, nitems, vc_quarter_rounds(nitems), sendbuf, recvbuf, stage, header,
+                           guard, window);
+        return;
+    }
+    const auto wave = window ? vc_copy_chains_kernel<VC_WAVE, GUARDED, true> : vc_copy_chains_kernel<VC_WAVE, GUARDED, false>;
+    const auto workgroup = window ? vc_copy_chains_kernel<VC_THREADS, GUARDED, true> : vc_copy_chains_kernel<VC_THREADS, GUARDED, false>;
+    hipLaunchKernelGGL(lanes == VC_WAVE ? wave : workgroup, grid, dim3(lanes == VC_WAVE ? VC_WAVE : VC_THREADS), 0, st, items, stride, nitems, sendbuf,
+                       recvbuf, stage, header, guard, window);
+}
+
 hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf,
-                                 char *stage, hipStream_t st) {
+                                 char *stage, hipStream_t st, int window) {
     const int64_t step = vc_items_per_launch(lanes);
     for (int64_t done = 0; done < nitems; done += step) {
         const int64_t now = nitems - done < step ? nitems - done : step;
-        const dim3 grid(vc_grid_for(now, lanes));
-        const int64_t *first = items + done * stride;
-        if (lanes == VC_QUARTER)
-            hipLaunchKernelGGL(vc_copy_chains_quarter_kernel<false>, grid, dim3(VC_WAVE), 0, st, first, stride, (unsigned)now,
-                               vc_quarter_rounds(now), sendbuf, recvbuf, stage, nullptr, VcChainGuard());
-        else if (lanes == VC_WAVE)
-            hipLaunchKernelGGL((vc_copy_chains_kernel<VC_WAVE, false>), grid, dim3(VC_WAVE), 0, st, first, stride, (unsigned)now, sendbuf, recvbuf,
-                               stage, nullptr, VcChainGuard());
-        else
-            hipLaunchKernelGGL((vc_copy_chains_kernel<VC_THREADS, false>), grid, dim3(VC_THREADS), 0, st, first, stride, (unsigned)now, sendbuf,
-                               recvbuf, stage, nullptr, VcChainGuard());
+        vc_launch_chains_once<false>(items + done * stride, stride, (unsigned)now, lanes, sendbuf, recvbuf, stage, st, nullptr, VcChainGuard(), window);
     }
     return hipGetLastError();
 }
 
 // One launch (a guessed list longer than a launch holds is cut to what one holds; the rest is the caller's second launch).
 hipError_t vc_launch_copy_chains_guarded(const int64_t *items, int stride, int64_t grid_items, int lanes, const char *sendbuf,
-                                         char *recvbuf, char *stage, hipStream_t st, const int64_t *header, VcChainGuard guard, int64_t *covered) {
+                                         char *recvbuf, char *stage, hipStream_t st, const int64_t *header, VcChainGuard guard, int64_t *covered,
+                                         int window) {
     const int64_t step = vc_items_per_launch(lanes);
     const int64_t now = grid_items < step ? grid_items : step;
     *covered = now > 0 ? now : 0;
     if (now <= 0) return hipSuccess;
-    const dim3 grid(vc_grid_for(now, lanes));
-    if (lanes == VC_QUARTER)
-        hipLaunchKernelGGL(vc_copy_chains_quarter_kernel<true>, grid, dim3(VC_WAVE), 0, st, items, stride, (unsigned)now, vc_quarter_rounds(now),
-                           sendbuf, recvbuf, stage, header, guard);
-    else if (lanes == VC_WAVE)
-        hipLaunchKernelGGL((vc_copy_chains_kernel<VC_WAVE, true>), grid, dim3(VC_WAVE), 0, st, items, stride, (unsigned)now, sendbuf, recvbuf,
-                           stage, header, guard);
-    else
-        hipLaunchKernelGGL((vc_copy_chains_kernel<VC_THREADS, true>), grid, dim3(VC_THREADS), 0, st, items, stride, (unsigned)now, sendbuf,
-                           recvbuf, stage, header, guard);
+    vc_launch_chains_once<true>(items, stride, (unsigned)now, lanes, sendbuf, recvbuf, stage, st, header, guard, window);
     return hipGetLastError();
 }
 

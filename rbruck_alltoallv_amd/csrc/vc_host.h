@@ -104,6 +104,7 @@ struct vc_comm {
     double cal_copy_bytes_per_s = 0, cal_launch_s = 0, cal_sync_s = 0;   // calibrate(): the plain copy's rate, the cost of a
                                           // launch, of a launch the host waits for
     int bound_staging = 1;                // vc_comm_set_staging_bound
+    bool own_allowance = false;           // ... with an allowance of the caller's
     int64_t staging_allowance = 0;        // bytes of staging a forwarded call may take whatever its payload (set with the bound)
     int live_plans = 0;                   // plans created on this communicator and not yet freed
     std::vector<void *> retired_stage;    // staging arenas that were outgrown while plans existed: a HIP graph captured from
@@ -116,6 +117,7 @@ struct vc_comm {
         const char *sendbuf = nullptr;
         char *recvbuf = nullptr;
         int lanes = 0;                    // 0: only planned so far
+        int64_t max_pieces = 0;           // VcListlessGuard::max_pieces of the launch
         int n_launch_infos = 0;
         hipStream_t own_stream = nullptr; // the communicator's stream while the call runs on the caller's
         CallParams q;                     // what was asked for (the call may have to be run again another way)
@@ -218,6 +220,7 @@ template <class Launch> inline hipError_t vc_run_meta(vc_comm *c, Launch launch)
 
 // ---- defined in vc_api.hip, used by vc_tools.hip ----
 int ensure_events(vc_comm *c, size_t n);
+bool stages_in_window(const vc_comm *c);
 bool staging_out_of_bound(const vc_comm *c, int64_t stage_bytes, int64_t payload_bytes);
 int staging_batches(const vc_comm *c, int64_t stage_bytes);
 VcTables make_tables(vc_comm *c, const int *sc, const int *sd, const int *rc, const int *rd);

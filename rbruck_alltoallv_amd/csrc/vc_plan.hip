@@ -500,7 +500,7 @@ __global__ __launch_bounds__(VC_THREADS) void vc_plan_forward(VcSched S, VcTable
     vc_block_totals(sum, lds);
     if (threadIdx.x != 0) return;
     // every staged block is one hop, every block's last hop ends in recvbuf
-    const int64_t words[VC_HEADER_MAX_LEN + 1] = {carry, sum[0], items, sum[2], sum[3], sum[0] + sum[1], sum[4]};
+    const int64_t words[VC_HEADER_MAX_LEN + 1] = {vc_window_bytes(carry, S.window), sum[0], items, sum[2], sum[3], sum[0] + sum[1], sum[4]};
 #pragma unroll
     for (int k = 0; k <= VC_HEADER_MAX_LEN; k++) { header[k] = words[k]; header_host[k] = words[k]; }
 }

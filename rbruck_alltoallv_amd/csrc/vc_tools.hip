@@ -161,7 +161,7 @@ extern "C" int vc_suggest_tunables(const int *sendcounts, int elem_size, int n, 
         const double plan = 2 * c->cal_sync_s + 3 * launch + (double)P * P * (w + 2) * 16.0 / rate;
         // (a forwarded call whose staging, the bytes of all hops but the last, is out of bound runs in batches or per digit)
         const int64_t staged = (int64_t)(moved - payload);
-        const bool forwarded = c->forward != 0 && (!staging_out_of_bound(c, staged, (int64_t)payload) || staging_batches(c, staged));
+        const bool forwarded = c->forward != 0 && (stages_in_window(c) || !staging_out_of_bound(c, staged, (int64_t)payload) || staging_batches(c, staged));
         const double t = forwarded
             ? plan + launch + (payload + moved + 2.0 * pieces * (24 + 8 * (w + 1))) / rate
             : plan + launch * launches_for(n, cand[k], n < P) + (2.0 * moved + 2.0 * 32 * hop_pieces) / rate;

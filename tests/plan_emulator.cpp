@@ -273,6 +273,11 @@ extern "C" int plan_emulate(int func, int P, int n, int r, int batch, int esz, i
                         line = ph;
                         if (plen + ph > VC_CHUNK) errors++;
                         if (c > 0 && ph != 0) errors++;
+                        // ... and so does its place in a window of staging, whatever the window's size
+                        for (int window : {VC_CHUNK, 4 * VC_CHUNK, VC_STAGE_WINDOW}) {
+                            const int64_t place = dof & vc_window_mask(window);
+                            if (dspace == 2 && (place + plen > vc_window_bytes(stage_bytes, window) || ((place ^ dof) & (VC_LINE - 1)))) errors++;
+                        }
                         dst_ranges.push_back({dof, dof + plen, dspace});
                         memcpy((dspace == 1 ? recv_final : stage2.data()) + dof, send + so, (size_t)plen);
                         chain_moved += plen;

@@ -1,0 +1,105 @@
+"""Staging in a window (the default mode): layouts below, at and beyond it, through every kind of copy kernel, against the definition."""
+import numpy as np
+import pytest
+import torch
+
+from rbruck_alltoallv_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+WINDOW, CHUNK = 32 << 20, 8192
+
+
+def _equal(P, length):
+    return np.full((P, P), length, dtype=np.int32)
+
+
+def _mixed(P, hi, seed=5):
+    counts = np.random.default_rng(seed).integers(0, hi, (P, P)).astype(np.int32)
+    counts[::5, ::7] = min(10 * hi, 150_001)
+    return counts
+
+
+# function, tunables, counts, element size, layout of the arenas.  Four ranks at radix 2 stage four blocks: 8 MiB blocks fill the window exactly.
+CASES = {
+    "at the window": ("twophase_rbruck_alltoallv", (2,), _equal(4, 8 << 20), 1, 0),
+    "one line beyond": ("twophase_rbruck_alltoallv_om", (2,), _equal(4, (8 << 20) + 128), 1, 0),
+    "below": ("twophase_rbruck_alltoallv", (3,), _equal(4, 1 << 20), 1, 1),
+    "workgroups, odd addresses": ("tuna_algorithm", (2, 0), _mixed(40, 60_000), 1, 1),
+    "wavefronts": ("TTPL_rbruck_alltoallv", (8, 2), _mixed(160, 2_100), 1, 1),
+    "quarters from the list": ("TTPL_BT_alltoallv_s1", (64, 2, 0), np.where(_mixed(512, 60) > 60, 2_000, _mixed(512, 60)).astype(np.int32), 4, 1),
+    "quarters": ("TTPL_BT_alltoallv", (30, 2, 0), np.random.default_rng(1).integers(0, 1100, (300, 300)).astype(np.int32), 1, 0),
+    "batches, a lane a block": ("tuna_algorithm", (2, 0), np.random.default_rng(2).integers(0, 17, (512, 512)).astype(np.int32), 1, 0),
+    "batches, a quarter a block": ("twophase_rbruck_alltoallv", (4,), np.random.default_rng(3).integers(0, 300, (512, 512)).astype(np.int32), 1, 1),
+    "one launch": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(4).integers(0, 2500, (100, 100)).astype(np.int32), 1, 1),
+    "one launch that signals its end": ("twophase_rbruck_alltoallv_om", (2,), np.random.default_rng(4).integers(0, 12_000, (31, 31)).astype(np.int32), 1, 1),
+}
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_staging_window(case):
+    from rbruck_alltoallv_amd import api
+    name, tun, counts, esz, layout = CASES[case]
+    packed = name == "TTPL_BT_alltoallv"
+    prob = W.make_problem(counts, esz, layout, 0 if packed else layout)
+    dp = api.DeviceProblem(prob)
+    fn = getattr(api, name)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 9, ds)
+    dp.comm.set_forwarding(2)
+    dp.comm.set_staging_bound(0)
+    assert fn(*tun, dp, ds, dr) == 0 and dp.verify(ds, dr, packed) == 0, dp.comm.error()
+    want, slots = dr.clone(), dp.comm.last_stats().staging_bytes      # every slot in a place of its own
+    dp.comm.free()
+    dp = api.DeviceProblem(prob)
+    dp.comm.set_forwarding(1)
+    ran = []
+    for _ in range(4):                                    # through the list, then on the hint of the call before
+        dr.fill_(0xEE)
+        assert fn(*tun, dp, ds, dr) == 0, dp.comm.error()
+        assert torch.equal(dr, want), (case, ran)
+        st = dp.comm.last_stats()
+        ran.append((int(st.execution), int(st.lanes_per_item), int(st.staging_bytes)))
+        if st.execution != 3:                             # (slots of a fixed stride take more)
+            assert st.staging_bytes == (slots if slots <= WINDOW else WINDOW + CHUNK), (ran, slots)
+    print(case, slots, ran, flush=True)
+    plan = api.Plan(name, dp, dr, n=tun[0] if len(tun) == 3 or "TTPL" in name else 0, r=tun[1] if "TTPL" in name else tun[0])
+    assert plan.rc == 0, dp.comm.error()
+    for _ in range(2):
+        dr.fill_(0xEE)
+        assert plan.execute(ds, dr) == 0 and torch.equal(dr, want)
+    plan.free()
+    if name in ("twophase_rbruck_alltoallv", "twophase_rbruck_alltoallv_om", "tuna_algorithm", "TTPL_BT_alltoallv", "TTPL_BT_alltoallv_s1"):
+        for _ in range(2):
+            dr.fill_(0xEE)
+            assert api.call_async(name, tun, dp, ds, dr, torch.cuda.current_stream()) == 0 and dp.comm.wait() == 0, dp.comm.error()
+            assert torch.equal(dr, want)
+    dp.comm.free()
+
+
+def test_plan_with_a_window_in_a_graph():
+    """Replays of a captured plan, with another call on the communicator between them, leave what an eager call leaves."""
+    from rbruck_alltoallv_amd import api
+    prob = W.make_problem(_mixed(64, 9_000), 4, 1, 1)
+    dp = api.DeviceProblem(prob)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 4, ds)
+    plan = api.Plan("tuna_algorithm", dp, dr, r=2)
+    assert plan.rc == 0 and plan.execute(ds, dr) == 0 and dp.comm.last_stats().staging_bytes == WINDOW + CHUNK
+    want = dr.clone()
+    assert dp.verify(ds, dr) == 0
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        dp.comm.use_current_stream()
+        assert plan.execute_async(ds, dr) == 0
+    dp.comm.use_current_stream()
+    for _ in range(4):
+        dr.fill_(0xEE)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(dr, want)
+        dr.fill_(0xEE)
+        assert api.twophase_rbruck_alltoallv(8, dp, ds, dr) == 0 and torch.equal(dr, want)
+    del graph
+    plan.free()
+    dp.comm.free()

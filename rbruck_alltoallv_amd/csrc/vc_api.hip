@@ -628,6 +628,78 @@ static int run_batches(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, VcTa
     return rc ? rc : 1;
 }
 
+// ---- forwarded calls without a list whose slots have closed-form places: those that stage in a window, and those that stage nothing ----
+// The planner (vc_plan_check) only checks and counts, and the copy kernel, enqueued behind it, reads no plan table.
+static bool plans_without_tables(const VcSched &S) { return S.window || !vc_may_stage(S); }
+
+// Gives S the slots for blocks of up to `longest` bytes (a call that stages nothing takes any), makes room for them, and puts
+// the limits that come with them into `guard`.  False: blocks too long for slots of a fixed stride.
+static int place_in_window(vc_comm *c, VcSched &S, int64_t longest, VcListlessGuard &guard, int64_t &stage_bytes, bool &fits) {
+    const bool stages = vc_may_stage(S);
+    S.stride = stages ? vc_window_stride(longest) : VC_LINE;
+    fits = S.stride > 0;
+    if (!fits) return VC_OK;
+    const unsigned __int128 layout = (unsigned __int128)(S.w + S.w2) * (unsigned)S.P * (unsigned)S.P * (unsigned)S.stride;
+    stage_bytes = !stages ? 0 : (layout > (unsigned __int128)S.window ? vc_window_bytes((int64_t)S.window + 1, S.window) : (int64_t)layout);
+    HIP_TRY(reserve_stage(c, (size_t)stage_bytes + 64));
+    guard.stage_cap = (int64_t)c->stage.cap - 64;
+    guard.max_len = stages ? S.stride - VC_LINE + 1 : 0;
+    return VC_OK;
+}
+
+static int reserve_check_bufs(vc_comm *c, const VcSched &S) {
+    HIP_TRY(c->header.reserve(sizeof(int64_t) * VC_HEADER_WORDS(VC_MAX_LAUNCHES)));
+    HIP_TRY(c->row_bytes.reserve(vc_check_bytes(S.P)));
+    if (S.packed_recv) HIP_TRY(c->rd_packed.reserve(sizeof(int) * (size_t)S.P * S.P));
+    return VC_OK;
+}
+
+static int enqueue_check(vc_comm *c, const VcSched &S, VcTables &T, int64_t stage_bytes) {
+    HIP_TRY(vc_launch_plan_check(S, T, c->rd_packed.as<int>(), c->row_bytes.as<int64_t>(), stage_bytes, c->header.as<int64_t>(), c->h_header_dev,
+                                 c->of_call.ticket, c->stream));
+    T.rd_packed = c->rd_packed.as<int>();
+    return VC_OK;
+}
+
+// A blocking call: check and copy kernel go out together, the slots from the longest block of the last call (`longest`); one with longer blocks
+// has moved nothing and goes out once more.  Returns 1: served; 0: not a call for this kernel, nothing moved; < 0: errors.
+static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf, VcTables T, const VcDispatch &d,
+                              int64_t longest) {
+    int rc = reserve_check_bufs(c, S);
+    if (rc) return rc;
+    if (c->timing) { rc = ensure_events(c, 5); if (rc) return rc; }
+    hipStream_t st = c->stream;
+    VcListlessGuard guard = d.guard;
+    for (int attempt = 0; attempt < 2; attempt++) {
+        int64_t stage_bytes = 0;
+        bool fits;
+        rc = place_in_window(c, S, longest, guard, stage_bytes, fits);
+        if (rc || !fits) return rc;
+        if (c->timing) HIP_TRY(hipEventRecord(c->events[0], st));
+        c->plan_end = 2;
+        rc = enqueue_check(c, S, T, stage_bytes);
+        if (rc) return rc;
+        if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
+        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+        if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
+        HIP_TRY(VC_WAIT(c));
+        PlanInfo pi;
+        rc = plan_read(c, S, L, pi, true);
+        if (rc) return rc;
+        if (vc_listless_ok(c->h_header, guard)) {
+            pi.listless = true;
+            pi.chain_lanes = d.lanes;
+            rc = finish_stats(c, pi, nullptr, true);
+            return rc ? rc : 1;
+        }
+        VcListlessGuard any_length = guard;
+        any_length.max_len = 0;
+        if (!vc_listless_ok(c->h_header, any_length)) return 0;
+        longest = pi.max_len;
+    }
+    return 0;
+}
+
 static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, char *recvbuf, VcTables T, bool forward, bool reuse = false) {
     VcSched S;
     std::vector<VcLaunchInfo> L;
@@ -640,10 +712,15 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     const int pair_lanes = d.lanes;
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;
+    if (pair_lanes && plans_without_tables(S)) {
+        // (a refused single launch has left its own longest block in the header)
+        rc = try_without_tables(c, S, L, sendbuf, recvbuf, T, d, std::max(c->hint.max_len, d.stride > 0 ? c->h_header[VC_HEADER_MAX_LEN] : 0));
+        if (rc) return rc < 0 ? rc : VC_OK;
+    }
     rc = plan_sizes(c, S, L, T, forward);
     if (rc) return rc;
     bool synced = false;
-    if (pair_lanes) {
+    if (pair_lanes && !plans_without_tables(S)) {
         // the copy kernel goes out right behind the planning kernels and checks their verdict on the device: when the
         // staging arena turns out too small it has touched nothing and goes out once more behind a larger arena; when the
         // call is not of the kind the last one made the host expect, the call continues through the list
@@ -693,6 +770,45 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     return run_items(c, pi, c->desc.p, sendbuf, recvbuf, true);
 }
 
+static void keep_pending(vc_comm *c, const CallParams &q, const VcSched &S, const std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf,
+                         const VcTables &T, int lanes, const VcListlessGuard &guard) {
+    c->pending.active = true;
+    c->pending.S = S; c->pending.T = T; c->pending.sendbuf = sendbuf; c->pending.recvbuf = recvbuf; c->pending.lanes = lanes;
+    c->pending.guard = guard;
+    c->pending.n_launch_infos = (int)L.size();
+    c->pending.q = q;
+}
+
+// An _async call without plan tables (try_without_tables).  One that stages is only checked, and copied in vc_comm_wait, while there is no last call
+// to take slots and shape from; one of longer blocks than the last call's is copied there too, in the shape its own blocks ask for.
+static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf,
+                                  VcTables T) {
+    int rc = reserve_check_bufs(c, S);
+    if (rc) return rc;
+    if (c->timing) { rc = ensure_events(c, 5); if (rc) return rc; }
+    hipStream_t st = c->stream;
+    const bool stages = vc_may_stage(S);
+    int lanes = c->hint.valid || !stages ? vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes : 0;
+    VcListlessGuard guard = {0, stages && (lanes == VC_QUARTER || lanes == VC_BATCHED) ? VC_LISTLESS_MAX_PIECES : 0, 0, 0, 0};
+    int64_t stage_bytes = 0;
+    if (lanes) {
+        bool fits;
+        rc = place_in_window(c, S, c->hint.max_len, guard, stage_bytes, fits);
+        if (rc) return rc;
+        if (!fits) lanes = 0;
+    }
+    if (c->timing) HIP_TRY(hipEventRecord(c->events[0], st));
+    c->plan_end = 2;
+    rc = enqueue_check(c, S, T, stage_bytes);
+    if (rc) return rc;
+    if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
+    if (lanes)
+        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+    if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
+    keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
+    return VC_OK;
+}
+
 // The _async entry points: planning kernels and the listless copy kernel are enqueued and the call returns.  The copy
 // kernel checks the planner's verdict on the device (tables, staging arena) and touches nothing when it is bad;
 // vc_comm_wait reads the same verdict and reports it, or grows the arena and runs the copy again, in the shape the plan asks for.
@@ -701,22 +817,17 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
 // first call; planned, then batches 0.57).
 static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf,
                          VcTables T) {
+    if (plans_without_tables(S)) return enqueue_without_tables(c, q, S, L, sendbuf, recvbuf, T);
     int rc = plan_sizes(c, S, L, T, true);
     if (rc) return rc;
     hipStream_t st = c->stream;
     const int lanes = c->stage.cap || !vc_may_stage(S) ? vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes : 0;
-    // (an arena with a window holds any call: one of long blocks behind short ones must not run in the shape of these)
-    const int64_t max_pieces = S.window && vc_may_stage(S) && (lanes == VC_QUARTER || lanes == VC_BATCHED) ? VC_LISTLESS_MAX_PIECES : 0;
-    const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, max_pieces, 0, 0, 0};
+    const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
         HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
-    c->pending.active = true;
-    c->pending.S = S; c->pending.T = T; c->pending.sendbuf = sendbuf; c->pending.recvbuf = recvbuf; c->pending.lanes = lanes;
-    c->pending.max_pieces = max_pieces;
-    c->pending.n_launch_infos = (int)L.size();
-    c->pending.q = q;
+    keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
     return VC_OK;
 }
 
@@ -738,27 +849,36 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
         }
     } release{c};
     HIP_TRY(VC_WAIT(c));
-    const VcSched &S = c->pending.S;
+    VcSched &S = c->pending.S;
     std::vector<VcLaunchInfo> L((size_t)c->pending.n_launch_infos);     // plan_read only needs their number here
     PlanInfo pi;
     int rc = plan_read(c, S, L, pi, true);
     if (rc) return rc;
-    VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, c->pending.max_pieces, 0, 0, 0};
+    VcListlessGuard guard = c->pending.guard;
     int lanes = c->pending.lanes;
     if (!lanes || !vc_listless_ok(c->h_header, guard)) {  // no arena, or one too small, or longer blocks: nothing has been moved yet
         // a call whose forwarded staging is out of the communicator's bound runs one launch per digit on reused staging (its blocking
         // twin: in batches of receivers where it can)
         if (staging_out_of_bound(c, pi.stage_bytes, pi.payload_bytes))
             return run_schedule(c, c->pending.q, c->pending.sendbuf, c->pending.recvbuf, c->pending.T, false, true);
-        HIP_TRY(reserve_stage(c, (size_t)pi.stage_bytes + 64));
-        guard = {(int64_t)c->stage.cap - 64, 0, 0, 0, 0};
+        if (plans_without_tables(S)) {
+            bool fits;
+            rc = place_in_window(c, S, pi.max_len, guard, pi.stage_bytes, fits);
+            if (rc) return rc;
+            if (!fits) return run_schedule(c, c->pending.q, c->pending.sendbuf, c->pending.recvbuf, c->pending.T, true);
+        } else {
+            HIP_TRY(reserve_stage(c, (size_t)pi.stage_bytes + 64));
+        }
+        // (the plan is in order and has its room: whatever the arena held when its header was written)
+        guard = {INT64_MAX, 0, 0, 0, 0};
         lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, VcHint{1, pi.chain_items, pi.payload_bytes, pi.max_pieces, pi.max_len}, S).lanes;
         if (c->timing) {
             std::swap(c->events[1], c->events[2]);        // (the planning ended where the first attempt began)
             c->plan_end = 1;
             HIP_TRY(hipEventRecord(c->events[2], c->stream));
         }
-        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes,
+        const bool tables = !plans_without_tables(S);
+        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, tables ? c->B.slot_lines() : nullptr, tables ? c->B.row_base : nullptr, c->header.as<int64_t>(), guard, lanes,
                                       c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], c->stream));
         HIP_TRY(VC_WAIT(c));

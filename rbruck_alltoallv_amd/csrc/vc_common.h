@@ -262,6 +262,11 @@ hipError_t vc_launch_plan_sizes(const VcSched &S, const VcLaunchInfo *launches_h
 hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_off, int64_t *row_tot, int64_t *row_base, int64_t *row_bytes,
                                   int64_t *chain_row_tot, int64_t *chain_row_base, int64_t *header, int64_t *header_host, unsigned *ticket,
                                   hipStream_t st);
+// Forwarded execution without a list on slots of a fixed stride (or without staging): the header alone.  rd_packed: where the packed receive
+// displacements go (with S.packed_recv); group_tot: vc_check_bytes(P) bytes; stage_bytes: header[0].
+size_t vc_check_bytes(int P);
+hipError_t vc_launch_plan_check(const VcSched &S, VcTables T, int *rd_packed, int64_t *group_tot, int64_t stage_bytes, int64_t *header,
+                                int64_t *header_host, unsigned *ticket, hipStream_t st);
 // Forwarded execution: staging[t] = bytes of staging the blocks for receiver t take (P int64, device).
 hipError_t vc_launch_receiver_staging(const VcSched &S, VcTables T, int64_t *staging, hipStream_t st);
 // Forwarded execution: the chain items (every block's route in closed form, staging addresses from the plan tables;

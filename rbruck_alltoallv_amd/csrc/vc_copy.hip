@@ -656,6 +656,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
                 hop[u].moves = 0; at_row[u] = 0; at[u] = 0;
                 if (k0 + u >= nslots) continue;
                 hop[u] = vc_walk_step(S, walk, s, t, k0 + u);
+                if (S.stride) { at_row[u] = vc_slot_addr(S, slot_off, row_base, hop[u]); continue; }
                 at_row[u] = row_base[hop[u].row];
                 at[u] = slot_off[(int64_t)hop[u].row * P + hop[u].id];
             }

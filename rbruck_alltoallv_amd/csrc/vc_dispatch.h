@@ -78,6 +78,13 @@ struct VcDispatch {
                              // against the plan (the hint is only a guess); stage_cap is the caller's to fill in
 };
 
+// Fixed stride of a call that stages in a window without being the single launch: the longest block at any cache-line phase, and an odd
+// number of lines, so that slots whose blocks are much shorter do not all start at the same few places of the window.  0: blocks too long for it.
+#define VC_STRIDE_MAX_LEN ((int64_t)1 << 30)
+VC_HD int vc_window_stride(int64_t longest) {
+    return longest > VC_STRIDE_MAX_LEN ? 0 : (int)((((longest + 2 * VC_LINE - 1) / VC_LINE) | 1) * VC_LINE);
+}
+
 VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 : (pairs < 8192 ? 1792 : 3072); }
 
 // mode: vc_comm_set_forwarding (0 launch per digit, 1 the library's choice, 2 the list, 3 / 4 / 5 listless with a workgroup / a

@@ -117,7 +117,7 @@ struct vc_comm {
         const char *sendbuf = nullptr;
         char *recvbuf = nullptr;
         int lanes = 0;                    // 0: only planned so far
-        int64_t max_pieces = 0;           // VcListlessGuard::max_pieces of the launch
+        VcListlessGuard guard = {0, 0, 0, 0, 0};      // of the launch
         int n_launch_infos = 0;
         hipStream_t own_stream = nullptr; // the communicator's stream while the call runs on the caller's
         CallParams q;                     // what was asked for (the call may have to be run again another way)

@@ -515,6 +515,197 @@ hipError_t vc_launch_plan_forward(const VcSched &S, VcTables T, uint32_t *slot_o
     return hipGetLastError();
 }
 
+// ---- calls without a list on slots of a fixed stride: nothing has to be summed up but what the header holds ----
+#define VC_CHECK_RANKS 4
+struct __attribute__((packed, aligned(4))) VcFour { int v[VC_CHECK_RANKS]; };
+enum { VC_CHECK_PAYLOAD, VC_CHECK_MOVED, VC_CHECK_BAD, VC_CHECK_ITEMS, VC_CHECK_MOST, VC_CHECK_LONGEST, VC_CHECK_WORDS };
+
+// Hops of a block (vc_block_hops) whose offsets inside the node and between the nodes are j and jg.
+__device__ __forceinline__ int vc_offset_hops(const VcSched &S, int j, int jg) {
+    int hops = S.last_hop == 2 || (S.last_hop == 1 && jg) || !(j | jg) ? 1 : 0;
+    for (int x = 0; x < S.w; x++) { const int q = vc_div(j, S.dr); hops += q * S.r != j; j = q; }
+    for (int x = 0; x < S.w2; x++) { const int q = vc_div(jg, S.dr); hops += q * S.r != jg; jg = q; }
+    return hops;
+}
+
+// A workgroup has four receivers, a thread one source at a time: what the source sends to the four is one read of 16 bytes (a column of the
+// table, which costs a request per entry when it is read one at a time as in vc_plan_forward), the receivers' own rows are read along.
+// PACKED (S.packed_recv): writes the packed receive displacements on the way (rd_packed), which took a kernel of their own before.
+// Bound by the latency of one round of reads, all of a thread's at once, and of the count of the workgroups: 7.0 us on 200 ranks, 7.5 on 256,
+// 12.8 on 1024, 18.9 there with packed displacements (vc_plan_forward 7.6, 9.6, 24 - 29, 29 + 6.8 for vc_row_scan_kernel and a boundary).
+// A thread with four sources, a tile of 4 x 4 entries, takes 10, 12.1 and 14.6: too few wavefronts.  Those whose blocks are all no longer than
+// VC_CHECK_SHORT bytes add up in 32 bits.
+// group_tot: VC_CHECK_WORDS words per four receivers.  Header as vc_plan_forward leaves it, its first word `stage_bytes`.  short_elems:
+// the elements of VC_CHECK_SHORT bytes.
+#define VC_CHECK_SHORT (1u << 18)                         // (64 lanes x 4 blocks x 32 hops of them are 2^31 bytes)
+template <int THREADS, bool PACKED>
+__global__ __launch_bounds__(THREADS) void vc_plan_check(VcSched S, VcTables T, int *__restrict__ rd_packed, int64_t *group_tot, int64_t stage_bytes,
+                                                         unsigned short_elems, int64_t *__restrict__ header, int64_t *__restrict__ header_host,
+                                                         unsigned *ticket) {
+    constexpr int R = VC_CHECK_RANKS, WAVES = THREADS / VC_WAVE;
+    static_assert((uint64_t)VC_CHECK_SHORT * R * VC_WAVE * VC_MAX_HOP_SLOTS <= (uint64_t)1 << 31, "sums of a wavefront in 32 bits");
+    __shared__ int64_t of_wave[WAVES][VC_CHECK_WORDS];
+    __shared__ int is_last;
+    const int P = S.P, groups = (P + R - 1) / R, groups_per_xcd = (groups + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS;
+    const int group = (int)(blockIdx.x % VC_PLAN_XCDS) * groups_per_xcd + (int)blockIdx.x / VC_PLAN_XCDS;      // (grid: VC_PLAN_XCDS x groups_per_xcd)
+    const int lane = threadIdx.x % VC_WAVE, wave = threadIdx.x / VC_WAVE, t0 = group * R;
+    int64_t sum[VC_CHECK_WORDS] = {0, 0, 0, 0, 0, 0};     // (of the wavefront, in its last lane)
+    if (group < groups) {
+        int64_t carry[R] = {0, 0, 0, 0};
+        for (int base = 0; base < P; base += THREADS) {
+            const bool live = base + (int)threadIdx.x < P;
+            const int s = live ? base + (int)threadIdx.x : 0;
+            VcPairEntries e[R];
+            int64_t rbase[R];
+            if (t0 + R <= P && S.table_mask) {            // (the same branch in every thread)
+                const VcFour column = *reinterpret_cast<const VcFour *>(reinterpret_cast<const char *>(T.sc) + ((unsigned)(s * P + t0) << 2));
+#pragma unroll
+                for (int j = 0; j < R; j++) e[j].sent = column.v[j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < R; j++) e[j].sent = vc_sc(S, T, s, t0 + j < P ? t0 + j : 0);
+            }
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                const int t = t0 + j < P ? t0 + j : 0;
+                e[j].expected = vc_rc(S, T, t, s);
+                e[j].rd = PACKED ? 0 : vc_rd(S, T, t, s);
+                e[j].own = vc_sc(S, T, t, s) | vc_sd(S, T, t, s);
+                rbase[j] = T.rbase[t];
+            }
+            if (PACKED) {
+                int64_t incl[R];
+#pragma unroll
+                for (int j = 0; j < R; j++) incl[j] = vc_wave_inclusive_scan(live ? e[j].expected : 0);
+                __syncthreads();
+                if (lane == VC_WAVE - 1)
+#pragma unroll
+                    for (int j = 0; j < R; j++) of_wave[wave][j] = incl[j];
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < R; j++) {
+                    const int64_t upto = vc_wave_inclusive_scan(lane < WAVES ? of_wave[lane][j] : 0);      // of wavefronts 0 .. lane
+                    const int64_t before = __shfl(upto, wave ? wave - 1 : 0, VC_WAVE);
+                    e[j].rd = (int)(carry[j] + (wave ? before : 0) + incl[j] - e[j].expected);
+                    carry[j] += vc_last_lane(upto);
+                    if (live && t0 + j < P) rd_packed[(int64_t)(t0 + j) * P + s] = e[j].rd;
+                }
+            }
+            const int gs = vc_div(s, S.dn), ls = s - gs * S.n;
+            bool brief = true;
+#pragma unroll
+            for (int j = 0; j < R; j++) brief = brief && (unsigned)e[j].sent <= short_elems && (unsigned)e[j].expected <= short_elems;
+            const bool all_brief = __ballot(!brief) == 0;
+            unsigned payload = 0, moved = 0, bad = 0, items = 0, most = 0, longest = 0;
+            int64_t wide[VC_CHECK_WORDS] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                const int t = t0 + j, gt = vc_div(t, S.dn), lt = t - gt * S.n;
+                const bool there = live && t < P;
+                const int hops = there ? vc_offset_hops(S, vc_wrap(ls - lt + S.n, S.n), vc_wrap(gs - gt + S.G, S.G)) : 0;
+                // (a power of two of the byte address: 32 bits that wrap around do)
+                const unsigned cut = ((unsigned)rbase[j] + (unsigned)e[j].rd * (unsigned)S.esz + (unsigned)S.recv_lo) & (VC_PIECE - 1), phase = cut & (VC_LINE - 1);
+                bad += there ? vc_bad_entries(S, e[j]) : 0;
+                if (all_brief) {
+                    const unsigned len = there ? (unsigned)e[j].sent * (unsigned)S.esz : 0;
+                    const unsigned cnt = len == 0 ? 0 : (len + phase <= VC_CHUNK ? 1 : (len + cut + VC_PIECE - 1) / VC_PIECE);
+                    payload += there ? (unsigned)e[j].expected * (unsigned)S.esz : 0;
+                    moved += len * hops;
+                    items += cnt;
+                    most = cnt > most ? cnt : most;
+                    longest = len > longest ? len : longest;
+                } else if (there) {
+                    const int64_t len = (int64_t)e[j].sent * S.esz, cnt = vc_chunk_count(len, (int)phase, (int)cut);
+                    wide[VC_CHECK_PAYLOAD] += (int64_t)e[j].expected * S.esz;
+                    wide[VC_CHECK_MOVED] += len * hops;
+                    wide[VC_CHECK_ITEMS] += cnt;
+                    wide[VC_CHECK_MOST] = cnt > wide[VC_CHECK_MOST] ? cnt : wide[VC_CHECK_MOST];
+                    wide[VC_CHECK_LONGEST] = len > wide[VC_CHECK_LONGEST] ? len : wide[VC_CHECK_LONGEST];
+                }
+            }
+            if (all_brief) {
+                wide[VC_CHECK_PAYLOAD] = vc_wave_join_last<false>(payload);
+                wide[VC_CHECK_MOVED] = vc_wave_join_last<false>(moved);
+                wide[VC_CHECK_ITEMS] = vc_wave_join_last<false>(items);
+                wide[VC_CHECK_MOST] = vc_wave_join_last<true>(most);
+                wide[VC_CHECK_LONGEST] = vc_wave_join_last<true>(longest);
+            } else {
+                wide[VC_CHECK_PAYLOAD] = vc_wave_inclusive_scan(wide[VC_CHECK_PAYLOAD]);
+                wide[VC_CHECK_MOVED] = vc_wave_inclusive_scan(wide[VC_CHECK_MOVED]);
+                wide[VC_CHECK_ITEMS] = vc_wave_inclusive_scan(wide[VC_CHECK_ITEMS]);
+                wide[VC_CHECK_MOST] = vc_wave_max_last(wide[VC_CHECK_MOST]);
+                wide[VC_CHECK_LONGEST] = vc_wave_max_last(wide[VC_CHECK_LONGEST]);
+            }
+            wide[VC_CHECK_BAD] = vc_wave_join_last<false>(bad);
+#pragma unroll
+            for (int k = 0; k < VC_CHECK_WORDS; k++) sum[k] = k < VC_CHECK_MOST ? sum[k] + wide[k] : (wide[k] > sum[k] ? wide[k] : sum[k]);
+        }
+        // the packed receive layout is an int prefix sum of the rank's receive counts, like the reference's displacements
+        if (PACKED && threadIdx.x == VC_WAVE - 1)
+#pragma unroll
+            for (int j = 0; j < R; j++)
+                if (carry[j] > 0x7FFFFFFF && t0 + j < P) sum[VC_CHECK_BAD] += VC_BAD_OVERFLOW;
+    }
+    for (int round = 0; round < 2; round++) {             // of the workgroup's receivers; in the last workgroup, of all
+        __syncthreads();
+        if (lane == VC_WAVE - 1)
+#pragma unroll
+            for (int k = 0; k < VC_CHECK_WORDS; k++) of_wave[wave][k] = sum[k];
+        __syncthreads();
+        int64_t all = 0;                                  // total `lane` of the workgroup
+        if (threadIdx.x < VC_CHECK_WORDS)
+#pragma unroll
+            for (int q = 0; q < WAVES; q++) {
+                const int64_t v = of_wave[q][lane];
+                all = lane < VC_CHECK_MOST ? all + v : (v > all ? v : all);
+            }
+        if (round) {
+            // every staged block is one hop, every block's last hop ends in recvbuf
+            constexpr int word[VC_CHECK_WORDS] = {1, VC_HEADER_FIXED, VC_HEADER_BAD, 2, VC_HEADER_MAX_PIECES, VC_HEADER_MAX_LEN};
+            if (threadIdx.x < VC_CHECK_WORDS) {
+                int to = word[0];
+#pragma unroll
+                for (int k = 1; k < VC_CHECK_WORDS; k++) to = lane == k ? word[k] : to;
+                header[to] = all;
+                header_host[to] = all;
+            } else if (threadIdx.x == VC_CHECK_WORDS) {
+                header[0] = stage_bytes;
+                header_host[0] = stage_bytes;
+            }
+            return;
+        }
+        if (group < groups && threadIdx.x < VC_CHECK_WORDS) vc_share(&group_tot[(int64_t)group * VC_CHECK_WORDS + lane], all);
+        if (threadIdx.x < VC_WAVE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the totals are where the last workgroup will look
+        if (threadIdx.x == 0) is_last = vc_last_workgroup(ticket);
+        __syncthreads();
+        if (!is_last) return;
+#pragma unroll
+        for (int k = 0; k < VC_CHECK_WORDS; k++) sum[k] = 0;
+        for (int g = threadIdx.x; g < groups; g += THREADS)
+#pragma unroll
+            for (int k = 0; k < VC_CHECK_WORDS; k++) {
+                const int64_t v = vc_shared(&group_tot[(int64_t)g * VC_CHECK_WORDS + k]);
+                sum[k] = k < VC_CHECK_MOST ? sum[k] + v : (v > sum[k] ? v : sum[k]);
+            }
+#pragma unroll
+        for (int k = 0; k < VC_CHECK_WORDS; k++) sum[k] = k < VC_CHECK_MOST ? vc_wave_inclusive_scan(sum[k]) : vc_wave_max_last(sum[k]);
+    }
+}
+
+size_t vc_check_bytes(int P) { return sizeof(int64_t) * VC_CHECK_WORDS * (size_t)((P + VC_CHECK_RANKS - 1) / VC_CHECK_RANKS); }
+
+hipError_t vc_launch_plan_check(const VcSched &S, VcTables T, int *rd_packed, int64_t *group_tot, int64_t stage_bytes, int64_t *header,
+                                int64_t *header_host, unsigned *ticket, hipStream_t st) {
+    const int groups = (S.P + VC_CHECK_RANKS - 1) / VC_CHECK_RANKS, grid = (groups + VC_PLAN_XCDS - 1) / VC_PLAN_XCDS * VC_PLAN_XCDS;
+    // all sources in one round up to 1024 ranks
+    const int threads = S.P <= 128 ? 128 : (S.P <= 256 ? 256 : (S.P <= 512 ? 512 : 1024));
+    const auto packed = threads == 128 ? vc_plan_check<128, true> : (threads == 256 ? vc_plan_check<256, true> : (threads == 512 ? vc_plan_check<512, true> : vc_plan_check<1024, true>));
+    const auto plain = threads == 128 ? vc_plan_check<128, false> : (threads == 256 ? vc_plan_check<256, false> : (threads == 512 ? vc_plan_check<512, false> : vc_plan_check<1024, false>));
+    hipLaunchKernelGGL(S.packed_recv ? packed : plain, dim3(grid), dim3(threads), 0, st, S, T, rd_packed, group_tot, stage_bytes,
+                       VC_CHECK_SHORT / (unsigned)S.esz, header, header_host, ticket);
+    return hipGetLastError();
+}
+
 // What a call that runs in batches of receivers has to know before the first of them: grid (P).
 __global__ __launch_bounds__(VC_THREADS) void vc_receiver_staging_kernel(VcSched S, VcTables T, int64_t *__restrict__ staging) {
     __shared__ int64_t lds[VC_WAVES_PER_BLOCK];

@@ -651,6 +651,8 @@ VC_HD int64_t vc_slot_bytes(uint32_t lines) { return (int64_t)lines * VC_LINE; }
 
 template <class Slot>
 VC_HD int64_t vc_slot_addr(const VcSched &S, const Slot *slot_off, const int64_t *row_base, const VcHop &h) {
+    // (in a window, a power of two of no more than 2^31 bytes, the place: products that wrap around change nothing)
+    if (S.stride && S.window) return ((unsigned)h.row * (unsigned)S.P + (unsigned)h.id) * (unsigned)S.stride & (unsigned)(S.window - 1);
     if (S.stride) return ((int64_t)h.row * S.P + h.id) * S.stride;
     return row_base[h.row] + vc_slot_bytes(slot_off[(int64_t)h.row * S.P + h.id]);
 }

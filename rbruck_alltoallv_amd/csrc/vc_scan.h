@@ -52,6 +52,21 @@ __device__ __forceinline__ int64_t vc_wave_max_last(int64_t v) {
     return vc_dpp_max<VC_DPP_BCAST31, 0xc>(v);
 }
 
+// Lane 63 receives the sum, or the maximum, of the wavefront's values: 32 bits, an instruction a step.
+template <int CTRL, int ROWS, bool MAX> __device__ __forceinline__ unsigned vc_dpp_join(unsigned v) {
+    const unsigned u = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+    return MAX ? (u > v ? u : v) : v + u;
+}
+
+template <bool MAX> __device__ __forceinline__ unsigned vc_wave_join_last(unsigned v) {
+    v = vc_dpp_join<VC_DPP_SHR(1), 0xf, MAX>(v);
+    v = vc_dpp_join<VC_DPP_SHR(2), 0xf, MAX>(v);
+    v = vc_dpp_join<VC_DPP_SHR(4), 0xf, MAX>(v);
+    v = vc_dpp_join<VC_DPP_SHR(8), 0xf, MAX>(v);
+    v = vc_dpp_join<VC_DPP_BCAST15, 0xa, MAX>(v);
+    return vc_dpp_join<VC_DPP_BCAST31, 0xc, MAX>(v);
+}
+
 // Lane 63's value, in every lane.
 __device__ __forceinline__ int64_t vc_last_lane(int64_t v) {
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, VC_WAVE - 1), hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), VC_WAVE - 1);

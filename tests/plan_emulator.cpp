@@ -250,6 +250,12 @@ extern "C" int plan_emulate(int func, int P, int n, int r, int batch, int esz, i
                     const bool moves = vc_block_hop(S, T, slot_off.data(), row_base.data(), s0, t, k, d);
                     const int64_t cell = hop_dst[(int64_t)k * PP + key0];
                     if (moves ? cell != d : cell != -1) errors++;
+                    if (moves && S.stride && (int)(d >> VC_SPACE_SHIFT) == 2) {       // the same slot in a window: its place, worked out in 32 bits
+                        VcSched in_window = S;
+                        in_window.window = 4 * VC_CHUNK;
+                        const VcHop h = vc_hop_place(S, s0, t, k);
+                        if (vc_slot_addr(in_window, slot_off.data(), row_base.data(), h) != (vc_slot_addr(S, slot_off.data(), row_base.data(), h) & vc_window_mask(in_window.window))) errors++;
+                    }
                 }
                 if (hop_src[key0] != (VC_SPACE_SEND | vc_send_offset(S, T, s0, t))) errors++;
                 for (int64_t c = 0; c < cnt; c++) {

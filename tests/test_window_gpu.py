@@ -59,7 +59,8 @@ def test_staging_window(case):
         assert torch.equal(dr, want), (case, ran)
         st = dp.comm.last_stats()
         ran.append((int(st.execution), int(st.lanes_per_item), int(st.staging_bytes)))
-        if st.execution != 3:                             # (slots of a fixed stride take more)
+        assert st.execution == 3 or st.staging_bytes <= WINDOW + CHUNK
+        if st.execution == 1:                             # (slots of a fixed stride take more)
             assert st.staging_bytes == (slots if slots <= WINDOW else WINDOW + CHUNK), (ran, slots)
     print(case, slots, ran, flush=True)
     plan = api.Plan(name, dp, dr, n=tun[0] if len(tun) == 3 or "TTPL" in name else 0, r=tun[1] if "TTPL" in name else tun[0])
@@ -102,4 +103,67 @@ def test_plan_with_a_window_in_a_graph():
         assert api.twophase_rbruck_alltoallv(8, dp, ds, dr) == 0 and torch.equal(dr, want)
     del graph
     plan.free()
+    dp.comm.free()
+
+
+@pytest.mark.parametrize("P,name,tun", [(193, "tuna_algorithm", (3, 0)), (256, "twophase_rbruck_alltoallv", (2,)), (510, "TTPL_BT_alltoallv", (30, 4, 0)),
+                                        (513, "TTPL_rbruck_alltoallv", (27, 3)), (1024, "TTPL_BT_alltoallv_s1", (32, 32, 0)),
+                                        (1027, "twophase_rbruck_alltoallv_om", (32,)), (1030, "TTPL_BT_alltoallv", (103, 103, 0)), (201, "spreadout_alltoallv", ())])
+def test_the_check_counts_what_the_planner_counts(P, name, tun):
+    """Calls without a list are checked and counted by a kernel of their own: same totals, same verdict, same bytes as through the list."""
+    from rbruck_alltoallv_amd import api
+    packed = name == "TTPL_BT_alltoallv"
+    counts = np.random.default_rng(P).integers(0, 250, (P, P)).astype(np.int32)
+    counts[::7, ::3] = 0
+    counts[P - 1, P - 1], counts[3, P - 2] = 9_001, 20_003
+    prob = W.make_problem(counts, 1, 1, 0 if packed else 1)
+    dp = api.DeviceProblem(prob)
+    fn = getattr(api, name)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 9, ds)
+
+    def totals(mode, rc=0):
+        dp.comm.set_forwarding(mode)
+        dr.fill_(0xEE)
+        assert fn(*tun, dp, ds, dr) == rc, dp.comm.error()
+        assert bool((dr == 0xEE).all()) if rc else dp.verify(ds, dr, packed) == 0
+        st = dp.comm.last_stats()
+        return int(st.execution), (st.payload_bytes, st.moved_bytes, st.block_pieces, st.max_block_pieces, st.max_block_bytes, st.bad_table_entries)
+
+    listed, checked = totals(2), totals(1)
+    assert (listed[0], checked[0]) == (1, 2) and checked[1] == listed[1]
+    for table, at, value in (("recvcounts", (P - 1, 0), 77), ("sdispls", (P - 2, 5), -3), ("sendcounts", (0, P - 1), -1)) + (() if packed else (("rdispls", (5, P - 1), -9),)):
+        t = getattr(dp, table)
+        keep = int(t[at])
+        t[at] = value
+        want = totals(2, -7)[1][-1]
+        assert totals(1, -7)[1][-1] == want > 0, table
+        t[at] = keep
+    assert totals(1) == checked                           # (the hint is still that of the last good call)
+    dp.comm.free()
+
+
+@pytest.mark.parametrize("P,esz", [(21, 1), (20, 24), (130, 8)])
+def test_the_check_on_long_blocks(P, esz):
+    """Blocks beyond the check's 32-bit sums, through the _async twin of a communicator's first call, which has nothing to choose a shape by."""
+    from rbruck_alltoallv_amd import api
+    counts = np.random.default_rng(P).integers(0, 40_000 // esz, (P, P)).astype(np.int32)
+    counts[1::5, ::4] = 300_001 // esz
+    counts[P - 1, 0] = 20_000_011 // esz
+    prob = W.make_problem(counts, esz, 0, 1)
+    dp = api.DeviceProblem(prob)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 9, ds)
+    dp.comm.set_forwarding(2)
+    assert api.twophase_rbruck_alltoallv(2, dp, ds, dr) == 0
+    want, st = dr.clone(), dp.comm.last_stats()
+    listed = (st.payload_bytes, st.moved_bytes, st.block_pieces, st.max_block_pieces, st.max_block_bytes)
+    dp.comm.free()
+    dp = api.DeviceProblem(prob)
+    for _ in range(2):
+        dr.fill_(0xEE)
+        assert api.call_async("twophase_rbruck_alltoallv", (2,), dp, ds, dr, torch.cuda.current_stream()) == 0 and dp.comm.wait() == 0, dp.comm.error()
+        st = dp.comm.last_stats()
+        assert torch.equal(dr, want) and st.execution == 2
+        assert (st.payload_bytes, st.moved_bytes, st.block_pieces, st.max_block_pieces, st.max_block_bytes) == listed
     dp.comm.free()

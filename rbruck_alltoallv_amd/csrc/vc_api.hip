@@ -680,7 +680,8 @@ static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &
         rc = enqueue_check(c, S, T, stage_bytes);
         if (rc) return rc;
         if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
-        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+                                      nullptr, nullptr, nullptr, VcSignal(), d.batch));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
         HIP_TRY(VC_WAIT(c));
         PlanInfo pi;
@@ -708,7 +709,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     S.recv_lo = (int)((uintptr_t)recvbuf & 4095);
     PlanInfo pi;
     hipStream_t st = c->stream;
-    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, false, {0, 0, 0, 0, 0}};
+    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, false, 0, {0, 0, 0, 0, 0}};
     const int pair_lanes = d.lanes;
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;
@@ -734,7 +735,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
                 HIP_TRY(hipEventRecord(c->events[2], st));
             }
             HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, pair_lanes, sendbuf, recvbuf,
-                                          c->stage.as<char>(), st));
+                                          c->stage.as<char>(), st, nullptr, nullptr, nullptr, VcSignal(), d.batch));
             if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
             HIP_TRY(VC_WAIT(c));
             synced = true;
@@ -788,7 +789,8 @@ static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, st
     if (c->timing) { rc = ensure_events(c, 5); if (rc) return rc; }
     hipStream_t st = c->stream;
     const bool stages = vc_may_stage(S);
-    int lanes = c->hint.valid || !stages ? vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes : 0;
+    const VcDispatch d = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S);
+    int lanes = c->hint.valid || !stages ? d.lanes : 0;
     VcListlessGuard guard = {0, stages && (lanes == VC_QUARTER || lanes == VC_BATCHED) ? VC_LISTLESS_MAX_PIECES : 0, 0, 0, 0};
     int64_t stage_bytes = 0;
     if (lanes) {
@@ -803,7 +805,8 @@ static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, st
     if (rc) return rc;
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
-        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+                                      nullptr, nullptr, nullptr, VcSignal(), d.batch));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
     return VC_OK;
@@ -821,11 +824,13 @@ static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std:
     int rc = plan_sizes(c, S, L, T, true);
     if (rc) return rc;
     hipStream_t st = c->stream;
-    const int lanes = c->stage.cap || !vc_may_stage(S) ? vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes : 0;
+    const VcDispatch d = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S);
+    const int lanes = c->stage.cap || !vc_may_stage(S) ? d.lanes : 0;
     const VcListlessGuard guard = {c->stage.cap >= 64 ? (int64_t)c->stage.cap - 64 : 0, 0, 0, 0, 0};
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
-        HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st));
+        HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+                                      nullptr, nullptr, nullptr, VcSignal(), d.batch));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
     return VC_OK;
@@ -871,7 +876,8 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
         }
         // (the plan is in order and has its room: whatever the arena held when its header was written)
         guard = {INT64_MAX, 0, 0, 0, 0};
-        lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, VcHint{1, pi.chain_items, pi.payload_bytes, pi.max_pieces, pi.max_len}, S).lanes;
+        const VcDispatch d = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, VcHint{1, pi.chain_items, pi.payload_bytes, pi.max_pieces, pi.max_len}, S);
+        lanes = d.lanes;
         if (c->timing) {
             std::swap(c->events[1], c->events[2]);        // (the planning ended where the first attempt began)
             c->plan_end = 1;
@@ -879,7 +885,8 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
         }
         const bool tables = !plans_without_tables(S);
         HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, tables ? c->B.slot_lines() : nullptr, tables ? c->B.row_base : nullptr, c->header.as<int64_t>(), guard, lanes,
-                                      c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream));
+                                      c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream, nullptr,
+                                      nullptr, nullptr, VcSignal(), d.batch));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], c->stream));
         HIP_TRY(VC_WAIT(c));
     }
@@ -1048,8 +1055,10 @@ extern "C" int twophase_rbruck_alltoallv_noalloc(int r, char *sendbuf, int *send
     VcTables T = make_tables(c, sendcounts, sdispls, recvcounts, rdispls);
     rc = enqueue_plan_sizes(c, S, L, T, true, false);
     if (rc) return rc;
-    const int lanes = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S).lanes;
-    HIP_TRY(vc_launch_copy_blocks(S, T, B.slot_lines(), B.row_base, B.header, guard, lanes, sendbuf, recvbuf, stage, c->stream));
+    const VcDispatch d = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S);
+    const int lanes = d.lanes;
+    HIP_TRY(vc_launch_copy_blocks(S, T, B.slot_lines(), B.row_base, B.header, guard, lanes, sendbuf, recvbuf, stage, c->stream, nullptr, nullptr,
+                                  nullptr, VcSignal(), d.batch));
     HIP_TRY(VC_WAIT(c));
     PlanInfo pi;
     rc = plan_read(c, S, L, pi, true);

@@ -17,6 +17,8 @@
 // lane code of the listless copy kernel that gives a wavefront a batch of pairs: a lane per pair works out the route, then
 // the quarters of the wavefront carry the blocks one after the other
 #define VC_BATCHED 1
+// ... where blocks of no more than this many bytes are moved by one lane each
+#define VC_LANE_BLOCK 128
 // window of one workgroup of the copy kernel: 256 lanes x 2 vectors x 16 bytes, starting at a cache-line boundary
 #define VC_CHUNK 8192
 #define VC_LINE 128
@@ -332,8 +334,8 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 // Forwarded execution without a work-item list: one workgroup (or a quarter of a wavefront) per (source, destination)
 // pair works out the route of its block from the plan tables and carries it through.  Reads the device `header` the
 // planning kernels before it on the stream have written and does nothing unless vc_listless_ok(header, guard).
-// lanes: VC_THREADS (a workgroup per pair), VC_WAVE (a wavefront per pair, blocks of a KiB or two) or VC_QUARTER (a quarter of a
-// wavefront per pair, for blocks of a few hundred bytes).
+// lanes: VC_THREADS (a workgroup per pair), VC_WAVE (a wavefront per pair, blocks of a KiB or two), VC_QUARTER (a quarter of a
+// wavefront per pair, for blocks of a few hundred bytes) or VC_BATCHED (`batch` pairs per wavefront, vc_batch_pairs).
 // verdict (device, non-null: fixed-stride staging, S.stride > 0, at most VC_MAX_GRID pairs): the kernel needs no planner
 // before it and `header` is not read.  Its first wavefronts check the tables, count themselves in the VC_VERDICTS words at `verdict` (zero at the
 // start; the kernel clears those at `verdict_next` for the call after this one) and leave what the host wants to know — payload, block pieces, longest block, ... —
@@ -346,6 +348,6 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  unsigned long long *verdict = nullptr, unsigned long long *verdict_next = nullptr,
-                                 int64_t *totals = nullptr, VcSignal sig = VcSignal());
+                                 int64_t *totals = nullptr, VcSignal sig = VcSignal(), int batch = 16);
 // dst2 non-null: every vector is stored twice (one read, two writes)
 hipError_t vc_launch_calibration_copy(const char *src, char *dst, char *dst2, int64_t nbytes, hipStream_t st);

@@ -226,9 +226,10 @@ struct __attribute__((packed, aligned(1))) VcU64 { unsigned long long v; };
 struct __attribute__((packed, aligned(1))) VcU32 { unsigned v; };
 struct __attribute__((packed, aligned(1))) VcU16 { unsigned short v; };
 
-// A block of 1 .. VC_LANE_BLOCK bytes in one lane's registers: its first and its last 16 (8, 4, 2, 1) bytes, which overlap.
-#define VC_LANE_BLOCK 32
-struct VcLaneBlock { vc_u32x4 first, last; };
+// A block of 1 .. VC_LANE_BLOCK bytes in one lane's registers: its first and its last 16 (8, 4, 2, 1) bytes, which overlap, and the
+// vectors between them.
+#define VC_LANE_MIDDLE (VC_LANE_BLOCK / 16 - 2)
+struct VcLaneBlock { vc_u32x4 first, last, middle[VC_LANE_MIDDLE]; };
 
 __device__ __forceinline__ VcLaneBlock vc_lane_load(const char *src, int len) {
     VcLaneBlock b;
@@ -236,6 +237,9 @@ __device__ __forceinline__ VcLaneBlock vc_lane_load(const char *src, int len) {
     if (len >= 16) {
         b.first = reinterpret_cast<const VcU128 *>(src)->v;
         b.last = reinterpret_cast<const VcU128 *>(src + len - 16)->v;
+#pragma unroll
+        for (int k = 0; k < VC_LANE_MIDDLE; k++)
+            if (len > 32 + 16 * k) b.middle[k] = reinterpret_cast<const VcU128 *>(src + 16 + 16 * k)->v;
     } else if (len >= 8) {
         const unsigned long long x = reinterpret_cast<const VcU64 *>(src)->v, y = reinterpret_cast<const VcU64 *>(src + len - 8)->v;
         b.first.x = (unsigned)x; b.first.y = (unsigned)(x >> 32); b.last.x = (unsigned)y; b.last.y = (unsigned)(y >> 32);
@@ -254,6 +258,9 @@ __device__ __forceinline__ VcLaneBlock vc_lane_load(const char *src, int len) {
 __device__ __forceinline__ void vc_lane_store(const VcLaneBlock &b, char *dst, int len) {
     if (len >= 16) {
         reinterpret_cast<VcU128 *>(dst)->v = b.first;
+#pragma unroll
+        for (int k = 0; k < VC_LANE_MIDDLE; k++)
+            if (len > 32 + 16 * k) reinterpret_cast<VcU128 *>(dst + 16 + 16 * k)->v = b.middle[k];
         reinterpret_cast<VcU128 *>(dst + len - 16)->v = b.last;
     } else if (len >= 8) {
         reinterpret_cast<VcU64 *>(dst)->v = (unsigned long long)b.first.y << 32 | b.first.x;
@@ -618,7 +625,9 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
 // 64 / BATCH lanes per pair evaluate its hop slots and leave the route in LDS.  Blocks of no more than VC_LANE_BLOCK bytes are then moved by
 // a lane each, when all blocks of the wavefront are that short; else every quarter of the wavefront carries BATCH / 4 of them, one
 // after the other.  Measured on MI355X, 1024 ranks, two hops for most blocks: 0 - 16 bytes 76 us (pairs of one receiver
-// in a row, every block a quarter of a wavefront) -> 28; 0 - 512 bytes 277 -> 250.
+// in a row, every block a quarter of a wavefront) -> 28; 0 - 64 bytes, calls 144 -> 82 (blocks of up to 32 bytes a lane before).
+// Two blocks of a quarter in flight at once make it slower (0 - 512 bytes, calls of 16 pairs a wavefront 202 us -> 240): the requests of a wavefront
+// queue up in the memory.
 template <int BATCH, bool WINDOW>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                        const int64_t *__restrict__ row_base,
@@ -725,13 +734,12 @@ static void vc_launch_batch(const VcSched &S, VcTables T, const uint32_t *slot_o
 
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
-                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig) {
+                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig, int batch) {
     const int64_t npairs = (int64_t)S.P * S.P;
     if (sig.word && (!verdict || S.window || (lanes != VC_WAVE && lanes != VC_THREADS))) return hipErrorInvalidValue;
     if (lanes == VC_BATCHED) {
         if (verdict) return hipErrorInvalidValue;         // the batches are for more pairs than one launch with totals takes
-        const int batch = vc_batch_pairs(npairs);
-        (batch == 64 ? vc_launch_batch<64> : (batch == 32 ? vc_launch_batch<32> : vc_launch_batch<16>))(
+        (batch == 64 ? vc_launch_batch<64> : vc_launch_batch<16>)(
             S, T, slot_off, row_base, header, guard, sendbuf, recvbuf, stage, st);
         return hipGetLastError();
     }

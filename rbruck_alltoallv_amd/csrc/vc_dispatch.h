@@ -12,7 +12,7 @@
 //    quarter wins only further down: never up to 32 ranks (1024 pairs leave room for as many workgroups: 26 either way,
 //    the workgroup up to 1.3 x faster on KiB blocks), below 1.75 KiB up to 90 ranks (64 ranks: 27 - 33 against 34 - 38),
 //    below 3 KiB above (128 ranks: 30 - 70 against 64 - 84).
-//  * ... a batch of 16 - 64 pairs per wavefront when the blocks are so short that working out the routes costs more than
+//  * ... a batch of 16 or 64 pairs per wavefront when the blocks are so short that working out the routes costs more than
 //    moving the bytes: on 192 - 2048 ranks 5 - 40 % faster than the quarter up to an average block of 256 bytes, even at
 //    512, 3 - 16 % slower beyond.  Not on at most 128 ranks, where batches would leave most of the chip without a wavefront.
 //  * ... for the functions that send every block straight to its destination (nothing is staged, the plan is the check of the
@@ -74,9 +74,16 @@ struct VcDispatch {
     int stride;              // > 0: first try one launch on fixed-stride staging with slots of this many bytes ...
     int stride_lanes;        // ... with this many lanes per pair (the batches come without the totals: a quarter of a wavefront)
     bool self;               // ... that tells the host itself when it is done
+    int batch;               // VC_BATCHED: pairs per wavefront
     VcListlessGuard guard;   // what the call must look like for the listless kernel to move anything, checked on the device
                              // against the plan (the hint is only a guess); stage_cap is the caller's to fill in
 };
+
+// Pairs per wavefront of the batched listless kernel.  Where a lane moves a block each, all 64 lanes have one; where quarters of the wavefront
+// carry the blocks one after the other, short wavefronts keep the chip fuller.  Microseconds a call with 64 / 32 / 16 pairs, blocks of 0 .. x bytes: 1024 ranks, x = 32 53 / 60 / 75, 64 82 (a lane a block)
+// / - / 102, 128 120 / - / 151; 256 174 / 165 / 157, 512 224 / 212 / 202, 700 270 / 256 / 245; 512 ranks, 16 30 / 32 / 36, 64 35 / - / 43, 256 82 / 75 / 65, 512
+// 91 / 92 / 81; 800 ranks, 512 232 / 223 / 219; 256 ranks, 16 23.5 / 23.5 / 25.3, 100 28 / 28 / 30.
+VC_HD int vc_batch_pairs(int64_t longest) { return longest > VC_LANE_BLOCK ? 16 : 64; }
 
 // Fixed stride of a call that stages in a window without being the single launch: the longest block at any cache-line phase, and an odd
 // number of lines, so that slots whose blocks are much shorter do not all start at the same few places of the window.  0: blocks too long for it.
@@ -90,7 +97,8 @@ VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 :
 // mode: vc_comm_set_forwarding (0 launch per digit, 1 the library's choice, 2 the list, 3 / 4 / 5 listless with a workgroup / a
 // quarter of a wavefront per pair / batches).  S: the call's schedule (ranks, digits, whether it has an organized region).
 inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const VcSched &S) {
-    VcDispatch d = {0, 0, 0, false, {0, 0, 0, 0, 0}};
+    VcDispatch d = {0, 0, 0, false, 0, {0, 0, 0, 0, 0}};
+    d.batch = vc_batch_pairs(h.valid ? h.max_len : VC_LANE_BLOCK + 1);
     if (mode == 3) { d.lanes = VC_THREADS; return d; }
     if (mode == 4) { d.lanes = VC_QUARTER; return d; }
     if (mode == 5) { d.lanes = VC_BATCHED; return d; }
@@ -144,7 +152,5 @@ VC_HD int vc_lanes_for_items(int64_t bytes, int64_t items) {
     return average < VC_ITEM_QUARTER_BELOW ? VC_QUARTER : (average < VC_ITEM_WAVE_BELOW ? VC_WAVE : VC_THREADS);
 }
 
-// Pairs per wavefront of the batched listless kernel, and groups of four items in a row per wavefront of the quarter kernels:
-// as many as leave every SIMD of the chip a few wavefronts.
-VC_HD int vc_batch_pairs(int64_t pairs) { return pairs >= ((int64_t)1 << 19) ? 64 : (pairs >= ((int64_t)1 << 17) ? 32 : 16); }
+// Groups of four items in a row per wavefront of the quarter kernels: as many as leave every SIMD of the chip a few wavefronts.
 VC_HD int vc_quarter_rounds(int64_t items) { return items >= ((int64_t)1 << 19) ? 4 : (items >= ((int64_t)1 << 17) ? 2 : 1); }

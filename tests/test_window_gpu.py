@@ -30,6 +30,9 @@ CASES = {
     "quarters": ("TTPL_BT_alltoallv", (30, 2, 0), np.random.default_rng(1).integers(0, 1100, (300, 300)).astype(np.int32), 1, 0),
     "batches, a lane a block": ("tuna_algorithm", (2, 0), np.random.default_rng(2).integers(0, 17, (512, 512)).astype(np.int32), 1, 0),
     "batches, a quarter a block": ("twophase_rbruck_alltoallv", (4,), np.random.default_rng(3).integers(0, 300, (512, 512)).astype(np.int32), 1, 1),
+    "a lane a block, every length": ("TTPL_BT_alltoallv_s1", (26, 5, 0), (np.arange(260 * 260).reshape(260, 260) % 129).astype(np.int32), 1, 1),
+    "one byte too long for a lane": ("twophase_rbruck_alltoallv", (3,), (np.arange(260 * 260).reshape(260, 260) % 130).astype(np.int32), 1, 1),
+    "direct, a lane a block": ("spreadout_alltoallv", (), (np.arange(260 * 260).reshape(260, 260) % 43).astype(np.int32), 3, 1),
     "one launch": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(4).integers(0, 2500, (100, 100)).astype(np.int32), 1, 1),
     "one launch that signals its end": ("twophase_rbruck_alltoallv_om", (2,), np.random.default_rng(4).integers(0, 12_000, (31, 31)).astype(np.int32), 1, 1),
 }
@@ -63,7 +66,7 @@ def test_staging_window(case):
         if st.execution == 1:                             # (slots of a fixed stride take more)
             assert st.staging_bytes == (slots if slots <= WINDOW else WINDOW + CHUNK), (ran, slots)
     print(case, slots, ran, flush=True)
-    plan = api.Plan(name, dp, dr, n=tun[0] if len(tun) == 3 or "TTPL" in name else 0, r=tun[1] if "TTPL" in name else tun[0])
+    plan = api.Plan(name, dp, dr, n=tun[0] if "TTPL" in name else 0, r=tun[1] if "TTPL" in name else (tun + (2,))[0])
     assert plan.rc == 0, dp.comm.error()
     for _ in range(2):
         dr.fill_(0xEE)

@@ -54,7 +54,7 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
         c->h_launches = reinterpret_cast<VcLaunchInfo *>(reinterpret_cast<char *>(c->h_header) + launches_at);
         memset(c->h_flags, 0, VC_FLAG_WORDS * sizeof(int));
     }
-    if (e == hipSuccess) e = c->counting.reserve(VC_COUNTING_BYTES);
+    if (e == hipSuccess) e = c->counting.reserve(VC_COUNTING_BYTES + VC_HEADER_BYTES + sizeof(VcLaunchInfo) * VC_MAX_LAUNCHES);
     if (e == hipSuccess) e = hipMemset(c->counting.p, 0, VC_COUNTING_BYTES);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);          // (the calls may run on a stream that does not wait for this one)
     if (e != hipSuccess) {
@@ -68,6 +68,8 @@ extern "C" int vc_comm_create(int nranks, vc_comm_t *comm_out) {
     c->of_call = done(VC_CALL_DONE_AT, 0);
     c->of_meta = done(VC_META_DONE_AT, 1);
     c->max_state = reinterpret_cast<int *>(c->counting.as<char>() + 2 * VC_TICKET_BYTES);
+    c->header = reinterpret_cast<int64_t *>(c->counting.as<char>() + VC_COUNTING_BYTES);
+    c->launches = reinterpret_cast<VcLaunchInfo *>(c->counting.as<char>() + VC_COUNTING_BYTES + VC_HEADER_BYTES);
     c->staging_allowance = default_staging_allowance();
     *comm_out = c;
     return VC_OK;
@@ -77,8 +79,7 @@ extern "C" int vc_comm_free(vc_comm_t c) {
     if (!c) return VC_OK;
     (void)hipStreamSynchronize(c->stream);
     c->pending.active = false;
-    for (DevBuf *b : {&c->slot_off, &c->row_tot, &c->row_base, &c->org_run_base, &c->item_row_tot, &c->item_row_base, &c->row_bytes, &c->desc, &c->header, &c->launches, &c->stage, &c->rd_packed,
-                      &c->scratch, &c->counting, &c->chain_row_tot, &c->chain_row_base, &c->verdicts})
+    for (DevBuf *b : {&c->plan, &c->desc, &c->stage, &c->rd_packed, &c->scratch, &c->counting, &c->verdicts})
         b->release();
     free_retired_stage(c);
     for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
@@ -237,31 +238,31 @@ static PlanBufSizes plan_buf_sizes(const VcSched &S, int nl, bool forward) {
     return z;
 }
 
-// The communicator's own buffers, grown to what the call needs.
+static size_t carve(size_t &at, size_t bytes) {
+    const size_t here = at;
+    at += (bytes + 255) & ~(size_t)255;
+    return here;
+}
+
+// The communicator's own plan tables, slices of one allocation grown to what the call needs (an allocation is 10 us, one of a size the runtime
+// has not met yet 300; with one for each table the first call of a communicator of 8 ranks took 58 us, now 48, of 256 ranks 225, now 206).
 static int reserve_plan_bufs(vc_comm *c, const VcSched &S, int nl, bool forward) {
     const PlanBufSizes z = plan_buf_sizes(S, nl, forward);
-    HIP_TRY(c->slot_off.reserve(z.slot_off));
-    HIP_TRY(c->row_tot.reserve(z.row_tot));
-    HIP_TRY(c->row_base.reserve(z.row_base));
-    HIP_TRY(c->org_run_base.reserve(z.org_run_base));
-    HIP_TRY(c->item_row_tot.reserve(z.item_row_tot));
-    HIP_TRY(c->item_row_base.reserve(z.item_row_base));
-    HIP_TRY(c->row_bytes.reserve(z.row_bytes));
-    HIP_TRY(c->header.reserve(z.header));
-    HIP_TRY(c->launches.reserve(z.launches));
-    if (forward) {
-        HIP_TRY(c->chain_row_tot.reserve(z.chain_row_tot));
-        HIP_TRY(c->chain_row_base.reserve(z.chain_row_base));
-    }
+    size_t at = 0;
+    const size_t slot_off = carve(at, z.slot_off), row_tot = carve(at, z.row_tot), row_base = carve(at, z.row_base), org_run_base = carve(at, z.org_run_base),
+                 item_row_tot = carve(at, z.item_row_tot), item_row_base = carve(at, z.item_row_base), row_bytes = carve(at, z.row_bytes),
+                 chain_row_tot = carve(at, z.chain_row_tot), chain_row_base = carve(at, z.chain_row_base);
+    HIP_TRY(c->plan.reserve(at));
     if (S.packed_recv) HIP_TRY(c->rd_packed.reserve(z.rd_packed));
+    char *const base = c->plan.as<char>();
+    const auto table = [base](size_t offset) { return reinterpret_cast<int64_t *>(base + offset); };
     PlanBufs &B = c->B;
-    B.slot_off = c->slot_off.as<int64_t>(); B.row_tot = c->row_tot.as<int64_t>(); B.row_base = c->row_base.as<int64_t>();
-    B.org_run_base = c->org_run_base.as<int64_t>(); B.item_row_tot = c->item_row_tot.as<int64_t>();
-    B.item_row_base = c->item_row_base.as<int64_t>(); B.row_bytes = c->row_bytes.as<int64_t>();
-    B.chain_row_tot = forward ? c->chain_row_tot.as<int64_t>() : nullptr;
-    B.chain_row_base = forward ? c->chain_row_base.as<int64_t>() : nullptr;
+    B.slot_off = table(slot_off); B.row_tot = table(row_tot); B.row_base = table(row_base); B.org_run_base = table(org_run_base);
+    B.item_row_tot = table(item_row_tot); B.item_row_base = table(item_row_base); B.row_bytes = table(row_bytes);
+    B.chain_row_tot = forward ? table(chain_row_tot) : nullptr;
+    B.chain_row_base = forward ? table(chain_row_base) : nullptr;
     B.ticket = c->of_call.ticket;
-    B.header = c->header.as<int64_t>(); B.launches = c->launches.as<VcLaunchInfo>(); B.rd_packed = c->rd_packed.as<int>();
+    B.header = c->header; B.launches = c->launches; B.rd_packed = c->rd_packed.as<int>();
     return VC_OK;
 }
 
@@ -648,14 +649,13 @@ static int place_in_window(vc_comm *c, VcSched &S, int64_t longest, VcListlessGu
 }
 
 static int reserve_check_bufs(vc_comm *c, const VcSched &S) {
-    HIP_TRY(c->header.reserve(sizeof(int64_t) * VC_HEADER_WORDS(VC_MAX_LAUNCHES)));
-    HIP_TRY(c->row_bytes.reserve(vc_check_bytes(S.P)));
+    HIP_TRY(c->plan.reserve(vc_check_bytes(S.P)));
     if (S.packed_recv) HIP_TRY(c->rd_packed.reserve(sizeof(int) * (size_t)S.P * S.P));
     return VC_OK;
 }
 
 static int enqueue_check(vc_comm *c, const VcSched &S, VcTables &T, int64_t stage_bytes) {
-    HIP_TRY(vc_launch_plan_check(S, T, c->rd_packed.as<int>(), c->row_bytes.as<int64_t>(), stage_bytes, c->header.as<int64_t>(), c->h_header_dev,
+    HIP_TRY(vc_launch_plan_check(S, T, c->rd_packed.as<int>(), c->plan.as<int64_t>(), stage_bytes, c->header, c->h_header_dev,
                                  c->of_call.ticket, c->stream));
     T.rd_packed = c->rd_packed.as<int>();
     return VC_OK;
@@ -680,7 +680,7 @@ static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &
         rc = enqueue_check(c, S, T, stage_bytes);
         if (rc) return rc;
         if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
-        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header, guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
                                       nullptr, nullptr, nullptr, VcSignal(), d.batch));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
         HIP_TRY(VC_WAIT(c));
@@ -805,7 +805,7 @@ static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, st
     if (rc) return rc;
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
-        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header.as<int64_t>(), guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
                                       nullptr, nullptr, nullptr, VcSignal(), d.batch));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
@@ -884,7 +884,7 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
             HIP_TRY(hipEventRecord(c->events[2], c->stream));
         }
         const bool tables = !plans_without_tables(S);
-        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, tables ? c->B.slot_lines() : nullptr, tables ? c->B.row_base : nullptr, c->header.as<int64_t>(), guard, lanes,
+        HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, tables ? c->B.slot_lines() : nullptr, tables ? c->B.row_base : nullptr, c->header, guard, lanes,
                                       c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream, nullptr,
                                       nullptr, nullptr, VcSignal(), d.batch));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], c->stream));
@@ -997,12 +997,6 @@ extern "C" int TTPL_rbruck_alltoallv(int n, int r, char *sendbuf, int *sendcount
 // a GPU uses that GPU's one array, so calls that overlap on one GPU race.  The first
 // words count the planning kernel's workgroups and are zero between the calls; of the rest nothing needs to start at zero: the
 // planning kernel overwrites every word it or the copy kernel later reads.
-static size_t carve(size_t &at, size_t bytes) {
-    const size_t here = at;
-    at += (bytes + 255) & ~(size_t)255;
-    return here;
-}
-
 extern "C" int twophase_rbruck_alltoallv_noalloc(int r, char *sendbuf, int *sendcounts, int *sdispls, int sendtype_size, char *recvbuf,
                                                  int *recvcounts, int *rdispls, int recvtype_size, vc_comm_t c) {
     (void)recvtype_size;

@@ -95,12 +95,13 @@ struct vc_comm {
     int plan_end = 2;                     // which event marks the end of the planning kernels of the call in progress
     int waits = 0;                        // times the host has waited for the stream in the call in progress
     int64_t items_before_last = 0;        // block pieces of the forwarded call before the one `hint` describes (0: there was none)
-    DevBuf chain_row_tot, chain_row_base;
     DevBuf verdicts;                      // fixed-stride calls: two sets of VC_VERDICTS words used in turn
     bool verdict_clean = false;           // ... and the set the next call will use is known to be zero
     int verdict_turn = 0;
-    DevBuf slot_off, row_tot, row_base, org_run_base, item_row_tot, item_row_base, row_bytes, desc, header, launches, stage, rd_packed,
-        scratch, counting;
+    DevBuf plan;                          // the plan tables of the current call, one allocation (reserve_plan_bufs)
+    DevBuf desc, stage, rd_packed, scratch, counting;
+    int64_t *header = nullptr;            // (in `counting`) the planner's header on the device
+    VcLaunchInfo *launches = nullptr;     // (there too) the launch table of calls of more launches than travel as an argument
     double cal_copy_bytes_per_s = 0, cal_launch_s = 0, cal_sync_s = 0;   // calibrate(): the plain copy's rate, the cost of a
                                           // launch, of a launch the host waits for
     int bound_staging = 1;                // vc_comm_set_staging_bound
@@ -176,9 +177,10 @@ struct BusyGuard {
 #define VC_CALL_DONE_AT 32
 #define VC_META_DONE_AT 64
 #define VC_FLAG_WORDS 96
-// `counting` (device, zero from the start): the tickets of of_call and of_meta, max_state
+// `counting` (device): the tickets of of_call and of_meta and max_state, zero from the start; header and launch table
 #define VC_MAX_STATE_BYTES 512
 #define VC_COUNTING_BYTES (2 * VC_TICKET_BYTES + VC_MAX_STATE_BYTES)
+#define VC_HEADER_BYTES ((sizeof(int64_t) * VC_HEADER_WORDS(VC_MAX_LAUNCHES) + 255) / 256 * 256)
 #define VC_SPIN_US 10000
 
 // Enqueues launch(st, sig), whose last kernel tells the host by `sig` that everything before it on the stream and it itself are done, and

@@ -78,7 +78,7 @@ int vc_comm_set_bases(vc_comm_t comm, const int64_t *sbase_bytes, const int64_t 
  *    cannot serve has moved nothing and is redone the usual way, a longer list than guessed gets a second launch.
  *    When the last call on the communicator consisted of
  *    short blocks, the next one goes without the list: every pair of ranks gets a workgroup (at most 128 ranks) or a
- *    quarter of a wavefront (short blocks: average piece below 768 B on any number of ranks, below 1.75 - 3 KiB on 33 - 128) that derives its block's route itself; the
+ *    quarter of a wavefront (short blocks: average piece below 1280 B, without a window 768 B, on any number of ranks, below 1.75 - 3 KiB on 33 - 192) that derives its block's route itself; the
  *    kernel is enqueued right behind the size computation and the call needs one host synchronisation instead of two.
  *    Such a call also gets the reference's own staging layout, every slot as long as the longest block
  *    (src/twophase_tunable_rbruckv.cpp:59; the stride comes from the last call's longest block): slot addresses are then
@@ -86,9 +86,9 @@ int vc_comm_set_bases(vc_comm_t comm, const int64_t *sbase_bytes, const int64_t 
  *    table entries, and that its block fits a slot, before it forms an address from them; the kernel's first wavefronts
  *    check all of the tables and add up what the host needs afterwards, and the copying wavefronts hold their stores
  *    back until those have reported the tables in order (a call that returns VC_ERR_TABLES has written nothing here
- *    either); a call with a longer block is redone the general way.  Only on at most 192 ranks and while
- *    regions x P x P x stride stays below 256 MiB.
- *    On more than 192 ranks and blocks below 384 B on average a wavefront takes a batch of 16 - 64 pairs instead: a lane per
+ *    either); a call with a longer block is redone the general way.  Only on at most 192 ranks and, without a window (vc_comm_set_staging_bound),
+ *    while regions x P x P x stride stays below 256 MiB.
+ *    On more than 192 ranks and blocks below 384 B on average (640 B on 512 and more, in a window) a wavefront takes a batch of 16 or 64 pairs instead: a lane per
  *    pair works out the route, then the quarters of the wavefront carry the blocks one after the other.
  * 2: forwarded, always through the list.   3 / 4 / 5: forwarded, always without it, a workgroup / a quarter of a
  *    wavefront per pair of ranks / a batch of pairs per wavefront (any sizes; not the fastest choice everywhere).
@@ -113,7 +113,7 @@ int vc_comm_set_forwarding(vc_comm_t comm, int enable);
  *  - forwarded execution in the default mode with the default bound (1) stages in a window of 32 MiB: a slot at offset x of the layout lies
  *    at x mod 32 MiB, piece by piece.  A piece makes its next hop out of the registers of the workgroup that staged it, so nothing reads
  *    what it left behind, and the window stays in the memory-side cache.  Calls on fixed-stride slots with a
- *    wavefront or a workgroup per pair of ranks have an arena of up to 256 MiB instead;
+ *    wavefront or a workgroup per pair of ranks have an arena of up to 256 MiB instead, if that holds them;
  *  - forwarded execution in another mode or with an allowance keeps every hop's copy of every block in a place of its own.  A call whose
  *    staging would pass both the allowance (an eighth of the device's memory, at least
  *    1 GiB) and three times its payload is run in batches of receivers that use the same staging memory one after

@@ -472,7 +472,8 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     if (d.stride <= 0) return 0;
     const int pair_lanes = d.stride_lanes;
     S.stride = d.stride;
-    if (pair_lanes != VC_QUARTER) S.window = 0;           // (no more than VC_STRIDED_MAX_BYTES: a window would only save memory)
+    // (a wavefront or a workgroup per pair: while there is room a window would only save memory, and its kernels take 1 % longer)
+    if (pair_lanes != VC_QUARTER && vc_strided_stage_bytes(S) <= VC_STRIDED_MAX_BYTES) S.window = 0;
     const int64_t need = vc_window_bytes(vc_strided_stage_bytes(S), S.window);
     hipStream_t st = c->stream;
     // two sets of words in turn: a launch counts in one, which must start from zero, and clears the other one for the next call

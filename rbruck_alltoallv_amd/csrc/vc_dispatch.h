@@ -27,7 +27,9 @@
 //    longest block (src/twophase_tunable_rbruckv.cpp:59), makes slot addresses closed forms, so the call needs no planner
 //    at all.  64 ranks with blocks of 0 - 4 KiB 41 -> 24.6; 128 ranks, 0 - 512 B: 41 -> 25.6; 160 ranks: 31 - 42 -> 26 - 34;
 //    192 ranks: 31 - 50 -> 30 - 42; but 256 ranks 34 - 68 -> 44 - 68 and 384 ranks 2 x slower (the atomics of the totals
-//    and the arena grow with the square of the ranks): only up to 192 ranks and 256 MiB of arena.
+//    and the arena grow with the square of the ranks): only up to 192 ranks and, where the slots do not lie in a window, 256 MiB of arena.
+//    In a window, list or planner and copy / one launch: 64 ranks, 0 - 16 KB 53 / 48; 100 ranks, 0 - 8 KB 56 / 52; 128 ranks, 0 - 3 KB 47 / 43; 40 ranks,
+//    0 - 30 KB 45 / 39; 150 ranks, power law up to 4 KB 44 / 37.
 #pragma once
 
 #include "vc_common.h"
@@ -39,6 +41,13 @@
 #define VC_LISTLESS_MAX_PIECES 8              // pieces of one block: quarter of a wavefront per pair, batches
 #define VC_LISTLESS_WG_MAX_PIECES 16          // pieces of one block: wavefront or workgroup per pair
 #define VC_LISTLESS_QUARTER_BELOW 768         // average piece below which pairs get a quarter of a wavefront, more than 128 ranks
+// ... of calls that stage in a window, which need no plan tables then (vc_plan_check), more than 192 ranks; up to 192 ranks, in one launch,
+// VC_LISTLESS_WAVE_BELOW.  Calls, list / quarters, by average block: 140 ranks, 1 KB 41 / 35, 2.5 KB 59 / 52; 192 ranks, 1 KB 55 / 51, 2.5 KB 85 / 82; 512
+// ranks, 1 KB 203 / 185, 1.5 KB 262 / 262; 1024 ranks, 1 KB 593 / 572, 1.5 KB 808 / 819; 256 ranks, 1 KB 61 / 61, 1.5 KB 74 / 77.
+#define VC_WINDOW_QUARTER_BELOW 1280
+// ... and batches from 512 ranks up: quarters / batches, 1024 ranks, 500 B 354 / 326, 700 B 435 / 439; 512 ranks, 500 B 129 / 121; 256 ranks, 700 B 51 / 49
+#define VC_WINDOW_BATCH_BELOW 640
+#define VC_WINDOW_BATCH_PAIRS (1 << 18)
 #define VC_LISTLESS_BATCH_BELOW 384           // average piece below which a wavefront takes a batch of pairs
 #define VC_LISTLESS_DIRECT_PAIRS (1 << 17)    // direct functions: a quarter of a wavefront per pair up to VC_LISTLESS_WAVE_BELOW
 #define VC_LISTLESS_WAVE_BELOW 3072           // average piece below which a pair gets a wavefront instead of a workgroup
@@ -107,10 +116,11 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
     const int64_t pairs = (int64_t)S.P * S.P;
     const bool small_comm = pairs <= VC_LISTLESS_MAX_PAIRS;
     const int64_t average = h.payload / (h.items > 0 ? h.items : 1);
-    const bool short_blocks = h.valid && h.max_pieces <= VC_LISTLESS_MAX_PIECES &&
-                              average < (small_comm ? vc_small_quarter_below(pairs) : VC_LISTLESS_QUARTER_BELOW);
+    const int64_t quarter_below = small_comm ? vc_small_quarter_below(pairs)
+                                             : (!S.window ? VC_LISTLESS_QUARTER_BELOW : (pairs <= VC_STRIDED_MAX_PAIRS ? VC_LISTLESS_WAVE_BELOW : VC_WINDOW_QUARTER_BELOW));
+    const bool short_blocks = h.valid && h.max_pieces <= VC_LISTLESS_MAX_PIECES && average < quarter_below;
     if (short_blocks)
-        d.lanes = !small_comm && average < VC_LISTLESS_BATCH_BELOW ? VC_BATCHED : VC_QUARTER;
+        d.lanes = !small_comm && average < (S.window && pairs >= VC_WINDOW_BATCH_PAIRS ? VC_WINDOW_BATCH_BELOW : VC_LISTLESS_BATCH_BELOW) ? VC_BATCHED : VC_QUARTER;
     else if (listless_only)
         d.lanes = VC_THREADS;
     else if (h.valid && small_comm && h.max_pieces <= VC_LISTLESS_WG_MAX_PIECES && h.items <= VC_LISTLESS_MAX_ITEMS)
@@ -130,7 +140,8 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
         const int64_t stride = (h.max_len + 2 * VC_LINE - 1) & ~(int64_t)(VC_LINE - 1);
         VcSched strided = S;
         strided.stride = (int)stride;
-        if (stride <= 0x7FFFFF80 && vc_strided_stage_bytes(strided) <= VC_STRIDED_MAX_BYTES) {
+        // (in a window the slots may take any room)
+        if (stride <= 0x7FFFFF80 && (S.window || vc_strided_stage_bytes(strided) <= VC_STRIDED_MAX_BYTES)) {
             d.stride = (int)stride;
             d.stride_lanes = d.lanes == VC_BATCHED ? VC_QUARTER : d.lanes;
             d.guard.max_len = stride - VC_LINE + 1;

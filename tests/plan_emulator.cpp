@@ -394,15 +394,16 @@ extern "C" int64_t staging_allocate(int w, int w2, int msd, int coalesce, const 
 // left the hint (valid, items, payload, max_pieces, max_len).  out: lanes, stride, stride_lanes, guard.max_pieces,
 // guard.max_items, guard.max_average, guard.max_len.  Returns the schedule's error code.
 extern "C" int dispatch_decision(int func, int P, int n, int r, int mode, int call_kind, int valid, int64_t items, int64_t payload,
-                                 int64_t max_pieces, int64_t max_len, int64_t *out) {
+                                 int64_t max_pieces, int64_t max_len, int window, int64_t *out) {
     VcSched S;
     std::vector<VcLaunchInfo> L;
     const int code = vc_make_schedule((VcFunc)func, P, n, r, 0, 1, 0, S, L, 0, true);
     if (code) return code;
+    S.window = window && vc_may_stage(S) ? VC_STAGE_WINDOW : 0;      // (make_schedule in csrc/vc_api.hip)
     const VcHint h = {valid, items, payload, max_pieces, max_len};
     const VcDispatch d = vc_dispatch(mode, call_kind, h, S);
     out[0] = d.lanes; out[1] = d.stride; out[2] = d.stride_lanes; out[3] = d.guard.max_pieces; out[4] = d.guard.max_items;
-    out[5] = d.guard.max_average; out[6] = d.guard.max_len;
+    out[5] = d.guard.max_average; out[6] = d.guard.max_len; out[7] = d.batch;
     return 0;
 }
 

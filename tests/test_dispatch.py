@@ -80,3 +80,25 @@ def test_lanes_per_work_item_of_the_list_kernels():
     for average, lanes in ((16, QUARTER), (447, QUARTER), (448, WAVE), (3071, WAVE), (3072, GROUP), (4096, GROUP)):
         assert E.lanes_for_items(average * 1000, 1000) == lanes
     assert E.lanes_for_items(0, 0) == GROUP
+
+
+# calls that stage in a window: quarters further up (one launch up to 192 ranks), batches further up from 512 ranks, any room for the fixed slots
+WINDOW_TABLE = {
+    32: [(WAVE, True), (WAVE, True), (WAVE, True), (WAVE, True), (GROUP, True), (LIST, False)],
+    64: [(QUARTER, True), (QUARTER, True), (QUARTER, True), (WAVE, True), (GROUP, True), (LIST, False)],
+    128: [(QUARTER, True), (QUARTER, True), (QUARTER, True), (QUARTER, True), (GROUP, True), (LIST, False)],
+    192: [(BATCH, True), (QUARTER, True), (QUARTER, True), (QUARTER, True), (LIST, False), (LIST, False)],
+    256: [(BATCH, False), (QUARTER, False), (QUARTER, False), (LIST, False), (LIST, False), (LIST, False)],
+    1024: [(BATCH, False), (BATCH, False), (QUARTER, False), (LIST, False), (LIST, False), (LIST, False)],
+}
+
+
+@pytest.mark.parametrize("P", sorted(WINDOW_TABLE))
+def test_decision_table_of_calls_that_stage_in_a_window(P):
+    for (name, h), (lanes, strided) in zip(HINTS.items(), WINDOW_TABLE[P]):
+        d = E.dispatch(E.F_TWOPHASE, P, _hint(P, *h), mode=1, r=2, window=True)
+        assert (d["lanes"], d["stride"] > 0) == (lanes, strided), (P, name, d)
+        assert E.dispatch(E.F_TWOPHASE, P, _hint(P, *h), window=True, batch=True) == (64 if h[2] <= 128 else 16)
+        # a direct function stages nothing: the same with and without
+        assert E.dispatch(E.F_SPREADOUT, P, _hint(P, *h), window=True) == E.dispatch(E.F_SPREADOUT, P, _hint(P, *h)), (P, name)
+    assert [E.dispatch(E.F_TWOPHASE, P, _hint(P, 60, 1, longest), window=True, batch=True) for longest in (128, 129)] == [64, 16]

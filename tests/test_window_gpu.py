@@ -34,6 +34,9 @@ CASES = {
     "one byte too long for a lane": ("twophase_rbruck_alltoallv", (3,), (np.arange(260 * 260).reshape(260, 260) % 130).astype(np.int32), 1, 1),
     "direct, a lane a block": ("spreadout_alltoallv", (), (np.arange(260 * 260).reshape(260, 260) % 43).astype(np.int32), 3, 1),
     "one launch": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(4).integers(0, 2500, (100, 100)).astype(np.int32), 1, 1),
+    "one launch, workgroups in a window": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(6).integers(0, 30_000, (41, 41)).astype(np.int32), 1, 1),
+    "one launch, wavefronts in a window": ("tuna_algorithm", (2, 0), np.random.default_rng(7).integers(0, 1700, (100, 100)).astype(np.int32), 3, 1),
+    "one launch, quarters": ("TTPL_BT_alltoallv", (48, 2, 0), np.random.default_rng(8).integers(0, 1200, (192, 192)).astype(np.int32), 4, 0),
     "one launch that signals its end": ("twophase_rbruck_alltoallv_om", (2,), np.random.default_rng(4).integers(0, 12_000, (31, 31)).astype(np.int32), 1, 1),
 }
 

@@ -202,6 +202,7 @@ struct PlanInfo {
     int batches = 1;                                // launches of forwarded execution
     int recv_lo = 0;
     int window = 0;                                 // VcSched::window
+    bool cached = false;                            // vc_reads_cached
     int64_t stage_bytes = 0, payload_bytes = 0;
     std::vector<int64_t> first, count, bytes;       // per launch: first work item, item count, bytes moved
     std::vector<char> inter;                        // per launch: its messages cross nodes
@@ -320,6 +321,7 @@ static int plan_read(vc_comm *c, const VcSched &S, const std::vector<VcLaunchInf
     if (forward) {
         out.bytes[0] = h[VC_HEADER_FIXED];
         out.chain = true;
+        out.cached = vc_reads_cached(S, out.payload_bytes);
         out.chain_stride = VC_CHAIN_HEAD + vc_hop_slots(S);
         out.chain_items = h[2];
         out.chain_lanes = vc_lanes_for_items(out.payload_bytes, out.chain_items);      // every chain item carries one piece of the payload
@@ -379,7 +381,7 @@ static int launch_items(vc_comm *c, const PlanInfo &pi, const void *items_any, c
     if (c->stage.cap < (size_t)pi.stage_bytes + 64) return fail_arg("staging arena smaller than the plan needs");
     if (pi.chain) {
         HIP_TRY(vc_launch_copy_chains(static_cast<const int64_t *>(items_any), pi.chain_stride, pi.chain_items,
-                                      pi.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), c->stream, pi.window));
+                                      pi.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), c->stream, pi.window, pi.cached));
         return VC_OK;
     }
     const VcDesc *items = static_cast<const VcDesc *>(items_any);
@@ -503,7 +505,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     // the tables have been found in order
     const auto launch = [&](hipStream_t, VcSignal sig) {
         const hipError_t e = vc_launch_copy_blocks(S, T, nullptr, nullptr, nullptr, guard, pair_lanes, sendbuf, recvbuf, c->stage.as<char>(), st, verdict,
-                                                   verdict_next, c->h_header_dev + VC_TOTALS_AT, sig);
+                                                   verdict_next, c->h_header_dev + VC_TOTALS_AT, sig, d.batch, d.cached);
         if (e == hipSuccess) c->verdict_clean = true;
         return e;
     };
@@ -559,12 +561,13 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
     if (c->hint.items > 2 * c->items_before_last) return 2;
     hipStream_t st = c->stream;
     const int lanes = vc_lanes_for_items(c->hint.payload, c->hint.items);
+    const bool cached = vc_reads_cached(S, c->hint.payload);
     HIP_TRY(vc_launch_chain_plan(S, T, c->B.slot_lines(), c->B.row_base, c->B.chain_row_base, c->B.chain_row_tot, c->desc.as<int64_t>(), guess, st,
                                  c->B.header, guard.cap_items));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     int64_t done = 0;                                     // items the guarded launch was sized for
     HIP_TRY(vc_launch_copy_chains_guarded(c->desc.as<int64_t>(), stride, guess, lanes, sendbuf, recvbuf, c->stage.as<char>(), st, c->B.header,
-                                          guard, &done, S.window));
+                                          guard, &done, S.window, cached));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     HIP_TRY(VC_WAIT(c));
     int rc = plan_read(c, S, L, pi, true);
@@ -573,7 +576,7 @@ static int try_enqueued_list(vc_comm *c, const VcSched &S, std::vector<VcLaunchI
     pi.chain_lanes = lanes;
     if (pi.chain_items > done) {                          // more pieces than the last call had
         HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>() + done * stride, stride, pi.chain_items - done, lanes, sendbuf, recvbuf,
-                                      c->stage.as<char>(), st, S.window));
+                                      c->stage.as<char>(), st, S.window, cached));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
         HIP_TRY(VC_WAIT(c));
     }
@@ -620,7 +623,7 @@ static int run_batches(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, VcTa
         if (rc) return rc;
         if (c->timing) HIP_TRY(hipEventRecord(c->events[2 + 2 * b], st));
         HIP_TRY(vc_launch_copy_chains(c->desc.as<int64_t>(), pi.chain_stride, pi.chain_items, all.chain_lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
-                                      S.window));
+                                      S.window, all.cached));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3 + 2 * b], st));
         all.bytes[b] = pi.bytes[0];
     }
@@ -682,7 +685,7 @@ static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &
         if (rc) return rc;
         if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
         HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header, guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
-                                      nullptr, nullptr, nullptr, VcSignal(), d.batch));
+                                      nullptr, nullptr, nullptr, VcSignal(), d.batch, d.cached));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
         HIP_TRY(VC_WAIT(c));
         PlanInfo pi;
@@ -710,7 +713,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     S.recv_lo = (int)((uintptr_t)recvbuf & 4095);
     PlanInfo pi;
     hipStream_t st = c->stream;
-    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, false, 0, {0, 0, 0, 0, 0}};
+    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, false, 0, false, {0, 0, 0, 0, 0}};
     const int pair_lanes = d.lanes;
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;
@@ -736,7 +739,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
                 HIP_TRY(hipEventRecord(c->events[2], st));
             }
             HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, pair_lanes, sendbuf, recvbuf,
-                                          c->stage.as<char>(), st, nullptr, nullptr, nullptr, VcSignal(), d.batch));
+                                          c->stage.as<char>(), st, nullptr, nullptr, nullptr, VcSignal(), d.batch, d.cached));
             if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
             HIP_TRY(VC_WAIT(c));
             synced = true;
@@ -807,7 +810,7 @@ static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, st
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
         HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
-                                      nullptr, nullptr, nullptr, VcSignal(), d.batch));
+                                      nullptr, nullptr, nullptr, VcSignal(), d.batch, d.cached));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
     return VC_OK;
@@ -831,7 +834,7 @@ static int enqueue_async(vc_comm *c, const CallParams &q, const VcSched &S, std:
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     if (lanes)
         HIP_TRY(vc_launch_copy_blocks(S, T, c->B.slot_lines(), c->B.row_base, c->B.header, guard, lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
-                                      nullptr, nullptr, nullptr, VcSignal(), d.batch));
+                                      nullptr, nullptr, nullptr, VcSignal(), d.batch, d.cached));
     if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
     keep_pending(c, q, S, L, sendbuf, recvbuf, T, lanes, guard);
     return VC_OK;
@@ -887,7 +890,7 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
         const bool tables = !plans_without_tables(S);
         HIP_TRY(vc_launch_copy_blocks(S, c->pending.T, tables ? c->B.slot_lines() : nullptr, tables ? c->B.row_base : nullptr, c->header, guard, lanes,
                                       c->pending.sendbuf, c->pending.recvbuf, c->stage.as<char>(), c->stream, nullptr,
-                                      nullptr, nullptr, VcSignal(), d.batch));
+                                      nullptr, nullptr, VcSignal(), d.batch, d.cached));
         if (c->timing) HIP_TRY(hipEventRecord(c->events[3], c->stream));
         HIP_TRY(VC_WAIT(c));
     }
@@ -1053,7 +1056,7 @@ extern "C" int twophase_rbruck_alltoallv_noalloc(int r, char *sendbuf, int *send
     const VcDispatch d = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S);
     const int lanes = d.lanes;
     HIP_TRY(vc_launch_copy_blocks(S, T, B.slot_lines(), B.row_base, B.header, guard, lanes, sendbuf, recvbuf, stage, c->stream, nullptr, nullptr,
-                                  nullptr, VcSignal(), d.batch));
+                                  nullptr, VcSignal(), d.batch, d.cached));
     HIP_TRY(VC_WAIT(c));
     PlanInfo pi;
     rc = plan_read(c, S, L, pi, true);

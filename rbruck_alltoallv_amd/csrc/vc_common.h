@@ -290,9 +290,9 @@ hipError_t vc_launch_traffic(const VcDesc *desc, int64_t ndesc, int64_t *matrix,
 // a wavefront, for lists of pieces of a few hundred bytes)
 hipError_t vc_launch_copy_items(const VcDesc *items, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf, char *stage,
                                 hipStream_t st);
-// window: VcSched::window of the plan the list was made for
+// window: VcSched::window of the plan the list was made for; cached: vc_reads_cached
 hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf,
-                                 char *stage, hipStream_t st, int window = 0);
+                                 char *stage, hipStream_t st, int window, bool cached);
 // What the plan of a call must look like for a list and a copy launch that were enqueued right behind the planning kernel,
 // before the host had seen the plan, to do their work.  Kernels and host evaluate it on the same header, so both agree on
 // whether anything was moved.
@@ -312,7 +312,7 @@ VC_HD bool vc_chain_guard_ok(const int64_t *header, const VcChainGuard &g) {
 // (header[2] items exist).  Items beyond `covered` (grid_items, or what one launch holds) are left for a second, ordinary launch.
 hipError_t vc_launch_copy_chains_guarded(const int64_t *items, int stride, int64_t grid_items, int lanes, const char *sendbuf,
                                          char *recvbuf, char *stage, hipStream_t st, const int64_t *header, VcChainGuard guard, int64_t *covered,
-                                         int window);
+                                         int window, bool cached);
 // What the plan of a call must look like for the listless kernels to run it; 0 = no limit.  The kernels evaluate it on
 // the device header, the host on its copy after the synchronisation: both then agree on whether anything was moved.
 struct VcListlessGuard {
@@ -348,6 +348,6 @@ VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  unsigned long long *verdict = nullptr, unsigned long long *verdict_next = nullptr,
-                                 int64_t *totals = nullptr, VcSignal sig = VcSignal(), int batch = 16);
+                                 int64_t *totals = nullptr, VcSignal sig = VcSignal(), int batch = 16, bool cached = false);
 // dst2 non-null: every vector is stored twice (one read, two writes)
 hipError_t vc_launch_calibration_copy(const char *src, char *dst, char *dst2, int64_t nbytes, hipStream_t st);

@@ -23,12 +23,16 @@
 #include "vc_plan_math.h"
 #include "vc_scan.h"
 
+#include <type_traits>
+
 typedef unsigned int vc_u32x4 __attribute__((ext_vector_type(4)));
 struct __attribute__((packed, aligned(1))) VcU128 { vc_u32x4 v; };
 
-// 16-byte load from any byte address (one global_load_dwordx4; the hardware handles the misalignment)
-__device__ __forceinline__ vc_u32x4 vc_load16(const char *p) {
-    return __builtin_nontemporal_load(&reinterpret_cast<const VcU128 *>(p)->v);
+// 16-byte load from any byte address (one global_load_dwordx4; the hardware handles the misalignment).  CACHED: an ordinary one, served by the
+// memory-side cache when the caller, or the last call, has left the input there, and leaving it there; see vc_reads_cached.
+template <bool CACHED> __device__ __forceinline__ vc_u32x4 vc_load16(const char *p) {
+    const vc_u32x4 *const v = &reinterpret_cast<const VcU128 *>(p)->v;
+    return CACHED ? reinterpret_cast<const VcU128 *>(p)->v : __builtin_nontemporal_load(v);
 }
 
 // 16-byte store to a 16-byte aligned address
@@ -77,7 +81,7 @@ __device__ __forceinline__ char *vc_resolve(int64_t loc, const char *sendbuf, ch
 #define VC_WAIT_VMCNT0 0x0F70              // s_waitcnt vmcnt(0): loads have arrived and stores have been acknowledged
 struct VcAlwaysGo { __device__ __forceinline__ bool operator()() const { return true; } };
 
-template <int LANES, bool THROUGH, bool WINDOW, class NextDst, class Go = VcAlwaysGo>
+template <int LANES, bool THROUGH, bool WINDOW, bool CACHED, class NextDst, class Go = VcAlwaysGo>
 __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, int nhop, int w, NextDst next_dst, Go go = Go()) {
     constexpr int VECS = VC_CHUNK / 16 / LANES;           // window vectors per lane: 2 for a workgroup of 256, 8 for one wavefront
     const int t = threadIdx.x;
@@ -90,7 +94,7 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
         constexpr int WHOLE = VC_PIECE / 16 / LANES;
         vc_u32x4 v[WHOLE];
 #pragma unroll
-        for (int i = 0; i < WHOLE; i++) v[i] = vc_load16(src + ((t + i * LANES) << 4));
+        for (int i = 0; i < WHOLE; i++) v[i] = vc_load16<CACHED>(src + ((t + i * LANES) << 4));
         if (!go()) return;
         for (int k = 0; k < nhop; k++) {
             char *dst = next_dst();
@@ -110,7 +114,7 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
     for (int i = 0; i < VECS; i++) {
         const int j = t + i * LANES;
         has[i] = (i > 0 || j >= first_full) && j < end_full;
-        if (has[i]) v[i] = vc_load16(sw + (j << 4));
+        if (has[i]) v[i] = vc_load16<CACHED>(sw + (j << 4));
     }
     int head = (first_full << 4) - w;
     if (head > n) head = n;
@@ -138,7 +142,7 @@ __device__ __forceinline__ void vc_forward_piece(const char *src, int64_t len, i
 // GUARDED: the launch was enqueued before the host had seen the plan (see VcChainGuard): `nitems` is a guess, header[2] the
 // truth, and nothing moves unless the plan is one this launch can serve.
 // WINDOW: the plan stages in a window of `window` bytes.
-template <int LANES, bool GUARDED, bool WINDOW>
+template <int LANES, bool GUARDED, bool WINDOW, bool CACHED>
 __global__ __launch_bounds__(LANES) void vc_copy_chains_kernel(const int64_t *__restrict__ items, int stride, unsigned nitems,
                                                                const char *__restrict__ sendbuf, char *__restrict__ recvbuf,
                                                                char *__restrict__ stage, const int64_t *__restrict__ header,
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_chains_kernel(const int64_t *__
     int64_t word = 0;
     if (lane < nhop) word = it[VC_CHAIN_HEAD + lane];
     int at = 0;
-    vc_forward_piece<LANES, false, WINDOW>(src, len, nhop, w, [&]() {
+    vc_forward_piece<LANES, false, WINDOW, CACHED>(src, len, nhop, w, [&]() {
         const unsigned lo = __builtin_amdgcn_readlane((int)word, at), hi = __builtin_amdgcn_readlane((int)(word >> 32), at);
         return at++ ? vc_resolve((int64_t)hi << 32 | lo, sendbuf, recvbuf, stage, mask) : dst;
     });
@@ -178,14 +182,14 @@ __global__ __launch_bounds__(LANES) void vc_copy_items_kernel(const VcDesc *__re
     const VcDesc d = items[idx];
     if (d.len <= 0) return;
     char *dst = vc_resolve(d.dst, sendbuf, recvbuf, stage);
-    vc_forward_piece<LANES, false, false>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, (int)((uintptr_t)dst & (VC_LINE - 1)), [&]() { return dst; });
+    vc_forward_piece<LANES, false, false, false>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, (int)((uintptr_t)dst & (VC_LINE - 1)), [&]() { return dst; });
 }
 
 // A quarter of a wavefront (16 lanes) per item, four items per wavefront, for lists of pieces of a few hundred bytes:
 // such a launch is bound by how many items are in flight, not by HBM, and a piece of 100 bytes has work for 7 lanes.
 // Every group of 16 lanes reads its own item; lane t of the group owns window vectors t, t + 16 of every 512-byte pass
 // (most items need one pass; longer ones loop), and moves head byte t and tail byte t.
-template <bool WINDOW, class DstOf>
+template <bool WINDOW, bool CACHED, class DstOf>
 __device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_t len, int nhop, DstOf dst_of) {
     const int t = threadIdx.x & 15;
     char *dst = dst_of(0);
@@ -204,8 +208,8 @@ __device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_
     for (int64_t j = t; first_pass || j < end_full; j += 32) {     // always one, also for a block without a full vector
         const bool has0 = j >= first_full && j < end_full, has1 = j + 16 >= first_full && j + 16 < end_full;
         vc_u32x4 v0, v1;
-        if (has0) v0 = vc_load16(sw + (j << 4));
-        if (has1) v1 = vc_load16(sw + ((j + 16) << 4));
+        if (has0) v0 = vc_load16<CACHED>(sw + (j << 4));
+        if (has1) v1 = vc_load16<CACHED>(sw + ((j + 16) << 4));
         for (int k = 0; k < nhop; k++) {
             if (k || !first_pass) dst = dst_of(k);
             char *dw = dst - w;
@@ -279,7 +283,7 @@ __device__ __forceinline__ void vc_lane_store(const VcLaneBlock &b, char *dst, i
 // A piece moved by LANES neighbouring lanes of a wavefront: lane t owns window vectors t, t + LANES, ... (the window starts at the
 // cache line of the destination, `w` bytes before it), VECS of them in flight at once.  Staging without a window is stored past the
 // caches (nothing reads it again); recvbuf is not: a line that two neighbouring blocks share is then put together in the L2.
-template <int LANES, int VECS, bool WINDOW, class DstOf, class Go = VcAlwaysGo>
+template <int LANES, int VECS, bool WINDOW, bool CACHED, class DstOf, class Go = VcAlwaysGo>
 __device__ __forceinline__ void vc_forward_short(const char *src, int len, int nhop, int w, DstOf dst_of, Go go = Go()) {
     const int t = threadIdx.x % LANES;
     if (len < 16) {
@@ -298,7 +302,7 @@ __device__ __forceinline__ void vc_forward_short(const char *src, int len, int n
         for (int i = 0; i < VECS; i++) {
             const int lo = ((j0 + i * LANES) << 4) - w;
             at[i] = lo <= -16 || lo >= len ? -1 : (lo < 0 ? 0 : (lo > len - 16 ? len - 16 : lo));
-            if (at[i] >= 0) v[i] = vc_load16(src + at[i]);
+            if (at[i] >= 0) v[i] = vc_load16<CACHED>(src + at[i]);
         }
         if (j0 == t && !go()) return;
         for (int k = 0; k < nhop - 1; k++) {
@@ -322,7 +326,7 @@ __device__ __forceinline__ void vc_forward_short(const char *src, int len, int n
 // gridDim.x wavefronts, a multiple of VC_XCDS; XCD k works through the k-th eighth of them, each taking four items in a row
 // `rounds`: groups of four items in a row a wavefront takes, one after the other (long lists of very short pieces: fewer
 // wavefronts, each paying its start-up once for more items)
-template <bool GUARDED, bool WINDOW>
+template <bool GUARDED, bool WINDOW, bool CACHED>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_chains_quarter_kernel(const int64_t *__restrict__ items, int stride, unsigned nitems,
                                                                          int rounds, const char *__restrict__ sendbuf,
                                                                          char *__restrict__ recvbuf, char *__restrict__ stage,
@@ -339,7 +343,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_chains_quarter_kernel(const i
         const int nhop = (int)it[VC_CHAIN_NHOP];
         if (len <= 0 || nhop <= 0) continue;
         const int64_t mask = WINDOW ? vc_window_mask(window) : -1;
-        vc_forward_piece_quarter<WINDOW>(vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage), len, nhop,
+        vc_forward_piece_quarter<WINDOW, CACHED>(vc_resolve(it[VC_CHAIN_SRC], sendbuf, recvbuf, stage), len, nhop,
                                          [&](int k) { return vc_resolve(it[VC_CHAIN_HEAD + k], sendbuf, recvbuf, stage, mask); });
     }
 }
@@ -355,7 +359,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_items_quarter_kernel(const Vc
         const VcDesc d = items[idx];
         if (d.len <= 0) continue;
         char *dst = vc_resolve(d.dst, sendbuf, recvbuf, stage);
-        vc_forward_piece_quarter<false>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, [&](int) { return dst; });
+        vc_forward_piece_quarter<false, false>(vc_resolve(d.src, sendbuf, recvbuf, stage), d.len, 1, [&](int) { return dst; });
     }
 }
 
@@ -495,7 +499,7 @@ __device__ __forceinline__ bool vc_pair_allowed(const VcSched &S, const VcPairRe
 // Everything the block's addresses depend on is read before the planner's verdict is looked at: the reads are
 // independent of each other and of the verdict (tables are always readable), so they travel together instead of one
 // memory round trip after the other; nothing is stored before the verdict is known.
-template <int LANES, bool SELF, bool WINDOW>
+template <int LANES, bool SELF, bool WINDOW, bool CACHED>
 __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T, const uint32_t *__restrict__ slot_off,
                                              const int64_t *__restrict__ row_base,
                                              const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -530,7 +534,7 @@ __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
         unsigned long long left = moves;
-        vc_forward_piece<LANES, SELF, WINDOW>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
+        vc_forward_piece<LANES, SELF, WINDOW, CACHED>(src + lo, hi - lo, __popcll(moves), c ? 0 : phase,
                                 [&]() {
                                     const int k = __ffsll(left) - 1;
                                     left &= left - 1;
@@ -546,7 +550,7 @@ __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T
 // 32 ranks of 0 - 2 KiB 14.0 -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3.  The quarter kernel has no such instance: its lanes' short stores past the caches each
 // cost a write to memory (64 ranks, 1 KiB blocks: 16.6 -> 21.9 us).
 // WINDOW: S.window.
-template <int LANES, bool SELF, bool WINDOW>
+template <int LANES, bool SELF, bool WINDOW, bool CACHED>
 __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                const int64_t *__restrict__ row_base,
                                                                const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -554,7 +558,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
                                                                char *__restrict__ recvbuf, char *__restrict__ stage,
                                                                unsigned long long *verdict, unsigned long long *verdict_next,
                                                                int64_t *totals, VcSignal sig) {
-    vc_copy_pair<LANES, SELF, WINDOW>(S, T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, verdict, verdict_next, totals);
+    vc_copy_pair<LANES, SELF, WINDOW, CACHED>(S, T, slot_off, row_base, header, guard, first_pair, sendbuf, recvbuf, stage, verdict, verdict_next, totals);
     if (SELF) vc_signal(sig);
 }
 
@@ -563,7 +567,7 @@ __global__ __launch_bounds__(LANES) void vc_copy_blocks_kernel(VcSched S, VcTabl
 // Eight vectors of a lane in flight, 2 KiB a group: 87 VGPRs, 5 wavefronts per SIMD.  With four (62 VGPRs, 7) the loads of a second round
 // wait for the stores of the first: calls of blocks of 512 B - 2.5 KiB on average on 64 - 200 ranks 3 - 5 % slower (128 ranks, 2 KiB 33.0
 // us -> 34.2; 192 ranks, 600 B 38.3 -> 40.4), 1024 ranks, 700 B 596 -> 605, and only direct calls on 300 ranks faster (91.9 -> 89.9).
-template <bool WINDOW>
+template <bool WINDOW, bool CACHED>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                          const int64_t *__restrict__ row_base,
                                                                          const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -612,7 +616,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
     for (int64_t c = 0; c < pieces; c++) {
         int64_t lo, hi;
         vc_piece_range(len, phase, cut, c, lo, hi);
-        vc_forward_short<VC_QUARTER, 8, WINDOW>(src + lo, (int)(hi - lo), nhop, c ? 0 : phase,
+        vc_forward_short<VC_QUARTER, 8, WINDOW, CACHED>(src + lo, (int)(hi - lo), nhop, c ? 0 : phase,
                                                 [&](int k) { return vc_resolve(route[g][k] + lo, sendbuf, recvbuf, stage, WINDOW ? vc_window_mask(S.window) : -1); },
                                                 [&]() { return gate(); });
     }
@@ -628,7 +632,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
 // in a row, every block a quarter of a wavefront) -> 28; 0 - 64 bytes, calls 144 -> 82 (blocks of up to 32 bytes a lane before).
 // Two blocks of a quarter in flight at once make it slower (0 - 512 bytes, calls of 16 pairs a wavefront 202 us -> 240): the requests of a wavefront
 // queue up in the memory.
-template <int BATCH, bool WINDOW>
+template <int BATCH, bool WINDOW, bool CACHED>
 __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S, VcTables T, const uint32_t *__restrict__ slot_off,
                                                                        const int64_t *__restrict__ row_base,
                                                                        const int64_t *__restrict__ header, VcListlessGuard guard,
@@ -713,20 +717,27 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_batch_kernel(VcSched S
         for (int64_t c = 0; c < pieces; c++) {            // the same cuts as the chain items of this block
             int64_t lo, hi;
             vc_piece_range(blen, phase, cut, c, lo, hi);
-            vc_forward_short<VC_QUARTER, 4, WINDOW>(src + lo, (int)(hi - lo), b_nhop[b], c ? 0 : phase,
+            vc_forward_short<VC_QUARTER, 4, WINDOW, CACHED>(src + lo, (int)(hi - lo), b_nhop[b], c ? 0 : phase,
                                                     [&](int k) { return vc_resolve(dsts[k] + lo, sendbuf, recvbuf, stage, mask); });
         }
     }
 }
 
+// The instance of a kernel for calls with or without a window, with ordinary or non-temporal loads: `of` names it.
+template <class Of> static auto vc_instance(bool window, bool cached, Of of) {
+    const std::true_type yes;
+    const std::false_type no;
+    return window ? (cached ? of(yes, yes) : of(yes, no)) : (cached ? of(no, yes) : of(no, no));
+}
+
 template <int BATCH>
 static void vc_launch_batch(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
-                            VcListlessGuard guard, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st) {
+                            VcListlessGuard guard, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st, bool cached) {
     const int64_t ts = BATCH == 16 ? 4 : 8, waves = ((S.P + ts - 1) / ts) * ((S.P + BATCH / ts - 1) / (BATCH / ts));
     const size_t lds = sizeof(int64_t) * BATCH * (vc_hop_slots(S) + 2) + sizeof(int) * BATCH * 2;
     for (int64_t done = 0; done < waves; done += VC_MAX_GRID) {
         const int64_t now = waves - done < VC_MAX_GRID ? waves - done : VC_MAX_GRID;
-        const auto kernel = S.window ? vc_copy_blocks_batch_kernel<BATCH, true> : vc_copy_blocks_batch_kernel<BATCH, false>;
+        const auto kernel = vc_instance(S.window, cached, [](auto w, auto k) { return vc_copy_blocks_batch_kernel<BATCH, w(), k()>; });
         hipLaunchKernelGGL(kernel, dim3((unsigned)((now + VC_XCDS - 1) / VC_XCDS * VC_XCDS)), dim3(VC_WAVE), lds, st, S,
                            T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage);
     }
@@ -734,13 +745,13 @@ static void vc_launch_batch(const VcSched &S, VcTables T, const uint32_t *slot_o
 
 hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *slot_off, const int64_t *row_base, const int64_t *header,
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
-                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig, int batch) {
+                                 unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig, int batch, bool cached) {
     const int64_t npairs = (int64_t)S.P * S.P;
     if (sig.word && (!verdict || S.window || (lanes != VC_WAVE && lanes != VC_THREADS))) return hipErrorInvalidValue;
     if (lanes == VC_BATCHED) {
         if (verdict) return hipErrorInvalidValue;         // the batches are for more pairs than one launch with totals takes
         (batch == 64 ? vc_launch_batch<64> : vc_launch_batch<16>)(
-            S, T, slot_off, row_base, header, guard, sendbuf, recvbuf, stage, st);
+            S, T, slot_off, row_base, header, guard, sendbuf, recvbuf, stage, st, cached);
         return hipGetLastError();
     }
     const int64_t step = lanes == VC_QUARTER ? VC_MAX_GRID * VC_ITEMS_PER_WAVE : VC_MAX_GRID;
@@ -750,14 +761,14 @@ hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *s
         if (verdict && done) return hipErrorInvalidValue;    // the totals belong to a call that one launch takes
         const dim3 grid((unsigned)((units + VC_XCDS - 1) / VC_XCDS * VC_XCDS) + vc_totals_blocks(S, verdict, lanes == VC_THREADS ? VC_THREADS : VC_WAVE));
         if (lanes == VC_QUARTER) {
-            const auto kernel = S.window ? vc_copy_blocks_quarter_kernel<true> : vc_copy_blocks_quarter_kernel<false>;
+            const auto kernel = vc_instance(S.window, cached, [](auto w, auto k) { return vc_copy_blocks_quarter_kernel<w(), k()>; });
             hipLaunchKernelGGL(kernel, grid, dim3(VC_WAVE), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, verdict,
                                verdict_next, totals);
             continue;
         }
         const bool self = sig.word != nullptr;
-        const auto wave = self ? vc_copy_blocks_kernel<VC_WAVE, true, false> : (S.window ? vc_copy_blocks_kernel<VC_WAVE, false, true> : vc_copy_blocks_kernel<VC_WAVE, false, false>);
-        const auto workgroup = self ? vc_copy_blocks_kernel<VC_THREADS, true, false> : (S.window ? vc_copy_blocks_kernel<VC_THREADS, false, true> : vc_copy_blocks_kernel<VC_THREADS, false, false>);
+        const auto wave = self ? vc_copy_blocks_kernel<VC_WAVE, true, false, false> : vc_instance(S.window, cached, [](auto w, auto k) { return vc_copy_blocks_kernel<VC_WAVE, false, w(), k()>; });
+        const auto workgroup = self ? vc_copy_blocks_kernel<VC_THREADS, true, false, false> : vc_instance(S.window, cached, [](auto w, auto k) { return vc_copy_blocks_kernel<VC_THREADS, false, w(), k()>; });
         const auto kernel = lanes == VC_WAVE ? wave : workgroup;
         hipLaunchKernelGGL(kernel, grid, dim3(lanes), 0, st, S, T, slot_off, row_base, header, guard, done, sendbuf, recvbuf, stage, verdict,
                            verdict_next, totals, sig);
@@ -777,26 +788,26 @@ static unsigned vc_grid_for(int64_t items, int lanes) {
 // One launch of the list-driven kernel with LANES lanes per item, in the instance for calls with or without a window.
 template <bool GUARDED>
 static void vc_launch_chains_once(const int64_t *items, int stride, unsigned nitems, int lanes, const char *sendbuf, char *recvbuf, char *stage,
-                                  hipStream_t st, const int64_t *header, VcChainGuard guard, int window) {
+                                  hipStream_t st, const int64_t *header, VcChainGuard guard, int window, bool cached) {
     const dim3 grid(vc_grid_for(nitems, lanes));
     if (lanes == VC_QUARTER) {
-        const auto kernel = window ? vc_copy_chains_quarter_kernel<GUARDED, true> : vc_copy_chains_quarter_kernel<GUARDED, false>;
+        const auto kernel = vc_instance(window, cached, [](auto w, auto k) { return vc_copy_chains_quarter_kernel<GUARDED, w(), k()>; });
         hipLaunchKernelGGL(kernel, grid, dim3(VC_WAVE), 0, st, items, stride, nitems, vc_quarter_rounds(nitems), sendbuf, recvbuf, stage, header,
                            guard, window);
         return;
     }
-    const auto wave = window ? vc_copy_chains_kernel<VC_WAVE, GUARDED, true> : vc_copy_chains_kernel<VC_WAVE, GUARDED, false>;
-    const auto workgroup = window ? vc_copy_chains_kernel<VC_THREADS, GUARDED, true> : vc_copy_chains_kernel<VC_THREADS, GUARDED, false>;
+    const auto wave = vc_instance(window, cached, [](auto w, auto k) { return vc_copy_chains_kernel<VC_WAVE, GUARDED, w(), k()>; });
+    const auto workgroup = vc_instance(window, cached, [](auto w, auto k) { return vc_copy_chains_kernel<VC_THREADS, GUARDED, w(), k()>; });
     hipLaunchKernelGGL(lanes == VC_WAVE ? wave : workgroup, grid, dim3(lanes == VC_WAVE ? VC_WAVE : VC_THREADS), 0, st, items, stride, nitems, sendbuf,
                        recvbuf, stage, header, guard, window);
 }
 
 hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf,
-                                 char *stage, hipStream_t st, int window) {
+                                 char *stage, hipStream_t st, int window, bool cached) {
     const int64_t step = vc_items_per_launch(lanes);
     for (int64_t done = 0; done < nitems; done += step) {
         const int64_t now = nitems - done < step ? nitems - done : step;
-        vc_launch_chains_once<false>(items + done * stride, stride, (unsigned)now, lanes, sendbuf, recvbuf, stage, st, nullptr, VcChainGuard(), window);
+        vc_launch_chains_once<false>(items + done * stride, stride, (unsigned)now, lanes, sendbuf, recvbuf, stage, st, nullptr, VcChainGuard(), window, cached);
     }
     return hipGetLastError();
 }
@@ -804,12 +815,12 @@ hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitem
 // One launch (a guessed list longer than a launch holds is cut to what one holds; the rest is the caller's second launch).
 hipError_t vc_launch_copy_chains_guarded(const int64_t *items, int stride, int64_t grid_items, int lanes, const char *sendbuf,
                                          char *recvbuf, char *stage, hipStream_t st, const int64_t *header, VcChainGuard guard, int64_t *covered,
-                                         int window) {
+                                         int window, bool cached) {
     const int64_t step = vc_items_per_launch(lanes);
     const int64_t now = grid_items < step ? grid_items : step;
     *covered = now > 0 ? now : 0;
     if (now <= 0) return hipSuccess;
-    vc_launch_chains_once<true>(items, stride, (unsigned)now, lanes, sendbuf, recvbuf, stage, st, header, guard, window);
+    vc_launch_chains_once<true>(items, stride, (unsigned)now, lanes, sendbuf, recvbuf, stage, st, header, guard, window, cached);
     return hipGetLastError();
 }
 

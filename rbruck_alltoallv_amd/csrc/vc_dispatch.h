@@ -84,6 +84,7 @@ struct VcDispatch {
     int stride_lanes;        // ... with this many lanes per pair (the batches come without the totals: a quarter of a wavefront)
     bool self;               // ... that tells the host itself when it is done
     int batch;               // VC_BATCHED: pairs per wavefront
+    bool cached;             // vc_reads_cached
     VcListlessGuard guard;   // what the call must look like for the listless kernel to move anything, checked on the device
                              // against the plan (the hint is only a guess); stage_cap is the caller's to fill in
 };
@@ -106,8 +107,9 @@ VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 :
 // mode: vc_comm_set_forwarding (0 launch per digit, 1 the library's choice, 2 the list, 3 / 4 / 5 listless with a workgroup / a
 // quarter of a wavefront per pair / batches).  S: the call's schedule (ranks, digits, whether it has an organized region).
 inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const VcSched &S) {
-    VcDispatch d = {0, 0, 0, false, 0, {0, 0, 0, 0, 0}};
+    VcDispatch d = {0, 0, 0, false, 0, false, {0, 0, 0, 0, 0}};
     d.batch = vc_batch_pairs(h.valid ? h.max_len : VC_LANE_BLOCK + 1);
+    d.cached = h.valid && vc_reads_cached(S, h.payload);
     if (mode == 3) { d.lanes = VC_THREADS; return d; }
     if (mode == 4) { d.lanes = VC_QUARTER; return d; }
     if (mode == 5) { d.lanes = VC_BATCHED; return d; }

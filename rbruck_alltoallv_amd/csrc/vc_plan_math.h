@@ -225,6 +225,16 @@ VC_HD int64_t vc_strided_stage_bytes(const VcSched &S) { return (int64_t)(S.w + 
 // Whether any block of a call can make two hops, the first one into staging.
 VC_HD bool vc_may_stage(const VcSched &S) { return S.w + S.w2 + (S.last_hop == 1 && S.G > 1 ? 1 : 0) > 1; }
 
+// Whether a forwarded call reads its input with ordinary loads, which keep it in the memory-side cache (256 MiB), or non-temporal ones, which
+// take no room there and, of lines two blocks share, fetch both parts from memory.  What a program exchanges it has mostly just computed, or
+// exchanges again: as long as input, output and window are a part of that cache, ordinary loads find them there.  Calls, non-temporal / ordinary, three
+// inputs in turn: 150 ranks, payload 4 MiB 23.1 / 23.0, 16 33.4 / 27.0, 24 40.4 / 31.6, 32 44.7 / 48.0, 48 54.6 / 55.4; nothing staged, 16 MiB
+// 25.5 / 23.3, 24 29.5 / 25.4, 32 32.0 / 26.8, 48 39.7 / 41.2; 16 ranks, 24 MiB through the list 40.7 / 38.1; 64 ranks, 16 MiB, planned 20.3 / 17.0; 256
+// ranks, 0 - 600 B 36.8 / 31.1; one call alone on 24 MiB that a kernel has just written 52.5 / 42.9, after 1 GiB of other writes 50.7 / 53.2.
+#define VC_CACHED_STAGED ((int64_t)24 << 20)
+#define VC_CACHED_DIRECT ((int64_t)32 << 20)
+VC_HD bool vc_reads_cached(const VcSched &S, int64_t payload) { return payload <= (vc_may_stage(S) ? VC_CACHED_STAGED : VC_CACHED_DIRECT); }
+
 // Hops of block (s, t): the digit rounds it moves in, plus the hop that is no digit round (vc_block_hop's last slot).
 VC_HD int vc_block_hops(const VcSched &S, int s, int t) {
     if (s == t) return 1;

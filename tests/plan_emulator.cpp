@@ -403,7 +403,7 @@ extern "C" int dispatch_decision(int func, int P, int n, int r, int mode, int ca
     const VcHint h = {valid, items, payload, max_pieces, max_len};
     const VcDispatch d = vc_dispatch(mode, call_kind, h, S);
     out[0] = d.lanes; out[1] = d.stride; out[2] = d.stride_lanes; out[3] = d.guard.max_pieces; out[4] = d.guard.max_items;
-    out[5] = d.guard.max_average; out[6] = d.guard.max_len; out[7] = d.batch;
+    out[5] = d.guard.max_average; out[6] = d.guard.max_len; out[7] = d.batch; out[8] = d.cached;
     return 0;
 }
 

@@ -102,3 +102,10 @@ def test_decision_table_of_calls_that_stage_in_a_window(P):
         # a direct function stages nothing: the same with and without
         assert E.dispatch(E.F_SPREADOUT, P, _hint(P, *h), window=True) == E.dispatch(E.F_SPREADOUT, P, _hint(P, *h)), (P, name)
     assert [E.dispatch(E.F_TWOPHASE, P, _hint(P, 60, 1, longest), window=True, batch=True) for longest in (128, 129)] == [64, 16]
+
+
+def test_input_that_the_memory_side_cache_holds_is_read_with_ordinary_loads():
+    for mode, kind in ((0, 0), (1, 0), (2, 0), (3, 0), (5, 0), (1, 1)):
+        for func, limit in ((E.F_TWOPHASE, 24 << 20), (E.F_TTPL, 24 << 20), (E.F_SPREADOUT, 32 << 20)):
+            at = lambda payload, valid=1: E.dispatch(func, 64, (valid, 8192, payload, 2, 1 << 13), mode=mode, call_kind=kind, n=8, window=True, cached=True)
+            assert [at(0), at(limit), at(limit + 1), at(limit, valid=0)] == [True, True, False, False], (mode, func)

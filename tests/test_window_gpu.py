@@ -83,6 +83,32 @@ def test_staging_window(case):
     dp.comm.free()
 
 
+@pytest.mark.parametrize("limit,name,tun,P", [(24, "twophase_rbruck_alltoallv", (2,), 16), (24, "tuna_algorithm", (2, 0), 40), (24, "twophase_rbruck_alltoallv", (4,), 110),
+                                              (24, "TTPL_BT_alltoallv_s1", (10, 2, 0), 190), (24, "TTPL_BT_alltoallv", (32, 4, 0), 256), (24, "TTPL_rbruck_alltoallv", (12, 3), 300),
+                                              (24, "twophase_rbruck_alltoallv_om", (8,), 520), (32, "spreadout_alltoallv", (), 100), (32, "MPICH_intra_scattered", (0,), 310)])
+def test_calls_at_the_limit_of_ordinary_loads(limit, name, tun, P):
+    """Payloads just below and just above the limit, the input rewritten between the calls."""
+    from rbruck_alltoallv_amd import api
+    for payload in ((limit << 20) * 63 // 64, (limit << 20) * 65 // 64):
+        mean = payload // P ** 2
+        counts = np.random.default_rng(P).integers(mean - mean // 8, mean + mean // 8 + 1, (P, P)).astype(np.int32)
+        assert (int(counts.sum()) > limit << 20) == (payload > limit << 20)
+        prob = W.make_problem(counts, 1, 1, 0 if name == "TTPL_BT_alltoallv" else 1)
+        dp = api.DeviceProblem(prob)
+        ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+        for turn in range(4):
+            dp.fill_payload(0, turn, ds)
+            dr.fill_(0xEE)
+            assert getattr(api, name)(*tun, dp, ds, dr) == 0, dp.comm.error()
+            assert dp.verify(ds, dr, name == "TTPL_BT_alltoallv") == 0, (payload, turn)
+        if name in ("tuna_algorithm", "TTPL_BT_alltoallv"):
+            plan = api.Plan(name, dp, dr, n=tun[0] if "TTPL" in name else 0, r=tun[1] if "TTPL" in name else tun[0])
+            dr.fill_(0xEE)
+            assert plan.rc == 0 and plan.execute(ds, dr) == 0 and dp.verify(ds, dr, name == "TTPL_BT_alltoallv") == 0
+            plan.free()
+        dp.comm.free()
+
+
 def test_plan_with_a_window_in_a_graph():
     """Replays of a captured plan, with another call on the communicator between them, leave what an eager call leaves."""
     from rbruck_alltoallv_amd import api

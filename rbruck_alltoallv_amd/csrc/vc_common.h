@@ -292,7 +292,7 @@ hipError_t vc_launch_copy_items(const VcDesc *items, int64_t nitems, int lanes, 
                                 hipStream_t st);
 // window: VcSched::window of the plan the list was made for; cached: vc_reads_cached
 hipError_t vc_launch_copy_chains(const int64_t *items, int stride, int64_t nitems, int lanes, const char *sendbuf, char *recvbuf,
-                                 char *stage, hipStream_t st, int window, bool cached);
+                                 char *stage, hipStream_t st, int window = 0, bool cached = false);
 // What the plan of a call must look like for a list and a copy launch that were enqueued right behind the planning kernel,
 // before the host had seen the plan, to do their work.  Kernels and host evaluate it on the same header, so both agree on
 // whether anything was moved.

@@ -58,7 +58,7 @@ __device__ __forceinline__ void piece_load(const char *src, int64_t len, const c
         for (int i = 0; i < 2; i++) {
             const int64_t j = t + i * VC_THREADS;
             R.has[i] = (i > 0 || j >= first_full) && j < end_full;
-            if (R.has[i]) R.v[i] = vc_load16(sw + (j << 4));
+            if (R.has[i]) R.v[i] = vc_load16<false>(sw + (j << 4));
         }
     } else {
         const unsigned delta = (unsigned)((uintptr_t)sw & 15);

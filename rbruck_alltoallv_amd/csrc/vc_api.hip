@@ -474,8 +474,9 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     if (d.stride <= 0) return 0;
     const int pair_lanes = d.stride_lanes;
     S.stride = d.stride;
-    // (a wavefront or a workgroup per pair: while there is room a window would only save memory, and its kernels take 1 % longer)
-    if (pair_lanes != VC_QUARTER && vc_strided_stage_bytes(S) <= VC_STRIDED_MAX_BYTES) S.window = 0;
+    // (a wavefront or a workgroup per pair: what little data stages is stored past the caches where there is room; 64 ranks, 1.2 KB 17.9 us, in a
+    // window 18.9, 48 ranks, 4 KB 18.5 / 19.3, but 64 ranks, 4 KB 25.4 / 23.2, 128 ranks, 2 KiB 33.2 / 31.3)
+    if (pair_lanes != VC_QUARTER && c->hint.payload <= VC_STRIDED_PAST_CACHES && vc_strided_stage_bytes(S) <= VC_STRIDED_MAX_BYTES) S.window = 0;
     const int64_t need = vc_window_bytes(vc_strided_stage_bytes(S), S.window);
     hipStream_t st = c->stream;
     // two sets of words in turn: a launch counts in one, which must start from zero, and clears the other one for the next call
@@ -795,7 +796,8 @@ static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, st
     const bool stages = vc_may_stage(S);
     const VcDispatch d = vc_dispatch(c->forward, VC_CALL_LISTLESS_ONLY, c->hint, S);
     int lanes = c->hint.valid || !stages ? d.lanes : 0;
-    VcListlessGuard guard = {0, stages && (lanes == VC_QUARTER || lanes == VC_BATCHED) ? VC_LISTLESS_MAX_PIECES : 0, 0, 0, 0};
+    const int most = lanes == VC_QUARTER || lanes == VC_BATCHED ? VC_LISTLESS_MAX_PIECES : (lanes == VC_WAVE ? VC_LISTLESS_WG_MAX_PIECES : 0);
+    VcListlessGuard guard = {0, stages ? most : 0, 0, 0, 0};
     int64_t stage_bytes = 0;
     if (lanes) {
         bool fits;

@@ -15,10 +15,9 @@
 //  * ... a batch of 16 or 64 pairs per wavefront when the blocks are so short that working out the routes costs more than
 //    moving the bytes: on 192 - 2048 ranks 5 - 40 % faster than the quarter up to an average block of 256 bytes, even at
 //    512, 3 - 16 % slower beyond.  Not on at most 128 ranks, where batches would leave most of the chip without a wavefront.
-//  * ... for the functions that send every block straight to its destination (nothing is staged, the plan is the check of the
-//    tables) a quarter of a wavefront up to an average block of 3 KiB on at most 362 ranks: 150 ranks, 1 and 2 KiB 31 -> 24 and
-//    39 -> 36, 300 ranks 61 -> 60 and 97 -> 91; even on 512 ranks, where a list makes up for itself.
-//  * ... a wavefront (average piece below 3 KiB) or a workgroup per pair: at most 128 ranks and 32768 pieces (26 - 42
+//  * ... for calls that stage in a window, or nothing, a wavefront per pair on 46 ranks and more instead of the list, whatever the average
+//    block, while none is more than 16 pieces (vc_closed_wave_from); direct calls on up to 362 ranks a quarter below that.
+//  * ... else a wavefront (average piece below 3 KiB) or a workgroup per pair: at most 128 ranks and 32768 pieces (26 - 42
 //    against 40 - 57 through the list at 16 and 64 ranks with blocks up to 8 KB, 31 - 77 against 48 - 92 up to 32 KB; a few
 //    per cent at 128 ranks; at 256 ranks the list wins).
 //  * never without the list after a call with a block of more than 8 (quarter, batch) / 16 (wavefront, workgroup) pieces:
@@ -41,18 +40,18 @@
 #define VC_LISTLESS_MAX_PIECES 8              // pieces of one block: quarter of a wavefront per pair, batches
 #define VC_LISTLESS_WG_MAX_PIECES 16          // pieces of one block: wavefront or workgroup per pair
 #define VC_LISTLESS_QUARTER_BELOW 768         // average piece below which pairs get a quarter of a wavefront, more than 128 ranks
-// ... of calls that stage in a window, which need no plan tables then (vc_plan_check), more than 192 ranks; up to 192 ranks, in one launch,
-// VC_LISTLESS_WAVE_BELOW.  Calls, list / quarters, by average block: 140 ranks, 1 KB 41 / 35, 2.5 KB 59 / 52; 192 ranks, 1 KB 55 / 51, 2.5 KB 85 / 82; 512
-// ranks, 1 KB 203 / 185, 1.5 KB 262 / 262; 1024 ranks, 1 KB 593 / 572, 1.5 KB 808 / 819; 256 ranks, 1 KB 61 / 61, 1.5 KB 74 / 77.
+// ... of calls that stage in a window, which need no plan tables then (vc_plan_check), more than 192 ranks.  Calls, list / quarters, by average
+// block: 512 ranks, 1 KB 203 / 185, 1.5 KB 262 / 262; 1024 ranks, 1 KB 593 / 572, 1.5 KB 808 / 819; 256 ranks, 1 KB 61 / 61, 1.5 KB 74 / 77.
 #define VC_WINDOW_QUARTER_BELOW 1280
 // ... and batches from 512 ranks up: quarters / batches, 1024 ranks, 500 B 354 / 326, 700 B 435 / 439; 512 ranks, 500 B 129 / 121; 256 ranks, 700 B 51 / 49
 #define VC_WINDOW_BATCH_BELOW 640
 #define VC_WINDOW_BATCH_PAIRS (1 << 18)
 #define VC_LISTLESS_BATCH_BELOW 384           // average piece below which a wavefront takes a batch of pairs
-#define VC_LISTLESS_DIRECT_PAIRS (1 << 17)    // direct functions: a quarter of a wavefront per pair up to VC_LISTLESS_WAVE_BELOW
+#define VC_LISTLESS_DIRECT_PAIRS (1 << 17)    // 362 ranks
 #define VC_LISTLESS_WAVE_BELOW 3072           // average piece below which a pair gets a wavefront instead of a workgroup
 #define VC_LISTLESS_MAX_AVERAGE 4096          // a call the short-block kernels were chosen for must stay below this average
 #define VC_STRIDED_MAX_BYTES ((int64_t)256 << 20)
+#define VC_STRIDED_PAST_CACHES ((int64_t)12 << 20)     // payload up to which a single launch that could use a window does without
 #define VC_STRIDED_MAX_PAIRS 36864            // 192 ranks
 // the launch signals its own end: gains up to 32 ranks (32 ranks of 0 - 2 KiB 14.0 us -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3), is even
 // on 48 (0 - 4 KiB 17.0), and on 64 loses with cold caches what it gains with warm ones (0 - 4 KiB 23.2 -> 25.1, 21.5 -> 19.9): stores past
@@ -104,6 +103,28 @@ VC_HD int vc_window_stride(int64_t longest) {
 
 VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 : (pairs < 8192 ? 1792 : 3072); }
 
+// Calls whose slots have closed-form places (they stage in a window, or nothing) need no plan tables, and then a wavefront per pair of ranks
+// beats the list wherever there are pairs enough to fill the chip, as long as no block is many pieces: it takes up to 8 KiB of a block
+// at once, reads no items, and nothing has to be planned and written down before it.  Average pieces from vc_closed_wave_from on get one, below
+// vc_closed_quarter_below a quarter or less.  Microseconds a call by average block, before (list, workgroups or quarters) / a wavefront per pair:
+//   48 ranks, 4 KB 21.6 / 18.4, 10 KB 31.4 / 28.8;  64, 1.7 KB 21.0 / 18.2, 9 KB 50.6 / 44.8;  100, 2.5 KB 32.1 / 29.1, 9 KB 94 / 75;
+//   128, 4 KB 83 / 63, 20 KB 265 / 237;  160, 1.2 KB 49.8 / 44.1, 12 KB 189 / 173;  256, 2 KB 103 / 93, 12 KB 436 / 410;
+//   512, 2 KB 326 / 308, 7 KB 1037 / 955;  1024, 4 KB 1980 / 1949;  nothing staged: 128, 5 KB 70 / 47;  300, 2 KB 105 / 87;  800, 2.5 KB 660 / 598.
+// Fewer ranks: 34 ranks, 12 KB 24.0 / 30.3, 40 27.0 / 30.5 (but 4 KB 18.9 / 15.6); blocks of up to 40 pieces on 64 ranks 230 / 261.
+// The lines: a quarter / a wavefront, 64 ranks, 800 B 17.2 / 17.9, 1.2 KB 19.6 / 18.0; 128, 1.2 KB 30.3 / 31.7, 1.5 KB 33.5 / 31.9; 150, 1030 B 33.1 / 37.6, and
+// past what vc_reads_cached holds 1130 B 43.9 / 40.4; 192, 1030 B 58.7 / 57.5; nothing staged 160,
+// 1.5 KB 35.9 / 34.8; a list / a wavefront 256, 1.3 KB 77.3 / 79.4; 350, 1.5 KB 150 / 135; 512, 1.65 KB 282 / 281; 800, 1.5 KB 532 / 583; nothing staged 512,
+// 1.5 KB 174 / 201, 2.4 KB 274 / 245.  Beyond 192 ranks direct calls of longer pieces stay with the list (256 ranks, 4 KB 119 / 115, 512 407 / 398).
+#define VC_CLOSED_WAVE_PAIRS 2048             // 46 ranks
+VC_HD int64_t vc_closed_quarter_below(int64_t pairs, bool stages, bool cached) {
+    if (pairs > VC_STRIDED_MAX_PAIRS) return stages ? VC_WINDOW_QUARTER_BELOW : (pairs <= VC_LISTLESS_DIRECT_PAIRS ? 1664 : VC_LISTLESS_QUARTER_BELOW);
+    return pairs <= 1024 ? 0 : (pairs < 8192 ? 960 : (stages ? (cached ? 1280 : 1024) : 1664));
+}
+VC_HD int64_t vc_closed_wave_from(int64_t pairs, bool stages, bool cached) {
+    if (pairs <= VC_STRIDED_MAX_PAIRS) return vc_closed_quarter_below(pairs, stages, cached);
+    return pairs <= VC_LISTLESS_DIRECT_PAIRS ? (stages ? 1344 : 1664) : (stages ? 1664 : 1920);
+}
+
 // mode: vc_comm_set_forwarding (0 launch per digit, 1 the library's choice, 2 the list, 3 / 4 / 5 listless with a workgroup / a
 // quarter of a wavefront per pair / batches).  S: the call's schedule (ranks, digits, whether it has an organized region).
 inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const VcSched &S) {
@@ -118,24 +139,26 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
     const int64_t pairs = (int64_t)S.P * S.P;
     const bool small_comm = pairs <= VC_LISTLESS_MAX_PAIRS;
     const int64_t average = h.payload / (h.items > 0 ? h.items : 1);
-    const int64_t quarter_below = small_comm ? vc_small_quarter_below(pairs)
-                                             : (!S.window ? VC_LISTLESS_QUARTER_BELOW : (pairs <= VC_STRIDED_MAX_PAIRS ? VC_LISTLESS_WAVE_BELOW : VC_WINDOW_QUARTER_BELOW));
+    const bool stages = vc_may_stage(S), closed = S.window || !stages;      // closed: no plan tables, whatever the shape
+    const int64_t quarter_below = closed ? vc_closed_quarter_below(pairs, stages, d.cached) : (small_comm ? vc_small_quarter_below(pairs) : VC_LISTLESS_QUARTER_BELOW);
+    const bool wave = closed && h.valid && pairs >= VC_CLOSED_WAVE_PAIRS && h.max_pieces <= VC_LISTLESS_WG_MAX_PIECES &&
+                      average >= vc_closed_wave_from(pairs, stages, d.cached) && (stages || pairs <= VC_STRIDED_MAX_PAIRS || average < VC_LISTLESS_WAVE_BELOW);
     const bool short_blocks = h.valid && h.max_pieces <= VC_LISTLESS_MAX_PIECES && average < quarter_below;
     if (short_blocks)
         d.lanes = !small_comm && average < (S.window && pairs >= VC_WINDOW_BATCH_PAIRS ? VC_WINDOW_BATCH_BELOW : VC_LISTLESS_BATCH_BELOW) ? VC_BATCHED : VC_QUARTER;
     else if (listless_only)
-        d.lanes = VC_THREADS;
+        d.lanes = wave && average < VC_LISTLESS_WAVE_BELOW ? VC_WAVE : VC_THREADS;
+    else if (wave)
+        d.lanes = VC_WAVE;
     else if (h.valid && small_comm && h.max_pieces <= VC_LISTLESS_WG_MAX_PIECES && h.items <= VC_LISTLESS_MAX_ITEMS)
         d.lanes = average < VC_LISTLESS_WAVE_BELOW ? VC_WAVE : VC_THREADS;
-    else if (h.valid && S.w + S.w2 == 0 && pairs <= VC_LISTLESS_DIRECT_PAIRS && h.max_pieces <= VC_LISTLESS_MAX_PIECES && average < VC_LISTLESS_WAVE_BELOW)
-        d.lanes = VC_QUARTER;
     else
         return d;                                         // no hint yet, or long blocks: the list
     if (listless_only) return d;                          // nothing to fall back to: whatever the call turns out to be, it runs
     // the hint may be wrong about this call: the kernel leaves a call of another kind alone and the host takes the list
     const bool quarter = d.lanes == VC_QUARTER || d.lanes == VC_BATCHED;
     d.guard.max_pieces = quarter ? VC_LISTLESS_MAX_PIECES : VC_LISTLESS_WG_MAX_PIECES;
-    d.guard.max_items = quarter ? 0 : VC_LISTLESS_MAX_ITEMS;
+    d.guard.max_items = quarter || wave ? 0 : VC_LISTLESS_MAX_ITEMS;
     d.guard.max_average = quarter ? VC_LISTLESS_MAX_AVERAGE : 0;
     // one launch on fixed-stride staging: the stride from the last call's longest block, at any cache-line phase
     if (!S.coalesce && vc_hop_slots(S) <= VC_MAX_HOP_SLOTS && pairs <= VC_STRIDED_MAX_PAIRS) {

@@ -82,14 +82,17 @@ def test_lanes_per_work_item_of_the_list_kernels():
     assert E.lanes_for_items(0, 0) == GROUP
 
 
-# calls that stage in a window: quarters further up (one launch up to 192 ranks), batches further up from 512 ranks, any room for the fixed slots
+# calls that stage in a window: a wavefront per pair from 46 ranks up, whatever the average, instead of the list and of workgroups (up to 192 ranks in
+# one launch with any room for the slots); batches further up from 512 ranks
 WINDOW_TABLE = {
     32: [(WAVE, True), (WAVE, True), (WAVE, True), (WAVE, True), (GROUP, True), (LIST, False)],
-    64: [(QUARTER, True), (QUARTER, True), (QUARTER, True), (WAVE, True), (GROUP, True), (LIST, False)],
-    128: [(QUARTER, True), (QUARTER, True), (QUARTER, True), (QUARTER, True), (GROUP, True), (LIST, False)],
-    192: [(BATCH, True), (QUARTER, True), (QUARTER, True), (QUARTER, True), (LIST, False), (LIST, False)],
-    256: [(BATCH, False), (QUARTER, False), (QUARTER, False), (LIST, False), (LIST, False), (LIST, False)],
-    1024: [(BATCH, False), (BATCH, False), (QUARTER, False), (LIST, False), (LIST, False), (LIST, False)],
+    45: [(QUARTER, True), (QUARTER, True), (WAVE, True), (WAVE, True), (GROUP, True), (LIST, False)],
+    46: [(QUARTER, True), (QUARTER, True), (WAVE, True), (WAVE, True), (WAVE, True), (LIST, False)],
+    64: [(QUARTER, True), (QUARTER, True), (WAVE, True), (WAVE, True), (WAVE, True), (LIST, False)],
+    128: [(QUARTER, True), (QUARTER, True), (QUARTER, True), (WAVE, True), (WAVE, True), (LIST, False)],
+    192: [(BATCH, True), (QUARTER, True), (QUARTER, True), (WAVE, True), (WAVE, True), (LIST, False)],
+    256: [(BATCH, False), (QUARTER, False), (QUARTER, False), (WAVE, False), (WAVE, False), (LIST, False)],
+    1024: [(BATCH, False), (BATCH, False), (QUARTER, False), (WAVE, False), (WAVE, False), (LIST, False)],
 }
 
 
@@ -98,10 +101,28 @@ def test_decision_table_of_calls_that_stage_in_a_window(P):
     for (name, h), (lanes, strided) in zip(HINTS.items(), WINDOW_TABLE[P]):
         d = E.dispatch(E.F_TWOPHASE, P, _hint(P, *h), mode=1, r=2, window=True)
         assert (d["lanes"], d["stride"] > 0) == (lanes, strided), (P, name, d)
+        if lanes == WAVE and P >= 46:
+            assert (d["max_pieces"], d["max_items"], d["max_average"]) == (16, 0, 0)
         assert E.dispatch(E.F_TWOPHASE, P, _hint(P, *h), window=True, batch=True) == (64 if h[2] <= 128 else 16)
         # a direct function stages nothing: the same with and without
         assert E.dispatch(E.F_SPREADOUT, P, _hint(P, *h), window=True) == E.dispatch(E.F_SPREADOUT, P, _hint(P, *h)), (P, name)
     assert [E.dispatch(E.F_TWOPHASE, P, _hint(P, 60, 1, longest), window=True, batch=True) for longest in (128, 129)] == [64, 16]
+
+
+@pytest.mark.parametrize("func,P,lines", [(E.F_TWOPHASE, 90, [(0, QUARTER), (960, WAVE)]), (E.F_TWOPHASE, 128, [(768, QUARTER), (1280, WAVE)]),
+                                          (E.F_TWOPHASE, 192, [(768, QUARTER), (1024, WAVE)]), (E.F_TWOPHASE, 362, [(768, QUARTER), (1280, LIST), (1344, WAVE)]),
+                                          (E.F_TWOPHASE, 363, [(768, QUARTER), (1280, LIST), (1664, WAVE)]), (E.F_SPREADOUT, 64, [(0, QUARTER), (960, WAVE)]),
+                                          (E.F_SPREADOUT, 192, [(768, QUARTER), (1664, WAVE)]), (E.F_SPREADOUT, 362, [(768, QUARTER), (1664, WAVE), (3072, LIST)]),
+                                          (E.F_SPREADOUT, 363, [(384, QUARTER), (768, LIST), (1920, WAVE), (3072, LIST)])])
+def test_lines_of_calls_with_slots_in_closed_form(func, P, lines):
+    """A quarter of a wavefront, the list, a wavefront per pair: by the average piece, and by nothing else while no block is more than 8 pieces."""
+    for (line, lanes), before in zip(lines, [None] + [lanes for _, lanes in lines]):
+        if before is not None:
+            assert E.dispatch(func, P, _hint(P, line - 1, 8, 30000), window=True)["lanes"] == before, line
+        assert E.dispatch(func, P, _hint(P, line, 8, 30000), window=True)["lanes"] == lanes, line
+    # the _async twins, which never use the list
+    for average, pieces, lanes in ((2000, 16, WAVE), (2000, 17, GROUP), (3071, 16, WAVE), (3072, 16, GROUP)):
+        assert E.dispatch(func, P, _hint(P, average, pieces, 60000), window=True, call_kind=1)["lanes"] == lanes, (average, pieces)
 
 
 def test_input_that_the_memory_side_cache_holds_is_read_with_ordinary_loads():

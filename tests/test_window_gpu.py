@@ -33,6 +33,11 @@ CASES = {
     "a lane a block, every length": ("TTPL_BT_alltoallv_s1", (26, 5, 0), (np.arange(260 * 260).reshape(260, 260) % 129).astype(np.int32), 1, 1),
     "one byte too long for a lane": ("twophase_rbruck_alltoallv", (3,), (np.arange(260 * 260).reshape(260, 260) % 130).astype(np.int32), 1, 1),
     "direct, a lane a block": ("spreadout_alltoallv", (), (np.arange(260 * 260).reshape(260, 260) % 43).astype(np.int32), 3, 1),
+    "a wavefront a pair, no list": ("TTPL_BT_alltoallv", (23, 3, 0), np.random.default_rng(9).integers(0, 6_000, (207, 207)).astype(np.int32), 1, 0),
+    "a wavefront a pair, no list, up to 16 pieces": ("twophase_rbruck_alltoallv", (14,), np.where(np.arange(196 * 196).reshape(196, 196) % 61 == 0, 61_000, 3_001).astype(np.int32), 1, 1),
+    "a wavefront a pair, one launch, whole pieces": ("tuna_algorithm", (4, 0), _equal(46, 16384), 1, 0),
+    "a wavefront a pair, one launch, odd addresses": ("TTPL_BT_alltoallv_s1", (12, 3, 0), np.random.default_rng(10).integers(0, 20_000, (180, 180)).astype(np.int32), 1, 1),
+    "direct, a wavefront a pair": ("MPICH_intra_scattered", (0,), np.random.default_rng(11).integers(0, 4_500, (210, 210)).astype(np.int32), 1, 1),
     "one launch": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(4).integers(0, 2500, (100, 100)).astype(np.int32), 1, 1),
     "one launch, workgroups in a window": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(6).integers(0, 30_000, (41, 41)).astype(np.int32), 1, 1),
     "one launch, wavefronts in a window": ("tuna_algorithm", (2, 0), np.random.default_rng(7).integers(0, 1700, (100, 100)).astype(np.int32), 3, 1),

@@ -116,6 +116,17 @@ VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 :
 // 1.5 KB 35.9 / 34.8; a list / a wavefront 256, 1.3 KB 77.3 / 79.4; 350, 1.5 KB 150 / 135; 512, 1.65 KB 282 / 281; 800, 1.5 KB 532 / 583; nothing staged 512,
 // 1.5 KB 174 / 201, 2.4 KB 274 / 245.  Beyond 192 ranks direct calls of longer pieces stay with the list (256 ranks, 4 KB 119 / 115, 512 407 / 398).
 #define VC_CLOSED_WAVE_PAIRS 2048             // 46 ranks
+// Both lines are for calls of at least VC_CLOSED_WAVE_PER_PAIR bytes for every pair of ranks, the empty ones included: a wavefront that starts to find an
+// empty block costs as much as any (before / a wavefront per pair, rows of ranks that exchange among themselves: 128 ranks, 750 B a pair in blocks of 6 KB 39 / 23;
+// 400, 600 B 93 / 89; 600, 400 B 135 / 159; 1000, 300 B 271 / 401; 64 ranks, 375 B in blocks of 1.5 KB 15.8 / 16.7; nothing staged 100, 660 B 26 / 18; 256,
+// 660 B 39 / 39; 600, 730 B 126 / 139).
+#define VC_CLOSED_WAVE_PER_PAIR 640
+#define VC_CLOSED_DIRECT_PER_PAIR 1920        // more than 362 ranks, nothing staged
+VC_HD int64_t vc_closed_sparse_quarter_below(int64_t pairs, bool stages) {
+    if (pairs <= VC_LISTLESS_MAX_PAIRS) return vc_small_quarter_below(pairs);
+    if (pairs <= (stages ? VC_STRIDED_MAX_PAIRS : VC_LISTLESS_DIRECT_PAIRS)) return VC_LISTLESS_WAVE_BELOW;
+    return stages ? VC_WINDOW_QUARTER_BELOW : VC_LISTLESS_QUARTER_BELOW;
+}
 VC_HD int64_t vc_closed_quarter_below(int64_t pairs, bool stages, bool cached) {
     if (pairs > VC_STRIDED_MAX_PAIRS) return stages ? VC_WINDOW_QUARTER_BELOW : (pairs <= VC_LISTLESS_DIRECT_PAIRS ? 1664 : VC_LISTLESS_QUARTER_BELOW);
     return pairs <= 1024 ? 0 : (pairs < 8192 ? 960 : (stages ? (cached ? 1280 : 1024) : 1664));
@@ -140,8 +151,10 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
     const bool small_comm = pairs <= VC_LISTLESS_MAX_PAIRS;
     const int64_t average = h.payload / (h.items > 0 ? h.items : 1);
     const bool stages = vc_may_stage(S), closed = S.window || !stages;      // closed: no plan tables, whatever the shape
-    const int64_t quarter_below = closed ? vc_closed_quarter_below(pairs, stages, d.cached) : (small_comm ? vc_small_quarter_below(pairs) : VC_LISTLESS_QUARTER_BELOW);
-    const bool wave = closed && h.valid && pairs >= VC_CLOSED_WAVE_PAIRS && h.max_pieces <= VC_LISTLESS_WG_MAX_PIECES &&
+    const bool dense = h.payload >= (stages || pairs <= VC_LISTLESS_DIRECT_PAIRS ? VC_CLOSED_WAVE_PER_PAIR : VC_CLOSED_DIRECT_PER_PAIR) * pairs;
+    const int64_t quarter_below = closed ? (dense ? vc_closed_quarter_below(pairs, stages, d.cached) : vc_closed_sparse_quarter_below(pairs, stages))
+                                         : (small_comm ? vc_small_quarter_below(pairs) : VC_LISTLESS_QUARTER_BELOW);
+    const bool wave = closed && dense && h.valid && pairs >= VC_CLOSED_WAVE_PAIRS && h.max_pieces <= VC_LISTLESS_WG_MAX_PIECES &&
                       average >= vc_closed_wave_from(pairs, stages, d.cached) && (stages || pairs <= VC_STRIDED_MAX_PAIRS || average < VC_LISTLESS_WAVE_BELOW);
     const bool short_blocks = h.valid && h.max_pieces <= VC_LISTLESS_MAX_PIECES && average < quarter_below;
     if (short_blocks)

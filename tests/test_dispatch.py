@@ -120,6 +120,9 @@ def test_lines_of_calls_with_slots_in_closed_form(func, P, lines):
         if before is not None:
             assert E.dispatch(func, P, _hint(P, line - 1, 8, 30000), window=True)["lanes"] == before, line
         assert E.dispatch(func, P, _hint(P, line, 8, 30000), window=True)["lanes"] == lanes, line
+        if lanes == WAVE:                                 # rows of ranks: the same blocks, most pairs empty
+            kept = E.dispatch(func, P, (1, P * P // 8, line * (P * P // 8), 8, 30000), window=True)["lanes"]
+            assert kept == (QUARTER if line < (1792 if P < 91 else 3072 if P <= 192 or (func == E.F_SPREADOUT and P <= 362) else 1280) else LIST), line
     # the _async twins, which never use the list
     for average, pieces, lanes in ((2000, 16, WAVE), (2000, 17, GROUP), (3071, 16, WAVE), (3072, 16, GROUP)):
         assert E.dispatch(func, P, _hint(P, average, pieces, 60000), window=True, call_kind=1)["lanes"] == lanes, (average, pieces)

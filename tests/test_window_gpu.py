@@ -38,6 +38,8 @@ CASES = {
     "a wavefront a pair, one launch, whole pieces": ("tuna_algorithm", (4, 0), _equal(46, 16384), 1, 0),
     "a wavefront a pair, one launch, odd addresses": ("TTPL_BT_alltoallv_s1", (12, 3, 0), np.random.default_rng(10).integers(0, 20_000, (180, 180)).astype(np.int32), 1, 1),
     "direct, a wavefront a pair": ("MPICH_intra_scattered", (0,), np.random.default_rng(11).integers(0, 4_500, (210, 210)).astype(np.int32), 1, 1),
+    "nearly all of one hop, whole pieces": ("tuna_algorithm", (63, 0), _equal(64, 100_000), 1, 0),
+    "nearly all of one hop, odd addresses": ("twophase_rbruck_alltoallv", (100,), np.random.default_rng(12).integers(0, 12_000, (110, 110)).astype(np.int32), 1, 1),
     "one launch": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(4).integers(0, 2500, (100, 100)).astype(np.int32), 1, 1),
     "one launch, workgroups in a window": ("twophase_rbruck_alltoallv", (2,), np.random.default_rng(6).integers(0, 30_000, (41, 41)).astype(np.int32), 1, 1),
     "one launch, wavefronts in a window": ("tuna_algorithm", (2, 0), np.random.default_rng(7).integers(0, 1700, (100, 100)).astype(np.int32), 3, 1),

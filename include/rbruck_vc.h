@@ -77,9 +77,10 @@ int vc_comm_set_bases(vc_comm_t comm, const int64_t *sbase_bytes, const int64_t 
  *    device instead (tables, room in the list and in the staging arena, the staging bound: host_waits 1); a call they
  *    cannot serve has moved nothing and is redone the usual way, a longer list than guessed gets a second launch.
  *    When the last call on the communicator consisted of
- *    short blocks, the next one goes without the list: every pair of ranks gets a workgroup (at most 128 ranks) or a
- *    quarter of a wavefront (short blocks: average piece below 1280 B, without a window 768 B, on any number of ranks, below 1.75 - 3 KiB on 33 - 192) that derives its block's route itself; the
- *    kernel is enqueued right behind the size computation and the call needs one host synchronisation instead of two.
+ *    short blocks, or, with the default staging bound, of blocks of no more than 16 pieces on 46 ranks or more that most pairs have, the next one goes without the
+ *    list: every pair of ranks gets a workgroup or a wavefront, or a
+ *    quarter of a wavefront (average piece below about 1 - 1.3 KB, nothing staged 1 - 1.7 KB; with another staging bound 768 B, on up to 128 ranks 1.75 - 3 KiB) that derives
+ *    its block's route itself; the kernel is enqueued right behind the size computation and the call needs one host synchronisation instead of two.
  *    Such a call also gets the reference's own staging layout, every slot as long as the longest block
  *    (src/twophase_tunable_rbruckv.cpp:59; the stride comes from the last call's longest block): slot addresses are then
  *    closed forms and the call is a single kernel launch, without a planner before it.  Every pair of ranks checks its own
@@ -112,8 +113,8 @@ int vc_comm_set_forwarding(vc_comm_t comm, int enable);
  *    (hops - 1) x bytes (configuration 5 with radix 2: 60 GB);
  *  - forwarded execution in the default mode with the default bound (1) stages in a window of 32 MiB: a slot at offset x of the layout lies
  *    at x mod 32 MiB, piece by piece.  A piece makes its next hop out of the registers of the workgroup that staged it, so nothing reads
- *    what it left behind, and the window stays in the memory-side cache.  Calls on fixed-stride slots with a
- *    wavefront or a workgroup per pair of ranks have an arena of up to 256 MiB instead, if that holds them;
+ *    what it left behind, and the window stays in the memory-side cache.  Single launches with a
+ *    wavefront or a workgroup per pair of ranks and a payload of up to 12 MiB have an arena of up to 256 MiB instead, if that holds them;
  *  - forwarded execution in another mode or with an allowance keeps every hop's copy of every block in a place of its own.  A call whose
  *    staging would pass both the allowance (an eighth of the device's memory, at least
  *    1 GiB) and three times its payload is run in batches of receivers that use the same staging memory one after

@@ -474,9 +474,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     if (d.stride <= 0) return 0;
     const int pair_lanes = d.stride_lanes;
     S.stride = d.stride;
-    // (a wavefront or a workgroup per pair: what little data stages is stored past the caches where there is room; 64 ranks, 1.2 KB 17.9 us, in a
-    // window 18.9, 48 ranks, 4 KB 18.5 / 19.3, but 64 ranks, 4 KB 25.4 / 23.2, 128 ranks, 2 KiB 33.2 / 31.3)
-    if (pair_lanes != VC_QUARTER && c->hint.payload <= VC_STRIDED_PAST_CACHES && vc_strided_stage_bytes(S) <= VC_STRIDED_MAX_BYTES) S.window = 0;
+    S.window = d.stride_window;
     const int64_t need = vc_window_bytes(vc_strided_stage_bytes(S), S.window);
     hipStream_t st = c->stream;
     // two sets of words in turn: a launch counts in one, which must start from zero, and clears the other one for the next call
@@ -714,7 +712,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     S.recv_lo = (int)((uintptr_t)recvbuf & 4095);
     PlanInfo pi;
     hipStream_t st = c->stream;
-    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch{0, 0, 0, false, 0, false, {0, 0, 0, 0, 0}};
+    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch();
     const int pair_lanes = d.lanes;
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;

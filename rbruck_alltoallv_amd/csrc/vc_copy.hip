@@ -773,7 +773,7 @@ hipError_t vc_launch_copy_blocks(const VcSched &S, VcTables T, const uint32_t *s
                                  VcListlessGuard guard, int lanes, const char *sendbuf, char *recvbuf, char *stage, hipStream_t st,
                                  unsigned long long *verdict, unsigned long long *verdict_next, int64_t *totals, VcSignal sig, int batch, bool cached) {
     const int64_t npairs = (int64_t)S.P * S.P;
-    if (sig.word && (!verdict || S.window || (lanes != VC_WAVE && lanes != VC_THREADS))) return hipErrorInvalidValue;
+    if (sig.word && (!verdict || !vc_may_signal(lanes, S.window))) return hipErrorInvalidValue;
     if (lanes == VC_BATCHED) {
         if (verdict) return hipErrorInvalidValue;         // the batches are for more pairs than one launch with totals takes
         (batch == 64 ? vc_launch_batch<64> : vc_launch_batch<16>)(

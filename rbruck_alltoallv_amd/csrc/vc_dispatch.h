@@ -51,7 +51,12 @@
 #define VC_LISTLESS_WAVE_BELOW 3072           // average piece below which a pair gets a wavefront instead of a workgroup
 #define VC_LISTLESS_MAX_AVERAGE 4096          // a call the short-block kernels were chosen for must stay below this average
 #define VC_STRIDED_MAX_BYTES ((int64_t)256 << 20)
-#define VC_STRIDED_PAST_CACHES ((int64_t)12 << 20)     // payload up to which a single launch that could use a window does without
+// Payload up to which a single launch of wavefronts or workgroups that could use a window does without, where there is room: what little data stages is
+// stored past the caches.  64 ranks, 1.2 KB 17.9 us, in a window 18.9; 48 ranks, 4 KB 18.5 / 19.3; but 64 ranks, 4 KB 25.4 / 23.2, 128 ranks, 2 KiB
+// 33.2 / 31.3.  Up to 32 ranks the line also decides who signals its own end (VC_SELF_MAX_PAIRS).  Above it, signalled on slots of their own / in a window and
+// waited for: 16 ranks, 48 KB 25.7 / 25.5; 20 ranks, 32 KB 23.5 / 21.1, 0 - 68 KB 28.9 / 25.8; 24 ranks, 22 KB 21.4 / 20.3, 32 KB 25.8 / 23.2; 28 ranks, 12.5 KB 21.9 / 21.6;
+// 32 ranks, 13 KB 21.3 / 20.9, 16 KiB at radix 4 22.6 / 21.7, 8 20.5 / 20.5, 31 20.5 / 19.1.
+#define VC_STRIDED_PAST_CACHES ((int64_t)12 << 20)
 #define VC_STRIDED_MAX_PAIRS 36864            // 192 ranks
 // the launch signals its own end: gains up to 32 ranks (32 ranks of 0 - 2 KiB 14.0 us -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3), is even
 // on 48 (0 - 4 KiB 17.0), and on 64 loses with cold caches what it gains with warm ones (0 - 4 KiB 23.2 -> 25.1, 21.5 -> 19.9): stores past
@@ -81,12 +86,17 @@ struct VcDispatch {
                              // VC_THREADS, VC_WAVE, VC_QUARTER, or VC_BATCHED (a batch of pairs per wavefront)
     int stride;              // > 0: first try one launch on fixed-stride staging with slots of this many bytes ...
     int stride_lanes;        // ... with this many lanes per pair (the batches come without the totals: a quarter of a wavefront)
+    int stride_window;       // ... in a window of this many bytes (VcSched::window), or with a place of its own for every slot (0)
     bool self;               // ... that tells the host itself when it is done
     int batch;               // VC_BATCHED: pairs per wavefront
     bool cached;             // vc_reads_cached
     VcListlessGuard guard;   // what the call must look like for the listless kernel to move anything, checked on the device
                              // against the plan (the hint is only a guess); stage_cap is the caller's to fill in
 };
+
+// Which single launches can tell the host that they are done: only instances without a window, with a wavefront or a workgroup per pair, store
+// past the caches (vc_copy_blocks_kernel).  vc_launch_copy_blocks refuses any other.
+VC_HD bool vc_may_signal(int lanes, int window) { return !window && (lanes == VC_WAVE || lanes == VC_THREADS); }
 
 // Pairs per wavefront of the batched listless kernel.  Where a lane moves a block each, all 64 lanes have one; where quarters of the wavefront
 // carry the blocks one after the other, short wavefronts keep the chip fuller.  Microseconds a call with 64 / 32 / 16 pairs, blocks of 0 .. x bytes: 1024 ranks, x = 32 53 / 60 / 75, 64 82 (a lane a block)
@@ -139,7 +149,7 @@ VC_HD int64_t vc_closed_wave_from(int64_t pairs, bool stages, bool cached) {
 // mode: vc_comm_set_forwarding (0 launch per digit, 1 the library's choice, 2 the list, 3 / 4 / 5 listless with a workgroup / a
 // quarter of a wavefront per pair / batches).  S: the call's schedule (ranks, digits, whether it has an organized region).
 inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const VcSched &S) {
-    VcDispatch d = {0, 0, 0, false, 0, false, {0, 0, 0, 0, 0}};
+    VcDispatch d = VcDispatch();
     d.batch = vc_batch_pairs(h.valid ? h.max_len : VC_LANE_BLOCK + 1);
     d.cached = h.valid && vc_reads_cached(S, h.payload);
     if (mode == 3) { d.lanes = VC_THREADS; return d; }
@@ -179,11 +189,13 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
         VcSched strided = S;
         strided.stride = (int)stride;
         // (in a window the slots may take any room)
-        if (stride <= 0x7FFFFF80 && (S.window || vc_strided_stage_bytes(strided) <= VC_STRIDED_MAX_BYTES)) {
+        const bool room = vc_strided_stage_bytes(strided) <= VC_STRIDED_MAX_BYTES;
+        if (stride <= 0x7FFFFF80 && (S.window || room)) {
             d.stride = (int)stride;
             d.stride_lanes = d.lanes == VC_BATCHED ? VC_QUARTER : d.lanes;
             d.guard.max_len = stride - VC_LINE + 1;
-            d.self = d.stride_lanes != VC_QUARTER && pairs <= VC_SELF_MAX_PAIRS && h.payload * vc_hop_slots(S) <= VC_SELF_MAX_BYTES;
+            d.stride_window = room && vc_may_signal(d.stride_lanes, 0) && h.payload <= VC_STRIDED_PAST_CACHES ? 0 : S.window;
+            d.self = vc_may_signal(d.stride_lanes, d.stride_window) && pairs <= VC_SELF_MAX_PAIRS && h.payload * vc_hop_slots(S) <= VC_SELF_MAX_BYTES;
         }
     }
     return d;

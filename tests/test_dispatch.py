@@ -133,3 +133,30 @@ def test_input_that_the_memory_side_cache_holds_is_read_with_ordinary_loads():
         for func, limit in ((E.F_TWOPHASE, 24 << 20), (E.F_TTPL, 24 << 20), (E.F_SPREADOUT, 32 << 20)):
             at = lambda payload, valid=1: E.dispatch(func, 64, (valid, 8192, payload, 2, 1 << 13), mode=mode, call_kind=kind, n=8, window=True, cached=True)
             assert [at(0), at(limit), at(limit + 1), at(limit, valid=0)] == [True, True, False, False], (mode, func)
+
+
+def test_no_single_launch_is_chosen_that_the_launcher_refuses():
+    """Only instances without a window signal their own end: who signals and who stages in a window is decided in one place."""
+    chosen = set()
+    for P in range(3, 33):
+        for r in range(2, P):
+            digits = next(w for w in range(1, 6) if r ** w >= P)
+            for length in list(range(1 << 10, 65537, 3 << 10)) + [50_000, 61_000]:
+                pieces = 1 if length <= 8064 else length // 4096 + 2
+                for payload in sorted({min(share * P * P * length // 8, 64 << 20) for share in (1, 5, 8)}):
+                    hint = (1, max(1, payload // length) * pieces, payload, pieces, length)
+                    for window in (False, True):
+                        d = E.dispatch(E.F_TWOPHASE, P, hint, r=r, window=window, single=True)
+                        assert not d["refused"] and not (d["window"] and not window), (P, r, length, payload, d)
+                        assert d["window"] or d["stride"] * P * P * digits <= 256 << 20, (P, r, length, payload, d)
+                        chosen.add((d["stride"] > 0, d["self"], d["window"]))
+    W = 32 << 20
+    assert chosen == {(False, False, 0), (True, True, 0), (True, False, 0), (True, False, W)}
+    # above 12 MiB on 16 - 32 ranks: in a window, and then without a signal; and slots that have no room of their own
+    for P, r, length in ((32, 4, 16384), (32, 8, 16384), (24, 6, 32768), (16, 2, 50_000)):
+        hint = (1, P * P * 5, P * P * length, length // 4096 + 2, length)
+        d = E.dispatch(E.F_TWOPHASE, P, hint, r=r, window=True, single=True)
+        assert (d["self"], d["window"]) == (False, W), (P, r, length, d)
+        assert E.dispatch(E.F_TWOPHASE, P, hint, r=r, single=True)["self"]
+    d = E.dispatch(E.F_TWOPHASE, 31, (1, 31 * 31 * 2, 31 * 31 * 6000, 16, 60_000), r=2, window=True, single=True)
+    assert (d["self"], d["window"]) == (False, W)

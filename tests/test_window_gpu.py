@@ -206,3 +206,32 @@ def test_the_check_on_long_blocks(P, esz):
         assert torch.equal(dr, want) and st.execution == 2
         assert (st.payload_bytes, st.moved_bytes, st.block_pieces, st.max_block_pieces, st.max_block_bytes) == listed
     dp.comm.free()
+
+
+def _few_long(P, length, longest):
+    counts = _equal(P, length)
+    counts[1, P - 1] = counts[P - 2, 0] = longest
+    return counts
+
+
+@pytest.mark.parametrize("r,counts", [(4, _equal(32, 16384)), (8, _equal(32, 16384)), (6, _equal(24, 32768)), (16, _equal(24, 32768)), (4, _equal(20, 32768)),
+                                      (2, _equal(16, 50_000)), (5, _mixed(27, 30_000, 3).clip(0, 60_000)), (5, _mixed(27, 40_000, 3).clip(0, 60_000)),
+                                      (2, _few_long(31, 8_000, 60_000)), (2, _few_long(20, 8_000, 60_000))])
+def test_single_launch_on_few_ranks_with_long_blocks(r, counts):
+    """Up to 32 ranks: one launch that signals its own end has no window; one of more than 12 MiB, or whose slots have no room of their own,
+    stages in the window and is waited for."""
+    from rbruck_alltoallv_amd import api
+    prob = W.make_problem(counts, 1, 1, 1)
+    dp = api.DeviceProblem(prob)
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    for turn in range(3):
+        dp.fill_payload(0, turn, ds)
+        dr.fill_(0xEE)
+        assert api.twophase_rbruck_alltoallv(r, dp, ds, dr) == 0, (turn, dp.comm.error())
+        assert dp.verify(ds, dr) == 0
+        st = dp.comm.last_stats()
+        assert st.execution == (3 if turn else 1), turn
+    P, stride = len(counts), -(-(int(counts.max()) + 127) // 128) * 128
+    slots = next(w for w in range(1, 6) if r ** w >= P) * P * P * stride
+    assert st.staging_bytes == (slots if int(counts.sum()) <= 12 << 20 and slots <= 256 << 20 else min(slots, WINDOW + CHUNK))
+    dp.comm.free()

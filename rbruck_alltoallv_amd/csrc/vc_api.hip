@@ -475,7 +475,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     const int pair_lanes = d.stride_lanes;
     S.stride = d.stride;
     S.window = d.stride_window;
-    const int64_t need = vc_window_bytes(vc_strided_stage_bytes(S), S.window);
+    const int64_t need = S.window ? vc_window_arena(S.window) : vc_strided_stage_bytes(S);
     hipStream_t st = c->stream;
     // two sets of words in turn: a launch counts in one, which must start from zero, and clears the other one for the next call
     if (!c->verdicts.p) {
@@ -529,7 +529,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
     int rc = plan_read(c, S, L, pi, true);
     if (rc) return rc;
     if (totals[VC_TOTALS_STALLED]) return 0;          // a copying wavefront gave up waiting for the verdict and moved nothing
-    if (!vc_listless_ok(c->h_header, guard)) return 0;     // longer blocks than the last call's, or not a call for this kernel
+    if (!vc_listless_ok(c->h_header, guard)) return 0;     // longer blocks than the slots hold, or not a call for this kernel
     pi.listless = pi.strided = true;
     pi.chain_lanes = pair_lanes;
     rc = finish_stats(c, pi, nullptr, true);
@@ -636,18 +636,17 @@ static int run_batches(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, VcTa
 // The planner (vc_plan_check) only checks and counts, and the copy kernel, enqueued behind it, reads no plan table.
 static bool plans_without_tables(const VcSched &S) { return S.window || !vc_may_stage(S); }
 
-// Gives S the slots for blocks of up to `longest` bytes (a call that stages nothing takes any), makes room for them, and puts
-// the limits that come with them into `guard`.  False: blocks too long for slots of a fixed stride.
+// Gives S slots spread for blocks of `longest` bytes, which longer ones may pass (vc_window_arena), and makes room for them.  `fits` is false with
+// blocks too long for slots of a fixed stride.
 static int place_in_window(vc_comm *c, VcSched &S, int64_t longest, VcListlessGuard &guard, int64_t &stage_bytes, bool &fits) {
     const bool stages = vc_may_stage(S);
     S.stride = stages ? vc_window_stride(longest) : VC_LINE;
     fits = S.stride > 0;
     if (!fits) return VC_OK;
-    const unsigned __int128 layout = (unsigned __int128)(S.w + S.w2) * (unsigned)S.P * (unsigned)S.P * (unsigned)S.stride;
-    stage_bytes = !stages ? 0 : (layout > (unsigned __int128)S.window ? vc_window_bytes((int64_t)S.window + 1, S.window) : (int64_t)layout);
+    stage_bytes = stages ? vc_window_arena(S.window) : 0;
     HIP_TRY(reserve_stage(c, (size_t)stage_bytes + 64));
     guard.stage_cap = (int64_t)c->stage.cap - 64;
-    guard.max_len = stages ? S.stride - VC_LINE + 1 : 0;
+    guard.max_len = 0;
     return VC_OK;
 }
 
@@ -664,44 +663,35 @@ static int enqueue_check(vc_comm *c, const VcSched &S, VcTables &T, int64_t stag
     return VC_OK;
 }
 
-// A blocking call: check and copy kernel go out together, the slots from the longest block of the last call (`longest`); one with longer blocks
-// has moved nothing and goes out once more.  Returns 1: served; 0: not a call for this kernel, nothing moved; < 0: errors.
-static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf, VcTables T, const VcDispatch &d,
-                              int64_t longest) {
+// A blocking call: check and copy kernel go out together, the slots spread for the longest block of the last call.
+// Returns 1: served; 0: not a call for this kernel, nothing moved; < 0: errors.
+static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf, VcTables T, const VcDispatch &d) {
     int rc = reserve_check_bufs(c, S);
     if (rc) return rc;
     if (c->timing) { rc = ensure_events(c, 5); if (rc) return rc; }
     hipStream_t st = c->stream;
     VcListlessGuard guard = d.guard;
-    for (int attempt = 0; attempt < 2; attempt++) {
-        int64_t stage_bytes = 0;
-        bool fits;
-        rc = place_in_window(c, S, longest, guard, stage_bytes, fits);
-        if (rc || !fits) return rc;
-        if (c->timing) HIP_TRY(hipEventRecord(c->events[0], st));
-        c->plan_end = 2;
-        rc = enqueue_check(c, S, T, stage_bytes);
-        if (rc) return rc;
-        if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
-        HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header, guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
-                                      nullptr, nullptr, nullptr, VcSignal(), d.batch, d.cached));
-        if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
-        HIP_TRY(VC_WAIT(c));
-        PlanInfo pi;
-        rc = plan_read(c, S, L, pi, true);
-        if (rc) return rc;
-        if (vc_listless_ok(c->h_header, guard)) {
-            pi.listless = true;
-            pi.chain_lanes = d.lanes;
-            rc = finish_stats(c, pi, nullptr, true);
-            return rc ? rc : 1;
-        }
-        VcListlessGuard any_length = guard;
-        any_length.max_len = 0;
-        if (!vc_listless_ok(c->h_header, any_length)) return 0;
-        longest = pi.max_len;
-    }
-    return 0;
+    int64_t stage_bytes = 0;
+    bool fits;
+    rc = place_in_window(c, S, c->hint.max_len, guard, stage_bytes, fits);
+    if (rc || !fits) return rc;
+    if (c->timing) HIP_TRY(hipEventRecord(c->events[0], st));
+    c->plan_end = 2;
+    rc = enqueue_check(c, S, T, stage_bytes);
+    if (rc) return rc;
+    if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
+    HIP_TRY(vc_launch_copy_blocks(S, T, nullptr, nullptr, c->header, guard, d.lanes, sendbuf, recvbuf, c->stage.as<char>(), st,
+                                  nullptr, nullptr, nullptr, VcSignal(), d.batch, d.cached));
+    if (c->timing) HIP_TRY(hipEventRecord(c->events[3], st));
+    HIP_TRY(VC_WAIT(c));
+    PlanInfo pi;
+    rc = plan_read(c, S, L, pi, true);
+    if (rc) return rc;
+    if (!vc_listless_ok(c->h_header, guard)) return 0;
+    pi.listless = true;
+    pi.chain_lanes = d.lanes;
+    rc = finish_stats(c, pi, nullptr, true);
+    return rc ? rc : 1;
 }
 
 static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, char *recvbuf, VcTables T, bool forward, bool reuse = false) {
@@ -717,8 +707,7 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;
     if (pair_lanes && plans_without_tables(S)) {
-        // (a refused single launch has left its own longest block in the header)
-        rc = try_without_tables(c, S, L, sendbuf, recvbuf, T, d, std::max(c->hint.max_len, d.stride > 0 ? c->h_header[VC_HEADER_MAX_LEN] : 0));
+        rc = try_without_tables(c, S, L, sendbuf, recvbuf, T, d);
         if (rc) return rc < 0 ? rc : VC_OK;
     }
     rc = plan_sizes(c, S, L, T, forward);
@@ -784,7 +773,9 @@ static void keep_pending(vc_comm *c, const CallParams &q, const VcSched &S, cons
 }
 
 // An _async call without plan tables (try_without_tables).  One that stages is only checked, and copied in vc_comm_wait, while there is no last call
-// to take slots and shape from; one of longer blocks than the last call's is copied there too, in the shape its own blocks ask for.
+// to take slots and shape from; one with a block of more pieces than its shape is for is copied there too, in the shape its own blocks ask for (in the
+// wrong shape at once / in vc_comm_wait, calls of 0 - 600 B and others in turn, microseconds a call: 256 ranks, one block of 4 MB 2947 / 543, a few of 200 KB
+// 270 / 221; 40 ranks, 0 - 400 KB 321 / 144).
 static int enqueue_without_tables(vc_comm *c, const CallParams &q, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf,
                                   VcTables T) {
     int rc = reserve_check_bufs(c, S);

@@ -58,6 +58,9 @@
 // 32 ranks, 13 KB 21.3 / 20.9, 16 KiB at radix 4 22.6 / 21.7, 8 20.5 / 20.5, 31 20.5 / 19.1.
 #define VC_STRIDED_PAST_CACHES ((int64_t)12 << 20)
 #define VC_STRIDED_MAX_PAIRS 36864            // 192 ranks
+// In a window a slot may hold more than its stride (vc_window_arena): a single launch there takes blocks of up to this many times the last call's longest, so
+// that one that grows a little from call to call does not have every call go out twice (100 ranks, 0 - 600 B, 256 B longer each call 37.1 us -> 18.1).
+#define VC_WINDOW_GROWTH 4
 // the launch signals its own end: gains up to 32 ranks (32 ranks of 0 - 2 KiB 14.0 us -> 13.5, 24 ranks of 0 - 32 KiB 26.6 -> 22.3), is even
 // on 48 (0 - 4 KiB 17.0), and on 64 loses with cold caches what it gains with warm ones (0 - 4 KiB 23.2 -> 25.1, 21.5 -> 19.9): stores past
 // the caches fill a memory queue that the L2s would have filled later
@@ -104,7 +107,7 @@ VC_HD bool vc_may_signal(int lanes, int window) { return !window && (lanes == VC
 // 91 / 92 / 81; 800 ranks, 512 232 / 223 / 219; 256 ranks, 16 23.5 / 23.5 / 25.3, 100 28 / 28 / 30.
 VC_HD int vc_batch_pairs(int64_t longest) { return longest > VC_LANE_BLOCK ? 16 : 64; }
 
-// Fixed stride of a call that stages in a window without being the single launch: the longest block at any cache-line phase, and an odd
+// Fixed stride of a call that stages in a window without being the single launch: the last call's longest block at any cache-line phase, and an odd
 // number of lines, so that slots whose blocks are much shorter do not all start at the same few places of the window.  0: blocks too long for it.
 #define VC_STRIDE_MAX_LEN ((int64_t)1 << 30)
 VC_HD int vc_window_stride(int64_t longest) {
@@ -193,9 +196,9 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
         if (stride <= 0x7FFFFF80 && (S.window || room)) {
             d.stride = (int)stride;
             d.stride_lanes = d.lanes == VC_BATCHED ? VC_QUARTER : d.lanes;
-            d.guard.max_len = stride - VC_LINE + 1;
             d.stride_window = room && vc_may_signal(d.stride_lanes, 0) && h.payload <= VC_STRIDED_PAST_CACHES ? 0 : S.window;
             d.self = vc_may_signal(d.stride_lanes, d.stride_window) && pairs <= VC_SELF_MAX_PAIRS && h.payload * vc_hop_slots(S) <= VC_SELF_MAX_BYTES;
+            d.guard.max_len = (d.stride_window ? VC_WINDOW_GROWTH : 1) * (stride - VC_LINE + 1);
         }
     }
     return d;

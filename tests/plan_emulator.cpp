@@ -284,6 +284,19 @@ extern "C" int plan_emulate(int func, int P, int n, int r, int batch, int esz, i
                             const int64_t place = dof & vc_window_mask(window);
                             if (dspace == 2 && (place + plen > vc_window_bytes(stage_bytes, window) || ((place ^ dof) & (VC_LINE - 1)))) errors++;
                         }
+                        // ... also where the slots of a fixed stride are shorter than the block: the piece stays in the window's arena
+                        if (dspace == 2 && S.stride)
+                            for (int window : {VC_CHUNK, 4 * VC_CHUNK, VC_STAGE_WINDOW}) {
+                                VcSched in_window = S;
+                                in_window.window = window;
+                                in_window.stride = VC_LINE;
+                                const int phase = vc_phase(S, T, s0, t);
+                                const int64_t slot = (dof - (so - (hop_src[key0] & VC_OFFSET_MASK)) - phase) / S.stride;      // row * P + id
+                                VcHop h = {1, 1, (int)(slot / P), (int)(slot % P)};
+                                const int64_t place = (vc_hop_dst(in_window, h, vc_slot_addr(in_window, slot_off.data(), row_base.data(), h), vc_recv_offset(S, T, s0, t)) +
+                                                       (so - (hop_src[key0] & VC_OFFSET_MASK))) & VC_OFFSET_MASK & vc_window_mask(window);
+                                if (place + plen > vc_window_arena(window) || ((place ^ dof) & (VC_LINE - 1))) errors++;
+                            }
                         dst_ranges.push_back({dof, dof + plen, dspace});
                         memcpy((dspace == 1 ? recv_final : stage2.data()) + dof, send + so, (size_t)plen);
                         chain_moved += plen;

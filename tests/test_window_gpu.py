@@ -235,3 +235,44 @@ def test_single_launch_on_few_ranks_with_long_blocks(r, counts):
     slots = next(w for w in range(1, 6) if r ** w >= P) * P * P * stride
     assert st.staging_bytes == (slots if int(counts.sum()) <= 12 << 20 and slots <= 256 << 20 else min(slots, WINDOW + CHUNK))
     dp.comm.free()
+
+
+@pytest.mark.parametrize("P,name,tun,hi,execution", [(1024, "TTPL_BT_alltoallv", (32, 32, 0), 40, 2), (530, "twophase_rbruck_alltoallv", (9,), 700, 2), (256, "tuna_algorithm", (4, 0), 1500, 2),
+                                                     (210, "TTPL_BT_alltoallv_s1", (30, 5, 0), 90, 2), (194, "TTPL_BT_alltoallv", (97, 97, 0), 3, 2), (150, "twophase_rbruck_alltoallv_om", (3,), 500, 3),
+                                                     (40, "tuna_algorithm", (2, 0), 60, 3), (101, "twophase_rbruck_alltoallv", (2,), 4_000, 3)])
+def test_a_longest_block_that_grows_from_call_to_call(P, name, tun, hi, execution):
+    """Slots in a window have no limit of length: the next call's longer blocks, at the ends of the window too, are delivered by the first launch, that of
+    an _async call before it is waited for."""
+    from rbruck_alltoallv_amd import api
+    packed = name == "TTPL_BT_alltoallv"
+    counts = np.random.default_rng(P).integers(0, hi + 1, (P, P)).astype(np.int32)
+    comm = api.VirtualComm(P)
+    longest = hi
+    for turn in range(7):
+        if turn > 1:
+            longest = longest * 3 // 2 + 200              # (up to 8 pieces, what a quarter of a wavefront takes)
+            at = np.random.default_rng(turn).integers(0, P, (2, 5))
+            counts[at[0], at[1]] = min(longest, 28_000)
+            counts[P - 1, :3] = counts[:3, P - 1] = min(longest, 28_000)
+        prob = W.make_problem(counts, 1, 1, 0 if packed else 1)
+        dp = api.DeviceProblem(prob, comm=comm)
+        ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+        dp.fill_payload(0, turn, ds)
+        assert getattr(api, name)(*tun, dp, ds, dr) == 0, (turn, comm.error())
+        st = comm.last_stats()
+        assert dp.verify(ds, dr, packed) == 0, turn
+        if turn:
+            assert (st.execution, st.host_waits, st.staging_bytes) == (execution, 1, WINDOW + CHUNK), (turn, st.lanes_per_item)
+        if turn < 2 or name not in ("twophase_rbruck_alltoallv", "twophase_rbruck_alltoallv_om", "tuna_algorithm", "TTPL_BT_alltoallv", "TTPL_BT_alltoallv_s1"):
+            continue
+        counts[at[0], at[1] - 1] = min(longest + 300, 28_000)
+        prob = W.make_problem(counts, 1, 1, 0 if packed else 1)
+        dp = api.DeviceProblem(prob, comm=comm)
+        ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+        dp.fill_payload(0, turn, ds)
+        assert api.call_async(name, tun, dp, ds, dr, torch.cuda.current_stream()) == 0, comm.error()
+        torch.cuda.synchronize()
+        early = dr.clone()
+        assert comm.wait() == 0 and dp.verify(ds, dr, packed) == 0, turn
+        assert torch.equal(early, dr), turn
+    comm.free()

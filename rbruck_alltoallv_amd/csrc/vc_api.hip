@@ -495,6 +495,7 @@ static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, cons
         T.rd_packed = c->rd_packed.as<int>();
     }
     VcListlessGuard guard = d.guard;
+    guard.min_payload = 0;                                // (no pair knows the payload of the call)
     guard.stage_cap = (int64_t)c->stage.cap - 64;
     if (c->timing) HIP_TRY(hipEventRecord(c->events[2], st));
     int64_t *totals = c->h_header + VC_TOTALS_AT;
@@ -663,9 +664,10 @@ static int enqueue_check(vc_comm *c, const VcSched &S, VcTables &T, int64_t stag
     return VC_OK;
 }
 
-// A blocking call: check and copy kernel go out together, the slots spread for the longest block of the last call.
+// A blocking call: check and copy kernel go out together, the slots spread for blocks of `longest` bytes.
 // Returns 1: served; 0: not a call for this kernel, nothing moved; < 0: errors.
-static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf, VcTables T, const VcDispatch &d) {
+static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf, VcTables T, const VcDispatch &d,
+                              int64_t longest) {
     int rc = reserve_check_bufs(c, S);
     if (rc) return rc;
     if (c->timing) { rc = ensure_events(c, 5); if (rc) return rc; }
@@ -673,7 +675,7 @@ static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &
     VcListlessGuard guard = d.guard;
     int64_t stage_bytes = 0;
     bool fits;
-    rc = place_in_window(c, S, c->hint.max_len, guard, stage_bytes, fits);
+    rc = place_in_window(c, S, longest, guard, stage_bytes, fits);
     if (rc || !fits) return rc;
     if (c->timing) HIP_TRY(hipEventRecord(c->events[0], st));
     c->plan_end = 2;
@@ -694,6 +696,11 @@ static int try_without_tables(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &
     return rc ? rc : 1;
 }
 
+// What a call is, from the header its planner or its single launch has left.
+static VcHint hint_of(const int64_t *header) {
+    return VcHint{1, header[2], header[1], header[VC_HEADER_MAX_PIECES], header[VC_HEADER_MAX_LEN]};
+}
+
 static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, char *recvbuf, VcTables T, bool forward, bool reuse = false) {
     VcSched S;
     std::vector<VcLaunchInfo> L;
@@ -702,18 +709,25 @@ static int run_schedule(vc_comm *c, const CallParams &q, const char *sendbuf, ch
     S.recv_lo = (int)((uintptr_t)recvbuf & 4095);
     PlanInfo pi;
     hipStream_t st = c->stream;
-    const VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch();
-    const int pair_lanes = d.lanes;
+    VcDispatch d = forward ? vc_dispatch(c->forward, VC_CALL_BLOCKING, c->hint, S) : VcDispatch();
     int rc = try_strided(c, S, L, sendbuf, recvbuf, T, d);
     if (rc) return rc < 0 ? rc : VC_OK;
-    if (pair_lanes && plans_without_tables(S)) {
-        rc = try_without_tables(c, S, L, sendbuf, recvbuf, T, d);
+    // A launch that the device refused has left what the call is: the next one's shape is no guess.  Calls of two kinds in turn, microseconds a call, the second
+    // launch in the shape of the call before / of the call itself: 150 ranks, 0 - 500 B and 0 - 50 KB 268 / 193; 190, 0 - 100 B and 0 - 20 KB 427 / 148; 128, 0 - 600 B and 0 - 40 KB
+    // 184 / 130; 24, 0 - 2 KB and 0 - 100 KB 56 / 48.
+    VcHint known = c->hint;
+    const auto look_again = [&] { known = hint_of(c->h_header); d = vc_dispatch(c->forward, VC_CALL_BLOCKING, known, S); };
+    if (d.stride > 0) look_again();
+    for (int attempt = 0; attempt < 2 && d.lanes && plans_without_tables(S); attempt++) {
+        rc = try_without_tables(c, S, L, sendbuf, recvbuf, T, d, known.max_len);
         if (rc) return rc < 0 ? rc : VC_OK;
+        look_again();
     }
+    const int pair_lanes = plans_without_tables(S) ? 0 : d.lanes;
     rc = plan_sizes(c, S, L, T, forward);
     if (rc) return rc;
     bool synced = false;
-    if (pair_lanes && !plans_without_tables(S)) {
+    if (pair_lanes) {
         // the copy kernel goes out right behind the planning kernels and checks their verdict on the device: when the
         // staging arena turns out too small it has touched nothing and goes out once more behind a larger arena; when the
         // call is not of the kind the last one made the host expect, the call continues through the list

@@ -326,10 +326,11 @@ struct VcListlessGuard {
     int64_t max_items;      // block pieces in all
     int64_t max_average;    // average piece, bytes
     int64_t max_len;        // longest block, bytes (slots of a fixed stride with places of their own: what one holds at any phase; VC_WINDOW_GROWTH)
+    int64_t min_payload;    // fewest bytes in all
 };
 
 VC_HD bool vc_listless_ok(const int64_t *header, const VcListlessGuard &g) {
-    if (header[0] > g.stage_cap || header[VC_HEADER_BAD] != 0) return false;
+    if (header[0] > g.stage_cap || header[VC_HEADER_BAD] != 0 || header[1] < g.min_payload) return false;
     if (g.max_len && header[VC_HEADER_MAX_LEN] > g.max_len) return false;
     if (g.max_pieces && header[VC_HEADER_MAX_PIECES] > g.max_pieces) return false;
     if (g.max_items && header[2] > g.max_items) return false;

@@ -50,6 +50,16 @@
 #define VC_LISTLESS_DIRECT_PAIRS (1 << 17)    // 362 ranks
 #define VC_LISTLESS_WAVE_BELOW 3072           // average piece below which a pair gets a wavefront instead of a workgroup
 #define VC_LISTLESS_MAX_AVERAGE 4096          // a call the short-block kernels were chosen for must stay below this average
+// ... and without plan tables on more than 192 ranks, where the check in front of the copy kernel says what the call is and another shape is two launches
+// away: quarters and batches that find an average above VC_CLOSED_MAX_AVERAGE, batches of 64 pairs (a lane a block) on up to 362 ranks one above
+// VC_CLOSED_LANE_MAX_AVERAGE, and wavefronts that find fewer bytes for every pair than VC_CLOSED_WAVE_MIN_PER_PAIR leave the call to the shape it asks for.
+// Microseconds a call, two kinds in turn, refused from 4096 / 2048 / 1024 / (64 pairs) 512 on: 256 ranks, 0 - 100 and 0 - 1500 B 61 / 61 / 61 / 54, 0 - 100 and 0 - 5000 142 / 93 / 93 / 93,
+// 0 - 300 and 0 - 5000 97 / 93 / 93, 0 - 300 and 0 - 3000 78 / 79 / 85; 512, 0 - 100 and 0 - 3000 207 / 206 / 249 / 250, 0 - 300 and 0 - 20000 860 / 770 / 775.  The call
+// of 0 - x bytes behind one of long blocks, wavefronts / refused below 320 bytes a pair / 480: 256 ranks, x = 100 69 / 62 / 62, 600 71 / 75 / 74, 900 71 / 71 / 81;
+// 350, 100 116 / 91 / 91; 512, 300 233 / 168 / 169; 1024, 300 894 / 565 / 562.
+#define VC_CLOSED_MAX_AVERAGE 2048
+#define VC_CLOSED_LANE_MAX_AVERAGE 512
+#define VC_CLOSED_WAVE_MIN_PER_PAIR 320
 #define VC_STRIDED_MAX_BYTES ((int64_t)256 << 20)
 // Payload up to which a single launch of wavefronts or workgroups that could use a window does without, where there is room: what little data stages is
 // stored past the caches.  64 ranks, 1.2 KB 17.9 us, in a window 18.9; 48 ranks, 4 KB 18.5 / 19.3; but 64 ranks, 4 KB 25.4 / 23.2, 128 ranks, 2 KiB
@@ -185,7 +195,10 @@ inline VcDispatch vc_dispatch(int mode, int call_kind, const VcHint &h, const Vc
     const bool quarter = d.lanes == VC_QUARTER || d.lanes == VC_BATCHED;
     d.guard.max_pieces = quarter ? VC_LISTLESS_MAX_PIECES : VC_LISTLESS_WG_MAX_PIECES;
     d.guard.max_items = quarter || wave ? 0 : VC_LISTLESS_MAX_ITEMS;
-    d.guard.max_average = quarter ? VC_LISTLESS_MAX_AVERAGE : 0;
+    d.guard.max_average = !quarter ? 0 : (!closed || pairs <= VC_STRIDED_MAX_PAIRS ? VC_LISTLESS_MAX_AVERAGE :
+                                          (d.lanes == VC_BATCHED && d.batch == 64 && pairs <= VC_LISTLESS_DIRECT_PAIRS ? VC_CLOSED_LANE_MAX_AVERAGE :
+                                           (quarter_below > VC_CLOSED_MAX_AVERAGE ? VC_LISTLESS_MAX_AVERAGE : VC_CLOSED_MAX_AVERAGE)));
+    d.guard.min_payload = wave ? VC_CLOSED_WAVE_MIN_PER_PAIR * pairs : 0;
     // one launch on fixed-stride staging: the stride from the last call's longest block, at any cache-line phase
     if (!S.coalesce && vc_hop_slots(S) <= VC_MAX_HOP_SLOTS && pairs <= VC_STRIDED_MAX_PAIRS) {
         const int64_t stride = (h.max_len + 2 * VC_LINE - 1) & ~(int64_t)(VC_LINE - 1);

@@ -160,3 +160,20 @@ def test_no_single_launch_is_chosen_that_the_launcher_refuses():
         assert E.dispatch(E.F_TWOPHASE, P, hint, r=r, single=True)["self"]
     d = E.dispatch(E.F_TWOPHASE, 31, (1, 31 * 31 * 2, 31 * 31 * 6000, 16, 60_000), r=2, window=True, single=True)
     assert (d["self"], d["window"]) == (False, W)
+
+
+def test_a_call_like_the_last_one_passes_the_guard_of_its_own_shape():
+    """What the device refuses is dispatched once more on what it is: that shape must take it."""
+    lanes = set()
+    for f, P, n in ((E.F_TWOPHASE, 12, 0), (E.F_TWOPHASE, 60, 0), (E.F_TWOPHASE, 128, 0), (E.F_TTPL, 160, 16), (E.F_TWOPHASE, 200, 0), (E.F_TTPL, 352, 32), (E.F_TWOPHASE, 400, 0),
+                    (E.F_TTPL_S1, 1024, 32), (E.F_SPREADOUT, 60, 0), (E.F_SPREADOUT, 200, 0), (E.F_SPREADOUT, 362, 0), (E.F_SPREADOUT, 500, 0)):
+        for window in (False, True):
+            for share in (1, 2, 5, 50):                   # one pair in so many has a block
+                for length in [1, 60, 128, 129, 200, 383, 384, 511, 513, 600, 767, 900, 1000, 1100, 1279, 1300, 1400, 1700, 1900, 2040, 2050, 2500, 3071, 3100, 5000, 9000, 20000, 40000]:
+                    for uneven in (1, 4):
+                        blocks = P * P // share
+                        pieces = 1 if length <= 8064 else length // 4096 + 2
+                        h = (1, blocks * pieces, blocks * length, pieces * uneven, length * uneven)
+                        assert E.dispatch(f, P, h, n=n, window=window, single=True)["passes"], (f, P, window, h)
+                        lanes.add(E.dispatch(f, P, h, n=n, window=window)["lanes"])
+    assert lanes == {LIST, BATCH, QUARTER, WAVE, GROUP}

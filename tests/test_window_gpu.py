@@ -276,3 +276,44 @@ def test_a_longest_block_that_grows_from_call_to_call(P, name, tun, hi, executio
         assert comm.wait() == 0 and dp.verify(ds, dr, packed) == 0, turn
         assert torch.equal(early, dr), turn
     comm.free()
+
+
+@pytest.mark.parametrize("P", [40, 128])
+def test_a_call_of_another_kind_goes_straight_to_the_list(P):
+    """What the single launch is refused for, but for the length of a block, the other kernels without a list would be refused for too."""
+    from rbruck_alltoallv_amd import api
+    comm = api.VirtualComm(P)
+    waits = []
+    for turn, hi in enumerate((600, 600, 90_000, 600, 600)):      # 90 000 bytes are at least 21 pieces; no shape without a list takes more than 16
+        dp = api.DeviceProblem(W.make_problem(np.random.default_rng(turn).integers(0, hi + 1, (P, P)).astype(np.int32), 1, 1, 1), comm=comm)
+        ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+        dp.fill_payload(0, turn, ds)
+        assert api.twophase_rbruck_alltoallv(4, dp, ds, dr) == 0, comm.error()
+        st = comm.last_stats()
+        waits.append((int(st.execution), int(st.host_waits)))
+        assert dp.verify(ds, dr) == 0, turn
+    # the first call; one launch; refused, then planned for the list and copied; a list again, as the blocks of the last call were long; one launch
+    assert [e for e, _ in waits] == [1, 3, 1, 1, 3] and waits[1][1] == waits[4][1] == 1 and waits[2][1] == 3, waits
+    comm.free()
+
+
+@pytest.mark.parametrize("P,name,tun,kinds", [(230, "twophase_rbruck_alltoallv", (4,), [(100, 1), (5_000, 64)]), (300, "TTPL_BT_alltoallv", (30, 30, 0), [(300, 1), (9_000, 64)]),
+                                              (150, "tuna_algorithm", (4, 0), [(80, 16), (20_000, 64)]), (256, "spreadout_alltoallv", (), [(90, 1), (5_000, 64)])])
+def test_a_refused_call_gets_the_shape_of_its_own_blocks(P, name, tun, kinds):
+    """Calls of short and of long blocks in turn: what the device refuses goes out once more, in no shape of the call before."""
+    from rbruck_alltoallv_amd import api
+    packed = name == "TTPL_BT_alltoallv"
+    comm = api.VirtualComm(P)
+    seen = []
+    for turn in range(6):
+        hi, lanes = kinds[turn > 1 and turn % 2]
+        dp = api.DeviceProblem(W.make_problem(np.random.default_rng(turn).integers(0, hi + 1, (P, P)).astype(np.int32), 1, 1, 0 if packed else 1), comm=comm)
+        ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+        dp.fill_payload(0, turn, ds)
+        assert getattr(api, name)(*tun, dp, ds, dr) == 0, comm.error()
+        st = comm.last_stats()
+        assert dp.verify(ds, dr, packed) == 0, turn
+        seen.append((int(st.lanes_per_item), int(st.host_waits)))
+        # (the single launch takes short blocks in any shape: no pair knows the payload of the call)
+        assert turn == 0 or (seen[-1][0] == lanes and seen[-1][1] <= 2) or (P <= 192 and hi < 100), (turn, seen)
+    comm.free()

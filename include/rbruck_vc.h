@@ -87,7 +87,8 @@ int vc_comm_set_bases(vc_comm_t comm, const int64_t *sbase_bytes, const int64_t 
  *    table entries, and that its block fits a slot, before it forms an address from them; the kernel's first wavefronts
  *    check all of the tables and add up what the host needs afterwards, and the copying wavefronts hold their stores
  *    back until those have reported the tables in order (a call that returns VC_ERR_TABLES has written nothing here
- *    either); a call with a longer block is redone the general way.  Only on at most 192 ranks and, without a window (vc_comm_set_staging_bound),
+ *    either); a call with a longer block (in a window, see vc_comm_set_staging_bound: one more than four times as long), or of another kind, is redone
+ *    the general way, in the kernel that its own blocks ask for.  Only on at most 192 ranks and, without a window,
  *    while regions x P x P x stride stays below 256 MiB.
  *    On more than 192 ranks and blocks below 384 B on average (640 B on 512 and more, in a window) a wavefront takes a batch of 16 or 64 pairs instead: a lane per
  *    pair works out the route, then the quarters of the wavefront carry the blocks one after the other.

@@ -467,8 +467,8 @@ static int run_items(vc_comm *c, const PlanInfo &pi, const void *items_any, cons
 // own table entries, and that its block fits a slot, before it forms an address from them, and holds its stores back
 // until all of those wavefronts have reported the tables in order (their verdict comes after one round of loads, about
 // when the copying wavefronts have their data): as everywhere else, a call with bad tables has touched nothing when it
-// returns.  A call with a longer block than the stride holds is redone the general way (the blocks that did fit have
-// been delivered by then, and are delivered again).
+// returns.  A call with a longer block than the slots take (VcListlessGuard::max_len), or of another kind, is redone the general way (the blocks
+// that did fit have been delivered by then, and are delivered again).
 // Returns 1 when the call has been served, 0 when it must go the general way, < 0 on errors.
 static int try_strided(vc_comm *c, VcSched S, std::vector<VcLaunchInfo> &L, const char *sendbuf, char *recvbuf, VcTables T, const VcDispatch &d) {
     if (d.stride <= 0) return 0;
@@ -870,7 +870,7 @@ extern "C" int vc_comm_wait(vc_comm_t c) {
     if (rc) return rc;
     VcListlessGuard guard = c->pending.guard;
     int lanes = c->pending.lanes;
-    if (!lanes || !vc_listless_ok(c->h_header, guard)) {  // no arena, or one too small, or longer blocks: nothing has been moved yet
+    if (!lanes || !vc_listless_ok(c->h_header, guard)) {  // no arena, or one too small, or blocks of more pieces: nothing has been moved yet
         // a call whose forwarded staging is out of the communicator's bound runs one launch per digit on reused staging (its blocking
         // twin: in batches of receivers where it can)
         if (staging_out_of_bound(c, pi.stage_bytes, pi.payload_bytes))

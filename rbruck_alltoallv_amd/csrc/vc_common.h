@@ -33,13 +33,13 @@
 #define VC_OFFSET_MASK ((1ll << VC_SPACE_SHIFT) - 1)
 
 // Forwarded execution in the default mode keeps its staging in a window: a piece (at most VC_CHUNK bytes) of a slot at offset x of the
-// layout lies at x mod `window` of the arena.  The piece has made its next hop by the time another one takes its place (one group of
-// lanes performs all hops of a piece and reads the staging of none), so slots that share a place need no order between them.
+// layout lies at x mod `window` of the arena.  One group of lanes performs all hops of a piece from its registers and nothing reads staging, so slots that
+// share a place need no order between them, whichever pieces are in flight (with 512 or 1024 ranks the slots of all digits begin at the same place).
 // What bounds calls that stage is the traffic of the memory; 32 MiB of staging stay in the 256 MiB memory-side cache, and its writes
 // to HBM with them, if they are stored with an ordinary store (a non-temporal one bypasses that cache).  Contiguous copy with a second write to
 // a window: window >= 512 MiB 2250 us, <= 256 MiB 1705 (plain); 2110 - 2190 (non-temporal, any size).  Calls, no window / 128 / 64 / 32 MiB:
 // 1024 ranks, 4 KiB 2447 / 2234 / 1973 / 1893 us; 256 ranks, Zipf 166 / 156 / 138 / 135; 512 ranks, 1 MiB, radix 2 14400 / 12060 / 11330 / 10680.
-// No smaller one: about 29 MiB of pieces are in flight at once on routes of nine digits.
+// Not smaller: the L2s hold 32 MiB together, and a hop whose store stays in one of them would be none.
 #define VC_STAGE_WINDOW (32 << 20)
 
 // One block copy: `len` bytes from `src` to `dst` (space-tagged offsets), sent by
@@ -124,7 +124,7 @@ struct VcSched {
                       // itself: 0 none (one-layer Bruck; Bruck over the nodes), 1 those that change node (inter-node
                       // messages), 2 all (direct one-hop functions)
     int stride;       // > 0: staging slots at a fixed stride of this many bytes (a multiple of VC_LINE that holds the longest block
-                      //    at any cache-line phase), the reference's own layout (src/twophase_tunable_rbruckv.cpp:59): slot `id`
+                      //    at any cache-line phase; in a window blocks may be longer, vc_window_arena), the reference's own layout (src/twophase_tunable_rbruckv.cpp:59): slot `id`
                       //    of rank `holder` in region x starts at ((x P + holder) P + id) stride, a closed form, and the planner's
                       //    prefix sums and slot tables are not needed.  0: compact slots at prefix-sum offsets.
     int recycle;      // 1 (launch-per-digit execution only): staging memory is reused.  A staged block arrives in one hop slot and

@@ -135,9 +135,13 @@ VC_HD int64_t vc_small_quarter_below(int64_t pairs) { return pairs <= 1024 ? 0 :
 //   512, 2 KB 326 / 308, 7 KB 1037 / 955;  1024, 4 KB 1980 / 1949;  nothing staged: 128, 5 KB 70 / 47;  300, 2 KB 105 / 87;  800, 2.5 KB 660 / 598.
 // Fewer ranks: 34 ranks, 12 KB 24.0 / 30.3, 40 27.0 / 30.5 (but 4 KB 18.9 / 15.6); blocks of up to 40 pieces on 64 ranks 230 / 261.
 // The lines: a quarter / a wavefront, 64 ranks, 800 B 17.2 / 17.9, 1.2 KB 19.6 / 18.0; 128, 1.2 KB 30.3 / 31.7, 1.5 KB 33.5 / 31.9; 150, 1030 B 33.1 / 37.6, and
-// past what vc_reads_cached holds 1130 B 43.9 / 40.4; 192, 1030 B 58.7 / 57.5; nothing staged 160,
+// past what vc_reads_cached holds 1130 B 43.9 / 40.4; 192, 1030 B 58.7 / 57.5; blocks of 0 - 2 x the average, below that limit 95, 1030 B 21.8 / 21.7, 1275 B 22.9 / 21.8; 120,
+// 1030 B 25.1 / 28.2, 1275 B 27.0 / 28.4; 140, 1275 B 30.4 / 33.4; beyond it 150, 1150 B 40.8 / 38.7; 160, 1030 B 42.5 / 41.2, 1275 B 46.1 / 42.5; 175, 1030 B 46.9 / 47.4, 1150 B 49.8 / 47.9;
+// 190, 1030 B 51.0 / 52.4, 1150 B 54.4 / 52.9; nothing staged 160,
 // 1.5 KB 35.9 / 34.8; a list / a wavefront 256, 1.3 KB 77.3 / 79.4; 350, 1.5 KB 150 / 135; 512, 1.65 KB 282 / 281; 800, 1.5 KB 532 / 583; nothing staged 512,
-// 1.5 KB 174 / 201, 2.4 KB 274 / 245.  Beyond 192 ranks direct calls of longer pieces stay with the list (256 ranks, 4 KB 119 / 115, 512 407 / 398).
+// 1.5 KB 174 / 201, 2.4 KB 274 / 245.  What stages on more than 192 ranks has the list between its two lines: even with quarters on blocks of 0 - 2 x the average (above), slower than them on normal
+// ones from 300 ranks up (quarters / list / wavefronts: 256, 1330 B 71.9 / 69.2 / 74.4; 350, 1290 B 113 / 123 / 126; 400, 1450 B 153 / 167 / 161; 512, 1450 B 234 / 248 / 256; 700, 1450 B 420 / 455 / 467; 1024, 1600 B 853 / 867 / 920).
+// Beyond 192 ranks direct calls of longer pieces stay with the list (256 ranks, 4 KB 119 / 115, 512 407 / 398).
 #define VC_CLOSED_WAVE_PAIRS 2048             // 46 ranks
 // Both lines are for calls of at least VC_CLOSED_WAVE_PER_PAIR bytes for every pair of ranks, the empty ones included: a wavefront that starts to find an
 // empty block costs as much as any (before / a wavefront per pair, rows of ranks that exchange among themselves: 128 ranks, 750 B a pair in blocks of 6 KB 39 / 23;

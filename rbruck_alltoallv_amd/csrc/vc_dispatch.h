@@ -129,6 +129,9 @@ VC_HD int vc_batch_pairs(int64_t longest) { return longest > VC_LANE_BLOCK ? 16 
 // radix 3 132 / 118, 600 38.7 / 39.0; 1000, direct, 36.4 / 38.0).  Runs of more than one vector take LDS that wavefronts without any miss: calls whose blocks average less than
 // a VC_RUN_FILLth of the longest do without (900 ranks in rows of 60 that exchange 50 B among themselves 28.3 / 30.2).  Layouts with gaps, whose wavefronts fall back to
 // lanes, lose up to 1 % (1024 ranks of 0 - 60 B 70.8 / 71.2); with runs of 8 vectors, 11 KB a wavefront, it would be 9 % (0 - 100 B 90.8 / 100.3; packed 85.6 / 78.5).
+// Where a call stages outside a window, a tile with a block of two hops moves a lane a block (vc_copy_blocks_batch_kernel).  The tiles without are those of neighbouring
+// offsets below the radix, of one node: about r of P.  Runs for them / none, blocks of 0 - 60 B, every slot with a place of its own: 1000 ranks at radix 999 60.4 / 66.6, 500 92.2 / 96.0,
+// 250 103.6 / 105.2; 512 at 256 34.0 / 34.8, 128 36.5 / 36.1, 23 36.5 / 36.0; 1024 at 32 113.6 / 112.8 (0 - 32 B 33.6 / 33.2 at 23, 53.2 / 59.0 at 999; 0 - 16 B 50.7 / 53.4 at 999).
 #define VC_RUN_PAIRS (1 << 18)
 #define VC_RUN_ABOVE 4                        // bytes
 #define VC_RUN_SLOTS 7
@@ -136,8 +139,10 @@ VC_HD int vc_batch_pairs(int64_t longest) { return longest > VC_LANE_BLOCK ? 16 
 #define VC_RUN_WORD_SLOTS 4
 #define VC_RUN_WORD_PAIRS (1 << 19)
 #define VC_RUN_FILL 8
+#define VC_RUN_DIRECT_SHARE 4
 VC_HD int vc_run_vectors(const VcSched &S, int64_t longest, int64_t payload) {
     const int64_t pairs = (int64_t)S.P * S.P;
+    if (vc_may_stage(S) && !S.window && S.r * VC_RUN_DIRECT_SHARE < S.P) return 0;
     if (pairs < VC_RUN_PAIRS || S.esz % 8 == 0 || longest <= VC_RUN_ABOVE || longest > 64) return 0;
     if (longest <= 32 && vc_hop_slots(S) > VC_RUN_SLOTS && pairs < VC_RUN_MANY_PAIRS) return 0;
     if (longest <= 16) return 1;

@@ -161,21 +161,23 @@ def twolayer_communicator_linear_s2(n, bblock1, bblock2, prob, send, recv):
     return _run(F_TWOLAYER_LINEAR_S2, prob, send, recv, n=n, batch=bblock1, batch2=bblock2)
 
 
-def dispatch(func, P, hint, mode=1, call_kind=0, n=0, r=2, window=False, batch=False, cached=False, single=False):
+def dispatch(func, P, hint, mode=1, call_kind=0, n=0, r=2, window=False, batch=False, cached=False, single=False, run=False, esz=1):
     """csrc/vc_dispatch.h on the CPU: hint = (valid, block pieces, payload bytes, most pieces of a block, longest block); window: a
     call that stages does so in a window.
-    Returns dict(lanes, stride, stride_lanes, max_pieces, max_items, max_average, max_len), or with `batch` the pairs of a batch, with `cached` whether
-    the input is read with ordinary loads, with `single` dict(stride, self, window, refused, passes) of the single launch and the guard."""
+    Returns dict(lanes, stride, stride_lanes, max_pieces, max_items, max_average, max_len), or with `batch` the pairs of a batch, with `run` the vectors
+    of a block that moves in a run, with `cached` whether the input is read with ordinary loads, with `single` dict(stride, self, window, refused, passes) of the single launch and the guard."""
     global _lib
     if _lib is None:
         _lib = C.CDLL(build())
-    out = np.zeros(13, dtype=np.int64)
+    out = np.zeros(14, dtype=np.int64)
     valid, items, payload, max_pieces, max_len = hint
-    rc = _lib.dispatch_decision(C.c_int(func), C.c_int(P), C.c_int(n), C.c_int(r), C.c_int(mode), C.c_int(call_kind), C.c_int(int(valid)),
+    rc = _lib.dispatch_decision(C.c_int(func), C.c_int(P), C.c_int(n), C.c_int(r), C.c_int(esz), C.c_int(mode), C.c_int(call_kind), C.c_int(int(valid)),
                                 C.c_int64(items), C.c_int64(payload), C.c_int64(max_pieces), C.c_int64(max_len), C.c_int(int(window)), _p(out))
     assert rc == 0, rc
     if batch:
         return int(out[7])
+    if run:
+        return int(out[13])
     if cached:
         return bool(out[8])
     if single:

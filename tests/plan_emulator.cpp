@@ -406,12 +406,12 @@ extern "C" int64_t staging_allocate(int w, int w2, int msd, int coalesce, const 
 // The library's choice of kernel (csrc/vc_dispatch.h) for a call of function `func` on P ranks whose last forwarded call
 // left the hint (valid, items, payload, max_pieces, max_len).  out: lanes, stride, stride_lanes, guard.max_pieces,
 // guard.max_items, guard.max_average, guard.max_len, batch, cached, self, stride_window, whether vc_launch_copy_blocks refuses the
-// single launch of that kind, whether the guard lets a call like the last one pass.  Returns the schedule's error code.
-extern "C" int dispatch_decision(int func, int P, int n, int r, int mode, int call_kind, int valid, int64_t items, int64_t payload,
+// single launch of that kind, whether the guard lets a call like the last one pass, run.  Returns the schedule's error code.
+extern "C" int dispatch_decision(int func, int P, int n, int r, int esz, int mode, int call_kind, int valid, int64_t items, int64_t payload,
                                  int64_t max_pieces, int64_t max_len, int window, int64_t *out) {
     VcSched S;
     std::vector<VcLaunchInfo> L;
-    const int code = vc_make_schedule((VcFunc)func, P, n, r, 0, 1, 0, S, L, 0, true);
+    const int code = vc_make_schedule((VcFunc)func, P, n, r, 0, esz, 0, S, L, 0, true);
     if (code) return code;
     S.window = window && vc_may_stage(S) ? VC_STAGE_WINDOW : 0;      // (make_schedule in csrc/vc_api.hip)
     const VcHint h = {valid, items, payload, max_pieces, max_len};
@@ -421,6 +421,7 @@ extern "C" int dispatch_decision(int func, int P, int n, int r, int mode, int ca
     out[9] = d.self; out[10] = d.stride_window; out[11] = d.self && !vc_may_signal(d.stride_lanes, d.stride_window);
     int64_t header[VC_HEADER_MAX_LEN + 1] = {0, payload, items, 0, max_pieces, 0, max_len};
     out[12] = !d.lanes || vc_listless_ok(header, d.guard);
+    out[13] = d.run;
     return 0;
 }
 

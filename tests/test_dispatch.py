@@ -177,3 +177,16 @@ def test_a_call_like_the_last_one_passes_the_guard_of_its_own_shape():
                         assert E.dispatch(f, P, h, n=n, window=window, single=True)["passes"], (f, P, window, h)
                         lanes.add(E.dispatch(f, P, h, n=n, window=window)["lanes"])
     assert lanes == {LIST, BATCH, QUARTER, WAVE, GROUP}
+
+
+def test_runs_only_where_wavefronts_can_move_them():
+    """A call that stages outside a window (an allowance of its own, the forced batches, the entry point that allocates nothing) has a tile with a block of two
+    hops moved a lane a block: below a radix of a quarter of the ranks, where nearly every tile has one, it gets the instance without runs.  One that stages
+    nothing needs no window."""
+    for longest, vectors in ((16, 1), (32, 2), (64, 4)):
+        hint = _hint(512, longest // 2, 1, longest)
+        for mode, kind in ((1, 0), (1, 1), (5, 0)):
+            at = lambda func, window, n=16, r=2: E.dispatch(func, 512, hint, mode=mode, call_kind=kind, n=n, r=r, window=window, run=True)
+            assert [at(E.F_TWOPHASE, window, r=r) for r in (23, 127, 128, 511) for window in (True, False)] == [vectors, 0] * 2 + [vectors] * 4, (longest, mode, kind)
+            assert [at(E.F_TTPL, False, n, r) for n, r in ((16, 16), (128, 127), (256, 127), (256, 255))] == [0, 0, 0, vectors], (longest, mode, kind)
+            assert [at(E.F_SPREADOUT, window) for window in (True, False)] == [vectors] * 2, (longest, mode, kind)

@@ -48,3 +48,29 @@ def test_tiles_as_runs(most, esz, ranks, name, args, layouts):
         st = dp.comm.last_stats()
         assert st.execution == 2 and st.lanes_per_item == 1 and torch.equal(got, want)
     dp.comm.free()
+
+
+@pytest.mark.parametrize("how", ["forced", "allowance", "noalloc"])
+@pytest.mark.parametrize("most", [16, 32, 64])
+@pytest.mark.parametrize("r", [23, 300])
+def test_short_blocks_staged_outside_a_window(r, most, how):
+    """512 ranks, two digits: batches that give every slot a place of its own, forced, with an allowance of the caller's, and out of the static scratch array.  At
+    radix 23 a lane a block, at 300 tiles whose blocks have one hop as runs."""
+    from rbruck_alltoallv_amd import api
+    ranks = 512
+    dp = api.DeviceProblem(W.make_problem(counts_of(ranks, most - 1, 1), 1))
+    ds, got, want = dp.new_send_arena(), dp.new_recv_arena(0xEE), dp.new_recv_arena(0xEE)
+    dp.fill_payload(0, 9, ds)
+    dp.comm.set_forwarding(0)
+    assert api.twophase_rbruck_alltoallv(r, dp, ds, want) == 0 and dp.verify(ds, want) == 0
+    dp.comm.set_forwarding(5 if how == "forced" else 1)
+    if how == "allowance":
+        dp.comm.set_staging_bound(4096)
+    call = api.twophase_rbruck_alltoallv_noalloc if how == "noalloc" else api.twophase_rbruck_alltoallv
+    for turn in range(3):                                 # the later ones on the hint of the first
+        got.fill_(0xEE)
+        assert (call if turn else api.twophase_rbruck_alltoallv)(r, dp, ds, got) == 0, dp.comm.error()
+        assert torch.equal(got, want)
+    st = dp.comm.last_stats()
+    assert st.execution == 2 and st.lanes_per_item == 1 and st.staging_bytes > 0
+    dp.comm.free()

@@ -687,11 +687,13 @@ __global__ __launch_bounds__(THREADS) void vc_plan_check(VcSched S, VcTables T, 
                 if (carry[j] > 0x7FFFFFFF && t0 + j < P) sum[VC_CHECK_BAD] += VC_BAD_OVERFLOW;
     }
     // the workgroup's, then, in the last workgroup, all of them: a wavefront adds up one of the words
-    if (lane < VC_CHECK_WORDS && group < groups) {
+    if (group < groups) {
+        // (the last lane's sums are read by the whole wavefront: behind a branch that leaves that lane out they need not be complete)
         int64_t v = 0;
 #pragma unroll
         for (int k = 0; k < VC_CHECK_WORDS; k++) { const int64_t x = vc_last_lane(sum[k]); v = lane == k ? x : v; }
-        if (lane < VC_CHECK_MOST) atomicAdd(&of_group[lane], (unsigned long long)v); else atomicMax(&of_group[lane], (unsigned long long)v);
+        if (lane < VC_CHECK_MOST) atomicAdd(&of_group[lane], (unsigned long long)v);
+        else if (lane < VC_CHECK_WORDS) atomicMax(&of_group[lane], (unsigned long long)v);
     }
     __syncthreads();
     if (group < groups && threadIdx.x < VC_CHECK_WORDS) vc_share(&group_tot[(int64_t)lane * groups + group], (int64_t)of_group[lane]);

@@ -72,3 +72,34 @@ def test_header_of_the_check(P, name, args, esz, long):
     assert rc == _lib.VC_ERR_TABLES and checked[5] == planner[5] >= 9
     assert bool((got == 0x11).all())
     dp.comm.free()
+
+
+@pytest.mark.parametrize("P,n", [(200, 20), (514, 257), (1030, 10)])
+def test_packed_layouts_past_an_int(P, n):
+    """Receivers whose packed layout passes INT_MAX elements are counted apart from the bad entries, each once: the first one, neighbours of one workgroup, the last one, entries in
+    the first and the last wavefront of the sources.  One that ends at INT_MAX is none of them."""
+    from rbruck_alltoallv_amd import api
+    prob = W.make_problem(np.random.default_rng(P).integers(0, 60, (P, P)).astype(np.int32), 1)
+    dp = api.DeviceProblem(prob)
+    ds, got = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 9, ds)
+    for _ in range(2):
+        assert api.call_async("TTPL_BT_alltoallv", (n, 2, 0), dp, ds, got, torch.cuda.current_stream()) == 0 and dp.comm.wait() == 0, dp.comm.error()
+    assert int(dp.comm.last_stats().execution) == 2 and dp.verify(ds, got, True) == 0
+    top, over = 2 ** 31 - 1, [0, 101, 102, P - 1]
+    for t, total in [(t, top + 1) for t in over] + [(7, top)]:
+        dp.recvcounts[t] = 0
+        dp.recvcounts[t, 0], dp.recvcounts[t, P - 1] = 2 ** 30, total - 2 ** 30
+        dp.sendcounts[:, t] = dp.recvcounts[t]
+    dp.recvcounts[50, 50] += 1                            # and one bad entry
+    got.fill_(0x11)
+    for forwarding in (2, 1):                             # the planner, the check
+        dp.comm.set_forwarding(forwarding)
+        print("running", P, n, forwarding, flush=True)
+        if forwarding == 2:
+            rc = api.TTPL_BT_alltoallv(n, 2, 0, dp, ds, got)
+        else:
+            rc = api.call_async("TTPL_BT_alltoallv", (n, 2, 0), dp, ds, got, torch.cuda.current_stream()) or dp.comm.wait()
+        assert rc == _lib.VC_ERR_OVERFLOW and int(dp.comm.last_stats().bad_table_entries) == (len(over) << 40) + 1, forwarding
+    assert bool((got == 0x11).all())
+    dp.comm.free()

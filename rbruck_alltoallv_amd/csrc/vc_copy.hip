@@ -444,10 +444,10 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_items_quarter_kernel(const Vc
 // per wavefront on each of six shared words, and one verdict word that all wavefronts polled, these were what the launch waited for:
 // atomics on one address follow each other at about 10 ns.  Kernel times with warm caches: 128 ranks, 2 KiB blocks 27.6 us -> 24.5; 64 ranks
 // of 0 - 4 KiB 14.3 -> 12.8.)
-template <int LANES>
-__device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &T, unsigned long long *verdict, int64_t *totals) {
+// lanes: of the workgroup.
+__device__ __forceinline__ void vc_add_totals(const VcSched &S, const VcTables &T, unsigned long long *verdict, int64_t *totals, int lanes) {
     const int P = S.P, pairs = P * P, per_wave = VC_TOTALS_PER_WAVE, nwaves = (int)vc_totals_waves(P);      // P^2 <= VC_STRIDED_MAX_PAIRS
-    const int wave = (int)blockIdx.x * (LANES / VC_WAVE) + (int)threadIdx.x / VC_WAVE;
+    const int wave = (int)blockIdx.x * (lanes / VC_WAVE) + (int)threadIdx.x / VC_WAVE;
     if (wave >= nwaves) return;
     const int lane = threadIdx.x & (VC_WAVE - 1);
     // The verdict on the tables first, with nothing but one round of reads in front of it (all of a lane's pairs together): the
@@ -590,7 +590,11 @@ __device__ __forceinline__ void vc_copy_pair(const VcSched &S, const VcTables &T
                                              unsigned long long *verdict, unsigned long long *verdict_next,
                                              int64_t *totals) {
     const unsigned head = vc_totals_blocks(S, verdict, LANES);
-    if (blockIdx.x < head) { vc_add_totals<LANES>(S, T, verdict, totals); return; }
+    // Read from the launch where a workgroup has a pair and nothing is staged in a window: with a constant the compiler, short of scalar registers, there keeps 28 of the copying
+    // workgroups' in lanes of a vector register and reads them back in 138 places (64 ranks of 0 - 1500 B 33.3 us a call / 32.4, 220 161.8 / 149.3, 700 1368 / 1234).  The other
+    // instances take the constant, a read less in front of the verdict (wavefronts: 192 ranks of 2000 B 59.7 / 58.5, direct, 180 39.8 / 37.6; workgroups in a window, 8 registers in
+    // lanes, 600 ranks of 3500 B at radix 599 965 / 947, but of 9000 B at 25 1999 / 2030).
+    if (blockIdx.x < head) { vc_add_totals(S, T, verdict, totals, LANES == VC_WAVE || WINDOW ? LANES : (int)blockDim.x); return; }
     const unsigned block = blockIdx.x - head;
     const int64_t per = (gridDim.x - head) / VC_XCDS;
     const int64_t idx = first_pair + (int64_t)(block % VC_XCDS) * per + block / VC_XCDS;
@@ -659,7 +663,7 @@ __global__ __launch_bounds__(VC_WAVE) void vc_copy_blocks_quarter_kernel(VcSched
                                                                          int64_t *totals) {
     __shared__ char *route[VC_ITEMS_PER_WAVE][VC_MAX_HOP_SLOTS];
     const unsigned head = vc_totals_blocks(S, verdict, VC_WAVE);
-    if (blockIdx.x < head) { vc_add_totals<VC_WAVE>(S, T, verdict, totals); return; }
+    if (blockIdx.x < head) { vc_add_totals(S, T, verdict, totals, VC_WAVE); return; }
     const unsigned block = blockIdx.x - head;
     const int64_t per = (gridDim.x - head) / VC_XCDS;
     const int64_t wave = (int64_t)(block % VC_XCDS) * per + block / VC_XCDS;

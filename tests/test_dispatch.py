@@ -190,3 +190,34 @@ def test_runs_only_where_wavefronts_can_move_them():
             assert [at(E.F_TWOPHASE, window, r=r) for r in (23, 127, 128, 511) for window in (True, False)] == [vectors, 0] * 2 + [vectors] * 4, (longest, mode, kind)
             assert [at(E.F_TTPL, False, n, r) for n, r in ((16, 16), (128, 127), (256, 127), (256, 255))] == [0, 0, 0, vectors], (longest, mode, kind)
             assert [at(E.F_SPREADOUT, window) for window in (True, False)] == [vectors] * 2, (longest, mode, kind)
+
+
+def _run(P, longest, esz=1, r=2, func=E.F_TWOPHASE, payload=None):
+    """Vectors of a run of a call in a window behind one of blocks of `longest` bytes; payload: half of `longest` for every pair."""
+    return E.dispatch(func, P, (1, P * P, longest * P * P // 2 if payload is None else payload, 1, longest), r=r, esz=esz, window=True, run=True)
+
+
+def test_vectors_of_a_run():
+    """vc_run_vectors on both sides of each of its lines.  Hop slots of the Bruck functions here: digits of the ranks and one; of the direct ones, one."""
+    direct = lambda P, longest, esz=1: _run(P, longest, esz, func=E.F_SPREADOUT)
+    lengths = (4, 5, 16, 17, 32, 33, 64, 65)
+    # 512 ranks, two digits (three slots): by the longest block and the element
+    for esz, vectors in ((1, [0, 1, 1, 2, 2, 4, 4, 0]), (3, [0, 1, 1, 2, 2, 4, 4, 0]), (2, [0, 1, 1, 2, 2, 0, 0, 0]), (4, [0, 1, 1, 2, 2, 0, 0, 0]), (8, [0] * 8), (16, [0] * 8)):
+        assert [_run(512, longest, esz, r=23) for longest in lengths] == vectors, esz
+        assert [_run(511, longest, esz, r=23) for longest in lengths] == [0] * 8, esz          # too few ranks
+        # nothing staged: one slot
+        assert [direct(1000, longest, esz) for longest in lengths] == vectors, esz
+        assert [direct(511, longest, esz) for longest in lengths] == [0] * 8, esz
+    # runs of one and two vectors: routes of up to seven slots (six digits), from 2048 ranks on of any number
+    assert [_run(729, 16, r=3), _run(730, 16, r=3), _run(729, 32, r=3), _run(730, 32, r=3)] == [1, 0, 2, 0]
+    assert [_run(2047, 16), _run(2048, 16), _run(2047, 32), _run(2048, 32)] == [0, 1, 0, 2]
+    assert [_run(P, 64) for P in (512, 2047, 2048)] == [4] * 3
+    # elements of two and four bytes: two vectors with up to four slots; four where there is staging and 2^19 pairs
+    for esz in (2, 4):
+        assert [_run(512, 32, esz, r=r) for r in (8, 7)] == [2, 0], esz
+        assert [_run(P, 64, esz, r=32) for P in (724, 725)] == [0, 4] and direct(1000, 64, esz) == 0, esz
+    # more than one vector: blocks that average an eighth of the longest
+    for longest, vectors in ((16, 1), (17, 2), (32, 2), (64, 4)):
+        least = -(-512 * 512 * longest // 8)
+        assert [_run(512, longest, r=23, payload=p) for p in (least, least - 1)] == [vectors, 1 if longest == 16 else 0], longest
+    assert E.dispatch(E.F_TWOPHASE, 512, (0, 0, 0, 0, 0), r=23, window=True, run=True) == 0       # no hint

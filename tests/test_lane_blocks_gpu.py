@@ -74,5 +74,6 @@ def test_lanes_by_the_longest_block(ranks, name, args, longest):
         got.fill_(0xEE)
         print("running", ranks, name, longest, first, flush=True)
         assert getattr(api, name)(*args, dp, ds, got) == 0, dp.comm.error()
-        assert torch.equal(got, want), (first, int(dp.comm.last_stats().execution), int(dp.comm.last_stats().lanes_per_item))
+        st = dp.comm.last_stats()
+        assert torch.equal(got, want) and (st.execution, st.lanes_per_item) == (2, 1), (first, int(st.execution), int(st.lanes_per_item))
     dp.comm.free()

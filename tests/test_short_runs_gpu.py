@@ -5,8 +5,15 @@ import pytest
 import torch
 
 from rbruck_alltoallv_amd import workloads as W
+from tests import emulator as E
 
 pytestmark = pytest.mark.gpu
+
+SIZES = [(16, 1), (15, 1), (5, 1), (7, 2), (4, 4), (2, 8), (31, 1), (32, 1), (15, 2), (8, 4), (63, 1), (64, 1), (31, 2), (15, 4), (16, 4)]
+# vectors of a run behind a call whose longest block is `most` elements, by the entry of SIZES
+VECTORS = {512: [1, 1, 1, 1, 1, 0, 2, 2, 0, 0, 4, 4, 0, 0, 0], 736: [1, 1, 1, 1, 1, 0, 2, 2, 2, 2, 4, 4, 4, 4, 4]}
+OTHERS = [1, 1, 1, 1, 1, 0, 2, 2, 2, 2, 4, 4, 0, 0, 0]
+FUNCTION = {"tuna_algorithm": E.F_TUNA, "TTPL_BT_alltoallv": E.F_TTPL, "twophase_rbruck_alltoallv": E.F_TWOPHASE, "spreadout_alltoallv": E.F_SPREADOUT}
 
 
 def counts_of(ranks, most, esz):
@@ -23,7 +30,7 @@ def counts_of(ranks, most, esz):
 
 @pytest.mark.parametrize("layouts", [(0, 0), (0, 1), (1, 0)])
 @pytest.mark.parametrize("ranks,name,args", [(512, "tuna_algorithm", (3, 0)), (736, "tuna_algorithm", (27, 0)), (515, "TTPL_BT_alltoallv", (5, 2, 0)), (520, "twophase_rbruck_alltoallv", (519,)), (516, "spreadout_alltoallv", ())])
-@pytest.mark.parametrize("most,esz", [(16, 1), (15, 1), (5, 1), (7, 2), (4, 4), (2, 8), (31, 1), (32, 1), (15, 2), (8, 4), (63, 1), (64, 1), (31, 2), (15, 4), (16, 4)])
+@pytest.mark.parametrize("most,esz", SIZES)
 def test_tiles_as_runs(most, esz, ranks, name, args, layouts):
     from rbruck_alltoallv_amd import api
     packed = name == "TTPL_BT_alltoallv"
@@ -43,10 +50,67 @@ def test_tiles_as_runs(most, esz, ranks, name, args, layouts):
             if hinted:
                 dp.comm.set_bases(hp.sbase, hp.rbase)
                 assert getattr(api, name)(*args, hp, hs, hr) == 0, dp.comm.error()
+                # the instance that the call behind this one gets
+                st, n, r = dp.comm.last_stats(), args[0] if packed else 0, args[1] if packed else (args or (2,))[0]
+                last = (1, int(st.block_pieces), int(st.payload_bytes), int(st.max_block_pieces), int(st.max_block_bytes))
+                assert E.dispatch(FUNCTION[name], ranks, last, n=n, r=r, esz=esz, window=True, run=True) == VECTORS.get(ranks, OTHERS)[SIZES.index((most, esz))]
             dp.comm.set_bases(dp.sbase, dp.rbase)
             assert getattr(api, name)(*args, dp, ds, got) == 0, dp.comm.error()
         st = dp.comm.last_stats()
         assert st.execution == 2 and st.lanes_per_item == 1 and torch.equal(got, want)
+    dp.comm.free()
+
+
+@pytest.mark.parametrize("longest,vectors", [(16, 1), (32, 2), (64, 4), (128, 0)])
+def test_staged_hops_of_runs_lanes_and_four_lanes(longest, vectors):
+    """512 ranks, two digits, behind a call whose longest block is `longest`: every staged hop is where its slot starts (the slots of one region are 2^18 places of the window, all
+    different), and what is behind a block of less than a vector there says how its tile of 8 x 8 pairs moved: in a run the bytes that follow it, of a lane of its own
+    zeros (behind 4 and 8 bytes the block again), by four lanes what was there before."""
+    from rbruck_alltoallv_amd import api
+    P, R, STRIDE, WINDOW, BEFORE = 512, 23, 384, 32 << 20, 0xAB
+    rng = np.random.default_rng(longest)
+    tile = np.arange(P) // 8
+    kind = (tile[:, None] + 3 * tile[None, :]) % 5
+    counts = rng.integers(1, 17, (P, P))                  # (runs of 8 blocks of at least 2 bytes: a vector or more)
+    counts = np.where(counts == 1, 2, counts)
+    counts = np.where((kind == 1) | (kind == 2), np.minimum(rng.integers(2, 65, (P, P)), max(16 * vectors, 16)), counts)
+    counts[1::8, 2::8] = np.where(kind[1::8, 2::8] == 3, 80, counts[1::8, 2::8])           # too long for any run
+    counts[6::8, 7::8] = np.where(kind[6::8, 7::8] == 4, rng.integers(81, 129, kind[6::8, 7::8].shape), counts[6::8, 7::8])
+    dp = api.DeviceProblem(W.make_problem(counts.astype(np.int32), 1, align=1))
+    ds, dr = dp.new_send_arena(), dp.new_recv_arena()
+    dp.fill_payload(0, 9, ds)                             # (while the communicator has the bases of these arenas)
+    hp = api.DeviceProblem(W.make_problem(np.minimum(np.where(kind == 0, longest, counts), longest).astype(np.int32), 1), comm=dp.comm)
+    hs, hr = hp.new_send_arena(), hp.new_recv_arena()
+    for _ in range(3):
+        assert api.twophase_rbruck_alltoallv(R, hp, hs, hr) == 0, dp.comm.error()
+    address, size = dp.comm.staging()
+    assert size >= WINDOW
+    staged = torch.full((WINDOW,), BEFORE, dtype=torch.uint8, device="cuda:0")
+    assert dp.comm.lib.vc_calibration_copy(address, staged.data_ptr(), WINDOW, dp.comm.handle) == 0
+    dp.comm.set_bases(dp.sbase, dp.rbase)
+    assert api.twophase_rbruck_alltoallv(R, dp, ds, dr) == 0 and dp.verify(ds, dr) == 0, dp.comm.error()
+    st = dp.comm.last_stats()
+    assert st.execution == 2 and st.lanes_per_item == 1 and dp.comm.staging() == (address, size)
+    assert dp.comm.lib.vc_calibration_copy(staged.data_ptr(), address, WINDOW, dp.comm.handle) == 0
+    staged, sent = staged.cpu().numpy(), np.concatenate([ds.cpu().numpy().view(np.uint8).reshape(-1), np.zeros(128, np.uint8)])
+    s, t = np.divmod(np.arange(P * P), P)
+    j = (s - t) % P
+    s, t, j = (a[(j >= R) & (j % R != 0)] for a in (s, t, j))                              # two digits that are not zero
+    holder = (s - j // R * R) % P                         # after the most significant one
+    place = ((P + holder) * P + (j + holder) % P) * STRIDE % WINDOW
+    assert len(np.unique(place)) == len(place) > P * P * 9 // 10
+    n, at = counts[s, t], dp.host.sbase[s] + dp.host.sdispls[s, t]
+    k = np.arange(128)
+    got, follows = staged[place[:, None] + k], sent[at[:, None] + k]
+    assert np.array_equal(got[k < n[:, None]], follows[k < n[:, None]])
+    by_tile = counts.reshape(P // 8, 8, P // 8, 8).max((1, 3))[s // 8, t // 8]
+    runs, four = by_tile <= 16 * vectors, by_tile > 80
+    assert four.any() and runs.any() == (vectors > 0) and (~runs & ~four).any()
+    end = counts.reshape(P, P // 8, 8)[:, :, ::-1].cumsum(2)[:, :, ::-1].reshape(P, P)[s, t]      # bytes to the end of the run
+    behind = (k < 16) & (k >= n[:, None])
+    for moved, where, what in (("in runs", runs[:, None] & (k < end[:, None]), follows), ("a lane", (~runs & ~four & (n != 4) & (n != 8))[:, None], np.zeros_like(got)),
+                               ("four lanes", four[:, None], np.full_like(got, BEFORE))):
+        assert np.array_equal(got[where & behind], what[where & behind]), moved
     dp.comm.free()
 
 

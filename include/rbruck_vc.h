@@ -379,7 +379,7 @@ int vc_comm_last_traffic(vc_comm_t comm, int launch, int64_t *matrix_out);
 /* The staging arena as the last call left it: DEVICE pointer and the bytes that call used (what the reference keeps in
  * extra_buffer / temp_recv_buffer between rounds, src/twophase_tunable_rbruckv.cpp:59-61).  Where every slot has a place of
  * its own (vc_comm_set_staging_bound(comm, 0)) both execution modes leave the same bytes there; tests compare them.  A window holds what went
- * through it last.  The pointer is valid until a call on this communicator needs more. */
+ * through it last, blocks of a few hundred bytes at the start of their slots instead of at the line phase they have in recvbuf.  The pointer is valid until a call on this communicator needs more. */
 int vc_comm_staging(vc_comm_t comm, void **ptr_out, int64_t *bytes_out);
 
 /* ---- harness utilities (payload of the reference drivers, examples/rbruckv_example.cpp:88-92, and a

@@ -118,8 +118,8 @@ struct VcSched {
     int table_mask;   // -1; 0 in the uniform_* functions: equal blocks in rank order, there are no tables, and what is read in their
                       // place (anything readable) is masked out (vc_sc; a branch around the reads would split the batch of
                       // reads a block's addresses depend on: +10 us on 1 Mi blocks)
-    int recv_lo;      // low 12 bits of the recvbuf pointer: staging slots copy the final destination's cache-line phase,
-                      // long copies into recvbuf are cut at its 4 KiB boundaries
+    int recv_lo;      // low 12 bits of the recvbuf pointer: blocks in staging slots start at the final destination's cache-line phase (short
+                      // blocks of batches that stage in a window: at the slot's start), long copies into recvbuf are cut at its 4 KiB boundaries
     int last_hop;     // which blocks make a hop that is no digit round and ends in recvbuf, besides every rank's block to
                       // itself: 0 none (one-layer Bruck; Bruck over the nodes), 1 those that change node (inter-node
                       // messages), 2 all (direct one-hop functions)

@@ -249,7 +249,7 @@ __device__ __forceinline__ void vc_forward_piece_quarter(const char *src, int64_
 }
 
 // ---- blocks of a few hundred bytes, without byte-wise edges ----
-// What bounds these is the number of requests the copying sends to the L2 (about 75 per ns on this chip, whoever sends them: a
+// What bounds these is the number of requests the copying sends to the L2 (72 - 85 per ns on this chip by the kernel's mix of reads and writes: a
 // request writes at most 64 bytes), so every byte-wise head and tail counts as much as a whole vector.  Edges are moved as
 // 16-byte vectors that start or end with the block and overlap the aligned ones (the same bytes, twice).
 struct __attribute__((packed, aligned(1))) VcU64 { unsigned long long v; };

@@ -141,7 +141,8 @@ VC_HD int64_t vc_recv_offset(const VcSched &S, const VcTables &T, int s, int t) 
 
 // Staging slots start cache-line (VC_LINE) aligned; the data inside starts at the line phase
 // of the block's final address in recvbuf, so that every later hop copies between
-// equally aligned addresses.
+// equally aligned addresses.  (Batches that stage in a window, where nothing is copied on from staging, put short blocks at the slot's start:
+// vc_copy_blocks_batch_kernel.)
 VC_HD int vc_phase(const VcSched &S, const VcTables &T, int s, int t) {
     return (int)((vc_recv_offset(S, T, s, t) + S.recv_lo) & (VC_LINE - 1));
 }
